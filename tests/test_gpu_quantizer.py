@@ -89,6 +89,49 @@ def test_fit_layer_codebooks_matches_oracle(tq, oracle):
     assert rel < 0.05
 
 
+_FITS = {
+    # below and above the size from which only the cells the boundaries are expected to visit are sorted (2^22 samples)
+    "normal_small": lambda r: r.standard_normal(50_003),
+    "normal": lambda r: r.standard_normal((1 << 22) + 5),
+    "one_sample": lambda r: np.array([0.7]),
+    "seventeen": lambda r: r.standard_normal(17),
+    # all in one cell (everything is sorted then), values on the boundaries' own cells, values below the first octave
+    "zeros": lambda r: np.zeros(1 << 22),
+    "steps": lambda r: r.integers(-9, 10, (1 << 22) + 1) * 0.3,
+    "narrow": lambda r: r.standard_normal(1 << 22) * 1e-3,
+    # centroids that move far from where they start
+    "positive": lambda r: np.abs(r.standard_normal(1 << 22)) + 0.01,
+    # beyond the cells' range: one pass over the samples per step
+    "wide": lambda r: r.standard_normal(20_001) * 1e4,
+}
+
+
+@pytest.mark.parametrize("bits", [1, 4, 5])
+@pytest.mark.parametrize("data", sorted(_FITS))
+def test_codebook_fit_on_sorted_cells_matches_oracle(tq, oracle, data, bits):
+    """tq_generate_codebook_from_data: bins are those of the comparison, sums are exact and rounded once, so a centroid
+    differs from the oracle's (doubles added one after the other) by its last bits at most: 1e-6 relative to the data."""
+    import ctypes as C
+    f32p = C.POINTER(C.c_float)
+    d = np.ascontiguousarray(_FITS[data](np.random.default_rng(7)), np.float32)
+    got, want, bounds = np.empty(32, np.float32), np.empty(32, np.float32), np.empty(32, np.float32)
+    fit = tq.lib().tq_generate_codebook_from_data_host
+    fit.argtypes = [f32p, C.c_size_t, C.c_int, C.c_int, f32p, f32p]
+    assert fit(d.ctypes.data_as(f32p), d.size, bits, 100, got.ctypes.data_as(f32p), None) == 1 << bits, tq.last_error()
+    oracle.lib().tqo_lloyd_max(d.ctypes.data_as(f32p), d.size, bits, 100, want.ctypes.data_as(f32p), bounds.ctypes.data_as(f32p))
+    n = 1 << bits
+    assert np.abs(got[:n] - want[:n]).max() <= 1e-6 * max(1.0, np.abs(d).max())
+
+
+def test_layer_fit_above_the_sorting_threshold_matches_oracle(tq, oracle):
+    """Both codebooks of a layer of more than 2^22 weights: the residual's boundaries start far outside its samples."""
+    w = (np.random.default_rng(4).standard_normal((2051, 2048)) * 0.02).astype(np.float32)
+    want_p, want_r = oracle.fit_layer_codebooks(w, 512)
+    got_p, got_r = tq.fit_layer_codebooks(w, 512)
+    assert np.abs(got_p.centroids - want_p.centroids).max() < 1e-6
+    assert np.abs(got_r.centroids - want_r.centroids).max() < 1e-6
+
+
 def test_quantizer_error_conventions(tq):
     with pytest.raises(ValueError):
         tq.generate_codebook(6)

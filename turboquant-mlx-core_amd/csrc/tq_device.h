@@ -124,6 +124,20 @@ hipError_t launch_lloyd_pass(const float* data, size_t n, const float* bounds_de
                              const float* gcent_dev, const float* gbounds_dev, int ngc,
                              double* part_sum, unsigned long long* part_cnt, int workgroups, hipStream_t stream);
 
+// Lloyd-Max fits (tq_fit.hip): codebook 0 on the samples, codebook 1 (problems == 2) on their residuals against the
+// global codebook gtab_dev ([0..31] centroids, [32..62] boundaries).  state->bad: the samples are not all finite
+// numbers of ordinary size; nothing was fitted (launch_lloyd_pass takes those).  state->missed[p]: the boundaries of
+// codebook p left the cells whose samples were kept, after state->steps[p] steps: call again with first_round == false
+// and the same workspace (another expectation, from there on), or with everything == true, which cannot miss and
+// needs a larger workspace of its own (first_round == true again).
+struct FitCodebooks { int nc[2]; float init[2][32]; };
+struct FitResult { float cent[2][32]; int steps[2]; int bad; int missed[2]; unsigned kept[2]; };
+bool fit_supported(size_t n);
+bool fit_predicts(size_t n);         // large enough that keeping only the expected cells pays
+size_t fit_workspace_bytes(size_t n, int problems, bool everything);
+hipError_t launch_fit(const float* samples, size_t n, int problems, const float* gtab_dev, int ngc, const FitCodebooks& cb,
+                      int iterations, bool first_round, bool everything, void* workspace, FitResult* state, hipStream_t stream);
+
 hipError_t launch_codebook_quantize(const float* values, size_t n, const float* bounds_dev, int nc, uint8_t* indices,
                                     hipStream_t stream);
 hipError_t launch_codebook_lookup(const uint8_t* indices, size_t n, const float* centroids_dev, int nc, float* values,

@@ -61,7 +61,8 @@ void fill_tables(const float* cbp, int np, const float* cbr, int nr, float* t) {
     midpoints(cbr, nr, t + 80);
 }
 
-// generate_codebook_from_data_cpu (src/codebook.cpp:99-143) with the assignment pass on the GPU.
+// generate_codebook_from_data_cpu (src/codebook.cpp:99-143), one pass over all samples per step: samples that are not
+// all finite, or more than positions of 32 bits can number (fit_codebooks takes the rest).
 bool lloyd_max(const float* samples_dev, size_t n, int bits, int iterations, bool subtract,
                const float* gcent_dev, const float* gbounds_dev, int ngc, float* centroids_out) {
     float cent[32], bounds[32];
@@ -99,6 +100,48 @@ bool lloyd_max(const float* samples_dev, size_t n, int bits, int iterations, boo
     }
     std::memcpy(centroids_out, cent, nc * sizeof(float));
     return true;
+}
+
+// The codebook of the samples and, with residual_bits > 0, the one of their residuals against the global codebook
+// (gtab_dev: [0..31] centroids, [32..62] boundaries), each from the analytic start (src/codebook.cpp:99-143,
+// src/converter.cpp:345-357).
+bool fit_codebooks(const float* samples_dev, size_t n, int primary_bits, int residual_bits, int iterations,
+                   const float* gtab_dev, int ngc, float* cbp_out, float* cbr_out) {
+    const int problems = residual_bits > 0 ? 2 : 1;
+    if (tq::fit_supported(n)) {
+        tq::FitCodebooks cb{};
+        const int bits[2] = {primary_bits, residual_bits};
+        for (int p = 0; p < problems; ++p) {
+            cb.nc[p] = tq_generate_codebook(bits[p], cb.init[p], nullptr);
+            if (cb.nc[p] < 0) { set_error("tq_fit_layer_codebooks: unsupported bit width"); return false; }
+        }
+        DevBuf res;
+        tq::FitResult r{};
+        if (!res.alloc(sizeof(r), "hipMalloc(fit result)")) return false;
+        for (bool everything = !tq::fit_predicts(n);; everything = true) {
+            DevBuf work;
+            if (!work.alloc(tq::fit_workspace_bytes(n, problems, everything), "hipMalloc(fit)")) return false;
+            // (a round that misses costs what one that does not costs; data on which a fifth is needed is left to the
+            // sort of everything)
+            bool missed = true;
+            for (int round = 0; missed && !r.bad && round < (everything ? 1 : 4); ++round) {
+                if (!hip_ok(tq::launch_fit(samples_dev, n, problems, gtab_dev, ngc, cb, iterations, round == 0, everything, work.p,
+                                           res.as<tq::FitResult>(), nullptr), "fit launch") ||
+                    !hip_ok(hipMemcpy(&r, res.p, sizeof(r), hipMemcpyDeviceToHost), "copy centroids"))
+                    return false;
+                missed = r.missed[0] || (problems == 2 && r.missed[1]);
+                if (missed && (size_t)r.kept[0] + r.kept[1] > n / 2) break;      // more than the workspace holds
+            }
+            if (r.bad) break;
+            if (missed && everything) { set_error("tq_fit_layer_codebooks: cells do not cover the samples"); return false; }
+            if (missed) continue;
+            std::memcpy(cbp_out, r.cent[0], cb.nc[0] * sizeof(float));
+            if (problems == 2) std::memcpy(cbr_out, r.cent[1], cb.nc[1] * sizeof(float));
+            return true;
+        }
+    }
+    if (!lloyd_max(samples_dev, n, primary_bits, iterations, false, nullptr, nullptr, 0, cbp_out)) return false;
+    return problems == 1 || lloyd_max(samples_dev, n, residual_bits, iterations, true, gtab_dev, gtab_dev + 32, ngc, cbr_out);
 }
 
 }  // namespace
@@ -225,12 +268,8 @@ int tq_fit_layer_codebooks(const float* weight_dev, int out, int in, uint32_t bl
         a.inv_sqrt_bs = 1.0f / std::sqrt(static_cast<float>(block_size));
         a.quantize = 0;
         if (!hip_ok(tq::launch_quantize_rows(a, nullptr), "rotate samples")) return 1;
-        if (!lloyd_max(d_scaled.as<float>(), n, primary_bits, iterations, false, nullptr, nullptr, 0, cbp_out)) return 1;
-        if (residual_bits > 0 &&
-            !lloyd_max(d_scaled.as<float>(), n, residual_bits, iterations, true, d_g.as<float>(), d_g.as<float>() + 32,
-                       ngc, cbr_out))
-            return 1;
-        return 0;
+        return fit_codebooks(d_scaled.as<float>(), n, primary_bits, residual_bits, iterations, d_g.as<float>(), ngc, cbp_out,
+                             cbr_out) ? 0 : 1;
     } catch (...) { set_error("tq_fit_layer_codebooks: exception"); return 1; }
 }
 
@@ -283,7 +322,7 @@ int tq_generate_codebook_from_data_host(const float* data_host, size_t n, int bi
         DevBuf d;
         if (!d.alloc(n * sizeof(float), "hipMalloc(samples)") ||
             !hip_ok(hipMemcpy(d.p, data_host, n * sizeof(float), hipMemcpyHostToDevice), "copy samples") ||
-            !lloyd_max(d.as<float>(), n, bits, iterations, false, nullptr, nullptr, 0, centroids_out))
+            !fit_codebooks(d.as<float>(), n, bits, 0, iterations, nullptr, 0, centroids_out, nullptr))
             return -1;
         if (boundaries_out) midpoints(centroids_out, 1 << bits, boundaries_out);
         return 1 << bits;
