@@ -75,6 +75,12 @@ int tq_fit_layer_codebooks_host(const float* weight_host, int out_features, int 
                                 float* cb_primary_host_out, float* cb_residual_host_out);
 
 /**
+ * The conversion calls above keep up to 2 GiB of device memory per GPU between calls (the next call uses it again).
+ * This gives back what no running call uses; creating a layer and the end of a model's conversion do so too.
+ */
+void tq_quantizer_release_workspaces(void);
+
+/**
  * Largest power of two <= max_block_size that divides in_features
  * (src/converter.cpp:228-240).
  */

@@ -79,3 +79,43 @@ def test_forward_from_four_threads(tq, oracle):
         layer.close()
     for h in hips:
         h.close()
+
+
+def test_conversions_from_threads_share_kept_memory(tq, oracle):
+    """Fit and quantization of layers of different sizes from three threads at once, with the kept device memory given
+    back now and then: what a call returns is what it returns alone (a first call on fresh memory, checked against the
+    oracle), whatever the block held before."""
+    rng = np.random.default_rng(12)
+    weights = [(rng.standard_normal(s) * 0.02).astype(np.float32) for s in ((1030, 1024), (515, 2048), (4099, 1024))]
+    tq.lib().tq_quantizer_release_workspaces()
+
+    def convert(w):
+        p, r = tq.fit_layer_codebooks(w, 512)
+        q = tq.quantize_weight(w, p, r, 4, 4, 512, False)
+        return [p.centroids, r.centroids, q.packed_primary, q.packed_residual, q.norms, q.seeds], p, r
+
+    want = [convert(w)[0] for w in weights]
+    _, p, r = convert(weights[0])
+    ref = oracle.quantize_weight(weights[0], p, r, 4, 4, 512, False)
+    assert np.array_equal(ref.packed_primary, want[0][2])
+    failures = []
+
+    def work(i):
+        try:
+            for turn in range(8):
+                k = (i + turn) % len(weights)
+                got = convert(weights[k])[0]
+                if not all(np.array_equal(np.asarray(a), np.asarray(b)) for a, b in zip(got, want[k])):
+                    failures.append((i, turn, k))
+                if turn % 4 == i:
+                    tq.lib().tq_quantizer_release_workspaces()
+        except Exception as e:                                  # noqa: BLE001
+            failures.append((i, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    tq.lib().tq_quantizer_release_workspaces()
+    assert not failures, failures

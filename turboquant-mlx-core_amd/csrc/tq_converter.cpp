@@ -117,6 +117,7 @@ bool convert_model(const ConversionConfig& config) {
         }
     }
 
+    struct GiveBack { ~GiveBack() { tq_quantizer_release_workspaces(); } } give_back;    // (the quantizer's memory, also on a throw)
     int processed = 0, kept = 0, quantized = 0;
     for (const auto& shard : shards) {
         auto loaded = load_safetensors(shard.string());

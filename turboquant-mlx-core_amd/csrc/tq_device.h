@@ -104,6 +104,9 @@ hipError_t launch_combine_planes(const uint8_t* primary, const uint8_t* residual
 void set_error(const std::string& msg);
 bool hip_ok(hipError_t e, const char* what);
 
+// Device memory the conversion calls keep between calls, given back (tq_quantize_c.cpp).
+void release_conversion_memory();
+
 // Offline quantizer (tq_quantize.hip).
 struct QuantArgsHost {
     const float* w; float* orig_norm; double* recon_partial; float* scaled_out;

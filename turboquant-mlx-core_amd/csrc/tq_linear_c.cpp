@@ -216,6 +216,7 @@ tq_linear_t create_impl(int in_features, int out_features,
     // tq_linear_forward_static must not do runtime work on its first call (a caller may be capturing its
     // stream): the address of the static workspace on this device is looked up here, once.
     if (!static_scratch_ptr()) return nullptr;
+    tq::release_conversion_memory();
     tq_linear_s* h = new (std::nothrow) tq_linear_s();
     if (!h) { set_error("tq_linear_create: out of host memory"); return nullptr; }
     const size_t pbytes = (size_t)out_features * primary_cols;
