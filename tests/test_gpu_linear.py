@@ -317,6 +317,35 @@ def test_prefill_bf16_matches_dequant_matmul(tq, oracle, mode, out, inf, bs, bat
     assert _rel(y[3:4], y1) < 1e-3
 
 
+# ------------------------------------------------------------------ prefill, few output tiles: 32 x 32 to 128 x 128 tiles
+@pytest.mark.parametrize("mode", ["shared", "dual", "primary_only"])
+@pytest.mark.parametrize("out,inf,bs,batch", [(5, 64, 64, 33),             # one 64-column tile for eight waves, one ragged weight tile
+                                              (31, 192, 64, 64),           # odd number of tiles: no pairs of the nibble planes
+                                              (1030, 896, 128, 97),        # seven pairs; out no multiple of 4; one row in the last block
+                                              (4864, 896, 128, 77),        # 32 x 64 tiles
+                                              (2046, 2048, 1024, 513),     # 64 x 64 tiles, blocks wider than a wave's segment
+                                              (4864, 896, 128, 500),       # 128 x 128 tiles, the last row tile ragged
+                                              (132, 7680, 512, 160)])      # 15 and 30 pairs shared out among eight waves
+def test_prefill_small_tiles_match_dequant_matmul(tq, oracle, mode, out, inf, bs, batch):
+    """fp16 weights and rotated activations, fp32 sums, as the other prefill kernels: 1e-3 relative L2 for fp32 outputs, 5e-3 in
+    bf16; rows in front of and behind the edges of the 32-row blocks agree with the one-row kernel on the same row."""
+    qw, cbp, cbr = _make(oracle, out, inf, bs, mode)
+    x32 = np.random.default_rng(batch).standard_normal((batch, inf)).astype(np.float32)
+    xbits = oracle.f32_to_bf16_bits(x32)
+    want = oracle.linear_forward(qw, cbp, cbr, bs, oracle.bf16_bits_to_f32(xbits))
+    layer = tq.TurboQuantLinear(inf, out, qw, cbp, cbr, bs)
+    y = layer.forward(xbits, tq.BF16, tq.F32)
+    yb = oracle.bf16_bits_to_f32(layer.forward(xbits, tq.BF16, tq.BF16))
+    y16 = layer.forward(x32, tq.F32, tq.F16).view(np.float16).astype(np.float32)
+    rows = [0, 31, 32, batch - 1]
+    one = np.concatenate([layer.forward(xbits[r:r + 1], tq.BF16, tq.F32) for r in rows])
+    layer.close()
+    assert _rel(y, want) < 1e-3
+    assert _rel(yb, want) < 5e-3
+    assert _rel(y16, oracle.linear_forward(qw, cbp, cbr, bs, x32)) < 1.5e-3      # fp16 outputs: 2^-12 in the mean on top
+    assert _rel(y[rows], one) < 1e-3
+
+
 # ------------------------------------------------------------------ prefill, 512-row activation panels
 @pytest.mark.parametrize("mode", ["shared", "dual", "primary_only"])
 @pytest.mark.parametrize("out,inf,bs,batch", [(16500, 256, 256, 257),      # one ragged panel, ragged last weight tile

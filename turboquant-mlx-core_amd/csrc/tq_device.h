@@ -68,9 +68,11 @@ PrefillPlan prefill_plan(const LayerView& L, int batch, int num_cus, size_t capa
 size_t prefill_reserve_bytes(const LayerView& L, int max_batch, int num_cus);
 hipError_t launch_prefill(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
                           void* workspace, const PrefillPlan& plan, hipStream_t stream);
-// panel: fragment images of 512 rows for tq_prefill_panel_kernel instead of 256-row tile images.
+// Images of the rotated activations: 256-row tiles as tq_prefill_gemm_kernel keeps them in LDS, or fragment images of 512
+// rows (tq_prefill_panel_kernel) or 32 rows (tq_prefill_tile_kernel).
+enum : int { kTileImage = 0, kPanelImage = 1, kBlockImage = 2 };
 hipError_t launch_rotate_tiles(const LayerView& L, const void* x, int x_dtype, int batch, void* workspace,
-                               hipStream_t stream, bool panel = false);
+                               hipStream_t stream, int layout = kTileImage);
 // Small batches (tq_skinny.hip): 2..32 rows (any activation type) on shared-rotation layers, batch rows as
 // the M side of 16x16x32 MFMAs.  xt_workspace as for launch_prefill; partial: skinny_partial_bytes() for this batch.
 constexpr int kSkinnyMaxRows = 32;

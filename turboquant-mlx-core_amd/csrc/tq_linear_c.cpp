@@ -399,6 +399,19 @@ int forward_view(tq_linear_s* h, const tq::LayerView& V, bool generic_only, cons
     void* work = nullptr;
     float* partial = nullptr;
     tq::PrefillPlan plan{};
+    // (few output tiles: small ones, tq_prefill_tile.hip; a static workspace too small for 512-row images goes on)
+    const int tile = prefill ? tq::prefill_tile_shape(V, batch, device_cu_count()) : -1;
+    if (tile >= 0) {
+        const size_t need = tq::prefill_tile_workspace_bytes(V, batch);
+        void* ws = static_ws;
+        if (!static_ws) {
+            if (!ensure_stage(&h->d_work, &h->work_bytes, need, stream, &h->retired)) return 1;
+            ws = h->d_work;
+        }
+        if (!static_ws || need <= static_cap)
+            return hip_ok(tq::launch_prefill_tile(V, tile, x_dev, x_dtype, batch, y_dev, y_dtype, ws, stream),
+                          "tq_prefill_tile launch") ? 0 : 1;
+    }
     // (more than 256 rows and enough output tiles: 512-row activation panels, tq_prefill_panel.hip)
     const bool panel = prefill && tq::prefill_panel_supported(V, batch, device_cu_count(), static_ws ? static_cap : ~(size_t)0);
     if (prefill && !panel) plan = tq::prefill_plan(V, batch, device_cu_count(), static_ws ? static_cap : ~(size_t)0);

@@ -17,6 +17,9 @@
 // pipe fed during the decodes.
 #include "tq_prefill_common.h"
 
+#include <algorithm>
+#include <type_traits>
+
 namespace tq {
 
 constexpr int kBM = 256, kBN = 256;
@@ -393,6 +396,15 @@ __global__ __launch_bounds__(kGemmThreads) void tq_prefill_gemm_kernel(PrefillAr
     }
 }
 
+// Fragment images in 16-byte units: where row `row` of sub-step 0 begins (sub-steps are 1024 units apart in a panel image).
+// A block image, [M/32][K/16][64 lanes x 16 B] (sub-steps 64 units apart), is what tq_prefill_tile_kernel reads: its waves
+// walk one or a few row blocks along K, which in a panel image are pieces of 1 KB 16 KB apart, all on the same few
+// channels of the L2 (a wave's 64-column tile took 0.75 us whatever the number of workgroups).
+__device__ __forceinline__ size_t image_row_unit(int row, int u_all, bool blocks) {
+    if (blocks) return (size_t)(row >> 5) * u_all * 64 + (row & 31);
+    return (size_t)(row >> 9) * u_all * 1024 + (size_t)(((row >> 5) & 3) * 4 + ((row >> 7) & 3)) * 64 + (row & 31);
+}
+
 // ---------------------------------------------------------------------------
 // Rotate activations [M, K] (f32 / f16 / bf16) -> fp16 tile images: X~ = H (s (.) X) / sqrt(bs) per block,
 // stored as [M/256][K/32] images of 256 rows x 64 bytes in the exact byte order the GEMM keeps
@@ -402,12 +414,13 @@ __global__ __launch_bounds__(kGemmThreads) void tq_prefill_gemm_kernel(PrefillAr
 // workgroup with 1 KB loads and the images written in 1 KB runs through LDS, 21-27 us against 21-26 us for 2048
 // rows of 5120 columns and 10.9 against 8.5 us for 512 rows: the kernel is bound by neither its 64-byte accesses
 // nor, since the signs come from a table, its arithmetic.)
-// PANEL: fragment images for tq_prefill_panel_kernel instead, [M/512][K/16][4 waves][4 row blocks][64 lanes x 16 B]:
+// LAYOUT kPanelImage: fragment images for tq_prefill_panel_kernel instead, [M/512][K/16][4 waves][4 row blocks][64 lanes x 16 B]:
 // the 8 columns [16 u + 8 g, +8) of row r sit where lane 32 g + r % 32 of wave (r % 128) / 32 expects the
 // A operand of its row block (r % 512) / 128 in sub-step u (the first 128 rows of a panel are the first row block of
 // all four waves: a call of few rows keeps every SIMD busy with its first blocks).
 // ---------------------------------------------------------------------------
-template <bool PANEL>
+// (LAYOUT kBlockImage: the images of tq_prefill_tile_kernel, below)
+template <int LAYOUT>
 __global__ __launch_bounds__(256) void tq_rotate_f16_kernel(const void* __restrict__ x, int x_dtype,
                                                              uint16_t* __restrict__ out, int rows, int cols,
                                                              int chunks, uint32_t seed, uint32_t bs, float scale) {
@@ -444,14 +457,15 @@ __global__ __launch_bounds__(256) void tq_rotate_f16_kernel(const void* __restri
     if (active) {
         const int m_tile = row >> 8, r = row & 255;
         uint4* dst = reinterpret_cast<uint4*>(out + (((size_t)m_tile * chunks + chunk) * 256 + r) * kBK);
-        // (PANEL: 16-byte units; sub-step 2 chunk + i / 2 of panel row >> 9, block of (wave, row block), lane)
-        uint4* pdst = reinterpret_cast<uint4*>(out) + ((((size_t)(row >> 9) * chunks + chunk) * 2 * 4 + ((row >> 5) & 3)) * 4 + ((row >> 7) & 3)) * 64 + (row & 31);
+        // (16-byte units; sub-step 2 chunk + i / 2)
+        const int ustep = LAYOUT == kBlockImage ? 64 : 1024;
+        uint4* pdst = reinterpret_cast<uint4*>(out) + image_row_unit(row, 2 * chunks, LAYOUT == kBlockImage) + (size_t)(2 * chunk) * ustep;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             uint32_t w[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) w[j] = pack_f16_saturating(v[8 * i + 2 * j] * scale, v[8 * i + 2 * j + 1] * scale);
-            if constexpr (PANEL) pdst[(i >> 1) * 1024 + (i & 1) * 32] = make_uint4(w[0], w[1], w[2], w[3]);
+            if constexpr (LAYOUT != kTileImage) pdst[(i >> 1) * ustep + (i & 1) * 32] = make_uint4(w[0], w[1], w[2], w[3]);
             else dst[a_slot(r, i)] = make_uint4(w[0], w[1], w[2], w[3]);
         }
     }
@@ -473,7 +487,7 @@ constexpr int kRotPitch = 144;                 // bytes of a lane's 8 x 16 B in 
 template <int R>
 __global__ __launch_bounds__(256) void tq_rotate_panel_kernel(const void* __restrict__ x, int x_dtype,
                                                                uint16_t* __restrict__ out, uint16_t* __restrict__ out2,
-                                                               int rows, int cols, int segs, int planes,
+                                                               int rows, int cols, int segs, int planes, int blocks,
                                                                uint32_t seed, uint32_t seed2, uint32_t bs, float scale) {
     __shared__ __align__(16) char stage_all[R == 8 ? 4 * kWave * kRotPitch : 16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -497,7 +511,7 @@ __global__ __launch_bounds__(256) void tq_rotate_panel_kernel(const void* __rest
             raw[r][0] = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(x) + e);
         }
     }
-    const int U_all = cols >> 4;
+    const int U_all = cols >> 4, ustep = blocks ? 64 : 1024;
     const int g_own = seg * 64 + lane;                                 // this lane's 8-column group of the row
     for (int plane = 0; plane < planes; ++plane) {
         const uint32_t sd = plane ? seed2 : seed;
@@ -535,9 +549,7 @@ __global__ __launch_bounds__(256) void tq_rotate_panel_kernel(const void* __rest
                 *reinterpret_cast<uint4*>(stage + lane * kRotPitch + r * 16) = o;
             } else {
                 const int row = row0 + r;
-                if (active)
-                    img[((size_t)(row >> 9) * U_all + (g_own >> 1)) * 1024 + (size_t)(((row >> 5) & 3) * 4 + ((row >> 7) & 3)) * 64 +
-                        (row & 31) + (g_own & 1) * 32] = o;
+                if (active) img[image_row_unit(row, U_all, blocks) + (size_t)(g_own >> 1) * ustep + (g_own & 1) * 32] = o;
             }
         }
         if constexpr (R == 8) {
@@ -545,14 +557,14 @@ __global__ __launch_bounds__(256) void tq_rotate_panel_kernel(const void* __rest
             __builtin_amdgcn_wave_barrier();
             // Store instruction i: lane -> (column group 8 i + lane / 8, row lane % 8): eight lanes write one line.
             const int r = lane & 7, row = row0 + r;
-            const size_t row_unit = (size_t)(((row >> 5) & 3) * 4 + ((row >> 7) & 3)) * 64 + (row & 31);
+            const size_t row_unit = image_row_unit(row, U_all, blocks);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int g_in_seg = 8 * i + (lane >> 3);
                 const uint4 o = *reinterpret_cast<const uint4*>(stage + g_in_seg * kRotPitch + r * 16);
                 const int g = seg * 64 + g_in_seg;                      // 8-column group of the row
                 if (g * 8 < cols)
-                    img[((size_t)(row >> 9) * U_all + (g >> 1)) * 1024 + row_unit + (g & 1) * 32] = o;
+                    img[row_unit + (size_t)(g >> 1) * ustep + (g & 1) * 32] = o;
             }
             __builtin_amdgcn_wave_barrier();                           // (the next plane writes the piece again)
         }
@@ -632,6 +644,8 @@ size_t prefill_reserve_bytes(const LayerView& L, int max_batch, int num_cus) {
     look(16); look(kSkinnyMaxRows); look(kSkinnyMaxRows + 1); look(128); look(129);
     for (int rows = kBM; rows < max_batch + kBM; rows += kBM) { look(rows); look(rows + 1); }
     look(max_batch);
+    // (small tiles, whichever row counts take them: images of 512 rows)
+    if (max_batch >= 16) need = std::max(need, prefill_tile_workspace_bytes(L, max_batch));
     return need;
 }
 
@@ -645,42 +659,41 @@ bool prefill_supported(const LayerView& L, int x_dtype, int batch) {
     return L.in_features % kKLoad == 0;
 }
 
-// Rotated activations of `batch` rows as fp16 tile images in `workspace` (both rotations for dual mode).
+// Rotated activations of `batch` rows as fp16 images in `workspace` (both rotations for dual mode).
 hipError_t launch_rotate_tiles(const LayerView& L, const void* x, int x_dtype, int batch, void* workspace,
-                               hipStream_t stream, bool panel) {
+                               hipStream_t stream, int layout) {
     const int K = L.in_features, M = batch;
     uint16_t* xt = static_cast<uint16_t*>(workspace);
     const int chunks = K / kChunk;
     const dim3 rgrid((unsigned)(((long long)M * chunks + 4 * kWave - 1) / (4 * kWave)));   // 256 chunks per workgroup
-    const int tile_m = panel ? kPanelM : kBM;                      // rows of one image
+    const int tile_m = layout == kPanelImage ? kPanelM : layout == kBlockImage ? 32 : kBM;   // rows of one image
     uint16_t* const xt2 = xt + (size_t)((M + tile_m - 1) / tile_m) * tile_m * K;
-    if (panel && L.block_size <= 512) {
+    if (layout != kTileImage && L.block_size <= 512) {
         const int segs = (K + 511) / 512;
         const int planes = L.mode == kDual ? 2 : 1;
+        const int blocks = layout == kBlockImage;
         const long long tasks8 = (long long)((M + 7) / 8) * segs;
         if (tasks8 >= 2048) {
             hipLaunchKernelGGL(tq_rotate_panel_kernel<8>, dim3((unsigned)((tasks8 + 3) / 4)), dim3(256), 0, stream, x, x_dtype,
-                               xt, xt2, M, K, segs, planes, L.seed_primary, L.seed_residual, L.block_size, L.inv_sqrt_bs);
+                               xt, xt2, M, K, segs, planes, blocks, L.seed_primary, L.seed_residual, L.block_size, L.inv_sqrt_bs);
         } else {
             const long long tasks2 = (long long)((M + 1) / 2) * segs;
             hipLaunchKernelGGL(tq_rotate_panel_kernel<2>, dim3((unsigned)((tasks2 + 3) / 4)), dim3(256), 0, stream, x, x_dtype,
-                               xt, xt2, M, K, segs, planes, L.seed_primary, L.seed_residual, L.block_size, L.inv_sqrt_bs);
+                               xt, xt2, M, K, segs, planes, blocks, L.seed_primary, L.seed_residual, L.block_size, L.inv_sqrt_bs);
         }
         return hipGetLastError();
     }
-    if (panel) {
-        hipLaunchKernelGGL(tq_rotate_f16_kernel<true>, rgrid, dim3(256), 0, stream, x, x_dtype, xt, M, K, chunks,
-                           L.seed_primary, L.block_size, L.inv_sqrt_bs);
-        if (L.mode == kDual)
-            hipLaunchKernelGGL(tq_rotate_f16_kernel<true>, rgrid, dim3(256), 0, stream, x, x_dtype, xt2, M, K, chunks,
-                               L.seed_residual, L.block_size, L.inv_sqrt_bs);
-        return hipGetLastError();
+    auto rotate = [&](auto Layout, uint16_t* to, uint32_t seed) {
+        hipLaunchKernelGGL(tq_rotate_f16_kernel<decltype(Layout)::value>, rgrid, dim3(256), 0, stream, x, x_dtype, to, M, K, chunks,
+                           seed, L.block_size, L.inv_sqrt_bs);
+    };
+    for (int p = 0; p < (L.mode == kDual ? 2 : 1); ++p) {
+        uint16_t* const to = p ? xt2 : xt;
+        const uint32_t seed = p ? L.seed_residual : L.seed_primary;
+        if (layout == kPanelImage) rotate(std::integral_constant<int, kPanelImage>{}, to, seed);
+        else if (layout == kBlockImage) rotate(std::integral_constant<int, kBlockImage>{}, to, seed);
+        else rotate(std::integral_constant<int, kTileImage>{}, to, seed);
     }
-    hipLaunchKernelGGL(tq_rotate_f16_kernel<false>, rgrid, dim3(256), 0, stream, x, x_dtype, xt, M, K, chunks,
-                       L.seed_primary, L.block_size, L.inv_sqrt_bs);
-    if (L.mode == kDual)
-        hipLaunchKernelGGL(tq_rotate_f16_kernel<false>, rgrid, dim3(256), 0, stream, x, x_dtype, xt2, M, K, chunks,
-                           L.seed_residual, L.block_size, L.inv_sqrt_bs);
     return hipGetLastError();
 }
 

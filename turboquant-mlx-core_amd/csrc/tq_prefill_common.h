@@ -37,4 +37,11 @@ size_t prefill_panel_workspace_bytes(const LayerView& L, int batch, int num_cus,
 hipError_t launch_prefill_panel(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
                                 void* workspace, size_t workspace_bytes, int num_cus, hipStream_t stream);
 
+// The small-tile kernel (tq_prefill_tile.hip).  Its shape for a call that prefill_supported() takes, or -1: one of the
+// kernels with large tiles is faster.  Workspace: fragment images alone.
+int prefill_tile_shape(const LayerView& L, int batch, int num_cus);
+size_t prefill_tile_workspace_bytes(const LayerView& L, int batch);
+hipError_t launch_prefill_tile(const LayerView& L, int shape, const void* x, int x_dtype, int batch, void* y, int y_dtype,
+                               void* workspace, hipStream_t stream);
+
 }  // namespace tq

@@ -4,7 +4,7 @@
 // differently.  A workgroup is four waves, one per SIMD; wave w owns rows [128 w, 128 w + 128) of a 512-row panel
 // of activations and all 128 weight rows of the tile: a 128 x 128 accumulator tile (256 registers, the wave's
 // AccVGPRs).  What this buys:
-//   * the rotated activations never touch LDS.  tq_rotate_f16_kernel<PANEL> stores them as fragment images, i.e.
+//   * the rotated activations never touch LDS.  the rotation kernels store them as fragment images, i.e.
 //     in the exact register order of the MFMA A operand, so a wave fetches its operands with contiguous 1 KB
 //     global loads (four per 16-column sub-step) into a ring of eight sub-steps, seven sub-steps ahead;
 //   * a tile of weights (128 rows x 64 columns) is decoded once per workgroup and 512 rows of activations, through
@@ -683,7 +683,7 @@ bool prefill_panel_supported(const LayerView& L, int batch, int num_cus, size_t 
 hipError_t launch_prefill_panel(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
                                 void* workspace, size_t workspace_bytes, int num_cus, hipStream_t stream) {
     const PanelPlan plan = panel_plan(L, batch, num_cus, workspace_bytes);
-    hipError_t e = launch_rotate_tiles(L, x, x_dtype, batch, workspace, stream, true);
+    hipError_t e = launch_rotate_tiles(L, x, x_dtype, batch, workspace, stream, kPanelImage);
     if (e != hipSuccess) return e;
     PanelArgs a{};
     a.xt = static_cast<const char*>(workspace);
