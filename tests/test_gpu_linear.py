@@ -75,6 +75,25 @@ def test_dequantize_bit_exact(tq, oracle, mode, out, inf, bs):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("mode", list(MODES))
+@pytest.mark.parametrize("out,inf,bs", [(3, 4096, 2048), (5, 3072, 1024),      # stages across the 512-column groups of a wave
+                                        (70, 32, 2), (1, 32, 32),              # blocks inside a lane; one chunk in all
+                                        (37, 160, 32), (11, 1664, 128),        # rows that begin inside a group
+                                        (2500, 2560, 512)])                    # more chunks than the grid holds at once
+def test_dequantize_bit_exact_at_the_kernels_edges(tq, oracle, mode, out, inf, bs):
+    """Whole matrices in fp32, and their 16-bit forms: the fp32 value rounded to nearest-even."""
+    import ctypes
+    qw, cbp, cbr = _make(oracle, out, inf, bs, mode)
+    want = oracle.dequantize_weight_cpu(qw, cbp, cbr, bs)
+    layer = tq.TurboQuantLinear(inf, out, qw, cbp, cbr, bs)
+    assert np.array_equal(layer.dequantize(), want)
+    for dt, ref in ((tq.F16, want.astype(np.float16).view(np.uint16)), (tq.BF16, oracle.f32_to_bf16_bits(want))):
+        got = np.empty((out, inf), np.uint16)
+        assert tq.lib().tq_linear_dequantize_as_host(ctypes.c_void_p(layer._h), ctypes.c_void_p(got.ctypes.data), dt) == 0
+        assert np.array_equal(got, ref)
+    layer.close()
+
+
 def test_dequantize_fitted_codebooks_and_index_clamp(tq, oracle):
     qw, cbp, cbr = _make(oracle, 48, 1024, 512, "shared", fitted=True)
     assert np.array_equal(tq.dequantize_weight_gpu(qw, cbp, cbr, 512), oracle.dequantize_weight_cpu(qw, cbp, cbr, 512))

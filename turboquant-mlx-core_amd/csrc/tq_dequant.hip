@@ -7,158 +7,277 @@
 // Every step is a single fp32 operation in the reference's order (this file is
 // compiled with -ffp-contract=off), so the output is bit-identical to the CPU path.
 //
-// One wave handles one (row, 2048-column slab); a lane owns 32 consecutive columns.
+// A wave takes 64 consecutive 32-column chunks of the row-major matrix (whole blocks: a row holds a whole number of
+// them, and 2048 columns are a multiple of every block), one chunk per lane, and walks the matrix with the stride of the
+// grid: the position of a lane's columns in their block is the same in every step, so the signs are hashed once per wave.
+// The butterfly runs inside the lanes: five stages on the 32 columns of a chunk, then the 16 chunks of 512 columns change
+// places through LDS (lane p of 16 receives columns 2 p and 2 p + 1 of all 16 chunks) and four stages on those; only
+// blocks of 1024 and 2048 columns have stages across lanes.  Stage order and operations are the reference's.
 #include "tq_device.h"
+
+#include <type_traits>
 
 namespace tq {
 
 constexpr int kDqWaves = 4;   // waves per workgroup
 
-__device__ __forceinline__ void unpack_nibbles(const uint4& P, uint32_t (&idx)[kChunk]) {
-    const uint32_t w[4] = {P.x, P.y, P.z, P.w};
+// Exchange area of a wave: [4 groups of 512 columns][16 column pairs][16 chunks] x 8 bytes.  A group is padded so that two
+// of them lie on different halves of the banks; the 16-byte slots of a pair's 128 bytes are permuted by the pair, so that
+// the 16 lanes that read 16 bytes together find them on different banks.
+constexpr int kDqGroup = 16 * 128 + 128;
+constexpr int kDqExchange = 4 * kDqGroup;
+
+// v: 32 consecutive columns of a lane's chunk -> column pair p = lane % 16 of all 16 chunks of its 512 columns
+// (v[2 j], v[2 j + 1]: chunk j).  `area`: this wave's exchange area.
+__device__ __forceinline__ void chunks_to_pairs(float (&v)[kChunk], char* area, int lane) {
+    char* const base = area + (lane >> 4) * kDqGroup;
+    const int c = lane & 15, wr = ((c >> 1) << 4) | ((c & 1) << 3);
 #pragma unroll
-    for (int d = 0; d < 4; ++d)
+    for (int p = 0; p < 16; ++p)
+        *reinterpret_cast<float2*>(base + p * 128 + (wr ^ (((p >> 1) & 7) << 4))) = make_float2(v[2 * p], v[2 * p + 1]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const char* const rd = base + c * 128;
+    const int sw = ((c >> 1) & 7) << 4;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t byte = (w[d] >> (8 * j)) & 0xffu;
-            idx[8 * d + 2 * j]     = byte & 0x0fu;   // lo nibble = even column (src/dequantizer.cpp:46)
-            idx[8 * d + 2 * j + 1] = byte >> 4;      // hi nibble = odd column  (src/dequantizer.cpp:47)
-        }
+    for (int s = 0; s < 8; ++s) {
+        const float4 t = *reinterpret_cast<const float4*>(rd + ((s << 4) ^ sw));
+        v[4 * s] = t.x; v[4 * s + 1] = t.y; v[4 * s + 2] = t.z; v[4 * s + 3] = t.w;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();                       // (the area is written again)
 }
 
-__global__ __launch_bounds__(kDqWaves* kWave) void tq_dequant_kernel(LayerView L, void* __restrict__ Wout,
-                                                                      int w_dtype, int chunks, int slabs) {
-    __shared__ float tab[256];
-    for (int i = threadIdx.x; i < 256; i += blockDim.x) tab[i] = L.tables[i];
+// Stages 1 .. 16 of the butterfly on a lane's chunk, and 32 .. 1024 on its pairs.
+__device__ __forceinline__ void fwht_chunk(float (&v)[kChunk], uint32_t bs) {
+#pragma unroll
+    for (int h = 1; h < kChunk; h <<= 1) {
+        if ((uint32_t)h < bs) {
+#pragma unroll
+            for (int i = 0; i < kChunk; i += 2 * h)
+#pragma unroll
+                for (int j = i; j < i + h; ++j) { const float a = v[j], b = v[j + h]; v[j] = a + b; v[j + h] = a - b; }
+        }
+    }
+}
+__device__ __forceinline__ void fwht_pairs(float (&v)[kChunk], uint32_t bs, int lane) {
+#pragma unroll
+    for (int h = 2; h < kChunk; h <<= 1) {                 // (chunk j at 2 j: stage 16 h of the block)
+        if ((uint32_t)h * 16 < bs) {
+#pragma unroll
+            for (int i = 0; i < kChunk; i += 2 * h)
+#pragma unroll
+                for (int j = i; j < i + h; ++j) { const float a = v[j], b = v[j + h]; v[j] = a + b; v[j + h] = a - b; }
+        }
+    }
+    if (bs > 512) butterfly_lanes<16, kChunk>(v, lane);
+    if (bs > 1024) butterfly_lanes<32, kChunk>(v, lane);
+}
+
+// Index bytes of a chunk: 16 (nibbles) or 32.
+template <bool BYTES> struct ChunkBytes { uint4 v[BYTES ? 2 : 1]; };
+template <bool BYTES>
+__device__ __forceinline__ ChunkBytes<BYTES> load_chunk_bytes(const uint8_t* plane, long long chunk) {
+    ChunkBytes<BYTES> r;
+    const uint4* p = reinterpret_cast<const uint4*>(plane + (size_t)chunk * (BYTES ? 32 : 16));
+    r.v[0] = p[0];
+    if constexpr (BYTES) r.v[1] = p[1];
+    return r;
+}
+__device__ __forceinline__ uint32_t chunk_word(const ChunkBytes<false>& r, int d) {
+    return d == 0 ? r.v[0].x : d == 1 ? r.v[0].y : d == 2 ? r.v[0].z : r.v[0].w;
+}
+__device__ __forceinline__ uint32_t chunk_word(const ChunkBytes<true>& r, int d) {
+    const uint4& t = r.v[d >> 2];
+    const int e = d & 3;
+    return e == 0 ? t.x : e == 1 ? t.y : e == 2 ? t.z : t.w;
+}
+// tab[nibble k] of a chunk; the 16 entries of a table lie on 16 different banks.  Byte offsets 4 n straight from the word.
+__device__ __forceinline__ void lookup_nibbles(const ChunkBytes<false>& r, const char* tab, float (&v)[kChunk]) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const uint32_t w = chunk_word(r, d), lo = (w << 2) & 0x3c3c3c3cu, hi = (w >> 2) & 0x3c3c3c3cu;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            v[8 * d + 2 * j] = *reinterpret_cast<const float*>(tab + ((lo >> (8 * j)) & 0xffu));       // lo nibble = even column (src/dequantizer.cpp:46)
+            v[8 * d + 2 * j + 1] = *reinterpret_cast<const float*>(tab + ((hi >> (8 * j)) & 0xffu));   // hi nibble = odd column  (src/dequantizer.cpp:47)
+        }
+    }
+}
+
+// Which planes a layer has and how a centroid is found.
+template <int MODE> struct DequantMode {
+    static constexpr bool five = MODE == kShared5 || MODE == kPrimaryOnly5 || MODE == kDual5;
+    static constexpr bool dual = MODE == kDual || MODE == kDual5;
+};
+
+// COMBINED: the layer's one-byte-per-weight plane (kSharedLut; kShared5 and kPrimaryOnly5 where the residual index fits
+// the byte's top three bits).
+//
+// Bound by its vector instructions (about 30 per weight in dual rotation: two butterflies of 9, lookups and exchange,
+// signs, sum, norm and conversion; 16 in shared rotation) and by three waves per SIMD (registers, 11 KB of LDS per wave).
+// 27648 x 5120 to bf16: dual 364 -> 152 us (2.8 TB/s of planes and weights), shared 104.  Before, a lane kept 32 consecutive
+// columns throughout: four more stages across lanes at two to three instructions per value, two sign hashes per weight,
+// 64-byte pieces per lane in every store, and idle lanes behind the last 2048 columns of a row.
+template <int MODE, bool COMBINED>
+__global__ __launch_bounds__(kDqWaves* kWave, 3) void tq_dequant_kernel(LayerView L, void* __restrict__ Wout, int w_dtype,
+                                                                         int chunks_per_row, long long chunks) {
+    using M = DequantMode<MODE>;
+    constexpr bool bytes = COMBINED || M::five;            // of the primary plane
+    constexpr bool residual_plane = M::dual || (MODE == kShared5 && !COMBINED);
+    constexpr int kCopies = 8;                             // of the 256-entry table: a lane reads the copy lane % 8
+    __shared__ float tab[MODE == kSharedLut ? 256 * kCopies : 64];
+    __shared__ __align__(16) char exchange[kDqWaves * kDqExchange];
+    __shared__ __align__(16) float row_norm[kDqWaves * kWave];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    // (every centroid, or sum of two, is multiplied by 1/sqrt(in) before the butterfly: one fp32 product, whether formed
+    // here or per weight)
+    if constexpr (MODE == kSharedLut) {
+        for (int i = threadIdx.x; i < 256 * kCopies; i += blockDim.x) tab[i] = L.tables[i / kCopies] * L.inv_scale;
+    } else {
+        for (int i = threadIdx.x; i < 64; i += blockDim.x) tab[i] = MODE == kShared5 ? L.tables[i] : L.tables[i] * L.inv_scale;
+    }
+    // Signs of the residual's rotation over 2048 columns (a second set of 32 registers per lane does not fit).
+    __shared__ __align__(16) float signs_r[M::dual ? kSlab : 4];
+    if constexpr (M::dual)
+        for (int i = threadIdx.x; i < kSlab; i += blockDim.x)
+            signs_r[i] = L.inv_sqrt_bs * sign_of(L.seed_residual, (uint32_t)i & (L.block_size - 1));
     __syncthreads();
+    const char* const tab_p = reinterpret_cast<const char*>(tab);
+    const char* const tab_r = reinterpret_cast<const char*>(tab + (M::five ? 32 : 16));
+    char* const area = exchange + wave * kDqExchange;
+    float* const nrm_of = row_norm + wave * kWave;
 
-    const int lane = threadIdx.x & (kWave - 1);
-    const long long wid = (long long)blockIdx.x * kDqWaves + (threadIdx.x >> 6);
-    const int row = (int)(wid / slabs);
-    const int slab = (int)(wid % slabs);
-    if (row >= L.out_features) return;          // whole wave leaves together
-    const int chunk = slab * kWave + lane;
-    const bool active = chunk < chunks;
-    const int in = L.in_features;
     const uint32_t bs = L.block_size;
-    const bool five = (L.mode >= kShared5);
-    const bool has_res = (L.mode != kPrimaryOnly && L.mode != kPrimaryOnly5);
-    const bool shared = (L.mode == kSharedLut || L.mode == kShared5);
+    // Signs of this lane's 32 values after the exchange: columns 32 j + 2 p + (0, 1) of its 512.
+    float sp[kChunk];
+#pragma unroll
+    for (int k = 0; k < kChunk; ++k) {
+        const uint32_t col = (uint32_t)((lane >> 4) * 512 + (k >> 1) * 32 + 2 * (lane & 15) + (k & 1)) & (bs - 1);
+        sp[k] = L.inv_sqrt_bs * sign_of(L.seed_primary, col);
+    }
 
-    uint32_t pi[kChunk], ri[kChunk];
-    float v[kChunk];
-    if (active && L.mode == kSharedLut) {
-        // combined plane: one byte per weight, residual nibble high, primary nibble low
-        const uint4* p = reinterpret_cast<const uint4*>(L.packed_combined + (size_t)row * in + (size_t)chunk * 32);
-        const uint4 a = p[0], b = p[1];
-        const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int d = 0; d < 8; ++d)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t c = (w[d] >> (8 * j)) & 0xffu;
-                pi[4 * d + j] = c & 0x0fu;
-                ri[4 * d + j] = c >> 4;
-            }
-    } else if (active && five && L.packed_combined) {
-        // 5-bit primary with a residual of at most 3 bits: one byte per weight, residual index in
-        // the top 3 bits (both already clamped to their codebooks when the plane was built)
-        const uint4* p = reinterpret_cast<const uint4*>(L.packed_combined + (size_t)row * in + (size_t)chunk * 32);
-        const uint4 a = p[0], b = p[1];
-        const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int d = 0; d < 8; ++d)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t c = (w[d] >> (8 * j)) & 0xffu;
-                pi[4 * d + j] = c & 0x1fu;
-                ri[4 * d + j] = c >> 5;
-            }
-    } else if (active) {
-        if (five) {
-            const uint4* p = reinterpret_cast<const uint4*>(L.packed_primary + (size_t)row * in + (size_t)chunk * 32);
-            const uint4 a = p[0], b = p[1];
-            const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    const long long step = (long long)gridDim.x * (kDqWaves * kWave);
+    long long base = ((long long)blockIdx.x * kDqWaves + wave) * kWave;
+    if (base >= chunks) return;                            // whole wave leaves together; no workgroup barrier below
+    auto mine = [&](long long b) { return b + lane < chunks ? b + lane : chunks - 1; };     // (past the end: the last chunk again, not stored)
+    const uint8_t* const plane_p = COMBINED ? L.packed_combined : L.packed_primary;
+    ChunkBytes<bytes> P = load_chunk_bytes<bytes>(plane_p, mine(base));
+    ChunkBytes<false> R{};
+    if constexpr (residual_plane) R = load_chunk_bytes<false>(L.packed_residual, mine(base));
+    for (; base < chunks; base += step) {
+        const ChunkBytes<bytes> pb = P;
+        const ChunkBytes<false> rb = R;
+        const long long ahead = base + step < chunks ? base + step : base;
+        P = load_chunk_bytes<bytes>(plane_p, mine(ahead));
+        if constexpr (residual_plane) R = load_chunk_bytes<false>(L.packed_residual, mine(ahead));
+        nrm_of[lane] = L.norms[mine(base) / chunks_per_row];
+
+        float v[kChunk];
+        if constexpr (MODE == kSharedLut) {
+            // path A: 256-entry table of centroid sums (src/dequantizer.cpp:136-184)
 #pragma unroll
             for (int d = 0; d < 8; ++d)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) pi[4 * d + j] = (w[d] >> (8 * j)) & 0xffu;
+                for (int j = 0; j < 4; ++j)
+                    v[4 * d + j] = tab[((chunk_word(pb, d) >> (8 * j)) & 0xffu) * kCopies + (lane & (kCopies - 1))];
+        } else if constexpr (bytes) {
+            float t[kChunk];
+            if constexpr (MODE == kShared5 && !COMBINED) lookup_nibbles(rb, tab_r, t);
+#pragma unroll
+            for (int d = 0; d < 8; ++d)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t c = (chunk_word(pb, d) >> (8 * j)) & 0xffu;
+                    // (combined: residual index in the top three bits, both clamped when the plane was built)
+                    const uint32_t pi = COMBINED ? (c & 31u) : (c > 31u ? 31u : c);
+                    float x = tab[pi];
+                    if constexpr (MODE == kShared5)                                          // path B (src/dequantizer.cpp:186-212)
+                        x = (x + (COMBINED ? tab[32 + (c >> 5)] : t[4 * d + j])) * L.inv_scale;
+                    v[4 * d + j] = x;
+                }
         } else {
-            unpack_nibbles(*reinterpret_cast<const uint4*>(L.packed_primary + (size_t)row * (in >> 1) + (size_t)chunk * 16), pi);
+            lookup_nibbles(pb, tab_p, v);
         }
-        if (has_res)
-            unpack_nibbles(*reinterpret_cast<const uint4*>(L.packed_residual + (size_t)row * (in >> 1) + (size_t)chunk * 16), ri);
-    }
-
-    const uint32_t col0 = ((uint32_t)chunk * kChunk) & (bs - 1);
-    const float nrm = L.norms[row];
-
-    if (L.mode == kSharedLut) {
-        // path A: 256-entry table of centroid sums (src/dequantizer.cpp:136-184)
+        fwht_chunk(v, bs);
+        chunks_to_pairs(v, area, lane);
+        fwht_pairs(v, bs, lane);
 #pragma unroll
-        for (int k = 0; k < kChunk; ++k) v[k] = active ? tab[(ri[k] << 4) | pi[k]] * L.inv_scale : 0.0f;
-    } else {
-        const int roff = five ? 32 : 16;
+        for (int k = 0; k < kChunk; ++k) v[k] *= sp[k];
+        if constexpr (M::dual) {
+            // path C second plane (src/dequantizer.cpp:220-245)
+            float u[kChunk];
+            lookup_nibbles(rb, tab_r, u);
+            fwht_chunk(u, bs);
+            chunks_to_pairs(u, area, lane);
+            fwht_pairs(u, bs, lane);
 #pragma unroll
-        for (int k = 0; k < kChunk; ++k) {
-            float c = 0.0f;
-            if (active) {
-                c = tab[five ? (pi[k] > 31u ? 31u : pi[k]) : pi[k]];
-                if (shared) c = c + tab[roff + ri[k]];       // path B (src/dequantizer.cpp:186-212)
+            for (int j = 0; j < 16; ++j) {
+                const float2 sr = *reinterpret_cast<const float2*>(signs_r + (lane >> 4) * 512 + j * 32 + 2 * (lane & 15));
+                u[2 * j] *= sr.x; u[2 * j + 1] *= sr.y;
+                v[2 * j] = v[2 * j] + u[2 * j]; v[2 * j + 1] = v[2 * j + 1] + u[2 * j + 1];
             }
-            v[k] = c * L.inv_scale;
         }
-    }
-    fwht_lane32(v, bs, lane);
-#pragma unroll
-    for (int k = 0; k < kChunk; ++k) v[k] *= L.inv_sqrt_bs * sign_of(L.seed_primary, (col0 + k) & (bs - 1));
 
-    if (has_res && !shared) {
-        // path C second plane (src/dequantizer.cpp:220-245)
-        const int roff = five ? 32 : 16;
-        float u[kChunk];
+        const long long chunk0 = base + (lane >> 4) * 16;  // of the 16 chunks whose pair this lane holds
+        const float4* const np = reinterpret_cast<const float4*>(nrm_of + (lane >> 4) * 16);
+        const size_t elem = (size_t)chunk0 * kChunk + 2 * (lane & 15);
+        const int have = chunks - chunk0 < 16 ? (int)(chunks - chunk0) : 16;
+        auto store = [&](auto Tc) {
+            constexpr int T = decltype(Tc)::value;
+            typedef float f32x2_t __attribute__((ext_vector_type(2)));
+            typedef __bf16 b16x2_t __attribute__((ext_vector_type(2)));
+            typedef _Float16 h16x2_t __attribute__((ext_vector_type(2)));
 #pragma unroll
-        for (int k = 0; k < kChunk; ++k) u[k] = active ? tab[roff + ri[k]] * L.inv_scale : 0.0f;
-        fwht_lane32(u, bs, lane);
+            for (int q = 0; q < 4; ++q) {
+                const float4 n4 = np[q];
+                const float n[4] = {n4.x, n4.y, n4.z, n4.w};
 #pragma unroll
-        for (int k = 0; k < kChunk; ++k) {
-            u[k] *= L.inv_sqrt_bs * sign_of(L.seed_residual, (col0 + k) & (bs - 1));
-            v[k] = v[k] + u[k];
-        }
-    }
-
-    if (!active) return;
-    const size_t elem = (size_t)row * in + (size_t)chunk * kChunk;
-    if (w_dtype == kF32) {
-        float4* dst = reinterpret_cast<float4*>(static_cast<float*>(Wout) + elem);
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            dst[i] = make_float4(v[4 * i] * nrm, v[4 * i + 1] * nrm, v[4 * i + 2] * nrm, v[4 * i + 3] * nrm);
-    } else {
-        // The fp32 weight rounded to nearest-even, the cast src/turboquant_c_dequant.cpp:166 applies.
-        uint4* dst = reinterpret_cast<uint4*>(static_cast<uint16_t*>(Wout) + elem);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t h[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float f = v[8 * i + j] * nrm;
-                h[j] = (w_dtype == kBF16) ? (uint32_t)float_to_bf16_bits(f)
-                                          : (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)f);
+                for (int e = 0; e < 4; ++e) {
+                    const int j = 4 * q + e;
+                    const f32x2_t f = {v[2 * j] * n[e], v[2 * j + 1] * n[e]};
+                    if (j >= have) continue;
+                    // 16-bit: the fp32 weight rounded to nearest-even, the cast src/turboquant_c_dequant.cpp:166 applies.
+                    if constexpr (T == kF32) *reinterpret_cast<f32x2_t*>(static_cast<float*>(Wout) + elem + j * kChunk) = f;
+                    else if constexpr (T == kBF16)
+                        *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(Wout) + elem + j * kChunk) =
+                            __builtin_bit_cast(uint32_t, __builtin_convertvector(f, b16x2_t));
+                    else
+                        *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(Wout) + elem + j * kChunk) =
+                            __builtin_bit_cast(uint32_t, __builtin_convertvector(f, h16x2_t));
+                }
             }
-            dst[i] = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
-        }
+        };
+        if (w_dtype == kF32) store(std::integral_constant<int, kF32>{});
+        else if (w_dtype == kBF16) store(std::integral_constant<int, kBF16>{});
+        else store(std::integral_constant<int, kF16>{});
     }
 }
 
 hipError_t launch_dequant(const LayerView& L, void* w, int w_dtype, hipStream_t stream) {
-    const int chunks = L.in_features / kChunk;
-    const int slabs = (chunks + kWave - 1) / kWave;
-    const long long waves = (long long)L.out_features * slabs;
-    const long long grid = (waves + kDqWaves - 1) / kDqWaves;
-    if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(tq_dequant_kernel, dim3((unsigned)grid), dim3(kDqWaves * kWave), 0, stream, L, w, w_dtype, chunks,
-                       slabs);
+    const int per_row = L.in_features / kChunk;
+    const long long chunks = (long long)L.out_features * per_row;
+    const long long groups = (chunks + kDqWaves * kWave - 1) / (kDqWaves * kWave);
+    const dim3 grid((unsigned)(groups < 768 ? groups : 768)), block(kDqWaves * kWave);     // three workgroups per CU
+    auto go = [&](auto Mode, auto Combined) {
+        hipLaunchKernelGGL((tq_dequant_kernel<decltype(Mode)::value, decltype(Combined)::value>), grid, block, 0, stream, L, w,
+                           w_dtype, per_row, chunks);
+    };
+    const bool combined = L.packed_combined != nullptr;
+    switch (L.mode) {
+        case kSharedLut: go(std::integral_constant<int, kSharedLut>{}, std::true_type{}); break;
+        case kDual: go(std::integral_constant<int, kDual>{}, std::false_type{}); break;
+        case kPrimaryOnly: go(std::integral_constant<int, kPrimaryOnly>{}, std::false_type{}); break;
+        case kShared5:
+            if (combined) go(std::integral_constant<int, kShared5>{}, std::true_type{});
+            else go(std::integral_constant<int, kShared5>{}, std::false_type{});
+            break;
+        case kPrimaryOnly5:
+            if (combined) go(std::integral_constant<int, kPrimaryOnly5>{}, std::true_type{});
+            else go(std::integral_constant<int, kPrimaryOnly5>{}, std::false_type{});
+            break;
+        default: go(std::integral_constant<int, kDual5>{}, std::false_type{}); break;
+    }
     return hipGetLastError();
 }
 
