@@ -365,6 +365,49 @@ def test_prefill_small_tiles_match_dequant_matmul(tq, oracle, mode, out, inf, bs
     assert _rel(y[rows], one) < 1e-3
 
 
+# ------------------------------------------------------------------ prefill, two planes composed into one fp16 weight
+@pytest.mark.parametrize("mode,out,inf,bs,batch", [("dual", 8260, 256, 256, 513),       # half a 512-column segment; ragged last weight tile
+                                                   ("dual", 8322, 768, 128, 600),       # one segment and a half; out no multiple of 4
+                                                   ("dual", 6000, 512, 512, 1030),      # three panels, tail tiles in K ranges
+                                                   ("5+3dual", 16500, 256, 32, 385),    # one panel; 5-bit primary in bytes
+                                                   ("5+4shared", 16448, 512, 256, 400), # no rotation between the planes
+                                                   ("5+4dual", 8200, 1280, 256, 1024)])
+def test_prefill_composed_planes_match_dequant_matmul(tq, oracle, monkeypatch, mode, out, inf, bs, batch):
+    """Many rows of a layer with two planes: one fp16 weight (rounded once from fp32), fp16 activations, fp32 sums: 1e-3 relative
+    L2, 5e-3 in bf16."""
+    monkeypatch.setitem(MODES, "5+4dual", dict(pb=5, rb=4, shared=False))
+    monkeypatch.setitem(MODES, "5+4shared", dict(pb=5, rb=4, shared=True))
+    qw, cbp, cbr = _make(oracle, out, inf, bs, mode)
+    x32 = np.random.default_rng(batch).standard_normal((batch, inf)).astype(np.float32)
+    xbits = oracle.f32_to_bf16_bits(x32)
+    want = oracle.linear_forward(qw, cbp, cbr, bs, oracle.bf16_bits_to_f32(xbits))
+    layer = tq.TurboQuantLinear(inf, out, qw, cbp, cbr, bs)
+    layer.reserve(batch)
+    y = layer.forward(xbits, tq.BF16, tq.F32)
+    yb = oracle.bf16_bits_to_f32(layer.forward(xbits, tq.BF16, tq.BF16))
+    layer.close()
+    assert _rel(y, want) < 1e-3
+    assert _rel(yb, want) < 5e-3
+
+
+def test_prefill_composed_planes_in_slabs(tq, oracle):
+    """A weight of more than one slab (160 MB of fp16): rows of the call agree with the one-row kernel on the same rows, in
+    every slab's columns."""
+    rng = np.random.default_rng(3)
+    out, inf, bs, batch = 33100, 2560, 512, 520
+    cb = oracle.generate_codebook(4)
+    q = oracle.QuantizedWeight(rng.integers(0, 256, (out, inf // 2), dtype=np.uint8), rng.integers(0, 256, (out, inf // 2), dtype=np.uint8),
+                               rng.random(out, dtype=np.float32) + 0.5, np.array([99, 1234, bs], np.uint32))
+    x = oracle.f32_to_bf16_bits(rng.standard_normal((batch, inf)).astype(np.float32))
+    layer = tq.TurboQuantLinear(inf, out, q, cb, cb, bs)
+    y = layer.forward(x, tq.BF16, tq.F32)
+    rows = [0, 511, 512, 519]
+    one = np.concatenate([layer.forward(x[r:r + 1], tq.BF16, tq.F32) for r in rows])
+    layer.close()
+    for c0 in range(0, out, 4096):
+        assert _rel(y[rows, c0:c0 + 4096], one[:, c0:c0 + 4096]) < 1e-3, c0
+
+
 # ------------------------------------------------------------------ prefill, 512-row activation panels
 @pytest.mark.parametrize("mode", ["shared", "dual", "primary_only"])
 @pytest.mark.parametrize("out,inf,bs,batch", [(16500, 256, 256, 257),      # one ragged panel, ragged last weight tile

@@ -48,6 +48,24 @@ __device__ __forceinline__ void chunks_to_pairs(float (&v)[kChunk], char* area, 
     __builtin_amdgcn_wave_barrier();                       // (the area is written again)
 }
 
+// The way back.
+__device__ __forceinline__ void pairs_to_chunks(float (&v)[kChunk], char* area, int lane) {
+    char* const base = area + (lane >> 4) * kDqGroup;
+    const int c = lane & 15, wr = ((c >> 1) << 4) | ((c & 1) << 3), sw = ((c >> 1) & 7) << 4;
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+        *reinterpret_cast<float4*>(base + c * 128 + ((s << 4) ^ sw)) = make_float4(v[4 * s], v[4 * s + 1], v[4 * s + 2], v[4 * s + 3]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+        const float2 t = *reinterpret_cast<const float2*>(base + p * 128 + (wr ^ (((p >> 1) & 7) << 4)));
+        v[2 * p] = t.x; v[2 * p + 1] = t.y;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Stages 1 .. 16 of the butterfly on a lane's chunk, and 32 .. 1024 on its pairs.
 __device__ __forceinline__ void fwht_chunk(float (&v)[kChunk], uint32_t bs) {
 #pragma unroll
@@ -277,6 +295,114 @@ hipError_t launch_dequant(const LayerView& L, void* w, int w_dtype, hipStream_t 
             else go(std::integral_constant<int, kPrimaryOnly5>{}, std::false_type{});
             break;
         default: go(std::integral_constant<int, kDual5>{}, std::false_type{}); break;
+    }
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Two planes with rotations of their own as ONE fp16 weight in the primary's rotation, for prefill of many rows:
+//   sum_k cP[k] x~p[k] + cR[k] x~r[k]  =  sum_k (cP + H (s_p s_r (.) H cR) / bs)[k] x~p[k],     x~ = H (s (.) x)
+// so that the contraction runs once instead of once per plane.  The sum is formed in fp32 and rounded to fp16 once; the
+// planes multiplied one after the other round each centroid by itself.  kShared5: both planes in one rotation, a plain sum.
+// Rows [row0, row0 + rows) of the layer (row0 a multiple of 128), in the order in which tq_prefill_panel_kernel's threads
+// load them: [row / 128][K / 64][4 pieces of 8 columns][row % 128 / 32][half of the 64 columns][row % 32] x 16 bytes.
+// Bound by its vector instructions (28 per weight); 27648 x 5120 in 140 us, a sixth of the contraction it halves at 2048 rows.
+// Four waves per SIMD (128 registers) spill and are 10 % slower.
+// A wave takes 512 columns (whole blocks: at most 512) of four rows, 16 lanes each, and eight waves in a row the same
+// columns of 32 rows; exchange as above.
+// ---------------------------------------------------------------------------
+template <int MODE>
+__global__ __launch_bounds__(kDqWaves* kWave, 3) void tq_compose_kernel(LayerView L, char* __restrict__ out, int row0, int rows,
+                                                                         int segs, int tasks) {
+    constexpr bool bytes = DequantMode<MODE>::five, rotate = DequantMode<MODE>::dual;
+    __shared__ float tab[64];
+    __shared__ __align__(16) char exchange[rotate ? kDqWaves * kDqExchange : 16];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    if (threadIdx.x < 64) tab[threadIdx.x] = L.tables[threadIdx.x] * kComposeScale;
+    __syncthreads();
+    const char* const tab_p = reinterpret_cast<const char*>(tab);
+    const char* const tab_r = reinterpret_cast<const char*>(tab + (bytes ? 32 : 16));
+    char* const area = exchange + (rotate ? wave * kDqExchange : 0);
+    const uint32_t bs = L.block_size;
+    float sg[rotate ? kChunk : 1];
+    if constexpr (rotate) {
+        const float scale = 1.0f / (float)bs;              // (a power of two)
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+            const uint32_t col = (uint32_t)((k >> 1) * 32 + 2 * (lane & 15) + (k & 1)) & (bs - 1);
+            sg[k] = scale * sign_of(L.seed_primary, col) * sign_of(L.seed_residual, col);
+        }
+    }
+    const int per_row = L.in_features / kChunk, step = gridDim.x * kDqWaves;
+    int task = blockIdx.x * kDqWaves + wave;               // (32 rows, 512 columns, four of the rows)
+    if (task >= tasks) return;                             // whole wave leaves together; no workgroup barrier below
+    int r = 0, c = 0;                                      // this lane's row of the slab and chunk of the row
+    auto place = [&](int t) {
+        const int unit = t >> 3, rb = unit / segs;
+        r = rb * 32 + (t & 7) * 4 + (lane >> 4);
+        c = (unit - rb * segs) * 16 + (lane & 15);
+    };
+    // (past the last row or column: the last row, chunk 0 .. 15, not stored)
+    auto mine = [&]() { return (long long)(row0 + (r < rows ? r : rows - 1)) * per_row + (c < per_row ? c : 0); };
+    place(task);
+    ChunkBytes<bytes> P = load_chunk_bytes<bytes>(L.packed_primary, mine());
+    ChunkBytes<false> R = load_chunk_bytes<false>(L.packed_residual, mine());
+    for (; task < tasks; task += step) {
+        const ChunkBytes<bytes> pb = P;
+        const ChunkBytes<false> rb = R;
+        const int row = r, chunk = c;
+        place(task + step < tasks ? task + step : task);
+        P = load_chunk_bytes<bytes>(L.packed_primary, mine());
+        R = load_chunk_bytes<false>(L.packed_residual, mine());
+        float u[kChunk], v[kChunk];
+        lookup_nibbles(rb, tab_r, u);
+        if constexpr (rotate) {
+            fwht_chunk(u, bs);
+            chunks_to_pairs(u, area, lane);
+            fwht_pairs(u, bs, lane);
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) u[k] *= sg[k];
+            fwht_pairs(u, bs, lane);
+            pairs_to_chunks(u, area, lane);
+            fwht_chunk(u, bs);
+        }
+        if constexpr (bytes) {
+#pragma unroll
+            for (int d = 0; d < 8; ++d)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t c = (chunk_word(pb, d) >> (8 * j)) & 0xffu;
+                    v[4 * d + j] = tab[c > 31u ? 31u : c];
+                }
+        } else {
+            lookup_nibbles(pb, tab_p, v);
+        }
+        if (row >= rows || chunk >= per_row) continue;
+        char* const dst = out + ((size_t)(row >> 7) * (per_row >> 1) + (chunk >> 1)) * 16384 +
+                          (((row & 127) >> 5) * 64 + (chunk & 1) * 32 + (row & 31)) * 16;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            typedef float f32x8_t __attribute__((ext_vector_type(8)));
+            typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+            f32x8_t f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) f[j] = v[8 * i + j] + u[8 * i + j];
+            *reinterpret_cast<f16x8_t*>(dst + i * 4096) = __builtin_convertvector(f, f16x8_t);      // (in range: compose_ok)
+        }
+    }
+}
+
+hipError_t launch_compose(const LayerView& L, int row0, int rows, void* out, hipStream_t stream) {
+    const int segs = (L.in_features / kChunk + 15) / 16;
+    const long long tasks = (long long)((rows + 31) / 32) * segs * 8, groups = tasks / kDqWaves;
+    if (tasks > 0x3fffffff || (row0 & 127) || L.in_features % 64 || L.block_size > 512) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)(groups < 768 ? groups : 768)), block(kDqWaves * kWave);
+    char* const o = static_cast<char*>(out);
+    switch (L.mode) {
+        case kDual: hipLaunchKernelGGL(tq_compose_kernel<kDual>, grid, block, 0, stream, L, o, row0, rows, segs, (int)tasks); break;
+        case kDual5: hipLaunchKernelGGL(tq_compose_kernel<kDual5>, grid, block, 0, stream, L, o, row0, rows, segs, (int)tasks); break;
+        case kShared5: hipLaunchKernelGGL(tq_compose_kernel<kShared5>, grid, block, 0, stream, L, o, row0, rows, segs, (int)tasks); break;
+        default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }

@@ -318,6 +318,9 @@ tq_linear_t create_impl(int in_features, int out_features,
         for (int i = 0; i < np; ++i) big = std::fmax(big, std::fabs(cbp[i]));
         for (int i = 0; i < nr; ++i) big = std::fmax(big, std::fabs(cbr[i]));
         v.fp16_centroids_ok = (big < 30000.0f) ? 1 : 0;      // NaN compares false
+        // (the residual plane in the primary's rotation stays below sqrt(block) times its largest centroid)
+        v.compose_ok = block_size <= 512 && (mode == tq::kDual || mode == tq::kDual5 || (mode == tq::kShared5 && !fused5)) &&
+                       big * (1.0f + std::sqrt((float)block_size)) < 60000.0f;
     }
     if (fused5) {
         h->fwd_view = v;
@@ -364,6 +367,15 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 }  // namespace
 
+// Two planes as one composed weight (the caller has asked prefill_compose_supported with the static array's share).
+static int run_compose(tq_linear_s* h, const tq::LayerView& V, const void* x_dev, int x_dtype, int batch, void* y_dev, int y_dtype,
+                       hipStream_t stream, void* static_ws) {
+    if (!static_ws && !ensure_stage(&h->d_work, &h->work_bytes, tq::prefill_compose_workspace_bytes(V, batch, device_cu_count()),
+                                    stream, &h->retired)) return 1;
+    return hip_ok(tq::launch_prefill_compose(V, x_dev, x_dtype, batch, y_dev, y_dtype, static_ws ? static_ws : h->d_work,
+                                             device_cu_count(), stream), "tq_prefill_compose launch") ? 0 : 1;
+}
+
 // Shared by tq_linear_forward, tq_linear_forward_static and the MLP block.  gate: optional fp32
 // [batch, out]; the batch-1..15 kernel then stores silu(gate) * y.  static_ws: the workspaces of the
 // matrix-core paths come from there (TQ_STATIC_SCRATCH_BYTES) instead of the handle's own buffers,
@@ -399,6 +411,8 @@ int forward_view(tq_linear_s* h, const tq::LayerView& V, bool generic_only, cons
     void* work = nullptr;
     float* partial = nullptr;
     tq::PrefillPlan plan{};
+    if (prefill && tq::prefill_compose_supported(V, batch, device_cu_count(), static_ws ? static_cap : ~(size_t)0))
+        return run_compose(h, V, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws);
     // (few output tiles: small ones, tq_prefill_tile.hip; a static workspace too small for 512-row images goes on)
     const int tile = prefill ? tq::prefill_tile_shape(V, batch, device_cu_count()) : -1;
     if (tile >= 0) {
@@ -468,6 +482,9 @@ int forward_impl(tq_linear_s* h, const void* x_dev, int x_dtype, int batch, void
     // reference's kernel forms per element (metal/turboquant_dequant_mm.metal:240-248, 277-292).
     const bool two_plane5 = h->view.mode >= tq::kShared5 && !h->has_fwd_view;
     const size_t cap = (size_t)TQ_STATIC_SCRATCH_BYTES;
+    if (two_plane5 && !gate && h->has_plane_views &&
+        tq::prefill_compose_supported(h->view, batch, device_cu_count(), static_ws ? cap : ~(size_t)0))
+        return run_compose(h, h->view, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws);
     if (two_plane5 && batch >= 2 && !gate && h->has_plane_views) {
         const size_t one = align256((size_t)batch * h->view.out_features * sizeof(float));
         const size_t need = plane_sum_bytes(h, batch, y_dtype);
@@ -569,6 +586,11 @@ int tq_linear_reserve(tq_linear_t h, int max_batch) {
                 work = std::max(work, few_reserve_bytes(P, max_batch));
                 if (sk) part = std::max(part, tq::skinny_partial_bytes(P, rows));
             }
+            auto compose = [&](int r) {                    // (all rows at once: what prefill_reserve_bytes looks at)
+                if (r <= max_batch && tq::prefill_compose_supported(h->view, r, device_cu_count(), ~(size_t)0))
+                    work = std::max(work, tq::prefill_compose_workspace_bytes(h->view, r, device_cu_count()));
+            };
+            for (int r = tq::compose_min_rows(h->view); r <= max_batch; r = r / tq::kPanelM * tq::kPanelM + tq::kPanelM + 1) compose(r);
             if (!ensure_stage(&h->d_work, &h->work_bytes, work, nullptr, &h->retired)) return 1;
             if (!ensure_stage(&h->d_partial, &h->partial_bytes, part, nullptr, &h->retired)) return 1;
             if (!ensure_stage(&h->d_sum, &h->sum_bytes, plane_sum_bytes(h, max_batch, tq::kBF16), nullptr, &h->retired)) return 1;

@@ -37,6 +37,15 @@ size_t prefill_panel_workspace_bytes(const LayerView& L, int batch, int num_cus,
 hipError_t launch_prefill_panel(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
                                 void* workspace, size_t workspace_bytes, int num_cus, hipStream_t stream);
 
+// Layers of two planes (dual rotation; 5-bit primaries with a 4-bit residual) at many rows: the planes composed into one
+// fp16 weight first (tq_prefill_panel.hip).  Workspace: fragment images, parts, a slab of the weight.
+// (from the second panel of 512 rows on; 5-bit layers, whose planes are separate calls and a sum otherwise, in the first too)
+inline int compose_min_rows(const LayerView& L) { return L.mode == kDual ? kPanelM + 1 : 385; }
+bool prefill_compose_supported(const LayerView& L, int batch, int num_cus, size_t capacity);
+size_t prefill_compose_workspace_bytes(const LayerView& L, int batch, int num_cus);
+hipError_t launch_prefill_compose(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
+                                  void* workspace, int num_cus, hipStream_t stream);
+
 // The small-tile kernel (tq_prefill_tile.hip).  Its shape for a call that prefill_supported() takes, or -1: one of the
 // kernels with large tiles is faster.  Workspace: fragment images alone.
 int prefill_tile_shape(const LayerView& L, int batch, int num_cus);

@@ -56,12 +56,14 @@ struct PanelArgs {
     const char* xt;            // fragment images [planes][panels][K / 16][16 KB]
     const uint8_t* plane0;     // combined bytes [N, K] (shared rotation) or primary nibbles [N, K / 2]
     const uint8_t* plane1;     // residual nibbles [N, K / 2] (dual rotation) or NULL
+                               // kDense: plane0 holds the composed rows from n_first on
     const float* tables;       // 256 floats (build_tables in tq_linear_c.cpp)
     const float* norms;
     void* y;
     int y_dtype;
     int M, N, K;
     int panels, n_tiles, n_per_xcd;
+    int n_first;               // output column of the first weight tile (kDense: a call is run in slabs of columns)
     float out_scale;
     // The last `tail_tiles` tiles (in panel-major order; all tiles where the call has fewer tiles than the chip has
     // CUs) are cut into `parts` parts: K ranges of part_subs sub-steps, with the dual rotation one per (plane, K
@@ -78,8 +80,14 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-template <bool COMBINED> struct TileBytes { u32x4v v[2]; };     // index bytes of one thread for one weight tile
-template <> struct TileBytes<false> { u32x4v v[1]; };
+// Weights that launch_compose has written as fp16: a thread's 32 columns of a tile are copied to LDS instead of decoded.
+// They are stored in the order of these copies, [weight tile][K / 64][4 pieces][4 waves][64 lanes x 16 B], so that a
+// wave's load is 1 KB in one piece (row-major: 32 rows x 2 pieces of 16 bytes per load, and a tile's lines were out of the
+// CU's cache before their next piece was asked for: 880 TFLOP/s at 2048 x 16384 x 5120 instead of 1000).
+constexpr int kDense = 16;
+constexpr int kDenseTile = kPN * kTileK * 2;
+
+template <int PIECES> struct TileBytes { u32x4v v[PIECES]; };   // index bytes (kDense: fp16) of one thread for one weight tile
 
 }  // namespace
 
@@ -108,8 +116,10 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelA
     // Workgroup ids go round the XCDs (id % 8).  The workgroups an XCD runs side by side share a panel of
     // activations (the big operand: 512 x K fp16 per tile against 128 x K bytes of indices), so its L2
     // fetches the panel once for all of them; each takes another tile of weights.
-    constexpr bool combined = (MODE == kSharedLut);
+    constexpr bool combined = (MODE == kSharedLut), dense = (MODE == kDense);
+    static_assert(!dense || (NBLK == 4 && KG == 1), "composed weights: whole panels");
     constexpr int kPlanes = (MODE == kDual) ? 2 : 1;
+    constexpr int kRing = dense ? 2 : 4;                   // tiles of index bytes in registers
     const int U_all = a.K / kSubK;                         // sub-steps of a row (a multiple of kUnroll)
     const int id = blockIdx.x;
     int panel, n_tile, part = -1, part_slot = 0;            // part_slot: index of the part's fp32 product
@@ -146,7 +156,7 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelA
         const int half = (u_end - u_begin) >> 1;
         if (kg == 0) u_end = u_begin + half; else u_begin += half;
     }
-    const int m0 = panel * kPanelM, n0 = n_tile * kPN;
+    const int m0 = panel * kPanelM, n0 = a.n_first + n_tile * kPN;
     const int tiles_end = u_end / 4;                       // 64-column weight tiles end here
 
     // Decode mapping: thread -> (tile row, 32-column half).  The 16 lanes that write a 128-bit piece together
@@ -165,12 +175,13 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelA
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-    using Bytes = TileBytes<combined>;
+    using Bytes = TileBytes<dense ? 4 : (combined ? 2 : 1)>;
 
     for (int plane = plane_begin; plane < plane_end; ++plane) {
         if (plane > plane_begin) lds_barrier();            // the first plane's table and tiles are done with
         const char* const ap = a.xt + ((size_t)(plane * a.panels + panel) * U_all) * kSubImage + wave * 4096 + lane * 16;
-        const uint8_t* const bp = combined ? a.plane0 + (size_t)b_row * a.K + dh * 32
+        const uint8_t* const bp = dense ? a.plane0 + (size_t)n_tile * (a.K / kTileK) * kDenseTile + wave * 1024 + lane * 16
+                                  : combined ? a.plane0 + (size_t)b_row * a.K + dh * 32
                                            : (plane == 0 ? a.plane0 : a.plane1) + (size_t)b_row * (a.K >> 1) + dh * 16;
 
         // One row block per wave and no token among this wave's 32 rows: the wave re-reads the first image it was
@@ -179,7 +190,9 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelA
         const size_t a_step = (NBLK == 1 && m0 + wave * 32 >= a.M) ? 0 : (size_t)kSubImage;
         f16x8 A[8][NBLK];                                  // ring of eight sub-steps of this wave's 32 NBLK rows
         f16x8 Bf[2][4];                                    // weight fragments of the current and the next sub-step
-        Bytes By[4];                                       // ring of four tiles of index bytes
+        Bytes By[kRing];                                   // ring of tiles of index bytes
+        constexpr int kTileBytes = dense ? kDenseTile : (combined ? kTileK : kTileK / 2);
+        constexpr int kPieceStep = dense ? kDenseTile / 4 : 16;
 
         auto load_a = [&](auto Sc, int u) {
             constexpr int s = decltype(Sc)::value;
@@ -189,15 +202,18 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelA
         };
         auto load_bytes = [&](auto Sc, int tile) {
             constexpr int s = decltype(Sc)::value;
-            const uint8_t* p = bp + (size_t)(tile < tiles_end ? tile : tiles_end - 1) * (combined ? kTileK : kTileK / 2);
-            By[s].v[0] = *reinterpret_cast<const u32x4v*>(p);
-            if constexpr (combined) By[s].v[1] = *reinterpret_cast<const u32x4v*>(p + 16);
+            const uint8_t* p = bp + (size_t)(tile < tiles_end ? tile : tiles_end - 1) * kTileBytes;
+#pragma unroll
+            for (int i = 0; i < (int)(sizeof(Bytes) / 16); ++i) By[s].v[i] = *reinterpret_cast<const u32x4v*>(p + kPieceStep * i);
         };
         // Quarter q of a tile for this thread: 8 columns.  lookups() issues the table reads, finish() packs and
         // writes the 16 bytes of fp16.
         auto lookups = [&](auto Sc, auto Qc, uint32_t (&lv)[8]) {
             constexpr int s = decltype(Sc)::value, q = decltype(Qc)::value;
-            if constexpr (combined) {
+            if constexpr (dense) {
+                const u32x4v& src = By[s].v[q];
+                lv[0] = src.x; lv[1] = src.y; lv[2] = src.z; lv[3] = src.w;
+            } else if constexpr (combined) {
                 const u32x4v& src = By[s].v[q >> 1];
                 const uint32_t w0 = (q & 1) ? src.z : src.x, w1 = (q & 1) ? src.w : src.y;
 #pragma unroll
@@ -234,8 +250,10 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelA
         const int t_begin = u_begin >> 2;
         load_bytes(std::integral_constant<int, 0>{}, t_begin);
         load_bytes(std::integral_constant<int, 1>{}, t_begin + 1);
-        load_bytes(std::integral_constant<int, 2>{}, t_begin + 2);
-        load_bytes(std::integral_constant<int, 3>{}, t_begin + 3);
+        if constexpr (kRing == 4) {
+            load_bytes(std::integral_constant<int, 2>{}, t_begin + 2);
+            load_bytes(std::integral_constant<int, 3>{}, t_begin + 3);
+        }
         load_a(std::integral_constant<int, 0>{}, u_begin);
         load_a(std::integral_constant<int, 1>{}, u_begin + 1);
         load_a(std::integral_constant<int, 2>{}, u_begin + 2);
@@ -247,7 +265,7 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelA
         // The table, while those travel: wave w writes entries 64 w .. 64 w + 63, lane l into bytes 4 l .. of each
         // entry's 256.  Values come through scalar loads.  Shared rotation: entry b = fp16(lut[b]) in the upper half.
         // Nibble planes: entry b = the fp16 centroids of both nibbles of byte b (low nibble = even column).
-        {
+        if constexpr (!dense) {
             typedef const __attribute__((address_space(4))) float cfloat;
             cfloat* const src = (cfloat*)(a.tables + (plane == 0 ? 0 : 16));
             uint32_t* const dst = reinterpret_cast<uint32_t*>(smem) + lane;
@@ -275,7 +293,11 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelA
             lookups(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{}, lv);
             finish(std::integral_constant<int, 0>{}, 1, lv);
         }
-        load_bytes(std::integral_constant<int, 0>{}, t_begin + 4);
+        load_bytes(std::integral_constant<int, 0>{}, t_begin + kRing);
+        if constexpr (dense) {                             // (piece by piece from here on: the first of tile 1 is used up)
+            const int tile = t_begin + 1 + kRing < tiles_end ? t_begin + 1 + kRing : tiles_end - 1;
+            By[1].v[0] = *reinterpret_cast<const u32x4v*>(bp + (size_t)tile * kTileBytes);
+        }
         lds_barrier();
         read_frags(std::integral_constant<int, 0>{}, 0, 0);
 
@@ -290,12 +312,13 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelA
             constexpr int q = (U + 1) % 4;
             constexpr int dtile = (U + 1) / 4 + 1;                 // relative to tile ub / 4 (ub / 4 is a multiple of 4)
             constexpr int fbuf = ((U + 1) / 4) % 2, fks = (U + 1) % 4;
-            constexpr int sa = U % 8, san = (U + 7) % 8, sb = U % 2, sbn = (U + 1) % 2, sby = dtile % 4;
+            constexpr int sa = U % 8, san = (U + 7) % 8, sb = U % 2, sbn = (U + 1) % 2, sby = dtile % kRing;
             if constexpr (U % 4 == 3 && !(PANEL_ABL & 4)) lds_barrier();
             // This thread's index bytes of the quarter, the table addresses, the table values, the packed result.
-            uint32_t w0, w1 = 0, ad[8], lv[8];
+            uint32_t w0 = 0, w1 = 0, ad[8], lv[8];
             u32x4v o;
-            if constexpr (combined) {
+            if constexpr (dense) {
+            } else if constexpr (combined) {
                 const u32x4v& src = By[sby].v[q >> 1];
                 w0 = (q & 1) ? src.z : src.x;
                 w1 = (q & 1) ? src.w : src.y;
@@ -317,7 +340,9 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelA
                 if constexpr (k < 4 && !(PANEL_ABL & 16))
                     Bf[sbn][k] = *reinterpret_cast<const f16x8*>(bfrag + fbuf * kWTile + k * 32 * kWPitch + fks * 32);
                 if constexpr (!(PANEL_ABL & 2)) {
-                    if constexpr (combined) {
+                    if constexpr (dense) {
+                        if constexpr (k == 6) *reinterpret_cast<u32x4v*>(wdst + (dtile % 2) * kWTile + q * 16) = By[sby].v[q];
+                    } else if constexpr (combined) {
                         // addresses in even slots 0..6, reads in odd slots 1..7, packs in 9..12, write in 13
                         if constexpr (k < 8 && (k & 1) == 0) {
                             ad[k] = gemm_entry_addr(k < 4 ? w0 : w1, laneoff, k & 3);
@@ -350,9 +375,13 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelA
                 }
                 if constexpr (k >= 8 && k < 8 + NBLK && !(PANEL_ABL & 1))
                     A[san][k - 8] = *reinterpret_cast<const f16x8*>(pa + (k - 8) * 1024);
-                if constexpr (k == 14 && q == 3 && !(PANEL_ABL & 8)) {
+                if constexpr (dense && k == 14 && !(PANEL_ABL & 8)) {
+                    const int tile = (ub >> 2) + dtile + kRing;
+                    By[sby].v[q] = *reinterpret_cast<const u32x4v*>(bp + (size_t)(tile < tiles_end ? tile : tiles_end - 1) * kTileBytes + q * kPieceStep);
+                }
+                if constexpr (!dense && k == 14 && q == 3 && !(PANEL_ABL & 8)) {
                     const int tile = (ub >> 2) + dtile + 4;
-                    const uint8_t* p = bp + (size_t)(tile < tiles_end ? tile : tiles_end - 1) * (combined ? kTileK : kTileK / 2);
+                    const uint8_t* p = bp + (size_t)(tile < tiles_end ? tile : tiles_end - 1) * kTileBytes;
                     By[sby].v[0] = *reinterpret_cast<const u32x4v*>(p);
                     if constexpr (combined) By[sby].v[1] = *reinterpret_cast<const u32x4v*>(p + 16);
                 }
@@ -589,7 +618,7 @@ __global__ __launch_bounds__(256) void tq_prefill_panel_sum_kernel(PanelArgs a) 
     const int t = a.panels * a.n_tiles - a.tail_tiles + tile_k;
     const int panel = t / a.n_tiles, n_tile = t - panel * a.n_tiles;
     const int c4 = (threadIdx.x & 31) * 4, r = rows0 + (threadIdx.x >> 5);
-    const int col = n_tile * kPN + c4;
+    const int col = a.n_first + n_tile * kPN + c4;
 #pragma unroll
     for (int rr = 0; rr < 32; rr += 8) {
         const int row = panel * kPanelM + r + rr;
@@ -729,6 +758,97 @@ hipError_t launch_prefill_panel(const LayerView& L, const void* x, int x_dtype, 
     if (e != hipSuccess || a.tail_tiles == 0) return e;
     hipLaunchKernelGGL(tq_prefill_panel_sum_kernel, dim3((unsigned)(a.tail_tiles * 16)), dim3(256), 0, stream, a);
     return hipGetLastError();
+}
+
+
+// ---------------------------------------------------------------------------
+// Two planes as one fp16 weight (launch_compose), slab of output rows by slab, and one contraction over it instead of one
+// per plane.  Composing costs the same whatever the number of rows (1 us per million weights): with two or more panels
+// of activations it is less than what it saves.  us per call, bf16, before -> now, in x out: 5120 x 27648 at 2048 rows
+// 1119 -> 872, 5120 x 5120 at 2048 rows 252 -> 175, 3584 x 18944 at 700 rows 320 -> 256, 2048 x 10240 at 1024 rows 111 -> 97; in
+// one panel 5120 x 27648 at 512 rows 264, 393 composed (not taken), but the 5-bit layers, which are two calls and a sum
+// otherwise, gain there too: 3072 x 17000 at 512 rows 179 -> 141, 2048 x 8704 at 668 rows 140 -> 89, 5120 x 27648 at 1024 rows
+// 661 -> 489.  Against 64 bits the error is that of the two contractions (2.93e-4).  The slab bounds the workspace: the
+// whole weight in fp16 would be twice the layer.
+// ---------------------------------------------------------------------------
+namespace {
+
+constexpr size_t kComposeBytes = (size_t)160 << 20;        // of a slab
+
+struct ComposePlan { int slab_tiles; PanelPlan panel; size_t slab_at, total_bytes; };    // panel: of a whole slab, the largest need
+
+LayerView slab_view(const LayerView& L, int rows) {
+    LayerView s = L;
+    s.mode = kPrimaryOnly;                                 // one plane, one rotation
+    s.out_features = rows;
+    return s;
+}
+
+ComposePlan compose_plan(const LayerView& L, int batch, int num_cus) {
+    ComposePlan p{};
+    const int panels = (batch + kPanelM - 1) / kPanelM, tiles = (L.out_features + kPN - 1) / kPN;
+    const size_t tile_bytes = (size_t)kPN * L.in_features * sizeof(uint16_t);
+    int slab = (int)(kComposeBytes / tile_bytes);
+    if (slab < 1) slab = 1;
+    const int round = num_cus / panels;                    // weight tiles that fill the chip once
+    if (slab >= tiles) slab = tiles;
+    else if (round >= 1 && slab >= round) slab = slab / round * round;
+    else slab = (tiles + (tiles + slab - 1) / slab - 1) / ((tiles + slab - 1) / slab);       // slabs of equal length
+    p.slab_tiles = slab;
+    for (int t0 = 0; t0 < tiles; t0 += slab) {
+        const int n = t0 + slab < tiles ? slab * kPN : L.out_features - t0 * kPN;
+        const PanelPlan q = panel_plan(slab_view(L, n), batch, num_cus, ~(size_t)0);
+        if (q.total_bytes > p.panel.total_bytes) p.panel = q;
+    }
+    p.slab_at = (p.panel.total_bytes + 255) & ~(size_t)255;
+    p.total_bytes = p.slab_at + (size_t)slab * tile_bytes;
+    return p;
+}
+
+}  // namespace
+
+size_t prefill_compose_workspace_bytes(const LayerView& L, int batch, int num_cus) { return compose_plan(L, batch, num_cus).total_bytes; }
+
+bool prefill_compose_supported(const LayerView& L, int batch, int num_cus, size_t capacity) {
+    if (!L.compose_ok || batch < compose_min_rows(L)) return false;
+    if (!prefill_panel_supported(slab_view(L, L.out_features), batch, num_cus, capacity)) return false;
+    return compose_plan(L, batch, num_cus).total_bytes <= capacity;
+}
+
+hipError_t launch_prefill_compose(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
+                                  void* workspace, int num_cus, hipStream_t stream) {
+    const ComposePlan plan = compose_plan(L, batch, num_cus);
+    hipError_t e = launch_rotate_tiles(slab_view(L, L.out_features), x, x_dtype, batch, workspace, stream, kPanelImage);
+    if (e != hipSuccess) return e;
+    char* const slab = static_cast<char*>(workspace) + plan.slab_at;
+    const int tiles = (L.out_features + kPN - 1) / kPN;
+    for (int t0 = 0; t0 < tiles; t0 += plan.slab_tiles) {
+        const int row0 = t0 * kPN, rows = t0 + plan.slab_tiles < tiles ? plan.slab_tiles * kPN : L.out_features - row0;
+        if ((e = launch_compose(L, row0, rows, slab, stream)) != hipSuccess) return e;
+        const PanelPlan q = panel_plan(slab_view(L, rows), batch, num_cus, ~(size_t)0);
+        PanelArgs a{};
+        a.xt = static_cast<const char*>(workspace);
+        a.plane0 = reinterpret_cast<const uint8_t*>(slab);
+        a.norms = L.norms;
+        a.y = y; a.y_dtype = y_dtype;
+        a.M = batch; a.N = L.out_features; a.K = L.in_features;
+        a.panels = (batch + kPanelM - 1) / kPanelM;
+        a.n_tiles = (rows + kPN - 1) / kPN;
+        a.n_per_xcd = (a.n_tiles + 7) / 8;
+        a.n_first = row0;
+        a.out_scale = L.inv_scale / kComposeScale;
+        a.tail_tiles = q.tail_tiles; a.parts = q.parts; a.part_subs = q.part_subs;
+        a.first_part_wg = q.tail_tiles == a.panels * a.n_tiles ? 0 : 8 * a.n_per_xcd * a.panels;
+        a.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + q.xt_bytes);
+        hipLaunchKernelGGL((tq_prefill_panel_kernel<kDense, 4>), dim3((unsigned)(a.first_part_wg + a.tail_tiles * a.parts)),
+                           dim3(kPThreads), 0, stream, a);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if (a.tail_tiles) {
+            hipLaunchKernelGGL(tq_prefill_panel_sum_kernel, dim3((unsigned)(a.tail_tiles * 16)), dim3(256), 0, stream, a);
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+        }
+    }
+    return hipSuccess;
 }
 
 }  // namespace tq
