@@ -215,6 +215,37 @@ def test_five_bit_two_plane_forward(tq, oracle, rbits, shared, out_f, in_f, bs, 
     layer.close()
 
 
+@pytest.mark.parametrize("rbits,shared", [(4, False), (4, True), (0, False)], ids=["5+4dual", "5+4shared", "5+0"])
+@pytest.mark.parametrize("out_f,in_f,bs", [(1, 32, 2), (3, 96, 32), (5, 544, 32),        # one wave; a segment of one block
+                                           (2051, 1536, 512), (9, 8192, 512),            # rounds of rows; sixteen waves
+                                           (6, 8224, 4), (3, 16384, 512)])               # too wide: the generic kernel
+def test_five_bit_two_plane_one_row(tq, oracle, rbits, shared, out_f, in_f, bs):
+    """One row at the edges of the whole-row kernel, fp32 throughout: 2e-6 is 16 units of rounding, more than the 11
+    stages of a butterfly and of the sums leave in a 2-norm.  Bytes beyond 31 count as 31."""
+    o = oracle
+    rng = np.random.default_rng(out_f + in_f)
+    cbp = o.generate_codebook(5)
+    cbr = o.generate_codebook(rbits) if rbits else o.generate_codebook(4)
+    w = (rng.standard_normal((out_f, in_f)) * 0.03).astype(np.float32)
+    qw = o.quantize_weight(w, cbp, cbr, 5, rbits, bs, shared)
+    qw.packed_primary[0, :: 7] = 201
+    w_ref = o.dequantize_weight_cpu(qw, cbp, cbr, bs).astype(np.float64)
+    layer = tq.TurboQuantLinear(in_f, out_f, qw, cbp, cbr, bs)
+    x = rng.standard_normal((1, in_f)).astype(np.float32)
+
+    def rel(y, x):                                      # (a few sums may cancel: against what random signs leave)
+        want = x.astype(np.float64) @ w_ref.T
+        return np.linalg.norm(y - want) / max(np.linalg.norm(want), np.linalg.norm(x) * np.linalg.norm(w_ref) / in_f ** 0.5)
+
+    assert rel(layer.forward(x), x) < 2e-6
+    x16 = x.astype(np.float16)
+    assert rel(layer.forward(x16, tq.F16, tq.F32), x16.astype(np.float32)) < 2e-6
+    xb = o.f32_to_bf16_bits(x)
+    yb = o.bf16_bits_to_f32(layer.forward(xb, tq.BF16, tq.BF16))
+    assert rel(yb, o.bf16_bits_to_f32(xb)) < 4e-3          # the output's own rounding
+    layer.close()
+
+
 @pytest.mark.parametrize("shared", [True, False])
 @pytest.mark.parametrize("outs,in_f,bs,x_dt", [((640, 128, 131), 5120, 512, "bf16"),     # q, k, v: rows served in pairs
                                                  ((1100, 1000), 4096, 512, "f32"),         # gate, up: two slabs

@@ -158,6 +158,10 @@ hipError_t launch_codebook_lookup(const uint8_t* indices, size_t n, const float*
 // columns, all six modes.  Forward through the layer's fp32 scratch row (xrot_work); dequantiser and
 // rotation for blocks of at most 16 columns (widths that are not a multiple of 32).
 bool generic_supported(const LayerView& L);
+// One row of 5-bit layers of two planes (tq_gemv_five.hip); launch_gemv_generic takes it where it is supported.
+bool gemv_five_supported(const LayerView& L);
+hipError_t launch_gemv_five(const LayerView& L, const void* x, int x_dtype, void* y, int y_dtype, int num_cus,
+                            hipStream_t stream, const float* gate);
 hipError_t launch_gemv_generic(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
                                int num_cus, hipStream_t stream, const float* gate);
 hipError_t launch_dequant_small(const LayerView& L, void* w, int w_dtype, hipStream_t stream);

@@ -236,11 +236,19 @@ static hipError_t rotate_row_generic(const LayerView& L, const void* x, int x_dt
 hipError_t launch_gemv_generic(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
                                int num_cus, hipStream_t stream, const float* gate) {
     if (!generic_supported(L)) return hipErrorInvalidValue;
+    const bool five = gemv_five_supported(L);
     const size_t xe = (x_dtype == kF32) ? 4 : 2, ye = (y_dtype == kF32) ? 4 : 2;
     int grid = (L.out_features + 3) / 4;
     if (grid > num_cus * 8) grid = num_cus * 8;
     for (int b = 0; b < batch; ++b) {
-        hipError_t e = rotate_row_generic(L, static_cast<const char*>(x) + (size_t)b * L.in_features * xe, x_dtype, stream);
+        const void* const row = static_cast<const char*>(x) + (size_t)b * L.in_features * xe;
+        if (five) {
+            const hipError_t e = launch_gemv_five(L, row, x_dtype, static_cast<char*>(y) + (size_t)b * L.out_features * ye, y_dtype,
+                                                  num_cus, stream, gate ? gate + (size_t)b * L.out_features : nullptr);
+            if (e != hipSuccess) return e;
+            continue;
+        }
+        hipError_t e = rotate_row_generic(L, row, x_dtype, stream);
         if (e != hipSuccess) return e;
         GenericArgs a{};
         a.L = L;
