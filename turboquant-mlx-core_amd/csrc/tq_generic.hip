@@ -1,6 +1,7 @@
 // Fused TQ8 forward for every shape and mode the reference accepts and the tuned kernels do not take:
 // rows wider than 32768 columns, widths that are a multiple of the block size but not of 32 (blocks of
-// 1 to 16 columns), 5-bit primaries with their own residual rotation or a 4-bit residual
+// 1 to 16 columns), one row of 5-bit primaries with their own residual rotation or a 4-bit residual that
+// tq_gemv_five.hip does not take (wider than 8192 columns, blocks above 512)
 // (metal/turboquant_dequant_mm.metal:240-248, 277-292; src/dequantizer.cpp:625-626, 657).  The only
 // rule the reference has is in_features % block_size == 0 (src/rotation.cpp:374, 396).
 //

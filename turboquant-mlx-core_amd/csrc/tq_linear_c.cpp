@@ -477,7 +477,7 @@ size_t plane_sum_bytes(const tq_linear_s* h, int batch, int y_dtype) {
 int forward_impl(tq_linear_s* h, const void* x_dev, int x_dtype, int batch, void* y_dev, int y_dtype,
                  hipStream_t stream, const float* gate, void* static_ws = nullptr) {
     // 5-bit primaries with their own residual rotation or a 4-bit residual keep their two planes.  One
-    // row runs on the generic kernels (both planes in one pass); two or more rows run each plane through
+    // row runs both planes in one pass (tq_gemv_five.hip, tq_generic.hip); two or more rows run each plane through
     // the tuned kernels as a layer of its own and add the two results: y = P x~p + R x~r, the same sum the
     // reference's kernel forms per element (metal/turboquant_dequant_mm.metal:240-248, 277-292).
     const bool two_plane5 = h->view.mode >= tq::kShared5 && !h->has_fwd_view;
