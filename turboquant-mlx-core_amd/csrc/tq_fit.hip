@@ -636,7 +636,9 @@ static size_t fit_tiles(size_t n) {
 // codebook's boundaries visit 1 % of the samples and the residual's, which start from a far too wide codebook, a quarter.
 static size_t fit_capacity(size_t n, int problems, bool everything) { return everything ? problems * n : n / 2; }
 
-bool fit_supported(size_t n) { return n >= 1 && n < ((size_t)1 << 32) - 64; }
+// (positions and counters of 32 bits: tq_fit_refine_kernel walks a cell in strides of kFitMaxTile samples, and a cell may
+// hold all of them)
+bool fit_supported(size_t n) { return n >= 1 && n < ((size_t)1 << 32) - 2 * (size_t)kFitMaxTile; }
 bool fit_predicts(size_t n) { return n >= ((size_t)1 << 22); }
 
 size_t fit_workspace_bytes(size_t n, int problems, bool everything) {
