@@ -1,0 +1,152 @@
+// Host side of the conversion calls (csrc/tq_quantize_c.cpp) on a HIP runtime and kernels that are faked here, without a
+// GPU: a device of a given size whose memory is host memory, filled with 0xff when handed out.  One check per argument
+// (tests/test_host_rules.py).
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <new>
+#include <string>
+#include <vector>
+
+#include "tq_device.h"
+#include "turboquant_c/tq_quantizer.h"
+
+namespace {
+
+struct FakeDevice {
+    size_t size = ~(size_t)0, live = 0, peak = 0;
+    hipError_t last = hipSuccess;
+    std::map<void*, size_t> blocks;
+} dev;
+
+int lloyd_passes = 0;
+struct FitCall { bool first_round, everything; };
+std::vector<FitCall> fit_calls;
+enum { kFits, kMissesOnce, kNeedsAll } fit_outcome = kFits;
+bool host_memory_gone = false;
+
+int failures = 0;
+void expect(bool ok, const char* what, unsigned long long value = 0) {
+    if (!ok) { std::printf("failed: %s (%llu)\n", what, value); ++failures; }
+}
+
+}  // namespace
+
+void* operator new(size_t n) {
+    void* p = host_memory_gone ? nullptr : std::malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
+// --------------------------------------------------------------------------- the runtime
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) {
+    if (n > dev.size || dev.live + n > dev.size) return dev.last = hipErrorOutOfMemory;
+    *p = std::malloc(n);
+    std::memset(*p, 0xff, n);
+    const bool gone = host_memory_gone;                    // (the map is the fake's, not the library's)
+    host_memory_gone = false;
+    dev.blocks[*p] = n;
+    host_memory_gone = gone;
+    dev.live += n;
+    if (dev.live > dev.peak) dev.peak = dev.live;
+    return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+    if (!p) return hipSuccess;
+    expect(dev.blocks.count(p) == 1, "memory is freed once");
+    dev.live -= dev.blocks[p];
+    dev.blocks.erase(p);
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind) { std::memcpy(to, from, n); return hipSuccess; }
+hipError_t hipMemset(void* p, int v, size_t n) { std::memset(p, v, n); return hipSuccess; }
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipGetLastError() { const hipError_t e = dev.last; dev.last = hipSuccess; return e; }
+const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
+}
+
+// --------------------------------------------------------------------------- the kernels
+namespace tq {
+void set_error(const std::string&) {}
+bool hip_ok(hipError_t e, const char* what) {
+    if (e != hipSuccess) std::printf("(%s: %s)\n", what, hipGetErrorString(e));
+    return e == hipSuccess;
+}
+int quantize_partials_per_row(int, uint32_t) { return 1; }
+hipError_t launch_row_norms(const float*, float*, int, int, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_derive_seeds(const float*, size_t, uint32_t* s, hipStream_t) { s[0] = 1; s[1] = 2; return hipGetLastError(); }
+hipError_t launch_finish_norms(const float*, const double*, float*, int, int, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_quantize_rows(const QuantArgsHost&, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_codebook_quantize(const float*, size_t, const float*, int, uint8_t*, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_codebook_lookup(const uint8_t*, size_t, const float*, int, float*, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_lloyd_pass(const float*, size_t, const float*, int, int, const float*, const float*, int, double* sum,
+                             unsigned long long* cnt, int workgroups, hipStream_t) {
+    ++lloyd_passes;
+    std::memset(sum, 0, (size_t)workgroups * 32 * sizeof(double));
+    std::memset(cnt, 0, (size_t)workgroups * 32 * sizeof(unsigned long long));
+    return hipGetLastError();
+}
+bool fit_supported(size_t) { return true; }
+bool fit_predicts(size_t) { return true; }
+size_t fit_workspace_bytes(size_t n, int problems, bool everything) { return (everything ? 8 * (size_t)problems : 4) * n + (1 << 20); }
+// A codebook's fields are written for the codebooks that are fitted, as the kernels do.
+hipError_t launch_fit(const float*, size_t n, int problems, const float*, int, const FitCodebooks& cb, int iterations,
+                      bool first_round, bool everything, void*, FitResult* state, hipStream_t) {
+    fit_calls.push_back({first_round, everything});
+    state->bad = 0;
+    for (int p = 0; p < problems; ++p) {
+        std::memcpy(state->cent[p], cb.init[p], sizeof(cb.init[p]));
+        state->steps[p] = iterations;
+        state->missed[p] = fit_outcome == kMissesOnce ? fit_calls.size() == 1 : fit_outcome == kNeedsAll && !everything;
+        state->kept[p] = (unsigned)(fit_outcome == kNeedsAll ? n : n / 8);
+    }
+    return hipGetLastError();
+}
+}  // namespace tq
+
+namespace {
+
+constexpr int kOut = 1024, kIn = 1024;
+constexpr size_t kN = (size_t)kOut * kIn;
+
+int fit() {
+    static std::vector<float> w(kN, 0.5f);
+    float g[16], cp[16], cr[16];
+    tq_generate_codebook(4, g, nullptr);
+    return tq_fit_layer_codebooks(w.data(), kOut, kIn, 512, 4, 4, g, 16, 100, cp, cr);
+}
+
+// A block goes back to the pool while host memory is short: nothing may be thrown out of a destructor.
+void no_host_memory() {
+    std::vector<float> v(kN, 0.0f);
+    std::vector<uint8_t> idx(kN);
+    float bounds[15] = {0};
+    host_memory_gone = true;
+    const int rc = tq_codebook_quantize_host(v.data(), kN, bounds, 16, idx.data());
+    host_memory_gone = false;
+    expect(rc == 0, "the call needs no host memory of its own", rc);
+    tq_quantizer_release_workspaces();
+    expect(dev.live == 0, "all device memory is given back", dev.live);
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const struct { const char* name; void (*run)(); } checks[] = {{"no_host_memory", no_host_memory}};
+    for (const auto& c : checks)
+        if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
+            c.run();
+            if (!failures) std::printf("ok\n");
+            return failures ? 1 : 0;
+        }
+    (void)&fit;
+    std::fprintf(stderr, "usage: conversion_memory <check>\n");
+    return 2;
+}

@@ -1,4 +1,5 @@
-"""Dispatch rules and workspace sizes of the library's host code (tests/cpp/host_rules.cpp), without a GPU."""
+"""Host code of the library without a GPU: dispatch rules and workspace sizes (tests/cpp/host_rules.cpp), and the conversion
+calls on a faked runtime (tests/cpp/conversion_memory.cpp)."""
 import os
 import subprocess
 
@@ -6,11 +7,21 @@ import pytest
 
 import __graft_entry__ as entry
 
-EXE = os.path.join(entry.ROOT, "tests", "cpp", "bin", "host_rules")
+BIN = os.path.join(entry.ROOT, "tests", "cpp", "bin")
+
+
+def _check(program, check):
+    exe = os.path.join(BIN, program)
+    assert os.path.exists(exe), "build the test programs first (python __graft_entry__.py)"
+    p = subprocess.run([exe, check], capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, p.stdout + p.stderr
 
 
 @pytest.mark.parametrize("check", ["fit_limit"])
 def test_host_rules(check):
-    assert os.path.exists(EXE), "build the test programs first (python __graft_entry__.py)"
-    p = subprocess.run([EXE, check], capture_output=True, text=True, timeout=120)
-    assert p.returncode == 0, p.stdout + p.stderr
+    _check("host_rules", check)
+
+
+@pytest.mark.parametrize("check", ["no_host_memory"])
+def test_conversion_memory(check):
+    _check("conversion_memory", check)

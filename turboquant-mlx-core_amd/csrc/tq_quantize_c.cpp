@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "tq_device.h"
@@ -41,12 +42,22 @@ class KeptMemory {
     struct Block { void* p; size_t bytes; int device; };
     static constexpr size_t kKeepBytes = (size_t)2 << 30;
     static constexpr size_t kUnit = (size_t)2 << 20;       // sizes in whole units; smaller blocks are not kept
+    static constexpr int kMaxIdle = 64;                    // (an array: blocks come back in destructors, which must not throw)
     std::mutex mu_;
-    std::vector<Block> idle_;                              // oldest first
+    Block idle_[kMaxIdle];                                 // oldest first
+    int n_ = 0;
+
+    Block remove(int i) {
+        const Block b = idle_[i];
+        for (int k = i + 1; k < n_; ++k) idle_[k - 1] = idle_[k];
+        --n_;
+        return b;
+    }
 
 public:
     static KeptMemory& get() {
-        static KeptMemory* const kept = new KeptMemory();  // (never destroyed: the runtime may be gone by then)
+        alignas(KeptMemory) static unsigned char storage[sizeof(KeptMemory)];
+        static KeptMemory* const kept = new (storage) KeptMemory();        // (never destroyed: the runtime may be gone by then)
         return *kept;
     }
     // The smallest idle block that is large enough and not more than four times too large, or a new one.
@@ -56,15 +67,15 @@ public:
         if (e != hipSuccess) return e;
         if (*got >= kUnit) {
             std::lock_guard<std::mutex> lock(mu_);
-            size_t best = idle_.size();
-            for (size_t i = 0; i < idle_.size(); ++i)
+            int best = -1;
+            for (int i = 0; i < n_; ++i)
                 if (idle_[i].device == *device && idle_[i].bytes >= *got && idle_[i].bytes / 4 <= *got &&
-                    (best == idle_.size() || idle_[i].bytes < idle_[best].bytes))
+                    (best < 0 || idle_[i].bytes < idle_[best].bytes))
                     best = i;
-            if (best < idle_.size()) {
-                *p = idle_[best].p;
-                *got = idle_[best].bytes;
-                idle_.erase(idle_.begin() + (long)best);
+            if (best >= 0) {
+                const Block b = remove(best);
+                *p = b.p;
+                *got = b.bytes;
                 return hipSuccess;
             }
         }
@@ -75,30 +86,37 @@ public:
         return hipMalloc(p, *got);
     }
     // The calls work on the null stream; nothing of it may still run when another call gets the block.
-    void give(void* p, size_t bytes, int device) {
-        std::vector<void*> out;
+    void give(void* p, size_t bytes, int device) noexcept {
         int now = 0;
         if (bytes < kUnit || bytes > kKeepBytes || hipGetDevice(&now) != hipSuccess || now != device ||
             hipStreamSynchronize(nullptr) != hipSuccess) {
-            out.push_back(p);
-        } else {
+            (void)hipFree(p);
+            return;
+        }
+        Block out[kMaxIdle];
+        int n_out = 0;
+        {
             std::lock_guard<std::mutex> lock(mu_);
             size_t held = bytes;
-            for (const Block& b : idle_) held += b.device == device ? b.bytes : 0;
-            for (size_t i = 0; i < idle_.size() && held > kKeepBytes;) {
+            for (int i = 0; i < n_; ++i) held += idle_[i].device == device ? idle_[i].bytes : 0;
+            for (int i = 0; i < n_ && held > kKeepBytes;) {
                 if (idle_[i].device != device) { ++i; continue; }
                 held -= idle_[i].bytes;
-                out.push_back(idle_[i].p);
-                idle_.erase(idle_.begin() + (long)i);
+                out[n_out++] = remove(i);
             }
-            idle_.push_back({p, bytes, device});
+            if (n_ == kMaxIdle) out[n_out++] = remove(0);
+            idle_[n_++] = {p, bytes, device};
         }
-        for (void* q : out) (void)hipFree(q);
+        for (int i = 0; i < n_out; ++i) (void)hipFree(out[i].p);
     }
-    void release() {
-        std::vector<Block> out;
-        { std::lock_guard<std::mutex> lock(mu_); out.swap(idle_); }
-        for (const Block& b : out) (void)hipFree(b.p);
+    void release() noexcept {
+        Block out[kMaxIdle];
+        int n_out = 0;
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            while (n_ > 0) out[n_out++] = remove(n_ - 1);
+        }
+        for (int i = 0; i < n_out; ++i) (void)hipFree(out[i].p);
     }
 };
 
@@ -230,7 +248,7 @@ void release_conversion_memory() { KeptMemory::get().release(); }
 extern "C" {
 
 void tq_quantizer_release_workspaces(void) {
-    try { KeptMemory::get().release(); } catch (...) { set_error("tq_quantizer_release_workspaces: exception"); }
+    try { tq::release_conversion_memory(); } catch (...) { set_error("tq_quantizer_release_workspaces: exception"); }
 }
 
 int tq_generate_codebook(int bits, float* centroids, float* boundaries) {
