@@ -136,17 +136,30 @@ void no_host_memory() {
     expect(dev.live == 0, "all device memory is given back", dev.live);
 }
 
+// No room for the workspace of the fit: the pass per step needs next to nothing beside the samples.
+void fit_without_workspace() {
+    dev.size = 4 * kN + (4 << 20);                         // the rotated samples and small tables
+    expect(fit() == 0, "the fit falls back to a pass per step");
+    expect(lloyd_passes == 2 && fit_calls.empty(), "both codebooks were fitted that way", lloyd_passes);
+    // ... and where the larger workspace does not fit after the smaller one did
+    lloyd_passes = 0;
+    fit_outcome = kNeedsAll;
+    dev.size = 4 * kN + 4 * kN + (6 << 20);
+    expect(fit() == 0, "the fit falls back after the first workspace");
+    expect(lloyd_passes == 2 && fit_calls.size() == 1, "both codebooks were fitted that way", lloyd_passes);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-    const struct { const char* name; void (*run)(); } checks[] = {{"no_host_memory", no_host_memory}};
+    const struct { const char* name; void (*run)(); } checks[] = {{"no_host_memory", no_host_memory},
+                                                                    {"fit_without_workspace", fit_without_workspace}};
     for (const auto& c : checks)
         if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
             c.run();
             if (!failures) std::printf("ok\n");
             return failures ? 1 : 0;
         }
-    (void)&fit;
     std::fprintf(stderr, "usage: conversion_memory <check>\n");
     return 2;
 }

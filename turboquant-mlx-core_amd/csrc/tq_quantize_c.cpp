@@ -83,7 +83,9 @@ public:
         if (e != hipErrorOutOfMemory) return e;
         release();
         (void)hipGetLastError();
-        return hipMalloc(p, *got);
+        e = hipMalloc(p, *got);
+        if (e != hipSuccess) (void)hipGetLastError();      // (reported here; the launches that follow ask for the last error too)
+        return e;
     }
     // The calls work on the null stream; nothing of it may still run when another call gets the block.
     void give(void* p, size_t bytes, int device) noexcept {
@@ -128,6 +130,7 @@ struct DevBuf {
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
     ~DevBuf() { if (p) KeptMemory::get().give(p, bytes, device); }
+    void drop() { if (p) (void)hipFree(p); p = nullptr; }  // back to the device instead of the kept blocks
     bool alloc(size_t n, const char* what) { return hip_ok(KeptMemory::get().take(n, &p, &bytes, &device), what); }
     template <typename T> T* as() { return static_cast<T*>(p); }
 };
@@ -157,7 +160,8 @@ void fill_tables(const float* cbp, int np, const float* cbr, int nr, float* t) {
 }
 
 // generate_codebook_from_data_cpu (src/codebook.cpp:99-143), one pass over all samples per step: samples that are not
-// all finite, or more than positions of 32 bits can number (fit_codebooks takes the rest).
+// all finite, more than positions of 32 bits can number, or no memory for the workspace of the fit (fit_codebooks takes
+// the rest).
 bool lloyd_max(const float* samples_dev, size_t n, int bits, int iterations, bool subtract,
                const float* gcent_dev, const float* gbounds_dev, int ngc, float* centroids_out) {
     float cent[32], bounds[32];
@@ -212,10 +216,10 @@ bool fit_codebooks(const float* samples_dev, size_t n, int primary_bits, int res
         }
         DevBuf res;
         tq::FitResult r{};
-        if (!res.alloc(sizeof(r), "hipMalloc(fit result)")) return false;
+        if (!res.alloc(sizeof(r), "hipMalloc(fit result)")) return false;      // (the passes need as much)
         for (bool everything = !tq::fit_predicts(n);; everything = true) {
             DevBuf work;
-            if (!work.alloc(tq::fit_workspace_bytes(n, problems, everything), "hipMalloc(fit)")) return false;
+            if (!work.alloc(tq::fit_workspace_bytes(n, problems, everything), "hipMalloc(fit)")) break;    // (the passes below need none)
             // (a round that misses costs what one that does not costs; data on which a fifth is needed is left to the
             // sort of everything)
             bool missed = true;
@@ -229,7 +233,7 @@ bool fit_codebooks(const float* samples_dev, size_t n, int primary_bits, int res
             }
             if (r.bad) break;
             if (missed && everything) { set_error("tq_fit_layer_codebooks: cells do not cover the samples"); return false; }
-            if (missed) continue;
+            if (missed) { work.drop(); continue; }         // (room for the larger one)
             std::memcpy(cbp_out, r.cent[0], cb.nc[0] * sizeof(float));
             if (problems == 2) std::memcpy(cbr_out, r.cent[1], cb.nc[1] * sizeof(float));
             return true;
