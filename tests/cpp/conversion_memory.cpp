@@ -149,11 +149,22 @@ void fit_without_workspace() {
     expect(lloyd_passes == 2 && fit_calls.size() == 1, "both codebooks were fitted that way", lloyd_passes);
 }
 
+// One codebook: what the device holds for the second is nobody's.
+void one_codebook_that_misses() {
+    std::vector<float> d(kN, 0.5f);
+    float c[16];
+    fit_outcome = kMissesOnce;
+    expect(tq_generate_codebook_from_data_host(d.data(), kN, 4, 100, c, nullptr) == 16, "the fit ends");
+    expect(fit_calls.size() == 2 && !fit_calls[1].first_round && !fit_calls[1].everything,
+           "a fit that missed goes on with a new expectation", fit_calls.size());
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const struct { const char* name; void (*run)(); } checks[] = {{"no_host_memory", no_host_memory},
-                                                                    {"fit_without_workspace", fit_without_workspace}};
+                                                                    {"fit_without_workspace", fit_without_workspace},
+                                                                    {"one_codebook_that_misses", one_codebook_that_misses}};
     for (const auto& c : checks)
         if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
             c.run();

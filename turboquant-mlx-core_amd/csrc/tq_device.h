@@ -140,7 +140,7 @@ hipError_t launch_lloyd_pass(const float* data, size_t n, const float* bounds_de
 // numbers of ordinary size; nothing was fitted (launch_lloyd_pass takes those).  state->missed[p]: the boundaries of
 // codebook p left the cells whose samples were kept, after state->steps[p] steps: call again with first_round == false
 // and the same workspace (another expectation, from there on), or with everything == true, which cannot miss and
-// needs a larger workspace of its own (first_round == true again).
+// needs a larger workspace of its own (first_round == true again).  With one problem the second's fields are not written.
 struct FitCodebooks { int nc[2]; float init[2][32]; };
 struct FitResult { float cent[2][32]; int steps[2]; int bad; int missed[2]; unsigned kept[2]; };
 bool fit_supported(size_t n);

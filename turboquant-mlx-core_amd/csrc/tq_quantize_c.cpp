@@ -229,7 +229,8 @@ bool fit_codebooks(const float* samples_dev, size_t n, int primary_bits, int res
                     !hip_ok(hipMemcpy(&r, res.p, sizeof(r), hipMemcpyDeviceToHost), "copy centroids"))
                     return false;
                 missed = r.missed[0] || (problems == 2 && r.missed[1]);
-                if (missed && (size_t)r.kept[0] + r.kept[1] > n / 2) break;      // more than the workspace holds
+                const size_t kept = (size_t)r.kept[0] + (problems == 2 ? r.kept[1] : 0);
+                if (missed && kept > n / 2) break;         // more than the workspace holds
             }
             if (r.bad) break;
             if (missed && everything) { set_error("tq_fit_layer_codebooks: cells do not cover the samples"); return false; }
