@@ -104,6 +104,7 @@ hipError_t launch_fit(const float*, size_t n, int problems, const float*, int, c
     for (int p = 0; p < problems; ++p) {
         std::memcpy(state->cent[p], cb.init[p], sizeof(cb.init[p]));
         state->steps[p] = iterations;
+        state->coarse[p] = 0;
         state->missed[p] = fit_outcome == kMissesOnce ? fit_calls.size() == 1 : fit_outcome == kNeedsAll && !everything;
         state->kept[p] = (unsigned)(fit_outcome == kNeedsAll ? n : n / 8);
     }

@@ -123,6 +123,23 @@ def test_codebook_fit_on_sorted_cells_matches_oracle(tq, oracle, data, bits):
     assert np.abs(got[:n] - want[:n]).max() <= 1e-6 * max(1.0, np.abs(d).max())
 
 
+@pytest.mark.parametrize("sigma", [1e-5, 1e-3, 0.3])
+@pytest.mark.parametrize("n", [50_003, (1 << 22) + 5])
+def test_codebook_fit_of_samples_small_beside_the_largest(tq, oracle, sigma, n):
+    """One sample of 200 among small ones: centroids hold fp32 precision relative to themselves.  Both sides add in 53 bits
+    and more and round a centroid once (2^-24), and a last bit may shift the next step's boundaries: 2^-21 of each."""
+    import ctypes as C
+    f32p = C.POINTER(C.c_float)
+    d = (np.random.default_rng(7).standard_normal(n) * sigma).astype(np.float32)
+    d[n // 3] = 200.0
+    got, want, bounds = np.empty(32, np.float32), np.empty(32, np.float32), np.empty(32, np.float32)
+    fit = tq.lib().tq_generate_codebook_from_data_host
+    fit.argtypes = [f32p, C.c_size_t, C.c_int, C.c_int, f32p, f32p]
+    assert fit(d.ctypes.data_as(f32p), n, 4, 100, got.ctypes.data_as(f32p), None) == 16, tq.last_error()
+    oracle.lib().tqo_lloyd_max(d.ctypes.data_as(f32p), n, 4, 100, want.ctypes.data_as(f32p), bounds.ctypes.data_as(f32p))
+    assert (np.abs(got[:16] - want[:16]) <= np.abs(want[:16]) * 2.0 ** -21).all(), np.abs(got[:16] / want[:16] - 1).max()
+
+
 def test_layer_fit_above_the_sorting_threshold_matches_oracle(tq, oracle):
     """Both codebooks of a layer of more than 2^22 weights: the residual's boundaries start far outside its samples."""
     w = (np.random.default_rng(4).standard_normal((2051, 2048)) * 0.02).astype(np.float32)

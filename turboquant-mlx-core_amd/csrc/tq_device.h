@@ -137,12 +137,13 @@ hipError_t launch_lloyd_pass(const float* data, size_t n, const float* bounds_de
 
 // Lloyd-Max fits (tq_fit.hip): codebook 0 on the samples, codebook 1 (problems == 2) on their residuals against the
 // global codebook gtab_dev ([0..31] centroids, [32..62] boundaries).  state->bad: the samples are not all finite
-// numbers of ordinary size; nothing was fitted (launch_lloyd_pass takes those).  state->missed[p]: the boundaries of
+// numbers of ordinary size; nothing was fitted (launch_lloyd_pass takes those).  state->coarse[p]: samples of codebook p are
+// too small beside the largest for the units of its sums; the fit was given up (the same).  state->missed[p]: the boundaries of
 // codebook p left the cells whose samples were kept, after state->steps[p] steps: call again with first_round == false
 // and the same workspace (another expectation, from there on), or with everything == true, which cannot miss and
 // needs a larger workspace of its own (first_round == true again).  With one problem the second's fields are not written.
 struct FitCodebooks { int nc[2]; float init[2][32]; };
-struct FitResult { float cent[2][32]; int steps[2]; int bad; int missed[2]; unsigned kept[2]; };
+struct FitResult { float cent[2][32]; int steps[2]; int bad; int coarse[2]; int missed[2]; unsigned kept[2]; };
 bool fit_supported(size_t n);
 bool fit_predicts(size_t n);         // large enough that keeping only the expected cells pays
 size_t fit_workspace_bytes(size_t n, int problems, bool everything);

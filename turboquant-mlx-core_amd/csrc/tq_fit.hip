@@ -18,9 +18,11 @@
 //                           own part that compare below it
 //
 // Cells are a monotone function of the value (about 10 bits of mantissa), so a boundary splits one cell only and bins
-// are exactly those of the comparison `boundary < value`.  Sums are integers (every sample is a multiple of 2^-38 of
-// the scale, values below 2^-14 of it rounded to one), so they are exact whatever the order the samples arrive in
-// and are rounded once, where the reference adds doubles one after the other.
+// are exactly those of the comparison `boundary < value`.  Sums are integers in units of 2^-38 of the scale, exact whatever
+// the order the samples arrive in and rounded once, where the reference adds doubles one after the other.  Samples from
+// 2^-15 of the scale on are whole numbers of units; those below lose what is smaller than one.  Where that could
+// reach a quarter of the rounding of a centroid (samples that are tiny beside the largest: no rotated weight does
+// that) the fit says so and is left to the pass per step.
 //
 // 18944 x 3584 (68 M samples, 2 x 100 steps).  One pass over all samples per step took 230 ms, 1.1 ms each (thread-private
 // bins in 96 KB of LDS, one wave per SIMD) and a copy of the partial sums to the host; the kernels here take 1.13 ms:
@@ -37,7 +39,8 @@ constexpr int kFitLin = 1024;                         // cells of [0, 2^-6) of t
 constexpr int kFitHalf = kFitLin * 7;                 // ... and 1024 per octave from 2^-6 to 1
 constexpr int kFitCells = 2 * kFitHalf;               // negative values mirrored below
 constexpr int kFitThreads = 1024;
-constexpr int kFitMaxExp = 8;                         // units stay at or below 2^-30, far below an fp32 centroid's last bit
+constexpr int kFitMaxExp = 8;                         // of the scale: the pass per step takes samples of 2^8 and more
+constexpr int kFitCut = 2;                            // cells on either side of zero whose samples may be no whole number of units
 constexpr uint32_t kFitLinEnd = 0x3c800000u;          // 2^-6
 constexpr int kFitMaxTile = 1 << 19;                  // samples per tile: offset sums (22 bits each) stay below 2^41
 
@@ -535,7 +538,7 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_iterate_kernel(const FitPa
     __shared__ float cent[32];
     __shared__ unsigned long long left_n[33];
     __shared__ i128 left_q[33];
-    __shared__ int stop, missed;
+    __shared__ int stop, missed, coarse;
     const int p = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nc = cb.nc[p];
     const bool bad = P->bad != 0;
@@ -543,7 +546,8 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_iterate_kernel(const FitPa
         if (p == 0) out->bad = bad ? 1 : 0;
         out->kept[p] = bad ? 0 : kept[p];
         out->missed[p] = !bad && !fit_room(kept, gridDim.x, capacity) ? 1 : 0;
-        stop = 0; missed = 0;
+        out->coarse[p] = 0;
+        stop = 0; missed = 0; coarse = 0;
     }
     if (bad || !fit_room(kept, gridDim.x, capacity)) return;
     if (tid < nc) cent[tid] = out->cent[p][tid];
@@ -605,6 +609,10 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_iterate_kernel(const FitPa
                 if (c > 0) {                                                         // src/codebook.cpp:124-129
                     const double s = i128_to_double(left_q[lane + 1] - left_q[lane]) * unit;
                     const float nv = (float)(s / (double)c);
+                    // each of the bin's samples around zero may have lost up to one unit
+                    const unsigned long long from = max(left_n[lane], (unsigned long long)start[kFitHalf - kFitCut]);
+                    const unsigned long long to = min(left_n[lane + 1], (unsigned long long)start[kFitHalf + kFitCut]);
+                    if (from < to && (double)(to - from) * unit > (double)fabsf(nv) * 0x1p-26 * (double)c) coarse = 1;
                     shift = fabsf(nv - cent[lane]);
                     cent[lane] = nv;
                 }
@@ -613,10 +621,11 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_iterate_kernel(const FitPa
             if (lane == 0) stop = shift < 1e-6f ? 1 : 0;                             // src/codebook.cpp:132
         }
         __syncthreads();
-        if (stop) break;
+        if (stop || coarse) break;
     }
     if (tid == 0) {
         out->missed[p] = missed;
+        out->coarse[p] = coarse;
         out->steps[p] = stop ? iterations : iter;
     }
     if (tid < nc) out->cent[p][tid] = cent[tid];

@@ -160,7 +160,7 @@ void fill_tables(const float* cbp, int np, const float* cbr, int nr, float* t) {
 }
 
 // generate_codebook_from_data_cpu (src/codebook.cpp:99-143), one pass over all samples per step: samples that are not
-// all finite, more than positions of 32 bits can number, or no memory for the workspace of the fit (fit_codebooks takes
+// all finite, differ too much in size or are more than positions of 32 bits can number, or no memory for the workspace of the fit (fit_codebooks takes
 // the rest).
 bool lloyd_max(const float* samples_dev, size_t n, int bits, int iterations, bool subtract,
                const float* gcent_dev, const float* gbounds_dev, int ngc, float* centroids_out) {
@@ -222,17 +222,18 @@ bool fit_codebooks(const float* samples_dev, size_t n, int primary_bits, int res
             if (!work.alloc(tq::fit_workspace_bytes(n, problems, everything), "hipMalloc(fit)")) break;    // (the passes below need none)
             // (a round that misses costs what one that does not costs; data on which a fifth is needed is left to the
             // sort of everything)
-            bool missed = true;
-            for (int round = 0; missed && !r.bad && round < (everything ? 1 : 4); ++round) {
+            bool missed = true, passes = false;
+            for (int round = 0; missed && !passes && round < (everything ? 1 : 4); ++round) {
                 if (!hip_ok(tq::launch_fit(samples_dev, n, problems, gtab_dev, ngc, cb, iterations, round == 0, everything, work.p,
                                            res.as<tq::FitResult>(), nullptr), "fit launch") ||
                     !hip_ok(hipMemcpy(&r, res.p, sizeof(r), hipMemcpyDeviceToHost), "copy centroids"))
                     return false;
                 missed = r.missed[0] || (problems == 2 && r.missed[1]);
+                passes = r.bad || r.coarse[0] || (problems == 2 && r.coarse[1]);
                 const size_t kept = (size_t)r.kept[0] + (problems == 2 ? r.kept[1] : 0);
                 if (missed && kept > n / 2) break;         // more than the workspace holds
             }
-            if (r.bad) break;
+            if (passes) break;
             if (missed && everything) { set_error("tq_fit_layer_codebooks: cells do not cover the samples"); return false; }
             if (missed) { work.drop(); continue; }         // (room for the larger one)
             std::memcpy(cbp_out, r.cent[0], cb.nc[0] * sizeof(float));
