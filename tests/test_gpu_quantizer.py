@@ -149,6 +149,24 @@ def test_layer_fit_above_the_sorting_threshold_matches_oracle(tq, oracle):
     assert np.abs(got_r.centroids - want_r.centroids).max() < 1e-6
 
 
+@pytest.mark.parametrize("shape", [(64, 512), (2051, 2048)])
+def test_layer_fit_against_an_unsorted_codebook(tq, oracle, shape):
+    """A sample's bin is the number of boundaries below it, also where the global codebook is in no order; a residual may then
+    be larger than any centroid's distance from its own boundaries."""
+    w = (np.random.default_rng(4).standard_normal(shape) * 0.02).astype(np.float32)
+    c = oracle.generate_codebook(4).centroids.copy()
+    c[7] = 100.0
+    g = oracle.Codebook(c, 4)
+    norms = np.sqrt((w * w).astype(np.float64).sum(1).astype(np.float32))
+    v = oracle.wht_forward(w / norms[:, None], oracle.derive_seed(w, 0), 512) * np.float32(np.sqrt(np.float32(shape[1])))
+    bin_of = np.zeros(v.shape, np.int8)
+    for b in g.boundaries:
+        bin_of += b < v
+    want = oracle.generate_codebook_from_data(v - c[bin_of], 4).centroids
+    _, got = tq.fit_layer_codebooks(w, 512, global_primary=g)
+    assert (np.abs(got.centroids - want) <= 1e-6 * np.maximum(1.0, np.abs(want))).all()
+
+
 def test_quantizer_error_conventions(tq):
     with pytest.raises(ValueError):
         tq.generate_codebook(6)

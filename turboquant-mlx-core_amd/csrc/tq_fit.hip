@@ -129,7 +129,7 @@ __device__ void fit_scale(float biggest, FitParams* P, int p) {
 }
 
 // One workgroup: the largest |sample| and the scales.  A residual is at most half a gap of the global codebook, or
-// what lies beyond its last centroid.
+// what lies beyond its last centroid, where that codebook is sorted.
 __global__ __launch_bounds__(256) void tq_fit_absmax_fold_kernel(const uint32_t* __restrict__ part, int parts, FitProblem fp,
                                                                  int problems, FitParams* __restrict__ P, FitCodebooks cb,
                                                                  FitResult* __restrict__ state) {
@@ -151,7 +151,16 @@ __global__ __launch_bounds__(256) void tq_fit_absmax_fold_kernel(const uint32_t*
             const float* c = fp.gtab[p];
             const float* g = c + 32;
             b = fmaxf(fabsf(big - c[fp.ngc - 1]), fabsf(-big - c[0]));
-            for (int k = 0; k + 1 < fp.ngc; ++k) b = fmaxf(b, fmaxf(fabsf(g[k] - c[k]), fabsf(c[k + 1] - g[k])));
+            bool sorted = true;
+            float far = 0.0f;
+            for (int k = 0; k < fp.ngc; ++k) {
+                if (!(fabsf(c[k]) < 1e30f)) P->bad = 1;           // infinities and NaN: no residual is a number
+                far = fmaxf(far, fabsf(c[k]));
+                if (k + 1 == fp.ngc) break;
+                b = fmaxf(b, fmaxf(fabsf(g[k] - c[k]), fabsf(c[k + 1] - g[k])));
+                if (!(c[k] <= c[k + 1])) sorted = false;
+            }
+            if (!sorted) b = big + far;                           // (a bin may have any centroid)
             b *= 1.0001f;
             if (!(m < 0x7f800000u)) P->bad = 1;
         }
