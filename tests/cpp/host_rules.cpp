@@ -5,6 +5,7 @@
 #include <cstring>
 
 #include "tq_device.h"
+#include "tq_prefill_common.h"
 
 namespace {
 
@@ -30,10 +31,29 @@ void fit_limit() {
     expect(lo + stride < (1ull << 32), "a stride beyond the last sample is still a 32-bit number", lo);
 }
 
+tq::LayerView layer(int mode, int in, int out) {
+    tq::LayerView v{};
+    v.mode = mode;
+    v.in_features = in; v.out_features = out;
+    v.block_size = 512;
+    v.fp16_centroids_ok = 1;
+    v.compose_ok = 1;
+    return v;
+}
+
+// Planes are composed where there are two of them; the modes without are refused whatever the view's fields say.
+void compose_modes() {
+    for (int mode = tq::kPrimaryOnly; mode <= tq::kDual5; ++mode) {
+        const bool two = mode == tq::kDual || mode == tq::kDual5 || mode == tq::kShared5;
+        const bool got = tq::prefill_compose_supported(layer(mode, 5120, 27648), 2048, 256, ~(size_t)0);
+        expect(got == two, "composed planes by mode", mode);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-    const struct { const char* name; void (*run)(); } checks[] = {{"fit_limit", fit_limit}};
+    const struct { const char* name; void (*run)(); } checks[] = {{"fit_limit", fit_limit}, {"compose_modes", compose_modes}};
     for (const auto& c : checks)
         if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
             c.run();

@@ -345,6 +345,7 @@ tq_linear_t create_impl(int in_features, int out_features,
         a.packed_residual = nullptr;
         a.tables = h->d_tables_plane[0];
         a.seed_residual = 0;
+        a.compose_ok = 0;
         tq::LayerView& b = h->plane_view[1];
         b = v;
         b.mode = tq::kPrimaryOnly;
@@ -354,6 +355,7 @@ tq_linear_t create_impl(int in_features, int out_features,
         b.tables = h->d_tables_plane[1];
         b.seed_primary = mode == tq::kDual5 ? seeds[1] : seeds[0];
         b.seed_residual = 0;
+        b.compose_ok = 0;
         h->has_plane_views = true;
     }
     return h;

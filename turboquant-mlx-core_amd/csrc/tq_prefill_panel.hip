@@ -810,7 +810,8 @@ ComposePlan compose_plan(const LayerView& L, int batch, int num_cus) {
 size_t prefill_compose_workspace_bytes(const LayerView& L, int batch, int num_cus) { return compose_plan(L, batch, num_cus).total_bytes; }
 
 bool prefill_compose_supported(const LayerView& L, int batch, int num_cus, size_t capacity) {
-    if (!L.compose_ok || batch < compose_min_rows(L)) return false;
+    if (!L.compose_ok || (L.mode != kDual && L.mode != kDual5 && L.mode != kShared5)) return false;
+    if (batch < compose_min_rows(L)) return false;
     if (!prefill_panel_supported(slab_view(L, L.out_features), batch, num_cus, capacity)) return false;
     return compose_plan(L, batch, num_cus).total_bytes <= capacity;
 }
