@@ -1,11 +1,13 @@
 // Dispatch rules and workspace sizes: host code of the library, run without a GPU.  One check per argument
 // (tests/test_host_rules.py); a check that fails prints what it found and ends with status 1.
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
 
 #include "tq_device.h"
 #include "tq_prefill_common.h"
+#include "turboquant_c/tq_quantizer.h"
 
 namespace {
 
@@ -37,7 +39,7 @@ tq::LayerView layer(int mode, int in, int out) {
     v.in_features = in; v.out_features = out;
     v.block_size = 512;
     v.fp16_centroids_ok = 1;
-    v.compose_ok = 1;
+    v.compose_scale = 0.75f;
     return v;
 }
 
@@ -50,10 +52,30 @@ void compose_modes() {
     }
 }
 
+// Planes are composed where the rounding of the sum to fp16 is no larger than that of the centroids: never where these are
+// fp16 numbers already (and in range), and the scale is a plain factor.
+void compose_precision() {
+    float analytic[32], exact[32], wide[32];
+    const int n = tq_generate_codebook(4, analytic, nullptr);
+    for (int i = 0; i < n; ++i) {
+        exact[i] = std::nearbyint(analytic[i] * 256.0f) / 256.0f;        // (fp16 holds them, and sums of two)
+        wide[i] = analytic[i] * 20000.0f;
+    }
+    const float s = tq::compose_scale(tq::kDual, 512, analytic, n, analytic, n);
+    expect(s > 0.5f && s <= 1.0f, "the analytic codebooks are composed", (unsigned long long)(s * 1000));
+    expect(tq::compose_scale(tq::kDual, 512, exact, n, exact, n) == 0.0f, "exact centroids are not", 0);
+    expect(tq::compose_scale(tq::kShared5, 512, exact, n, exact, n) > 0.0f, "but their sum in one rotation is as exact", 0);
+    expect(tq::compose_scale(tq::kDual, 512, wide, n, wide, n) == 0.0f, "nor sums beyond the range of fp16", 0);
+    expect(tq::compose_scale(tq::kDual, 1024, analytic, n, analytic, n) == 0.0f, "nor blocks of 1024", 0);
+    wide[3] = NAN;
+    expect(tq::compose_scale(tq::kDual, 512, wide, n, analytic, n) == 0.0f, "nor what is no number", 0);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-    const struct { const char* name; void (*run)(); } checks[] = {{"fit_limit", fit_limit}, {"compose_modes", compose_modes}};
+    const struct { const char* name; void (*run)(); } checks[] = {{"fit_limit", fit_limit}, {"compose_modes", compose_modes},
+                                                                    {"compose_precision", compose_precision}};
     for (const auto& c : checks)
         if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
             c.run();

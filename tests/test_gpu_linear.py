@@ -390,6 +390,29 @@ def test_prefill_composed_planes_match_dequant_matmul(tq, oracle, monkeypatch, m
     assert _rel(yb, want) < 5e-3
 
 
+@pytest.mark.parametrize("codebook", ["analytic", "fp16", "fitted"])
+def test_prefill_composed_planes_lose_no_precision(tq, oracle, codebook):
+    """Rows of one 1 each: what is rounded is the weights alone (1/16 per rotated value is exact).  513 rows, which may compose
+    the planes, against the same 512 rows, which never do; one per cent, for what decides takes the weights as normally distributed
+    and two rotations mix a particular residual more or less well.  Centroids that fp16 holds: exact but for fp32 sums of
+    256 terms."""
+    out, inf, bs = 8322, 768, 256
+    cb = {"analytic": [oracle.generate_codebook(4)] * 2, "fp16": [oracle.generate_codebook(4)] * 2}.get(codebook)
+    w = (np.random.default_rng(8).standard_normal((out, inf)) * 0.02).astype(np.float32)
+    if codebook == "fitted":
+        cb = oracle.fit_layer_codebooks(w, bs)
+    if codebook == "fp16":
+        cb = [oracle.Codebook(c.centroids.astype(np.float16).astype(np.float32), 4) for c in cb]
+    qw = oracle.quantize_weight(w, *cb, 4, 4, bs, False)
+    want = oracle.dequantize_weight_cpu(qw, *cb, bs).T[:512]
+    x = np.zeros((513, inf), np.float32)
+    x[np.arange(513), np.arange(513)] = 1.0
+    layer = tq.TurboQuantLinear(inf, out, qw, *cb, bs)
+    many, few = _rel(layer.forward(x)[:512], want), _rel(layer.forward(x[:512]), want)
+    layer.close()
+    assert many <= (2e-6 if codebook == "fp16" else 1.01 * few), (many, few)
+
+
 def test_prefill_composed_planes_in_slabs(tq, oracle):
     """A weight of more than one slab (160 MB of fp16): rows of the call agree with the one-row kernel on the same rows, in
     every slab's columns."""

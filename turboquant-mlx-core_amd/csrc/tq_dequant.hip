@@ -303,7 +303,8 @@ hipError_t launch_dequant(const LayerView& L, void* w, int w_dtype, hipStream_t 
 // Two planes with rotations of their own as ONE fp16 weight in the primary's rotation, for prefill of many rows:
 //   sum_k cP[k] x~p[k] + cR[k] x~r[k]  =  sum_k (cP + H (s_p s_r (.) H cR) / bs)[k] x~p[k],     x~ = H (s (.) x)
 // so that the contraction runs once instead of once per plane.  The sum is formed in fp32 and rounded to fp16 once; the
-// planes multiplied one after the other round each centroid by itself.  kShared5: both planes in one rotation, a plain sum.
+// planes multiplied one after the other round each centroid by itself (compose_scale() looks at which of the two is
+// closer).  kShared5: both planes in one rotation, a plain sum.
 // Rows [row0, row0 + rows) of the layer (row0 a multiple of 128), in the order in which tq_prefill_panel_kernel's threads
 // load them: [row / 128][K / 64][4 pieces of 8 columns][row % 128 / 32][half of the 64 columns][row % 32] x 16 bytes.
 // Bound by its vector instructions (28 per weight); 27648 x 5120 in 140 us, a sixth of the contraction it halves at 2048 rows.
@@ -318,7 +319,7 @@ __global__ __launch_bounds__(kDqWaves* kWave, 3) void tq_compose_kernel(LayerVie
     __shared__ float tab[64];
     __shared__ __align__(16) char exchange[rotate ? kDqWaves * kDqExchange : 16];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
-    if (threadIdx.x < 64) tab[threadIdx.x] = L.tables[threadIdx.x] * kComposeScale;
+    if (threadIdx.x < 64) tab[threadIdx.x] = L.tables[threadIdx.x] * L.compose_scale;
     __syncthreads();
     const char* const tab_p = reinterpret_cast<const char*>(tab);
     const char* const tab_r = reinterpret_cast<const char*>(tab + (bytes ? 32 : 16));
@@ -387,7 +388,7 @@ __global__ __launch_bounds__(kDqWaves* kWave, 3) void tq_compose_kernel(LayerVie
             f32x8_t f;
 #pragma unroll
             for (int j = 0; j < 8; ++j) f[j] = v[8 * i + j] + u[8 * i + j];
-            *reinterpret_cast<f16x8_t*>(dst + i * 4096) = __builtin_convertvector(f, f16x8_t);      // (in range: compose_ok)
+            *reinterpret_cast<f16x8_t*>(dst + i * 4096) = __builtin_convertvector(f, f16x8_t);      // (in range: compose_scale)
         }
     }
 }

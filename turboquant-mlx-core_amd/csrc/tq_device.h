@@ -39,7 +39,7 @@ struct LayerView {
     float inv_sqrt_bs;               // 1/sqrt(block_size), host computed
     int fp16_centroids_ok;           // every centroid fits fp16 with room to spare (the byte-pair tables of the
                                      // batch-1 kernel hold fp16 values); otherwise fp32 tables are used
-    int compose_ok;                  // two planes kept as such, and their sum in the primary's rotation fits fp16 (launch_compose)
+    float compose_scale;             // two planes kept as such: what their fp16 sum is multiplied by (launch_compose); 0: not composed
     float* xrot_work;                // scratch of 2 * in_features floats (rows wider than 16384 columns: the
                                      // batch-1 path rotates the activations once, in a kernel of its own), or NULL
 };
@@ -60,9 +60,7 @@ hipError_t launch_combine_planes5(const uint8_t* primary, const uint8_t* residua
                                   size_t residual_bytes, int n_primary, int n_residual, hipStream_t stream);
 hipError_t launch_dequant(const LayerView& L, void* w, int w_dtype, hipStream_t stream);
 // Rows [row0, row0 + rows) of a two-plane layer (kDual, kDual5, kShared5) as one fp16 weight in the primary's rotation,
-// times kComposeScale: weights are close to normally distributed with unit variance, and 0.78 puts the fewest of them where
-// a binade's spacing is coarse for its values (0.8 % less rounding error than 1).
-constexpr float kComposeScale = 0.78f;
+// times L.compose_scale.
 hipError_t launch_compose(const LayerView& L, int row0, int rows, void* out, hipStream_t stream);
 // Prefill (tq_prefill.hip): rotate the activations to fp16 in `workspace`, then dequant + MFMA GEMM.
 bool prefill_supported(const LayerView& L, int x_dtype, int batch);

@@ -318,9 +318,7 @@ tq_linear_t create_impl(int in_features, int out_features,
         for (int i = 0; i < np; ++i) big = std::fmax(big, std::fabs(cbp[i]));
         for (int i = 0; i < nr; ++i) big = std::fmax(big, std::fabs(cbr[i]));
         v.fp16_centroids_ok = (big < 30000.0f) ? 1 : 0;      // NaN compares false
-        // (the residual plane in the primary's rotation stays below sqrt(block) times its largest centroid)
-        v.compose_ok = block_size <= 512 && (mode == tq::kDual || mode == tq::kDual5 || (mode == tq::kShared5 && !fused5)) &&
-                       big * (1.0f + std::sqrt((float)block_size)) < 60000.0f;
+        v.compose_scale = fused5 ? 0.0f : tq::compose_scale(mode, block_size, cbp, np, cbr, nr);
     }
     if (fused5) {
         h->fwd_view = v;
@@ -345,7 +343,7 @@ tq_linear_t create_impl(int in_features, int out_features,
         a.packed_residual = nullptr;
         a.tables = h->d_tables_plane[0];
         a.seed_residual = 0;
-        a.compose_ok = 0;
+        a.compose_scale = 0.0f;
         tq::LayerView& b = h->plane_view[1];
         b = v;
         b.mode = tq::kPrimaryOnly;
@@ -355,7 +353,7 @@ tq_linear_t create_impl(int in_features, int out_features,
         b.tables = h->d_tables_plane[1];
         b.seed_primary = mode == tq::kDual5 ? seeds[1] : seeds[0];
         b.seed_residual = 0;
-        b.compose_ok = 0;
+        b.compose_scale = 0.0f;
         h->has_plane_views = true;
     }
     return h;

@@ -41,6 +41,9 @@ hipError_t launch_prefill_panel(const LayerView& L, const void* x, int x_dtype, 
 // fp16 weight first (tq_prefill_panel.hip).  Workspace: fragment images, parts, a slab of the weight.
 // (from the second panel of 512 rows on; 5-bit layers, whose planes are separate calls and a sum otherwise, in the first too)
 inline int compose_min_rows(const LayerView& L) { return L.mode == kDual ? kPanelM + 1 : 385; }
+// What the sum of the planes is multiplied by before it is rounded to fp16, or 0: multiplying plane by plane is the more
+// precise, or the sum may leave fp16's range.  Codebooks as the layer was created with.
+float compose_scale(int mode, uint32_t block_size, const float* cbp, int np, const float* cbr, int nr);
 bool prefill_compose_supported(const LayerView& L, int batch, int num_cus, size_t capacity);
 size_t prefill_compose_workspace_bytes(const LayerView& L, int batch, int num_cus);
 hipError_t launch_prefill_compose(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,

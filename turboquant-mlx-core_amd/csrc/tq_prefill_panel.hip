@@ -26,6 +26,8 @@
 // per-row kernel).
 #include "tq_prefill_common.h"
 
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 // Measurement builds (make ablations; bench.py --prefill-ablations): -DTQ_PANEL_ABLATE=<mask> compiles parts of the
@@ -768,7 +770,7 @@ hipError_t launch_prefill_panel(const LayerView& L, const void* x, int x_dtype, 
 // 1119 -> 872, 5120 x 5120 at 2048 rows 252 -> 175, 3584 x 18944 at 700 rows 320 -> 256, 2048 x 10240 at 1024 rows 111 -> 97; in
 // one panel 5120 x 27648 at 512 rows 264, 393 composed (not taken), but the 5-bit layers, which are two calls and a sum
 // otherwise, gain there too: 3072 x 17000 at 512 rows 179 -> 141, 2048 x 8704 at 668 rows 140 -> 89, 5120 x 27648 at 1024 rows
-// 661 -> 489.  Against 64 bits the error is that of the two contractions (2.93e-4).  The slab bounds the workspace: the
+// 661 -> 489.  Against 64 bits the error is no larger than that of the two contractions (compose_scale).  The slab bounds the workspace: the
 // whole weight in fp16 would be twice the layer.
 // ---------------------------------------------------------------------------
 namespace {
@@ -807,10 +809,84 @@ ComposePlan compose_plan(const LayerView& L, int batch, int num_cus) {
 
 }  // namespace
 
+// A layer's weights (rows normalised, rotated) are close to normally distributed with unit variance.  From that and the
+// codebooks: the mean square of what rounding the centroids to fp16 changes, and of what rounding the sum does, which has
+// no centroids of its own to be lucky or unlucky with but a binade of fp16 for each weight; a scale moves the weights
+// among the binades.  Root mean squares, in 1e-4: the analytic codebooks 2.08 by planes and 2.06 composed at 0.878 (2.12 at
+// 0.78), fitted ones 1.49 to 2.37 by planes and 2.03 to 2.05 composed; 5-bit 2.13 to 2.26 and 2.04 to 2.08, with one rotation
+// for both planes (the sums are then a set of 512 values) 1.79 to 1.93 composed.  On weights quantized with them the
+// analytic pair has 2.06 to 2.07 and 2.05 to 2.08 (two rotations mix a residual more or less well).  The sum is taken where
+// it is no worse.  50 to 150 us on the host, once per layer.
+float compose_scale(int mode, uint32_t block_size, const float* cbp, int np, const float* cbr, int nr) {
+    if ((mode != kDual && mode != kDual5 && mode != kShared5) || block_size > 512) return 0.0f;
+    const int n_p = std::min(np, mode == kDual ? 16 : 32);
+    float big = 0.0f;
+    for (int i = 0; i < np; ++i) big = std::max(big, std::fabs(cbp[i]));
+    for (int i = 0; i < nr; ++i) big = std::max(big, std::fabs(cbr[i]));
+    // (the residual plane in the primary's rotation stays below sqrt(block) times its largest centroid)
+    if (!(big * (1.0f + std::sqrt((float)block_size)) < 60000.0f)) return 0.0f;
+    constexpr int kGrid = 192, kScales = 16;
+    double weight[kGrid], at[kGrid], total = 0.0;
+    for (int m = 0; m < kGrid; ++m) {
+        at[m] = (m + 0.5) / 16.0 - 6.0;
+        total += weight[m] = std::exp(-0.5 * at[m] * at[m]);
+    }
+    auto bin = [](const float* c, int n, double v) {
+        int k = 0;
+        for (int i = 0; i + 1 < n; ++i) k += 0.5 * ((double)c[i] + c[i + 1]) < v ? 1 : 0;
+        return k;
+    };
+    // A step of fp16 at v (2^-24 below 2^-14), and what rounding to the nearest loses.
+    auto step_at = [](float v) {
+        const uint32_t b = __builtin_bit_cast(uint32_t, v) & 0x7f800000u;
+        return __builtin_bit_cast(float, std::max(b, 113u << 23)) * 0x1p-10f;
+    };
+    auto lost = [&](double v) { const double s = step_at((float)v); return v - std::nearbyint(v / s) * s; };
+    double p[32] = {0}, q[16] = {0}, left = 0.0;           // how often a centroid is used; the residual's mean square
+    for (int m = 0; m < kGrid; ++m) {
+        weight[m] /= total;
+        const int i = bin(cbp, n_p, at[m]);
+        p[i] += weight[m];
+        left += weight[m] * (at[m] - cbp[i]) * (at[m] - cbp[i]);
+    }
+    double planes = 0.0, sum[kScales] = {0}, scale[kScales];
+    for (int k = 0; k < kScales; ++k) scale[k] = (double)(float)std::exp2(-k / (double)kScales);
+    if (mode == kShared5) {
+        for (int m = 0; m < kGrid; ++m) {
+            const int i = bin(cbp, n_p, at[m]), j = bin(cbr, nr, at[m] - cbp[i]);
+            const double v = (double)cbp[i] + cbr[j], e = lost(cbp[i]) + lost(cbr[j]);
+            planes += weight[m] * e * e;
+            for (int k = 0; k < kScales; ++k) {
+                const double d = lost(v * scale[k]) / scale[k];
+                sum[k] += weight[m] * d * d;
+            }
+        }
+    } else {
+        double power = 0.0;                                // of the residual plane, normally distributed in the other rotation
+        for (int m = 0; m < kGrid; ++m) q[bin(cbr, nr, at[m] * std::sqrt(left))] += weight[m];
+        for (int i = 0; i < n_p; ++i) planes += p[i] * lost(cbp[i]) * lost(cbp[i]);
+        for (int j = 0; j < nr; ++j) { planes += q[j] * lost(cbr[j]) * lost(cbr[j]); power += q[j] * cbr[j] * cbr[j]; }
+        for (int i = 0; i < n_p; ++i)
+            for (int m = 0; m < kGrid; ++m) {
+                const float v = (float)(cbp[i] + std::sqrt(power) * at[m]);
+                const double w = p[i] * weight[m] / 12.0;  // (a step's square / 12 on average)
+                for (int k = 0; k < kScales; ++k) {
+                    const double step = step_at(v * (float)scale[k]);
+                    sum[k] += w * step * step;
+                }
+            }
+        for (int k = 0; k < kScales; ++k) sum[k] /= scale[k] * scale[k];
+    }
+    int best = 0;
+    for (int k = 1; k < kScales; ++k)
+        if (sum[k] < sum[best]) best = k;
+    return sum[best] <= planes ? (float)scale[best] : 0.0f;
+}
+
 size_t prefill_compose_workspace_bytes(const LayerView& L, int batch, int num_cus) { return compose_plan(L, batch, num_cus).total_bytes; }
 
 bool prefill_compose_supported(const LayerView& L, int batch, int num_cus, size_t capacity) {
-    if (!L.compose_ok || (L.mode != kDual && L.mode != kDual5 && L.mode != kShared5)) return false;
+    if (!(L.compose_scale > 0.0f) || (L.mode != kDual && L.mode != kDual5 && L.mode != kShared5)) return false;
     if (batch < compose_min_rows(L)) return false;
     if (!prefill_panel_supported(slab_view(L, L.out_features), batch, num_cus, capacity)) return false;
     return compose_plan(L, batch, num_cus).total_bytes <= capacity;
@@ -837,7 +913,7 @@ hipError_t launch_prefill_compose(const LayerView& L, const void* x, int x_dtype
         a.n_tiles = (rows + kPN - 1) / kPN;
         a.n_per_xcd = (a.n_tiles + 7) / 8;
         a.n_first = row0;
-        a.out_scale = L.inv_scale / kComposeScale;
+        a.out_scale = L.inv_scale / L.compose_scale;
         a.tail_tiles = q.tail_tiles; a.parts = q.parts; a.part_subs = q.part_subs;
         a.first_part_wg = q.tail_tiles == a.panels * a.n_tiles ? 0 : 8 * a.n_per_xcd * a.panels;
         a.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + q.xt_bytes);
