@@ -71,11 +71,51 @@ void compose_precision() {
     expect(tq::compose_scale(tq::kDual, 512, wide, n, analytic, n) == 0.0f, "nor what is no number", 0);
 }
 
+// The workspace of composed planes: beside one rotation's images no more than the layer's planes, or 67 MB (a K part of a tile
+// per CU), or what the call takes plane by plane; within the capacity where one is given, and the parts before the slab.
+void compose_workspace() {
+    const int shapes[][2] = {{5120, 27648}, {27648, 5120}, {5120, 5120}, {3584, 18944}, {2048, 10240}, {4096, 14336}, {2048, 151936},
+                             {8192, 28672}, {1280, 8200}, {768, 8322}};
+    const int modes[] = {tq::kDual, tq::kDual5, tq::kShared5};
+    int composed = 0;
+    for (const auto& s : shapes)
+        for (int mode : modes)
+            for (int rows : {385, 512, 513, 700, 1024, 1025, 1536, 2048, 4096, 8192}) {
+                tq::LayerView v = layer(mode, s[0], s[1]);
+                v.block_size = 256;
+                const size_t all = ~(size_t)0;
+                if (!tq::prefill_compose_supported(v, rows, 256, all)) continue;
+                ++composed;
+                tq::LayerView one = v;
+                one.mode = mode == tq::kDual ? tq::kDual : tq::kPrimaryOnly;
+                const size_t images = ((size_t)rows + 511) / 512 * 512 * s[0] * 2, tiles = ((size_t)s[1] + 127) / 128;
+                const size_t planes = tiles * 128 * s[0] / 2 * (mode == tq::kDual ? 2 : 3), part = (size_t)256 * 512 * 128 * 4;
+                const size_t by_plane = tq::prefill_panel_workspace_bytes(one, rows, 256, all);
+                const size_t most = images + 512 + (planes > part ? planes : part);
+                const size_t need = tq::prefill_compose_workspace_bytes(v, rows, 256, all);
+                expect(need > images && need <= (by_plane > most ? by_plane : most), "workspace of composed planes", need);
+                for (size_t cap : {need, need - 1, (size_t)32 << 20})
+                    if (tq::prefill_compose_supported(v, rows, 256, cap))
+                        expect(tq::prefill_compose_workspace_bytes(v, rows, 256, cap) <= cap, "a capacity is kept to", cap);
+            }
+    expect(composed > 60, "most of these calls compose", composed);
+    // (the calls of the GPU tests of composed planes)
+    const int calls[][5] = {{tq::kDual, 8260, 1280, 256, 513}, {tq::kDual, 8322, 1792, 128, 600}, {tq::kDual, 8322, 1792, 256, 513},
+                            {tq::kDual, 6000, 1536, 512, 1030}, {tq::kDual5, 16500, 256, 32, 385}, {tq::kShared5, 16448, 512, 256, 400},
+                            {tq::kDual5, 8200, 1280, 256, 1024}, {tq::kDual, 33100, 2560, 512, 520}};
+    for (const auto& c : calls) {
+        tq::LayerView v = layer(c[0], c[2], c[1]);
+        v.block_size = c[3];
+        expect(tq::prefill_compose_supported(v, c[4], 256, ~(size_t)0), "a call that the GPU tests take to compose", c[1]);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const struct { const char* name; void (*run)(); } checks[] = {{"fit_limit", fit_limit}, {"compose_modes", compose_modes},
-                                                                    {"compose_precision", compose_precision}};
+                                                                    {"compose_precision", compose_precision},
+                                                                    {"compose_workspace", compose_workspace}};
     for (const auto& c : checks)
         if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
             c.run();

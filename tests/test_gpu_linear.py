@@ -366,9 +366,9 @@ def test_prefill_small_tiles_match_dequant_matmul(tq, oracle, mode, out, inf, bs
 
 
 # ------------------------------------------------------------------ prefill, two planes composed into one fp16 weight
-@pytest.mark.parametrize("mode,out,inf,bs,batch", [("dual", 8260, 256, 256, 513),       # half a 512-column segment; ragged last weight tile
-                                                   ("dual", 8322, 768, 128, 600),       # one segment and a half; out no multiple of 4
-                                                   ("dual", 6000, 512, 512, 1030),      # three panels, tail tiles in K ranges
+@pytest.mark.parametrize("mode,out,inf,bs,batch", [("dual", 8260, 1280, 256, 513),      # half a 512-column segment; ragged last weight tile
+                                                   ("dual", 8322, 1792, 128, 600),      # three segments and a half; out no multiple of 4
+                                                   ("dual", 6000, 1536, 512, 1030),     # three panels
                                                    ("5+3dual", 16500, 256, 32, 385),    # one panel; 5-bit primary in bytes
                                                    ("5+4shared", 16448, 512, 256, 400), # no rotation between the planes
                                                    ("5+4dual", 8200, 1280, 256, 1024)])
@@ -396,7 +396,7 @@ def test_prefill_composed_planes_lose_no_precision(tq, oracle, codebook):
     the planes, against the same 512 rows, which never do; one per cent, for what decides takes the weights as normally distributed
     and two rotations mix a particular residual more or less well.  Centroids that fp16 holds: exact but for fp32 sums of
     256 terms."""
-    out, inf, bs = 8322, 768, 256
+    out, inf, bs = 8322, 1792, 256
     cb = {"analytic": [oracle.generate_codebook(4)] * 2, "fp16": [oracle.generate_codebook(4)] * 2}.get(codebook)
     w = (np.random.default_rng(8).standard_normal((out, inf)) * 0.02).astype(np.float32)
     if codebook == "fitted":

@@ -369,10 +369,10 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // Two planes as one composed weight (the caller has asked prefill_compose_supported with the static array's share).
 static int run_compose(tq_linear_s* h, const tq::LayerView& V, const void* x_dev, int x_dtype, int batch, void* y_dev, int y_dtype,
-                       hipStream_t stream, void* static_ws) {
-    if (!static_ws && !ensure_stage(&h->d_work, &h->work_bytes, tq::prefill_compose_workspace_bytes(V, batch, device_cu_count()),
+                       hipStream_t stream, void* static_ws, size_t capacity) {
+    if (!static_ws && !ensure_stage(&h->d_work, &h->work_bytes, tq::prefill_compose_workspace_bytes(V, batch, device_cu_count(), capacity),
                                     stream, &h->retired)) return 1;
-    return hip_ok(tq::launch_prefill_compose(V, x_dev, x_dtype, batch, y_dev, y_dtype, static_ws ? static_ws : h->d_work,
+    return hip_ok(tq::launch_prefill_compose(V, x_dev, x_dtype, batch, y_dev, y_dtype, static_ws ? static_ws : h->d_work, capacity,
                                              device_cu_count(), stream), "tq_prefill_compose launch") ? 0 : 1;
 }
 
@@ -412,7 +412,7 @@ int forward_view(tq_linear_s* h, const tq::LayerView& V, bool generic_only, cons
     float* partial = nullptr;
     tq::PrefillPlan plan{};
     if (prefill && tq::prefill_compose_supported(V, batch, device_cu_count(), static_ws ? static_cap : ~(size_t)0))
-        return run_compose(h, V, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws);
+        return run_compose(h, V, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws, static_ws ? static_cap : ~(size_t)0);
     // (few output tiles: small ones, tq_prefill_tile.hip; a static workspace too small for 512-row images goes on)
     const int tile = prefill ? tq::prefill_tile_shape(V, batch, device_cu_count()) : -1;
     if (tile >= 0) {
@@ -484,7 +484,7 @@ int forward_impl(tq_linear_s* h, const void* x_dev, int x_dtype, int batch, void
     const size_t cap = (size_t)TQ_STATIC_SCRATCH_BYTES;
     if (two_plane5 && !gate && h->has_plane_views &&
         tq::prefill_compose_supported(h->view, batch, device_cu_count(), static_ws ? cap : ~(size_t)0))
-        return run_compose(h, h->view, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws);
+        return run_compose(h, h->view, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws, static_ws ? cap : ~(size_t)0);
     if (two_plane5 && batch >= 2 && !gate && h->has_plane_views) {
         const size_t one = align256((size_t)batch * h->view.out_features * sizeof(float));
         const size_t need = plane_sum_bytes(h, batch, y_dtype);
@@ -588,7 +588,7 @@ int tq_linear_reserve(tq_linear_t h, int max_batch) {
             }
             auto compose = [&](int r) {                    // (all rows at once: what prefill_reserve_bytes looks at)
                 if (r <= max_batch && tq::prefill_compose_supported(h->view, r, device_cu_count(), ~(size_t)0))
-                    work = std::max(work, tq::prefill_compose_workspace_bytes(h->view, r, device_cu_count()));
+                    work = std::max(work, tq::prefill_compose_workspace_bytes(h->view, r, device_cu_count(), ~(size_t)0));
             };
             for (int r = tq::compose_min_rows(h->view); r <= max_batch; r = r / tq::kPanelM * tq::kPanelM + tq::kPanelM + 1) compose(r);
             if (!ensure_stage(&h->d_work, &h->work_bytes, work, nullptr, &h->retired)) return 1;

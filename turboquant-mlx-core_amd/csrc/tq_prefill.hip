@@ -640,7 +640,7 @@ size_t prefill_reserve_bytes(const LayerView& L, int max_batch, int num_cus) {
         const size_t n = prefill_panel_supported(L, rows, num_cus, ~(size_t)0) ? prefill_panel_workspace_bytes(L, rows, num_cus, ~(size_t)0)
                                                                              : prefill_plan(L, rows, num_cus, ~(size_t)0).total_bytes;
         if (n > need) need = n;
-        if (prefill_compose_supported(L, rows, num_cus, ~(size_t)0)) need = std::max(need, prefill_compose_workspace_bytes(L, rows, num_cus));
+        if (prefill_compose_supported(L, rows, num_cus, ~(size_t)0)) need = std::max(need, prefill_compose_workspace_bytes(L, rows, num_cus, ~(size_t)0));
     };
     look(16); look(kSkinnyMaxRows); look(kSkinnyMaxRows + 1); look(128); look(129);
     for (int rows = kBM; rows < max_batch + kBM; rows += kBM) { look(rows); look(rows + 1); }

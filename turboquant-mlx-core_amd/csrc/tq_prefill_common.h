@@ -38,16 +38,17 @@ hipError_t launch_prefill_panel(const LayerView& L, const void* x, int x_dtype, 
                                 void* workspace, size_t workspace_bytes, int num_cus, hipStream_t stream);
 
 // Layers of two planes (dual rotation; 5-bit primaries with a 4-bit residual) at many rows: the planes composed into one
-// fp16 weight first (tq_prefill_panel.hip).  Workspace: fragment images, parts, a slab of the weight.
+// fp16 weight first (tq_prefill_panel.hip).  Workspace: fragment images, parts, a slab of the weight, cut to `capacity` (the
+// same for the three calls below).
 // (from the second panel of 512 rows on; 5-bit layers, whose planes are separate calls and a sum otherwise, in the first too)
 inline int compose_min_rows(const LayerView& L) { return L.mode == kDual ? kPanelM + 1 : 385; }
 // What the sum of the planes is multiplied by before it is rounded to fp16, or 0: multiplying plane by plane is the more
 // precise, or the sum may leave fp16's range.  Codebooks as the layer was created with.
 float compose_scale(int mode, uint32_t block_size, const float* cbp, int np, const float* cbr, int nr);
 bool prefill_compose_supported(const LayerView& L, int batch, int num_cus, size_t capacity);
-size_t prefill_compose_workspace_bytes(const LayerView& L, int batch, int num_cus);
+size_t prefill_compose_workspace_bytes(const LayerView& L, int batch, int num_cus, size_t capacity);
 hipError_t launch_prefill_compose(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
-                                  void* workspace, int num_cus, hipStream_t stream);
+                                  void* workspace, size_t capacity, int num_cus, hipStream_t stream);
 
 // The small-tile kernel (tq_prefill_tile.hip).  Its shape for a call that prefill_supported() takes, or -1: one of the
 // kernels with large tiles is faster.  Workspace: fragment images alone.

@@ -767,17 +767,16 @@ hipError_t launch_prefill_panel(const LayerView& L, const void* x, int x_dtype, 
 // Two planes as one fp16 weight (launch_compose), slab of output rows by slab, and one contraction over it instead of one
 // per plane.  Composing costs the same whatever the number of rows (1 us per million weights): with two or more panels
 // of activations it is less than what it saves.  us per call, bf16, before -> now, in x out: 5120 x 27648 at 2048 rows
-// 1119 -> 872, 5120 x 5120 at 2048 rows 252 -> 175, 3584 x 18944 at 700 rows 320 -> 256, 2048 x 10240 at 1024 rows 111 -> 97; in
-// one panel 5120 x 27648 at 512 rows 264, 393 composed (not taken), but the 5-bit layers, which are two calls and a sum
-// otherwise, gain there too: 3072 x 17000 at 512 rows 179 -> 141, 2048 x 8704 at 668 rows 140 -> 89, 5120 x 27648 at 1024 rows
-// 661 -> 489.  Against 64 bits the error is no larger than that of the two contractions (compose_scale).  The slab bounds the workspace: the
-// whole weight in fp16 would be twice the layer.
+// 1119 -> 872, 5120 x 5120 at 2048 rows 252 -> 175, 3584 x 18944 at 700 rows 320 -> 240, 2048 x 10240 at 1024 rows 111 -> 97; in
+// one panel 5120 x 27648 at 512 rows 264, 393 composed (not taken); 5-bit layers, which are two calls and a sum otherwise:
+// 1280 x 20000 at 500 rows 110 -> 71, 2048 x 8704 at 668 rows 140 -> 89, 5120 x 27648 at 1024 rows 661 -> 489.  Against 64 bits
+// the error is no larger than that of the two contractions (compose_scale).  The slab bounds the workspace.
 // ---------------------------------------------------------------------------
 namespace {
 
-constexpr size_t kComposeBytes = (size_t)160 << 20;        // of a slab
+constexpr size_t kSlabBytes = (size_t)160 << 20;           // largest slab: what the last-level cache still holds of it when it is read
 
-struct ComposePlan { int slab_tiles; PanelPlan panel; size_t slab_at, total_bytes; };    // panel: of a whole slab, the largest need
+struct ComposePlan { int slab_tiles; size_t slab_at, total_bytes; };     // slab_tiles == 0: plane by plane is cheaper
 
 LayerView slab_view(const LayerView& L, int rows) {
     LayerView s = L;
@@ -786,24 +785,64 @@ LayerView slab_view(const LayerView& L, int rows) {
     return s;
 }
 
-ComposePlan compose_plan(const LayerView& L, int batch, int num_cus) {
-    ComposePlan p{};
+// Workspace of a call: fragment images, the parts of a slab's tail tiles, the slab.  A handle keeps it, so it is bounded by
+// what the handle holds anyway: beside the images as many bytes as the layer's planes or as one K part of a tile per CU
+// (67 MB), or all that the call takes plane by plane; and by `capacity`.  The cut into slabs is the
+// cheapest by a count in rounds of the chip over whole rows, and taken if it is cheaper than the call plane by plane.  us,
+// in x out, random indices: 5120 x 27648, 2048 rows in two slabs 660, in four 679, in rounds of 64 weight tiles with a tail
+// cut along K 690 (plane by plane 965); 1536 rows in three 537, in two 607 (767); 3000 rows in two 895, in three that
+// leave one XCD a third round 1046 (1383); 4096 rows in three 1090, in seven 1179 (1829).  4096 x 14336 at 700 rows, where
+// 117 MB would be a slab and 67 are given: in two 236, plane by plane 195 (one slab: 163).
+ComposePlan compose_plan(const LayerView& L, int batch, int num_cus, size_t capacity) {
     const int panels = (batch + kPanelM - 1) / kPanelM, tiles = (L.out_features + kPN - 1) / kPN;
     const size_t tile_bytes = (size_t)kPN * L.in_features * sizeof(uint16_t);
-    int slab = (int)(kComposeBytes / tile_bytes);
-    if (slab < 1) slab = 1;
-    const int round = num_cus / panels;                    // weight tiles that fill the chip once
-    if (slab >= tiles) slab = tiles;
-    else if (round >= 1 && slab >= round) slab = slab / round * round;
-    else slab = (tiles + (tiles + slab - 1) / slab - 1) / ((tiles + slab - 1) / slab);       // slabs of equal length
-    p.slab_tiles = slab;
-    for (int t0 = 0; t0 < tiles; t0 += slab) {
-        const int n = t0 + slab < tiles ? slab * kPN : L.out_features - t0 * kPN;
-        const PanelPlan q = panel_plan(slab_view(L, n), batch, num_cus, ~(size_t)0);
-        if (q.total_bytes > p.panel.total_bytes) p.panel = q;
-    }
-    p.slab_at = (p.panel.total_bytes + 255) & ~(size_t)255;
-    p.total_bytes = p.slab_at + (size_t)slab * tile_bytes;
+    const LayerView whole = slab_view(L, L.out_features);
+    const size_t xt_bytes = panel_plan(whole, batch, num_cus, 0).xt_bytes;
+    const size_t packed = (size_t)tiles * kPN * L.in_features / 2 * (L.mode == kDual ? 2 : 3);
+    const size_t part_per_cu = (size_t)num_cus * kPanelM * kPN * sizeof(float);
+    const size_t extra = std::max(packed, part_per_cu);
+    const PanelPlan planes = panel_plan(L.mode == kDual ? L : whole, batch, num_cus, ~(size_t)0);
+    const size_t most = std::min(capacity, std::max(xt_bytes + 256 + extra, planes.total_bytes));
+    ComposePlan p{};
+    if (xt_bytes + 256 >= most) return p;
+    const int fits = (int)std::min<size_t>(std::min(most - xt_bytes - 256, kSlabBytes) / tile_bytes, (size_t)tiles);
+    if (fits < 1) return p;
+    const double round_us = L.in_features / 32.0;          // 0.5 us for a sub-step of 16 columns
+    // Rounds that `units` workgroups take, `passes` over a row each.  (A round that leaves CUs idle is shorter: the others get
+    // their power.  Without a tail the XCD with the most weight tiles decides.  Parts are written and added again.)
+    auto rounds = [&](int units) {
+        const int rest = units % num_cus;
+        return units / num_cus + (rest ? 0.5 + 0.5 * rest / num_cus : 0.0);
+    };
+    auto count = [&](const PanelPlan& q, int rows, int passes) {
+        const int n_tiles = (rows + kPN - 1) / kPN, units = q.tail_tiles * q.parts;
+        if (!units) return passes * rounds((n_tiles + 7) / 8 * 8 * panels);
+        return passes * rounds(panels * n_tiles - q.tail_tiles) + rounds(units) * q.part_subs * kSubK / L.in_features + 0.15 / round_us * units;
+    };
+    double best = L.mode == kDual ? count(planes, L.out_features, 2)
+                                  : 2 * count(planes, L.out_features, 1) + (double)batch * L.out_features * 12.0 / 5e6 / round_us;
+    best -= (double)L.out_features * L.in_features / 1e6 / round_us;       // composing
+    auto look = [&](int slab) {
+        const int slabs = (tiles + slab - 1) / slab, last = L.out_features - (slabs - 1) * slab * kPN;
+        const size_t slab_bytes = (size_t)slab * tile_bytes, room = most - 256 - slab_bytes;
+        size_t bytes = 0;
+        double cost = 14.0 / round_us * slabs;             // (the launches of a slab)
+        auto add = [&](int n, int rows) {
+            const PanelPlan q = panel_plan(slab_view(L, rows), batch, num_cus, room);
+            cost += n * count(q, rows, 1);
+            bytes = std::max(bytes, q.total_bytes);
+        };
+        if (slabs > 1) add(slabs - 1, slab * kPN);
+        add(1, last);
+        if (cost >= best) return;
+        best = cost;
+        p.slab_tiles = slab;
+        p.slab_at = (bytes + 255) & ~(size_t)255;
+        p.total_bytes = p.slab_at + slab_bytes;
+    };
+    const int fewest = (tiles + fits - 1) / fits, round = num_cus / panels;
+    for (int n = fewest; n < fewest + 6; ++n) look((tiles + n - 1) / n);               // of equal length
+    if (round >= 1 && fits >= round && fits < tiles) look(fits / round * round);       // whole rounds
     return p;
 }
 
@@ -883,18 +922,21 @@ float compose_scale(int mode, uint32_t block_size, const float* cbp, int np, con
     return sum[best] <= planes ? (float)scale[best] : 0.0f;
 }
 
-size_t prefill_compose_workspace_bytes(const LayerView& L, int batch, int num_cus) { return compose_plan(L, batch, num_cus).total_bytes; }
+size_t prefill_compose_workspace_bytes(const LayerView& L, int batch, int num_cus, size_t capacity) {
+    return compose_plan(L, batch, num_cus, capacity).total_bytes;
+}
 
 bool prefill_compose_supported(const LayerView& L, int batch, int num_cus, size_t capacity) {
     if (!(L.compose_scale > 0.0f) || (L.mode != kDual && L.mode != kDual5 && L.mode != kShared5)) return false;
     if (batch < compose_min_rows(L)) return false;
     if (!prefill_panel_supported(slab_view(L, L.out_features), batch, num_cus, capacity)) return false;
-    return compose_plan(L, batch, num_cus).total_bytes <= capacity;
+    return compose_plan(L, batch, num_cus, capacity).slab_tiles > 0;
 }
 
 hipError_t launch_prefill_compose(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
-                                  void* workspace, int num_cus, hipStream_t stream) {
-    const ComposePlan plan = compose_plan(L, batch, num_cus);
+                                  void* workspace, size_t capacity, int num_cus, hipStream_t stream) {
+    const ComposePlan plan = compose_plan(L, batch, num_cus, capacity);
+    if (!plan.slab_tiles) return hipErrorInvalidValue;
     hipError_t e = launch_rotate_tiles(slab_view(L, L.out_features), x, x_dtype, batch, workspace, stream, kPanelImage);
     if (e != hipSuccess) return e;
     char* const slab = static_cast<char*>(workspace) + plan.slab_at;
@@ -902,7 +944,7 @@ hipError_t launch_prefill_compose(const LayerView& L, const void* x, int x_dtype
     for (int t0 = 0; t0 < tiles; t0 += plan.slab_tiles) {
         const int row0 = t0 * kPN, rows = t0 + plan.slab_tiles < tiles ? plan.slab_tiles * kPN : L.out_features - row0;
         if ((e = launch_compose(L, row0, rows, slab, stream)) != hipSuccess) return e;
-        const PanelPlan q = panel_plan(slab_view(L, rows), batch, num_cus, ~(size_t)0);
+        const PanelPlan q = panel_plan(slab_view(L, rows), batch, num_cus, plan.slab_at);      // (the parts end where the slab begins)
         PanelArgs a{};
         a.xt = static_cast<const char*>(workspace);
         a.plane0 = reinterpret_cast<const uint8_t*>(slab);
