@@ -76,7 +76,8 @@ int tq_fit_layer_codebooks_host(const float* weight_host, int out_features, int 
 
 /**
  * The conversion calls above keep up to 2 GiB of device memory per GPU between calls (the next call uses it again).
- * This gives back what no running call uses; creating a layer and the end of a model's conversion do so too.
+ * This gives back what no running call uses; creating a layer, the end of a model's conversion and an allocation of this
+ * library that does not fit beside it do so too.  A program that allocates by other means calls this first.
  */
 void tq_quantizer_release_workspaces(void);
 

@@ -160,12 +160,29 @@ void one_codebook_that_misses() {
            "a fit that missed goes on with a new expectation", fit_calls.size());
 }
 
+// What the calls keep is there for the rest of the library: an allocation that does not fit beside it gets it.
+void kept_blocks_give_way() {
+    std::vector<float> v(4 * kN, 0.0f);
+    std::vector<uint8_t> idx(4 * kN);
+    float bounds[15] = {0};
+    expect(tq_codebook_quantize_host(v.data(), 4 * kN, bounds, 16, idx.data()) == 0, "a call that leaves blocks behind");
+    expect(dev.live >= 20 * kN, "blocks are kept", dev.live);
+    dev.size = 32 * kN;
+    void* p = nullptr;
+    expect(tq::device_malloc(&p, 24 * kN) == hipSuccess, "the blocks give way", dev.live);
+    void* q = nullptr;
+    expect(tq::device_malloc(&q, 24 * kN) == hipErrorOutOfMemory, "what does not fit is refused");
+    expect(hipGetLastError() == hipSuccess, "and the refusal is not left to the next launch");
+    (void)hipFree(p);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const struct { const char* name; void (*run)(); } checks[] = {{"no_host_memory", no_host_memory},
                                                                     {"fit_without_workspace", fit_without_workspace},
-                                                                    {"one_codebook_that_misses", one_codebook_that_misses}};
+                                                                    {"one_codebook_that_misses", one_codebook_that_misses},
+                                                                    {"kept_blocks_give_way", kept_blocks_give_way}};
     for (const auto& c : checks)
         if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
             c.run();

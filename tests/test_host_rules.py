@@ -22,6 +22,6 @@ def test_host_rules(check):
     _check("host_rules", check)
 
 
-@pytest.mark.parametrize("check", ["no_host_memory", "fit_without_workspace", "one_codebook_that_misses"])
+@pytest.mark.parametrize("check", ["no_host_memory", "fit_without_workspace", "one_codebook_that_misses", "kept_blocks_give_way"])
 def test_conversion_memory(check):
     _check("conversion_memory", check)

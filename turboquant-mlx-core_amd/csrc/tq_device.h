@@ -112,6 +112,8 @@ bool hip_ok(hipError_t e, const char* what);
 
 // Device memory the conversion calls keep between calls, given back (tq_quantize_c.cpp).
 void release_conversion_memory();
+// hipMalloc that gives that memory back and tries again before it fails; a failure is not left as the last error.
+hipError_t device_malloc(void** p, size_t bytes);
 
 // Offline quantizer (tq_quantize.hip).
 struct QuantArgsHost {

@@ -178,7 +178,7 @@ bool ensure_stage(void** buf, size_t* have, size_t need, hipStream_t stream = nu
     }
     void* fresh = nullptr;
     const size_t want = (retired && *buf && need < 2 * *have) ? 2 * *have : need;
-    if (!hip_ok(hipMalloc(&fresh, want), "hipMalloc(staging)")) return false;
+    if (!hip_ok(tq::device_malloc(&fresh, want), "hipMalloc(staging)")) return false;
     if (*buf) {
         if (retired) retired->push_back(*buf);
         else (void)hipFree(*buf);
@@ -222,10 +222,10 @@ tq_linear_t create_impl(int in_features, int out_features,
     const size_t pbytes = (size_t)out_features * primary_cols;
     const size_t rbytes = (size_t)out_features * residual_cols;
     const hipMemcpyKind kind = from_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-    bool ok = hip_ok(hipMalloc((void**)&h->d_primary, pbytes), "hipMalloc(packed_primary)") &&
-              hip_ok(hipMalloc((void**)&h->d_residual, rbytes), "hipMalloc(packed_residual)") &&
-              hip_ok(hipMalloc((void**)&h->d_norms, (size_t)out_features * sizeof(float)), "hipMalloc(norms)") &&
-              hip_ok(hipMalloc((void**)&h->d_tables, 256 * sizeof(float)), "hipMalloc(tables)") &&
+    bool ok = hip_ok(tq::device_malloc((void**)&h->d_primary, pbytes), "hipMalloc(packed_primary)") &&
+              hip_ok(tq::device_malloc((void**)&h->d_residual, rbytes), "hipMalloc(packed_residual)") &&
+              hip_ok(tq::device_malloc((void**)&h->d_norms, (size_t)out_features * sizeof(float)), "hipMalloc(norms)") &&
+              hip_ok(tq::device_malloc((void**)&h->d_tables, 256 * sizeof(float)), "hipMalloc(tables)") &&
               hip_ok(hipMemcpy(h->d_primary, pp, pbytes, kind), "copy packed_primary") &&
               hip_ok(hipMemcpy(h->d_residual, pr, rbytes, kind), "copy packed_residual") &&
               hip_ok(hipMemcpy(h->d_norms, norms, (size_t)out_features * sizeof(float), kind), "copy norms");
@@ -235,7 +235,7 @@ tq_linear_t create_impl(int in_features, int out_features,
     bool has_residual = false;
     if (from_device) {
         int* d_flag = nullptr; int flag = 0;
-        ok = hip_ok(hipMalloc((void**)&d_flag, sizeof(int)), "hipMalloc(flag)") &&
+        ok = hip_ok(tq::device_malloc((void**)&d_flag, sizeof(int)), "hipMalloc(flag)") &&
              hip_ok(hipMemset(d_flag, 0, sizeof(int)), "hipMemset(flag)") &&
              hip_ok(tq::launch_any_nonzero(h->d_residual, rbytes, d_flag, nullptr), "any_nonzero") &&
              hip_ok(hipMemcpy(&flag, d_flag, sizeof(int), hipMemcpyDeviceToHost), "copy flag");
@@ -260,7 +260,7 @@ tq_linear_t create_impl(int in_features, int out_features,
     if (mode == tq::kSharedLut) {
         // The shared-rotation kernels stream one byte per weight; interleave the planes once and drop them.
         const size_t cbytes = (size_t)out_features * in_features;
-        ok = hip_ok(hipMalloc((void**)&h->d_combined, cbytes), "hipMalloc(packed_combined)") &&
+        ok = hip_ok(tq::device_malloc((void**)&h->d_combined, cbytes), "hipMalloc(packed_combined)") &&
              hip_ok(tq::launch_combine_planes(h->d_primary, h->d_residual, h->d_combined, pbytes, nullptr), "combine_planes") &&
              hip_ok(hipDeviceSynchronize(), "combine_planes sync");
         if (!ok) { delete h; return nullptr; }
@@ -279,8 +279,8 @@ tq_linear_t create_impl(int in_features, int out_features,
                 const float c = cbp[p5 < np ? p5 : np - 1];
                 lut[(r << 5) | p5] = mode == tq::kShared5 ? c + cbr[r < nr ? r : nr - 1] : c;   // src/dequantizer.cpp:186-212
             }
-        ok = hip_ok(hipMalloc((void**)&h->d_combined, cbytes), "hipMalloc(packed_combined)") &&
-             hip_ok(hipMalloc((void**)&h->d_tables_fwd, sizeof(lut)), "hipMalloc(tables)") &&
+        ok = hip_ok(tq::device_malloc((void**)&h->d_combined, cbytes), "hipMalloc(packed_combined)") &&
+             hip_ok(tq::device_malloc((void**)&h->d_tables_fwd, sizeof(lut)), "hipMalloc(tables)") &&
              hip_ok(hipMemcpy(h->d_tables_fwd, lut, sizeof(lut), hipMemcpyHostToDevice), "copy tables") &&
              hip_ok(tq::launch_combine_planes5(h->d_primary, h->d_residual, h->d_combined, rbytes, np < 32 ? np : 32, nr,
                                                nullptr), "combine_planes5") &&
@@ -309,7 +309,7 @@ tq_linear_t create_impl(int in_features, int out_features,
     // Scratch row for the rotated activations of one batch row (both rotations): rows wider than 16384
     // columns and the generic kernels rotate in a kernel of their own.  Allocated here so that a forward
     // call never allocates on the batch-1 path.
-    if (!hip_ok(hipMalloc((void**)&h->d_xrot, (size_t)2 * in_features * sizeof(float)), "hipMalloc(rotated row)")) {
+    if (!hip_ok(tq::device_malloc((void**)&h->d_xrot, (size_t)2 * in_features * sizeof(float)), "hipMalloc(rotated row)")) {
         delete h; return nullptr;
     }
     v.xrot_work = h->d_xrot;
@@ -330,8 +330,8 @@ tq_linear_t create_impl(int in_features, int out_features,
         std::memset(tb, 0, sizeof(tb));
         for (int b = 0; b < 256; ++b) ta[b] = cbp[b < np ? b : np - 1];          // index clamp of src/dequantizer.cpp:94
         for (int i = 0; i < 16; ++i) tb[i] = cbr[i < nr ? i : nr - 1];            // :103
-        ok = hip_ok(hipMalloc((void**)&h->d_tables_plane[0], sizeof(ta)), "hipMalloc(tables)") &&
-             hip_ok(hipMalloc((void**)&h->d_tables_plane[1], sizeof(tb)), "hipMalloc(tables)") &&
+        ok = hip_ok(tq::device_malloc((void**)&h->d_tables_plane[0], sizeof(ta)), "hipMalloc(tables)") &&
+             hip_ok(tq::device_malloc((void**)&h->d_tables_plane[1], sizeof(tb)), "hipMalloc(tables)") &&
              hip_ok(hipMemcpy(h->d_tables_plane[0], ta, sizeof(ta), hipMemcpyHostToDevice), "copy tables") &&
              hip_ok(hipMemcpy(h->d_tables_plane[1], tb, sizeof(tb), hipMemcpyHostToDevice), "copy tables");
         if (!ok) { delete h; return nullptr; }
@@ -719,7 +719,7 @@ int tq_linear_dequantize_as_host(tq_linear_t h, void* w_host, int w_dtype) {
         if (!h || !w_host) { set_error("tq_linear_dequantize_host: NULL argument"); return 1; }
         const size_t bytes = (size_t)h->view.out_features * h->view.in_features * (w_dtype == tq::kF32 ? 4 : 2);
         void* d = nullptr;
-        if (!hip_ok(hipMalloc(&d, bytes), "hipMalloc(weight)")) return 1;
+        if (!hip_ok(tq::device_malloc(&d, bytes), "hipMalloc(weight)")) return 1;
         bool ok = tq_linear_dequantize_as(h, d, w_dtype, nullptr) == 0 &&
                   hip_ok(hipMemcpy(w_host, d, bytes, hipMemcpyDeviceToHost), "copy weight");
         (void)hipFree(d);
@@ -763,7 +763,7 @@ int tq_wht_rotate_host(const float* in_host, float* out_host, int rows, int cols
         if (!in_host || !out_host || rows <= 0 || cols <= 0) { set_error("tq_wht_rotate_host: bad argument"); return 1; }
         const size_t bytes = (size_t)rows * cols * sizeof(float);
         float* d = nullptr;
-        if (!hip_ok(hipMalloc((void**)&d, bytes), "hipMalloc(matrix)")) return 1;
+        if (!hip_ok(tq::device_malloc((void**)&d, bytes), "hipMalloc(matrix)")) return 1;
         bool ok = hip_ok(hipMemcpy(d, in_host, bytes, hipMemcpyHostToDevice), "copy in") &&
                   tq_wht_rotate(d, d, rows, cols, seed, block_size, inverse, nullptr) == 0 &&
                   hip_ok(hipMemcpy(out_host, d, bytes, hipMemcpyDeviceToHost), "copy out");
@@ -799,9 +799,9 @@ tq_mlp_t tq_mlp_create(tq_linear_t gate, tq_linear_t up, tq_linear_t down, int m
         tq_mlp_s* m = new (std::nothrow) tq_mlp_s{gate, up, down, max_batch};
         if (!m) { set_error("tq_mlp_create: out of host memory"); return nullptr; }
         const size_t n = (size_t)max_batch * inter;
-        bool ok = hip_ok(hipMalloc((void**)&m->d_gate, n * sizeof(float)), "hipMalloc(gate)") &&
-                  hip_ok(hipMalloc((void**)&m->d_up, n * sizeof(float)), "hipMalloc(up)") &&
-                  hip_ok(hipMalloc(&m->d_act, n * sizeof(float)), "hipMalloc(act)");
+        bool ok = hip_ok(tq::device_malloc((void**)&m->d_gate, n * sizeof(float)), "hipMalloc(gate)") &&
+                  hip_ok(tq::device_malloc((void**)&m->d_up, n * sizeof(float)), "hipMalloc(up)") &&
+                  hip_ok(tq::device_malloc(&m->d_act, n * sizeof(float)), "hipMalloc(act)");
         // The batched path of the three layers needs rotated-activation workspaces: size them now so
         // that tq_mlp_forward never allocates.
         for (tq_linear_t l : {gate, up, down})

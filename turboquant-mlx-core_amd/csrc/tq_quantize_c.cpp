@@ -37,7 +37,7 @@ void midpoints(const float* c, int n, float* b) {
 // 150 such calls hipMalloc waited for the wipe and a conversion of 18944 x 3584 took 18.5 ms instead of 3.3 (measured;
 // 3.2 throughout with the memory kept).  A block belongs to one call at a time; what is idle stays below kKeepBytes per
 // device and is given back by tq_quantizer_release_workspaces, by the creation of a layer (the conversion is over, the
-// weights want the memory), at the end of a model's conversion and where an allocation here fails.
+// weights want the memory), at the end of a model's conversion and where an allocation of this library fails.
 class KeptMemory {
     struct Block { void* p; size_t bytes; int device; };
     static constexpr size_t kKeepBytes = (size_t)2 << 30;
@@ -79,11 +79,14 @@ public:
                 return hipSuccess;
             }
         }
-        e = hipMalloc(p, *got);
+        return fresh(p, *got);
+    }
+    hipError_t fresh(void** p, size_t bytes) {
+        hipError_t e = hipMalloc(p, bytes);
         if (e != hipErrorOutOfMemory) return e;
         release();
         (void)hipGetLastError();
-        e = hipMalloc(p, *got);
+        e = hipMalloc(p, bytes);
         if (e != hipSuccess) (void)hipGetLastError();      // (reported here; the launches that follow ask for the last error too)
         return e;
     }
@@ -249,6 +252,7 @@ bool fit_codebooks(const float* samples_dev, size_t n, int primary_bits, int res
 
 namespace tq {
 void release_conversion_memory() { KeptMemory::get().release(); }
+hipError_t device_malloc(void** p, size_t bytes) { return KeptMemory::get().fresh(p, bytes); }
 }  // namespace tq
 
 extern "C" {
