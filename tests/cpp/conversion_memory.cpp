@@ -1,76 +1,21 @@
-// Host side of the conversion calls (csrc/tq_quantize_c.cpp) on a HIP runtime and kernels that are faked here, without a
-// GPU: a device of a given size whose memory is host memory, filled with 0xff when handed out.  One check per argument
-// (tests/test_host_rules.py).
-#include <cstdio>
-#include <cstdlib>
-#include <cstring>
-#include <map>
-#include <new>
-#include <string>
-#include <vector>
-
+// Host side of the conversion calls (csrc/tq_quantize_c.cpp) on a faked runtime (fake_hip.h) and kernels that are faked
+// here, without a GPU.  One check per argument (tests/test_host_rules.py).
+#include "fake_hip.h"
 #include "tq_device.h"
 #include "turboquant_c/tq_quantizer.h"
 
-namespace {
+using fake::dev;
+using fake::expect;
+using fake::host_memory_gone;
 
-struct FakeDevice {
-    size_t size = ~(size_t)0, live = 0, peak = 0;
-    hipError_t last = hipSuccess;
-    std::map<void*, size_t> blocks;
-} dev;
+namespace {
 
 int lloyd_passes = 0;
 struct FitCall { bool first_round, everything; };
 std::vector<FitCall> fit_calls;
 enum { kFits, kMissesOnce, kNeedsAll } fit_outcome = kFits;
-bool host_memory_gone = false;
-
-int failures = 0;
-void expect(bool ok, const char* what, unsigned long long value = 0) {
-    if (!ok) { std::printf("failed: %s (%llu)\n", what, value); ++failures; }
-}
 
 }  // namespace
-
-void* operator new(size_t n) {
-    void* p = host_memory_gone ? nullptr : std::malloc(n ? n : 1);
-    if (!p) throw std::bad_alloc();
-    return p;
-}
-void operator delete(void* p) noexcept { std::free(p); }
-void operator delete(void* p, size_t) noexcept { std::free(p); }
-
-// --------------------------------------------------------------------------- the runtime
-extern "C" {
-hipError_t hipMalloc(void** p, size_t n) {
-    if (n > dev.size || dev.live + n > dev.size) return dev.last = hipErrorOutOfMemory;
-    *p = std::malloc(n);
-    std::memset(*p, 0xff, n);
-    const bool gone = host_memory_gone;                    // (the map is the fake's, not the library's)
-    host_memory_gone = false;
-    dev.blocks[*p] = n;
-    host_memory_gone = gone;
-    dev.live += n;
-    if (dev.live > dev.peak) dev.peak = dev.live;
-    return hipSuccess;
-}
-hipError_t hipFree(void* p) {
-    if (!p) return hipSuccess;
-    expect(dev.blocks.count(p) == 1, "memory is freed once");
-    dev.live -= dev.blocks[p];
-    dev.blocks.erase(p);
-    std::free(p);
-    return hipSuccess;
-}
-hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind) { std::memcpy(to, from, n); return hipSuccess; }
-hipError_t hipMemset(void* p, int v, size_t n) { std::memset(p, v, n); return hipSuccess; }
-hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipDeviceSynchronize() { return hipSuccess; }
-hipError_t hipGetLastError() { const hipError_t e = dev.last; dev.last = hipSuccess; return e; }
-const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
-}
 
 // --------------------------------------------------------------------------- the kernels
 namespace tq {
@@ -179,16 +124,9 @@ void kept_blocks_give_way() {
 }  // namespace
 
 int main(int argc, char** argv) {
-    const struct { const char* name; void (*run)(); } checks[] = {{"no_host_memory", no_host_memory},
-                                                                    {"fit_without_workspace", fit_without_workspace},
-                                                                    {"one_codebook_that_misses", one_codebook_that_misses},
-                                                                    {"kept_blocks_give_way", kept_blocks_give_way}};
-    for (const auto& c : checks)
-        if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
-            c.run();
-            if (!failures) std::printf("ok\n");
-            return failures ? 1 : 0;
-        }
-    std::fprintf(stderr, "usage: conversion_memory <check>\n");
-    return 2;
+    const fake::Check checks[] = {{"no_host_memory", no_host_memory},
+                                  {"fit_without_workspace", fit_without_workspace},
+                                  {"one_codebook_that_misses", one_codebook_that_misses},
+                                  {"kept_blocks_give_way", kept_blocks_give_way}};
+    return fake::run(checks, argc, argv);
 }

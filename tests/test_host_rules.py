@@ -1,5 +1,5 @@
 """Host code of the library without a GPU: dispatch rules and workspace sizes (tests/cpp/host_rules.cpp), and the conversion
-calls on a faked runtime (tests/cpp/conversion_memory.cpp)."""
+calls and the forward calls on a faked runtime (tests/cpp/conversion_memory.cpp, tests/cpp/forward_routes.cpp)."""
 import os
 import subprocess
 
@@ -25,3 +25,8 @@ def test_host_rules(check):
 @pytest.mark.parametrize("check", ["no_host_memory", "fit_without_workspace", "one_codebook_that_misses", "kept_blocks_give_way"])
 def test_conversion_memory(check):
     _check("conversion_memory", check)
+
+
+@pytest.mark.parametrize("check", ["compose_without_memory", "reserve_without_memory"])
+def test_forward_routes(check):
+    _check("forward_routes", check)

@@ -367,11 +367,15 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 }  // namespace
 
-// Two planes as one composed weight (the caller has asked prefill_compose_supported with the static array's share).
+// Two planes as one composed weight, and whether this call is run that way: plane by plane where the workspace cannot be had,
+// which takes less of it.
+static bool takes_compose(tq_linear_s* h, const tq::LayerView& V, int batch, hipStream_t stream, void* static_ws, size_t capacity) {
+    return tq::prefill_compose_supported(V, batch, device_cu_count(), capacity) &&
+           (static_ws || ensure_stage(&h->d_work, &h->work_bytes, tq::prefill_compose_workspace_bytes(V, batch, device_cu_count(), capacity),
+                                      stream, &h->retired));
+}
 static int run_compose(tq_linear_s* h, const tq::LayerView& V, const void* x_dev, int x_dtype, int batch, void* y_dev, int y_dtype,
                        hipStream_t stream, void* static_ws, size_t capacity) {
-    if (!static_ws && !ensure_stage(&h->d_work, &h->work_bytes, tq::prefill_compose_workspace_bytes(V, batch, device_cu_count(), capacity),
-                                    stream, &h->retired)) return 1;
     return hip_ok(tq::launch_prefill_compose(V, x_dev, x_dtype, batch, y_dev, y_dtype, static_ws ? static_ws : h->d_work, capacity,
                                              device_cu_count(), stream), "tq_prefill_compose launch") ? 0 : 1;
 }
@@ -411,9 +415,9 @@ int forward_view(tq_linear_s* h, const tq::LayerView& V, bool generic_only, cons
     void* work = nullptr;
     float* partial = nullptr;
     tq::PrefillPlan plan{};
-    if (prefill && tq::prefill_compose_supported(V, batch, device_cu_count(), static_ws ? static_cap : ~(size_t)0))
+    if (prefill && takes_compose(h, V, batch, stream, static_ws, static_ws ? static_cap : ~(size_t)0))
         return run_compose(h, V, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws, static_ws ? static_cap : ~(size_t)0);
-    // (few output tiles: small ones, tq_prefill_tile.hip; a static workspace too small for 512-row images goes on)
+    // (few output tiles: small ones, tq_prefill_tile.hip; a static workspace too small for its images goes on)
     const int tile = prefill ? tq::prefill_tile_shape(V, batch, device_cu_count()) : -1;
     if (tile >= 0) {
         const size_t need = tq::prefill_tile_workspace_bytes(V, batch);
@@ -477,13 +481,13 @@ size_t plane_sum_bytes(const tq_linear_s* h, int batch, int y_dtype) {
 int forward_impl(tq_linear_s* h, const void* x_dev, int x_dtype, int batch, void* y_dev, int y_dtype,
                  hipStream_t stream, const float* gate, void* static_ws = nullptr) {
     // 5-bit primaries with their own residual rotation or a 4-bit residual keep their two planes.  One
-    // row runs both planes in one pass (tq_gemv_five.hip, tq_generic.hip); two or more rows run each plane through
+    // row runs both planes in one pass (tq_gemv_five.hip, tq_generic.hip); more rows run each plane through
     // the tuned kernels as a layer of its own and add the two results: y = P x~p + R x~r, the same sum the
-    // reference's kernel forms per element (metal/turboquant_dequant_mm.metal:240-248, 277-292).
+    // reference's kernel forms per element (metal/turboquant_dequant_mm.metal:240-248, 277-292); many rows
+    // (385 and more, where the count of prefill_compose_supported says so) compose the planes first.
     const bool two_plane5 = h->view.mode >= tq::kShared5 && !h->has_fwd_view;
     const size_t cap = (size_t)TQ_STATIC_SCRATCH_BYTES;
-    if (two_plane5 && !gate && h->has_plane_views &&
-        tq::prefill_compose_supported(h->view, batch, device_cu_count(), static_ws ? cap : ~(size_t)0))
+    if (two_plane5 && !gate && h->has_plane_views && takes_compose(h, h->view, batch, stream, static_ws, static_ws ? cap : ~(size_t)0))
         return run_compose(h, h->view, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws, static_ws ? cap : ~(size_t)0);
     if (two_plane5 && batch >= 2 && !gate && h->has_plane_views) {
         const size_t one = align256((size_t)batch * h->view.out_features * sizeof(float));
@@ -570,6 +574,14 @@ size_t few_reserve_bytes(const tq::LayerView& V, int max_batch) {
 }
 }  // namespace
 
+namespace {
+// The workspace with room for composed planes, or, where that cannot be had, without (such calls run plane by plane then).
+bool reserve_work(tq_linear_s* h, size_t bytes, size_t with_composed) {
+    return ensure_stage(&h->d_work, &h->work_bytes, with_composed, nullptr, &h->retired) ||
+           (bytes < with_composed && ensure_stage(&h->d_work, &h->work_bytes, bytes, nullptr, &h->retired));
+}
+}  // namespace
+
 int tq_linear_reserve(tq_linear_t h, int max_batch) {
     try {
         if (!h || max_batch <= 0) { set_error("tq_linear_reserve: bad argument"); return 1; }
@@ -586,12 +598,7 @@ int tq_linear_reserve(tq_linear_t h, int max_batch) {
                 work = std::max(work, few_reserve_bytes(P, max_batch));
                 if (sk) part = std::max(part, tq::skinny_partial_bytes(P, rows));
             }
-            auto compose = [&](int r) {                    // (all rows at once: what prefill_reserve_bytes looks at)
-                if (r <= max_batch && tq::prefill_compose_supported(h->view, r, device_cu_count(), ~(size_t)0))
-                    work = std::max(work, tq::prefill_compose_workspace_bytes(h->view, r, device_cu_count(), ~(size_t)0));
-            };
-            for (int r = tq::compose_min_rows(h->view); r <= max_batch; r = r / tq::kPanelM * tq::kPanelM + tq::kPanelM + 1) compose(r);
-            if (!ensure_stage(&h->d_work, &h->work_bytes, work, nullptr, &h->retired)) return 1;
+            if (!reserve_work(h, work, std::max(work, tq::prefill_compose_reserve_bytes(h->view, max_batch, device_cu_count())))) return 1;
             if (!ensure_stage(&h->d_partial, &h->partial_bytes, part, nullptr, &h->retired)) return 1;
             if (!ensure_stage(&h->d_sum, &h->sum_bytes, plane_sum_bytes(h, max_batch, tq::kBF16), nullptr, &h->retired)) return 1;
             return 0;
@@ -605,7 +612,8 @@ int tq_linear_reserve(tq_linear_t h, int max_batch) {
         const size_t big = pf ? tq::prefill_reserve_bytes(V, max_batch, device_cu_count()) : 0;
         const size_t few = few_reserve_bytes(V, max_batch);
         const size_t work = std::max(few, std::max(small, big));
-        if (work && !ensure_stage(&h->d_work, &h->work_bytes, work, nullptr, &h->retired)) return 1;
+        const size_t composed = pf ? tq::prefill_compose_reserve_bytes(V, max_batch, device_cu_count()) : 0;
+        if (!reserve_work(h, work, std::max(work, composed))) return 1;
         if (sk && !ensure_stage(&h->d_partial, &h->partial_bytes, tq::skinny_partial_bytes(V, rows), nullptr, &h->retired)) return 1;
         return 0;
     } catch (...) { set_error("tq_linear_reserve: exception"); return 1; }

@@ -631,7 +631,7 @@ PrefillPlan prefill_plan(const LayerView& L, int batch, int num_cus, size_t capa
     return p;
 }
 
-// Largest workspace any call of 16 .. max_batch rows needs (fewer rows can mean more ranges, and the two kernels
+// Largest workspace any call of 16 .. max_batch rows needs beside composed planes (fewer rows can mean more ranges, and the two kernels
 // cut differently: every row count at which the choice of kernel or the number of tiles changes is looked at).
 size_t prefill_reserve_bytes(const LayerView& L, int max_batch, int num_cus) {
     size_t need = 0;
@@ -640,12 +640,11 @@ size_t prefill_reserve_bytes(const LayerView& L, int max_batch, int num_cus) {
         const size_t n = prefill_panel_supported(L, rows, num_cus, ~(size_t)0) ? prefill_panel_workspace_bytes(L, rows, num_cus, ~(size_t)0)
                                                                              : prefill_plan(L, rows, num_cus, ~(size_t)0).total_bytes;
         if (n > need) need = n;
-        if (prefill_compose_supported(L, rows, num_cus, ~(size_t)0)) need = std::max(need, prefill_compose_workspace_bytes(L, rows, num_cus, ~(size_t)0));
     };
     look(16); look(kSkinnyMaxRows); look(kSkinnyMaxRows + 1); look(128); look(129);
     for (int rows = kBM; rows < max_batch + kBM; rows += kBM) { look(rows); look(rows + 1); }
     look(max_batch);
-    // (small tiles, whichever row counts take them: images of 512 rows)
+    // (small tiles, whichever row counts take them: images of 32 rows)
     if (max_batch >= 16) need = std::max(need, prefill_tile_workspace_bytes(L, max_batch));
     return need;
 }

@@ -39,7 +39,7 @@ hipError_t launch_prefill_panel(const LayerView& L, const void* x, int x_dtype, 
 
 // Layers of two planes (dual rotation; 5-bit primaries with a 4-bit residual) at many rows: the planes composed into one
 // fp16 weight first (tq_prefill_panel.hip).  Workspace: fragment images, parts, a slab of the weight, cut to `capacity` (the
-// same for the three calls below).
+// same for a call's rule, size and launch).
 // (from the second panel of 512 rows on; 5-bit layers, whose planes are separate calls and a sum otherwise, in the first too)
 inline int compose_min_rows(const LayerView& L) { return L.mode == kDual ? kPanelM + 1 : 385; }
 // What the sum of the planes is multiplied by before it is rounded to fp16, or 0: multiplying plane by plane is the more
@@ -47,6 +47,7 @@ inline int compose_min_rows(const LayerView& L) { return L.mode == kDual ? kPane
 float compose_scale(int mode, uint32_t block_size, const float* cbp, int np, const float* cbr, int nr);
 bool prefill_compose_supported(const LayerView& L, int batch, int num_cus, size_t capacity);
 size_t prefill_compose_workspace_bytes(const LayerView& L, int batch, int num_cus, size_t capacity);
+size_t prefill_compose_reserve_bytes(const LayerView& L, int max_batch, int num_cus);      // of all calls of up to max_batch rows
 hipError_t launch_prefill_compose(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
                                   void* workspace, size_t capacity, int num_cus, hipStream_t stream);
 

@@ -933,6 +933,16 @@ bool prefill_compose_supported(const LayerView& L, int batch, int num_cus, size_
     return compose_plan(L, batch, num_cus, capacity).slab_tiles > 0;
 }
 
+// (the number of panels decides, and from how many rows on)
+size_t prefill_compose_reserve_bytes(const LayerView& L, int max_batch, int num_cus) {
+    size_t need = 0;
+    for (int rows = compose_min_rows(L); rows <= max_batch; rows = rows / kPanelM * kPanelM + kPanelM + 1)
+        for (int r : {rows, std::min(max_batch, (rows + kPanelM - 1) / kPanelM * kPanelM)})
+            if (prefill_compose_supported(L, r, num_cus, ~(size_t)0))
+                need = std::max(need, prefill_compose_workspace_bytes(L, r, num_cus, ~(size_t)0));
+    return need;
+}
+
 hipError_t launch_prefill_compose(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
                                   void* workspace, size_t capacity, int num_cus, hipStream_t stream) {
     const ComposePlan plan = compose_plan(L, batch, num_cus, capacity);
