@@ -14,13 +14,15 @@ struct Layer {
     int in, out;
     std::vector<unsigned char> x, y;
     tq_linear_t h = nullptr;
-    explicit Layer(int in_, int out_, int rows) : in(in_), out(out_), x((size_t)rows * in_ * 4), y((size_t)rows * out_ * 4) {
-        float cb[16];
-        tq_generate_codebook(4, cb, nullptr);
-        std::vector<uint8_t> p((size_t)out * in / 2, 0x5a), r(p.size(), 0xa5);
+    explicit Layer(int in_, int out_, int rows, int bits = 4, bool residual = true, uint32_t seed_residual = 1234, uint32_t bs = 256)
+        : in(in_), out(out_), x((size_t)rows * in_ * 4), y((size_t)rows * out_ * 4) {
+        float cbp[32], cbr[16];
+        const int np = tq_generate_codebook(bits, cbp, nullptr), pc = bits == 5 ? in : in / 2;
+        tq_generate_codebook(4, cbr, nullptr);
+        std::vector<uint8_t> p((size_t)out * pc, 0x15), r((size_t)out * in / 2, residual ? 0xa5 : 0);
         std::vector<float> norms(out, 1.0f);
-        const uint32_t seeds[3] = {99, 1234, 256};
-        h = tq_linear_create(in, out, p.data(), in / 2, r.data(), in / 2, norms.data(), seeds, cb, 16, cb, 16, 256);
+        const uint32_t seeds[3] = {99, seed_residual, bs};
+        h = tq_linear_create(in, out, p.data(), pc, r.data(), in / 2, norms.data(), seeds, cbp, np, cbr, 16, bs);
         expect(h != nullptr, tq_last_error());
     }
     ~Layer() { tq_linear_free(h); }
@@ -58,10 +60,26 @@ void reserve_without_memory() {
     expect(!Layer::ran("tq_compose_kernel"), "plane by plane");
 }
 
+// One row of 5-bit layers: the whole-row kernel takes two planes up to 8192 columns and blocks of 512, a primary alone is
+// a layer of one byte per weight.
+void five_bit_one_row() {
+    const struct { int in; uint32_t bs; bool residual; uint32_t seed; bool five; } cases[] = {
+        {1536, 512, true, 1234, true}, {1536, 512, true, 0, true}, {1536, 512, false, 0, false}, {8192, 512, true, 1234, true},
+        {8224, 32, true, 1234, false}, {3072, 1024, true, 1234, false}, {32, 2, true, 1234, true}};
+    for (const auto& c : cases) {
+        Layer layer(c.in, 64, 1, 5, c.residual, c.seed, c.bs);
+        expect(layer.forward(1) == 0, tq_last_error());
+        expect(Layer::ran("tq_gemv_five_kernel") == c.five, "the whole-row kernel", c.in);
+        expect(Layer::ran("tq_gemv_generic_kernel") == (c.residual && !c.five), "the generic kernel", c.in);
+        expect(!c.five || dev.launched.size() == 1, "one launch", dev.launched.size());
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const fake::Check checks[] = {{"compose_without_memory", compose_without_memory},
-                                  {"reserve_without_memory", reserve_without_memory}};
+                                  {"reserve_without_memory", reserve_without_memory},
+                                  {"five_bit_one_row", five_bit_one_row}};
     return fake::run(checks, argc, argv);
 }

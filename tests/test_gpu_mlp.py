@@ -221,7 +221,8 @@ def test_five_bit_two_plane_forward(tq, oracle, rbits, shared, out_f, in_f, bs, 
                                            (6, 8224, 4), (3, 16384, 512)])               # too wide: the generic kernel
 def test_five_bit_two_plane_one_row(tq, oracle, rbits, shared, out_f, in_f, bs):
     """One row at the edges of the whole-row kernel, fp32 throughout: 2e-6 is 16 units of rounding, more than the 11
-    stages of a butterfly and of the sums leave in a 2-norm.  Bytes beyond 31 count as 31."""
+    stages of a butterfly and of the sums leave in a 2-norm.  Bytes beyond 31 count as 31.  A primary alone (5+0) is a layer of one
+    byte per weight and takes the one-row kernels of those, in fp32 too."""
     o = oracle
     rng = np.random.default_rng(out_f + in_f)
     cbp = o.generate_codebook(5)

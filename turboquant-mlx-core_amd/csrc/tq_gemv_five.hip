@@ -1,5 +1,4 @@
-// One row of 5-bit layers that keep two planes (own residual rotation, or a 4-bit residual; byte primaries alone too),
-// for gfx950: metal/turboquant_dequant_mm.metal:240-248, 277-292; src/dequantizer.cpp:625-626, 657.
+// One row of 5-bit layers that keep two planes (own residual rotation, or a 4-bit residual), for gfx950: metal/turboquant_dequant_mm.metal:240-248, 277-292; src/dequantizer.cpp:625-626, 657.
 //
 //   y[r] = norm[r] / sqrt(in * bs) * ( sum_i cP[p(r,i)] x~p[i]  +  sum_i cR[q(r,i)] x~r[i] )
 //
@@ -76,7 +75,7 @@ __device__ __forceinline__ int row_of_lane(int lane) { return (lane & 1) * 2 + (
 
 template <int MODE>
 __global__ __launch_bounds__(64 * kFiveMaxWaves) void tq_gemv_five_kernel(FiveArgs a) {
-    constexpr bool dual = (MODE == kDual5), has_res = (MODE != kPrimaryOnly5);
+    constexpr bool dual = (MODE == kDual5);
     constexpr int R = kFiveRows;
     __shared__ float tabp[256];                              // (a byte plane may hold more than 31: src/dequantizer.cpp:94)
     __shared__ float tabr[16];
@@ -93,8 +92,7 @@ __global__ __launch_bounds__(64 * kFiveMaxWaves) void tq_gemv_five_kernel(FiveAr
         for (int r = 0; r < R; ++r) {
             const int row = group * R + r < a.out ? group * R + r : a.out - 1;
             pp[r] = *reinterpret_cast<const uint2*>(a.primary + (size_t)row * a.in + col);
-            if constexpr (has_res) qq[r] = *reinterpret_cast<const uint32_t*>(a.residual + (size_t)row * (a.in >> 1) + (col >> 1));
-            else qq[r] = 0;
+            qq[r] = *reinterpret_cast<const uint32_t*>(a.residual + (size_t)row * (a.in >> 1) + (col >> 1));
         }
     };
     load((int)blockIdx.x, p, q);
@@ -126,16 +124,12 @@ __global__ __launch_bounds__(64 * kFiveMaxWaves) void tq_gemv_five_kernel(FiveAr
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const float cp = tabp[((j < 4 ? p[r].x : p[r].y) >> (8 * (j & 3))) & 255u];
-                if constexpr (has_res) {
-                    const float cr = tabr[((j & 1 ? hi : lo) >> (8 * (j >> 1))) & 15u];
-                    if constexpr (dual) {
-                        t = __builtin_fmaf(cp, x0[j], t);
-                        u = __builtin_fmaf(cr, x1[j], u);
-                    } else {
-                        t = __builtin_fmaf(cp + cr, x0[j], t);                  // (src/dequantizer.cpp:186-212)
-                    }
-                } else {
+                const float cr = tabr[((j & 1 ? hi : lo) >> (8 * (j >> 1))) & 15u];
+                if constexpr (dual) {
                     t = __builtin_fmaf(cp, x0[j], t);
+                    u = __builtin_fmaf(cr, x1[j], u);
+                } else {
+                    t = __builtin_fmaf(cp + cr, x0[j], t);                      // (src/dequantizer.cpp:186-212)
                 }
             }
             if constexpr (dual) t += u;
@@ -163,7 +157,7 @@ __global__ __launch_bounds__(64 * kFiveMaxWaves) void tq_gemv_five_kernel(FiveAr
 }
 
 bool gemv_five_supported(const LayerView& L) {
-    if (L.mode != kShared5 && L.mode != kPrimaryOnly5 && L.mode != kDual5) return false;
+    if (L.mode != kShared5 && L.mode != kDual5) return false;          // (byte primaries alone run as a one-byte-per-weight layer)
     return L.block_size >= 2 && L.block_size <= 512 && L.in_features % 32 == 0 && L.in_features % (int)L.block_size == 0 &&
            L.in_features <= kFiveMaxCols;
 }
@@ -188,7 +182,6 @@ hipError_t launch_gemv_five(const LayerView& L, const void* x, int x_dtype, void
     const dim3 g((unsigned)grid), t((unsigned)(64 * waves));
     switch (L.mode) {
         case kShared5: hipLaunchKernelGGL(tq_gemv_five_kernel<kShared5>, g, t, 0, stream, a); break;
-        case kPrimaryOnly5: hipLaunchKernelGGL(tq_gemv_five_kernel<kPrimaryOnly5>, g, t, 0, stream, a); break;
         default: hipLaunchKernelGGL(tq_gemv_five_kernel<kDual5>, g, t, 0, stream, a); break;
     }
     return hipGetLastError();
