@@ -121,11 +121,15 @@ int tq_linear_reserve(tq_linear_t layer, int max_batch);
  * tq_last_error says how many bytes were needed) when layer and batch need more than that.  (From 16
  * rows on, a layer with few output tiles cuts K into ranges whose fp32 products are added afterwards:
  * here into as many ranges as the array holds, so the last bits of a result can differ from
- * tq_linear_forward's by the order of those sums.)  Each GPU has one such array, shared
+ * tq_linear_forward's by the order of those sums.  Two-plane layers whose planes tq_linear_forward composes into one
+ * fp16 weight, see tq_linear_reserve, are multiplied plane by plane where the slab does not fit the array: results
+ * then differ by the rounding of the weights to fp16, 3e-4 in the 2-norm, each as close to the exact result as the other.)
+ * Each GPU has one such array, shared
  * by every call on it and keeping the previous call's contents: calls that overlap on one GPU
  * (different streams or threads) race.  One row uses no part of the array (layers wider than 16384 columns,
- * widths that are not a multiple of 32 and 5-bit layers that keep two planes use the handle's own rotated row
- * at one row too: serialise calls per handle on those, as with tq_linear_forward).  The array's address on the
+ * widths that are not a multiple of 32 and 5-bit layers that keep two planes, where these are wider than 8192 columns or
+ * have blocks of 1024 or 2048, use the handle's own rotated row at one row too: serialise calls per handle on those, as
+ * with tq_linear_forward).  The array's address on the
  * current device is looked up when a layer is created, so the first call does no runtime work either.
  */
 #define TQ_STATIC_SCRATCH_BYTES (32u << 20)

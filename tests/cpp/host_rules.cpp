@@ -102,12 +102,16 @@ void compose_workspace() {
     // (the calls of the GPU tests of composed planes)
     const int calls[][5] = {{tq::kDual, 8260, 1280, 256, 513}, {tq::kDual, 8322, 1792, 128, 600}, {tq::kDual, 8322, 1792, 256, 513},
                             {tq::kDual, 6000, 1536, 512, 1030}, {tq::kDual5, 16500, 256, 32, 385}, {tq::kShared5, 16448, 512, 256, 400},
-                            {tq::kDual5, 8200, 1280, 256, 1024}, {tq::kDual, 33100, 2560, 512, 520}};
+                            {tq::kDual5, 8200, 1280, 256, 1024}, {tq::kDual5, 8200, 1280, 256, 600}, {tq::kDual, 33100, 2560, 512, 520}};
     for (const auto& c : calls) {
         tq::LayerView v = layer(c[0], c[2], c[1]);
         v.block_size = c[3];
         expect(tq::prefill_compose_supported(v, c[4], 256, ~(size_t)0), "a call that the GPU tests take to compose", c[1]);
     }
+    tq::LayerView fits = layer(tq::kDual, 1280, 8260), not_fits = layer(tq::kDual, 1792, 8322);
+    fits.block_size = 256; not_fits.block_size = 128;
+    expect(tq::prefill_compose_supported(fits, 513, 256, (size_t)32 << 20), "composed in the static array", 1280);
+    expect(!tq::prefill_compose_supported(not_fits, 600, 256, (size_t)32 << 20), "too large for the static array", 1792);
 }
 
 }  // namespace

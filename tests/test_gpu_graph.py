@@ -127,7 +127,9 @@ PANEL_BATCHES = (40, 130, 300, 600)
 
 @pytest.mark.parametrize("mode,out,inf,bs,BATCHES", [("shared", 640, 2048, 512, BATCHES), ("dual", 640, 2048, 512, BATCHES),
                                                      ("primary_only", 640, 2048, 512, BATCHES), ("dual_5bit", 640, 2048, 512, BATCHES),
-                                                     ("shared", 16500, 512, 256, PANEL_BATCHES), ("dual", 16500, 512, 256, PANEL_BATCHES)])
+                                                     ("shared", 16500, 512, 256, PANEL_BATCHES), ("dual", 16500, 512, 256, PANEL_BATCHES),
+                                                     ("dual", 8260, 1280, 256, (130, 513)),          # 513 rows: composed planes
+                                                     ("dual_5bit", 8200, 1280, 256, (40, 600))])     # 600 rows, too
 def test_reserved_layer_is_captured_and_replayed(tq, oracle, mode, out, inf, bs, BATCHES):
     o, hip = oracle, _Hip()
     layer, qw, cb = _layer(tq, o, out, inf, bs, mode)

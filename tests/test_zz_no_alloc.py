@@ -172,6 +172,32 @@ def test_static_forward_cuts_k_into_fewer_ranges_when_the_array_is_short(tq, ora
     layer.close()
 
 
+@pytest.mark.parametrize("out,inf,bs,batch,composed", [(8260, 1280, 256, 513, True), (8322, 1792, 128, 600, False)])
+def test_static_forward_where_planes_are_composed(tq, oracle, out, inf, bs, batch, composed):
+    """Two planes as one fp16 weight: 24 MB of workspace fit the array, 34 do not and the planes are multiplied one after the
+    other.  The same weights and fp32 sums of 1280 terms in another order at most (1e-6), or two roundings of the weights to fp16
+    (2.1e-4 each, independent: 3e-4; twice that)."""
+    hip = _Hip()
+    o = oracle
+    qw, cb = _make(o, out, inf, bs, "dual")
+    layer = tq.TurboQuantLinear(inf, out, qw, cb, cb, bs)
+    o.set_threads(8)
+    xbits = o.f32_to_bf16_bits(np.random.default_rng(80).standard_normal((batch, inf)).astype(np.float32))
+    ref = o.matmul_xwT(o.bf16_bits_to_f32(xbits), o.dequantize_weight_cpu(qw, cb, cb, bs), acc_double=True)
+    o.set_threads(1)
+    x_dev = hip.upload(xbits)
+    y_ref_dev, y_dev = hip.alloc(batch * out * 4), hip.alloc(batch * out * 4)
+    layer.forward_device(x_dev, tq.BF16, batch, y_ref_dev, tq.F32)
+    want = hip.download(y_ref_dev, (batch, out), np.float32)
+    layer.forward_static_device(x_dev, tq.BF16, batch, y_dev, tq.F32)
+    got = hip.download(y_dev, (batch, out), np.float32)
+    assert _rel(want, ref) < 1e-3 and _rel(got, ref) < 1e-3
+    assert _rel(got, want) < (1e-6 if composed else 6e-4)
+    assert composed or _rel(got, want) > 1e-5                  # (the case is the one that differs)
+    hip.free(x_dev, y_ref_dev, y_dev)
+    layer.close()
+
+
 def test_static_forward_refuses_a_workspace_beyond_the_array(tq, oracle):
     hip = _Hip()
     o = oracle
