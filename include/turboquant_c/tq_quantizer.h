@@ -60,8 +60,9 @@ int tq_quantize_weight_host(const float* weight_host, int out_features, int in_f
  * against the GLOBAL primary codebook, both from the analytic start, at most
  * `iterations` Lloyd-Max steps (the reference uses 100), stop when no centroid
  * moves by 1e-6.  Outputs 2^bits centroids each (residual untouched when
- * residual_bits == 0).  Needs 8*out*in bytes of temporary device memory and 150 MB (20*out*in where the samples'
- * values are so lumpy that all of them are sorted).
+ * residual_bits == 0).  Takes 8*out*in bytes of temporary device memory (20*out*in where the samples' values are so
+ * lumpy that all of them are sorted), 25 MB, and 90 MB for every started 2^27 weights; where that cannot be had,
+ * 4*out*in bytes and a pass over all weights per step, some hundred times slower.
  */
 int tq_fit_layer_codebooks(const float* weight_dev, int out_features, int in_features,
                            uint32_t block_size, int primary_bits, int residual_bits,
