@@ -132,8 +132,8 @@ template <int MODE> struct DequantMode {
 // COMBINED: the layer's one-byte-per-weight plane (kSharedLut; kShared5 and kPrimaryOnly5 where the residual index fits
 // the byte's top three bits).
 //
-// Bound by its vector instructions (about 30 per weight in dual rotation: two butterflies of 9, lookups and exchange,
-// signs, sum, norm and conversion; 16 in shared rotation) and by three waves per SIMD (registers, 11 KB of LDS per wave).
+// Bound by its vector instructions (39 per weight in dual rotation: two butterflies of 9, lookups and exchange,
+// signs, sum, norm and conversion) and by three waves per SIMD (registers, 11 KB of LDS per wave).
 // 27648 x 5120 to bf16: dual 364 -> 152 us (2.8 TB/s of planes and weights), shared 104.  Before, a lane kept 32 consecutive
 // columns throughout: four more stages across lanes at two to three instructions per value, two sign hashes per weight,
 // 64-byte pieces per lane in every store, and idle lanes behind the last 2048 columns of a row.
@@ -307,7 +307,8 @@ hipError_t launch_dequant(const LayerView& L, void* w, int w_dtype, hipStream_t 
 // closer).  kShared5: both planes in one rotation, a plain sum.
 // Rows [row0, row0 + rows) of the layer (row0 a multiple of 128), in the order in which tq_prefill_panel_kernel's threads
 // load them: [row / 128][K / 64][4 pieces of 8 columns][row % 128 / 32][half of the 64 columns][row % 32] x 16 bytes.
-// Bound by its vector instructions (28 per weight); 27648 x 5120 in 140 us, a sixth of the contraction it halves at 2048 rows.
+// Bound by its vector instructions (38 per weight); 27648 x 5120 in two slabs of 76 us, a quarter of the contraction at 2048
+// rows.
 // Four waves per SIMD (128 registers) spill and are 10 % slower.
 // A wave takes 512 columns (whole blocks: at most 512) of four rows, 16 lanes each, and eight waves in a row the same
 // columns of 32 rows; exchange as above.

@@ -9,8 +9,9 @@
 // The generic kernel (tq_generic.hip) read both rotated rows again for every weight row, 8 bytes of them per weight from
 // the L1 against 1.5 of indices, and needed a launch for the rotation.  us per call, dual rotation, bf16, before -> now, in x
 // out: 5120 x 13824 44.4 -> 29.2 (3.6 TB/s), 5120 x 27648 78.9 -> 52.3 (4.1 TB/s), 3584 x 18944 41.3 -> 29.9, 8192 x 8192 41.8
-// -> 29.3, 2048 x 2048 9.8 -> 7.2.  What bounds it: two table reads and about five vector instructions per weight, and
-// the rotation every workgroup repeats (a few us, hence few workgroups: 20 waves per CU; 28 measured the same).  Two rows
+// -> 29.3, 2048 x 2048 9.8 -> 7.2.  What bounds it: ten vector instructions per weight with both planes (the vector
+// units are busy 82 % of the time) and two table reads, and the rotation every workgroup repeats (a few us, hence few
+// workgroups: 20 waves per CU; 28 measured the same).  Two rows
 // at a time took 38.0 us for 5120 x 13824.  Rows beyond 8192 columns would give a wave two segments and twice the rotation:
 // 13824 x 5120 45.4 -> 37.2, but 9728 x 3584 26.3 -> 30.6, so they stay with the generic kernel.
 #include "tq_device.h"

@@ -286,7 +286,7 @@ size_t prefill_tile_workspace_bytes(const LayerView& L, int batch) {
 // The shape with the shortest estimate, in us without the rotation, fitted to seven layer shapes x five row counts
 // (40 to 1024) per mode: rounds of workgroups on the CUs, each a fixed cost (table, first requests, sum over the waves,
 // stores) and a cost per 64-column tile of the row, which is what a CU's loads deliver (20 to 36 bytes per clock; the
-// matrix units are busy a fifth of the time with 32-row tiles, a third with 64 x 64).  The 256 x 256 tiles of
+// matrix units are busy 6 to 12 % of the time with 32-row tiles, 19 % with 64 x 64, the vector units 16 to 33 %).  The 256 x 256 tiles of
 // tq_prefill.hip: 0.8 us per 32-column step of a range, and the ranges' products written and read again.  Where
 // 512 x 128 tiles fill the chip (prefill_panel_supported) they are faster throughout.
 //   us per call before -> now, bf16:  dual rotation, in x out: 896 x 4864 at 77 rows 57.7 -> 17.9, at 512 rows 60.3 -> 36.2;
