@@ -377,10 +377,12 @@ def test_prefill_composed_planes_match_dequant_matmul(tq, oracle, monkeypatch, m
     L2, 5e-3 in bf16."""
     monkeypatch.setitem(MODES, "5+4dual", dict(pb=5, rb=4, shared=False))
     monkeypatch.setitem(MODES, "5+4shared", dict(pb=5, rb=4, shared=True))
+    oracle.set_threads(8)
     qw, cbp, cbr = _make(oracle, out, inf, bs, mode)
     x32 = np.random.default_rng(batch).standard_normal((batch, inf)).astype(np.float32)
     xbits = oracle.f32_to_bf16_bits(x32)
     want = oracle.linear_forward(qw, cbp, cbr, bs, oracle.bf16_bits_to_f32(xbits))
+    oracle.set_threads(1)
     layer = tq.TurboQuantLinear(inf, out, qw, cbp, cbr, bs)
     layer.reserve(batch)
     y = layer.forward(xbits, tq.BF16, tq.F32)
@@ -403,8 +405,10 @@ def test_prefill_composed_planes_lose_no_precision(tq, oracle, codebook):
         cb = oracle.fit_layer_codebooks(w, bs)
     if codebook == "fp16":
         cb = [oracle.Codebook(c.centroids.astype(np.float16).astype(np.float32), 4) for c in cb]
+    oracle.set_threads(8)
     qw = oracle.quantize_weight(w, *cb, 4, 4, bs, False)
     want = oracle.dequantize_weight_cpu(qw, *cb, bs).T[:512]
+    oracle.set_threads(1)
     x = np.zeros((513, inf), np.float32)
     x[np.arange(513), np.arange(513)] = 1.0
     layer = tq.TurboQuantLinear(inf, out, qw, *cb, bs)

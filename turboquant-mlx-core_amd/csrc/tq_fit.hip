@@ -569,6 +569,7 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_iterate_kernel(const FitPa
     const float* fine = fine_all + fit_region(kept, p);
     if (tid == 0) { left_n[0] = 0; left_q[0] = 0; left_n[nc] = n; left_q[nc] = below[kFitCells]; }
     __syncthreads();
+    const unsigned long long cut_lo = start[kFitHalf - kFitCut], cut_hi = start[kFitHalf + kFitCut];
     int iter = out->steps[p];
     for (; iter < iterations; ++iter) {
         for (int k = wave; k < nc - 1; k += kFitThreads / kWave) {
@@ -619,16 +620,16 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_iterate_kernel(const FitPa
                 if (c > 0) {                                                         // src/codebook.cpp:124-129
                     const double s = i128_to_double(left_q[lane + 1] - left_q[lane]) * unit;
                     const float nv = (float)(s / (double)c);
-                    // each of the bin's samples around zero may have lost up to one unit
-                    const unsigned long long from = max(left_n[lane], (unsigned long long)start[kFitHalf - kFitCut]);
-                    const unsigned long long to = min(left_n[lane + 1], (unsigned long long)start[kFitHalf + kFitCut]);
-                    if (from < to && (double)(to - from) * unit > (double)fabsf(nv) * 0x1p-26 * (double)c) coarse = 1;
                     shift = fabsf(nv - cent[lane]);
                     cent[lane] = nv;
                 }
             }
             for (int m = 32; m >= 1; m >>= 1) shift = fmaxf(shift, __shfl_xor(shift, m, kWave));
             if (lane == 0) stop = shift < 1e-6f ? 1 : 0;                             // src/codebook.cpp:132
+        } else if (wave == 1 && lane < nc) {
+            // each of a bin's samples around zero may have lost up to one unit; the centroid again, beside wave 0
+            const unsigned long long from = max(left_n[lane], cut_lo), to = min(left_n[lane + 1], cut_hi);
+            if (from < to && (double)(to - from) > fabs(i128_to_double(left_q[lane + 1] - left_q[lane])) * 0x1p-26) coarse = 1;
         }
         __syncthreads();
         if (stop || coarse) break;
