@@ -75,11 +75,38 @@ void five_bit_one_row() {
     }
 }
 
+// Which calls run on operands of two parts, and that those whose workspace cannot be had run on the fp32 kernels as before:
+// captured without a reservation, no memory.
+void two_parts() {
+    const struct { int in; uint32_t bs, seed; bool residual; int rows; const char* kernel; } cases[] = {
+        {1056, 32, 0, true, 4, "tq_gemv"},        {1056, 32, 0, true, 5, "tq_rotate_split"}, {1056, 32, 0, true, 300, "tq_rotate_split"},
+        {1056, 32, 1, true, 3, "tq_gemv"},        {1056, 32, 1, true, 4, "tq_rotate_split"}, {1056, 32, 1, false, 4, "tq_gemv"},
+        {1088, 64, 1, true, 15, "tq_rotate_split"}, {1088, 64, 1, true, 16, "tq_rotate_panel"}, {1088, 64, 0, true, 15, "tq_skinny"},
+        {1024, 512, 1, true, 15, "tq_skinny"},    {1048, 8, 1, true, 40, "tq_gemv_generic"}};
+    for (const auto& c : cases) {
+        Layer layer(c.in, 70, c.rows, 4, c.residual, c.seed, c.bs);
+        expect(layer.forward(c.rows) == 0, tq_last_error(), c.in);
+        expect(Layer::ran(c.kernel), c.kernel, c.in * 1000 + c.rows);
+        expect(Layer::ran("tq_rotate_split") == (std::strcmp(c.kernel, "tq_rotate_split") == 0), "two parts", c.in * 1000 + c.rows);
+    }
+    Layer captured(1056, 70, 40, 4, true, 0, 32), reserved(1056, 70, 40, 4, true, 0, 32), poor(1056, 70, 40, 4, true, 0, 32);
+    expect(tq_linear_reserve(reserved.h, 40) == 0, tq_last_error());
+    dev.capturing = true;
+    expect(captured.forward(40) == 0 && !Layer::ran("tq_rotate_split") && !dev.launched.empty(), "captured, not reserved");
+    expect(reserved.forward(40) == 0 && Layer::ran("tq_rotate_split"), "captured, reserved");
+    expect(reserved.forward(5) == 0 && Layer::ran("tq_rotate_split"), "captured, fewer rows than reserved");
+    dev.capturing = false;
+    dev.size = dev.live + 100000;                          // (what fewer rows need)
+    expect(tq_linear_reserve(poor.h, 40) == 0, tq_last_error());
+    expect(poor.forward(40) == 0 && !Layer::ran("tq_rotate_split") && !dev.launched.empty(), "no memory");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const fake::Check checks[] = {{"compose_without_memory", compose_without_memory},
                                   {"reserve_without_memory", reserve_without_memory},
-                                  {"five_bit_one_row", five_bit_one_row}};
+                                  {"five_bit_one_row", five_bit_one_row},
+                                  {"two_parts", two_parts}};
     return fake::run(checks, argc, argv);
 }

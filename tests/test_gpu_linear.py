@@ -678,6 +678,59 @@ def test_matrix_core_paths_hold_their_tolerance_over_the_fp16_range(tq, oracle, 
     layer.close()
 
 
+# Operands in two fp16 parts: what the fp16 kernels do not take (odd multiples of 32 columns; nibble planes of odd multiples of 64 below
+# 16 rows; centroids beyond fp16), at the precision of the fp32 kernels.
+@pytest.mark.parametrize("mode", ["shared", "dual", "primary_only", "shared_3bit_res"])
+@pytest.mark.parametrize("out,inf,bs,batch", [(3, 32, 32, 5),              # half a tile for eight waves, less than a tile of outputs
+                                              (130, 96, 32, 33), (65, 992, 16, 64), (257, 1056, 32, 31), (64, 4128, 32, 6),
+                                              (600, 544, 32, 700),         # many tiles of 64 x 128
+                                              (40, 1088, 64, 15),          # whole tiles (nibble planes alone)
+                                              (33, 16416, 32, 5)])         # rotated by nine waves
+def test_two_part_operands_keep_fp32_precision(tq, oracle, mode, out, inf, bs, batch):
+    if mode.startswith("shared") and inf % 64 == 0:         # (multiples of 64 have fp16 kernels)
+        inf, bs = inf - 32, 32
+    qw, cbp, cbr = _make(oracle, out, inf, bs, mode)
+    layer = tq.TurboQuantLinear(inf, out, qw, cbp, cbr, bs)
+    rng = np.random.default_rng(out + inf + batch)
+    x = rng.standard_normal((batch, inf)).astype(np.float32)
+    x[0] *= np.float32(2.0 ** 60)                           # (every row has a scale of its own)
+    x[1] *= np.float32(2.0 ** -60)
+    x[2, : inf // 2] = 0
+    x[3] = 0
+    w = oracle.dequantize_weight_cpu(qw, cbp, cbr, bs).astype(np.float64)
+    want = x.astype(np.float64) @ w.T
+    y = layer.forward(x)
+    # 1.6e-7 was the largest seen against 64 bits; the oracle's weights are rounded as often as the rotated activations are
+    # (1e-7), and 96 columns average less out than 1000.
+    tol = 6e-7
+    for b in range(batch):
+        if b != 3:
+            assert _rel(y[b], want[b]) < 4 * tol, b
+    assert _rel(y[4:], want[4:]) < tol and np.all(y[3] == 0)
+    x16 = oracle.f32_to_bf16_bits(x)
+    yb = layer.forward(x16, tq.BF16, tq.F32)
+    wantb = oracle.bf16_bits_to_f32(x16).astype(np.float64) @ w.T
+    assert _rel(yb[4:], wantb[4:]) < tol
+    layer.close()
+
+
+@pytest.mark.parametrize("mode", ["shared", "dual", "primary_only"])
+def test_two_part_operands_centroids_beyond_fp16(tq, oracle, mode):
+    out, inf, bs, batch = 70, 512, 512, 40
+    qw, cbp, cbr = _make(oracle, out, inf, bs, mode)
+    cbp, cbr = (oracle.Codebook(c.centroids * np.float32(1e6), c.bits) for c in (cbp, cbr))
+    layer = tq.TurboQuantLinear(inf, out, qw, cbp, cbr, bs)
+    x = np.random.default_rng(7).standard_normal((batch, inf)).astype(np.float32)
+    want = x.astype(np.float64) @ oracle.dequantize_weight_cpu(qw, cbp, cbr, bs).astype(np.float64).T
+    assert _rel(layer.forward(x), want) < 6e-7
+    x[5, 3] = np.inf
+    x[6, 9] = np.nan
+    y = layer.forward(x)
+    keep = [b for b in range(batch) if b not in (5, 6)]
+    assert _rel(y[keep], want[keep]) < 6e-7 and np.isnan(y[6]).all() and not np.isfinite(y[5]).any()
+    layer.close()
+
+
 def _random_cases(n, seed):
     rng = np.random.default_rng(seed)
     cases = []

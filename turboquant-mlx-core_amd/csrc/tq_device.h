@@ -40,6 +40,8 @@ struct LayerView {
     int fp16_centroids_ok;           // every centroid fits fp16 with room to spare (the byte-pair tables of the
                                      // batch-1 kernel hold fp16 values); otherwise fp32 tables are used
     float compose_scale;             // two planes kept as such: what their fp16 sum is multiplied by (launch_compose); 0: not composed
+    const uint32_t* split_tables;    // the entries of `tables` times 2^-split_exp as two fp16 parts, hi << 16 | lo (tq_prefill_tile.hip),
+    int split_exp;                   // or NULL: they do not fit
     float* xrot_work;                // scratch of 2 * in_features floats (rows wider than 16384 columns: the
                                      // batch-1 path rotates the activations once, in a kernel of its own), or NULL
 };

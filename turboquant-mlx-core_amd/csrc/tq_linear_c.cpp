@@ -163,6 +163,42 @@ void build_tables(int mode, const float* cbp, int np, const float* cbr, int nr, 
     for (int i = 0; i < 16; ++i) t[pn + i] = cbr[i < nr ? i : nr - 1];
 }
 
+// A decode table on its way to the device: 256 floats and, behind them, the first `used` of them as two fp16 parts each,
+// c * 2^-exp = hi + lo (hi << 16 | lo), exp such that the largest is between 2^14 and 2^15: what lo leaves off is at most
+// 2^-24 of the entry or 2^-40 of the largest.  Tables with entries that are not finite, or further apart than 2^16, have none
+// (entries of 0 aside).
+struct DecodeTable {
+    uint32_t words[512];
+    bool split;
+    int exp;
+    DecodeTable(const float* t, int used) : words{}, split(true), exp(0) {
+        std::memcpy(words, t, 256 * sizeof(float));
+        float big = 0.0f, small = INFINITY;
+        for (int i = 0; i < used; ++i) {
+            const float a = std::fabs(t[i]);
+            if (!(a < INFINITY)) split = false;
+            if (a > big) big = a;
+            if (a > 0.0f && a < small) small = a;
+        }
+        if (!split || big < 0x1p-100f || small < big * 0x1p-16f) { split = false; return; }
+        exp = std::ilogb(big) - 14;
+        for (int i = 0; i < used; ++i) {
+            const float c = std::ldexp(t[i], -exp);
+            const _Float16 hi = (_Float16)c, lo = (_Float16)(c - (float)hi);
+            uint16_t hb, lb;
+            std::memcpy(&hb, &hi, 2);
+            std::memcpy(&lb, &lo, 2);
+            words[256 + i] = (uint32_t)hb << 16 | lb;
+        }
+    }
+    bool upload(float* dev) const { return hip_ok(hipMemcpy(dev, words, sizeof(words), hipMemcpyHostToDevice), "copy tables"); }
+    void set(tq::LayerView& v, const float* dev) const {
+        v.tables = dev;
+        v.split_tables = split ? reinterpret_cast<const uint32_t*>(dev + 256) : nullptr;
+        v.split_exp = exp;
+    }
+};
+
 // Grows a workspace of a handle.  A buffer that a captured graph may still reference is never
 // replaced while the stream is being captured: growth during capture is an error.
 // Grows *buf to at least `need` bytes.  Refused while `stream` is being captured (an allocation cannot be
@@ -225,7 +261,7 @@ tq_linear_t create_impl(int in_features, int out_features,
     bool ok = hip_ok(tq::device_malloc((void**)&h->d_primary, pbytes), "hipMalloc(packed_primary)") &&
               hip_ok(tq::device_malloc((void**)&h->d_residual, rbytes), "hipMalloc(packed_residual)") &&
               hip_ok(tq::device_malloc((void**)&h->d_norms, (size_t)out_features * sizeof(float)), "hipMalloc(norms)") &&
-              hip_ok(tq::device_malloc((void**)&h->d_tables, 256 * sizeof(float)), "hipMalloc(tables)") &&
+              hip_ok(tq::device_malloc((void**)&h->d_tables, sizeof(DecodeTable::words)), "hipMalloc(tables)") &&
               hip_ok(hipMemcpy(h->d_primary, pp, pbytes, kind), "copy packed_primary") &&
               hip_ok(hipMemcpy(h->d_residual, pr, rbytes, kind), "copy packed_residual") &&
               hip_ok(hipMemcpy(h->d_norms, norms, (size_t)out_features * sizeof(float), kind), "copy norms");
@@ -253,9 +289,8 @@ tq_linear_t create_impl(int in_features, int out_features,
 
     float tables[256];
     build_tables(mode, cbp, np, cbr, nr, tables);
-    if (!hip_ok(hipMemcpy(h->d_tables, tables, sizeof(tables), hipMemcpyHostToDevice), "copy tables")) {
-        delete h; return nullptr;
-    }
+    const DecodeTable table(tables, mode == tq::kSharedLut ? 256 : mode == tq::kDual ? 32 : mode == tq::kPrimaryOnly ? 16 : 0);
+    if (!table.upload(h->d_tables)) { delete h; return nullptr; }
 
     if (mode == tq::kSharedLut) {
         // The shared-rotation kernels stream one byte per weight; interleave the planes once and drop them.
@@ -269,19 +304,19 @@ tq_linear_t create_impl(int in_features, int out_features,
     }
 
     // (a primary-only layer never reads its residual codebook, whatever its length)
+    float lut[256];
+    std::memset(lut, 0, sizeof(lut));
     const bool fused5 = (mode == tq::kShared5 && nr <= 8) || mode == tq::kPrimaryOnly5;
     if (fused5) {
         const size_t cbytes = (size_t)out_features * in_features;
-        float lut[256];
-        std::memset(lut, 0, sizeof(lut));
         for (int r = 0; r < 8; ++r)
             for (int p5 = 0; p5 < 32; ++p5) {
                 const float c = cbp[p5 < np ? p5 : np - 1];
                 lut[(r << 5) | p5] = mode == tq::kShared5 ? c + cbr[r < nr ? r : nr - 1] : c;   // src/dequantizer.cpp:186-212
             }
         ok = hip_ok(tq::device_malloc((void**)&h->d_combined, cbytes), "hipMalloc(packed_combined)") &&
-             hip_ok(tq::device_malloc((void**)&h->d_tables_fwd, sizeof(lut)), "hipMalloc(tables)") &&
-             hip_ok(hipMemcpy(h->d_tables_fwd, lut, sizeof(lut), hipMemcpyHostToDevice), "copy tables") &&
+             hip_ok(tq::device_malloc((void**)&h->d_tables_fwd, sizeof(DecodeTable::words)), "hipMalloc(tables)") &&
+             DecodeTable(lut, 256).upload(h->d_tables_fwd) &&
              hip_ok(tq::launch_combine_planes5(h->d_primary, h->d_residual, h->d_combined, rbytes, np < 32 ? np : 32, nr,
                                                nullptr), "combine_planes5") &&
              hip_ok(hipDeviceSynchronize(), "combine_planes5 sync");
@@ -297,7 +332,7 @@ tq_linear_t create_impl(int in_features, int out_features,
     v.packed_residual = h->d_residual;
     v.packed_combined = h->d_combined;
     v.norms = h->d_norms;
-    v.tables = h->d_tables;
+    table.set(v, h->d_tables);
     v.out_features = out_features;
     v.in_features = in_features;
     v.block_size = block_size;
@@ -323,17 +358,17 @@ tq_linear_t create_impl(int in_features, int out_features,
     if (fused5) {
         h->fwd_view = v;
         h->fwd_view.mode = tq::kSharedLut;
-        h->fwd_view.tables = h->d_tables_fwd;
+        DecodeTable(lut, 256).set(h->fwd_view, h->d_tables_fwd);
         h->has_fwd_view = true;
     } else if (mode >= tq::kShared5 && tq::lanes_supported(in_features, block_size)) {
         float ta[256], tb[256];
         std::memset(tb, 0, sizeof(tb));
         for (int b = 0; b < 256; ++b) ta[b] = cbp[b < np ? b : np - 1];          // index clamp of src/dequantizer.cpp:94
         for (int i = 0; i < 16; ++i) tb[i] = cbr[i < nr ? i : nr - 1];            // :103
-        ok = hip_ok(tq::device_malloc((void**)&h->d_tables_plane[0], sizeof(ta)), "hipMalloc(tables)") &&
-             hip_ok(tq::device_malloc((void**)&h->d_tables_plane[1], sizeof(tb)), "hipMalloc(tables)") &&
-             hip_ok(hipMemcpy(h->d_tables_plane[0], ta, sizeof(ta), hipMemcpyHostToDevice), "copy tables") &&
-             hip_ok(hipMemcpy(h->d_tables_plane[1], tb, sizeof(tb), hipMemcpyHostToDevice), "copy tables");
+        const DecodeTable planes[2] = {DecodeTable(ta, 256), DecodeTable(tb, 16)};
+        for (int k = 0; k < 2 && ok; ++k)
+            ok = hip_ok(tq::device_malloc((void**)&h->d_tables_plane[k], sizeof(DecodeTable::words)), "hipMalloc(tables)") &&
+                 planes[k].upload(h->d_tables_plane[k]);
         if (!ok) { delete h; return nullptr; }
         tq::LayerView& a = h->plane_view[0];
         a = v;
@@ -341,7 +376,7 @@ tq_linear_t create_impl(int in_features, int out_features,
         a.packed_combined = h->d_primary;
         a.packed_primary = nullptr;
         a.packed_residual = nullptr;
-        a.tables = h->d_tables_plane[0];
+        planes[0].set(a, h->d_tables_plane[0]);
         a.seed_residual = 0;
         a.compose_scale = 0.0f;
         tq::LayerView& b = h->plane_view[1];
@@ -350,7 +385,7 @@ tq_linear_t create_impl(int in_features, int out_features,
         b.packed_primary = h->d_residual;
         b.packed_residual = nullptr;
         b.packed_combined = nullptr;
-        b.tables = h->d_tables_plane[1];
+        planes[1].set(b, h->d_tables_plane[1]);
         b.seed_primary = mode == tq::kDual5 ? seeds[1] : seeds[0];
         b.seed_residual = 0;
         b.compose_scale = 0.0f;
@@ -407,6 +442,14 @@ int forward_view(tq_linear_s* h, const tq::LayerView& V, bool generic_only, cons
     }
     const bool skinny = lanes && !gate && tq::skinny_supported(V, x_dtype, batch);
     const bool prefill = lanes && !skinny && !gate && tq::prefill_supported(V, x_dtype, batch);
+    // (odd multiples of 32 columns, nibble planes of odd multiples of 64 at few rows, centroids beyond fp16: two fp16 parts per operand,
+    // where its workspace can be had without an allocation that is refused)
+    if (lanes && !skinny && !prefill && !gate && tq::prefill_split_supported(V, batch)) {
+        const size_t need = tq::prefill_split_workspace_bytes(V, batch);
+        if (static_ws ? need <= static_cap : ensure_stage(&h->d_work, &h->work_bytes, need, stream, &h->retired))
+            return hip_ok(tq::launch_prefill_split(V, x_dev, x_dtype, batch, y_dev, y_dtype, static_ws ? static_ws : h->d_work,
+                                                   device_cu_count(), stream), "tq_prefill_split launch") ? 0 : 1;
+    }
     if (!prefill && !skinny && (generic_only || !tq::shape_supported(V.in_features, V.block_size))) {
         if (!tq::generic_supported(V)) { set_error("tq_linear_forward: unsupported layer shape"); return 1; }
         return hip_ok(tq::launch_gemv_generic(V, x_dev, x_dtype, batch, y_dev, y_dtype, device_cu_count(), stream, gate),
@@ -567,6 +610,13 @@ int tq_linear_forward(tq_linear_t h, const void* x_dev, int x_dtype, int batch,
 namespace {
 // Workspace of the whole-row kernel (2..12 rows) for every batch up to max_batch, thrice: the first layer of a group holds
 // the rotated rows of all its layers.
+size_t split_reserve_bytes(const tq::LayerView& V, int max_batch) {
+    size_t need = 0;
+    for (int b : {15, max_batch})                          // (16 rows and more of some layers take other kernels)
+        if (b <= max_batch && tq::prefill_split_supported(V, b) && !tq::prefill_supported(V, tq::kBF16, b))
+            need = std::max(need, tq::prefill_split_workspace_bytes(V, b));
+    return need;
+}
 size_t few_reserve_bytes(const tq::LayerView& V, int max_batch) {
     size_t need = 0;
     for (int b = 2; b <= max_batch && b <= 12; ++b) need = std::max(need, 3 * tq::gemv_few_workspace_bytes(V, b));
@@ -575,10 +625,11 @@ size_t few_reserve_bytes(const tq::LayerView& V, int max_batch) {
 }  // namespace
 
 namespace {
-// The workspace with room for composed planes, or, where that cannot be had, without (such calls run plane by plane then).
-bool reserve_work(tq_linear_s* h, size_t bytes, size_t with_composed) {
-    return ensure_stage(&h->d_work, &h->work_bytes, with_composed, nullptr, &h->retired) ||
-           (bytes < with_composed && ensure_stage(&h->d_work, &h->work_bytes, bytes, nullptr, &h->retired));
+// The workspace with room for composed planes and operands in two parts, or, where that cannot be had, without (such calls run
+// plane by plane, or on the fp32 kernels, then).
+bool reserve_work(tq_linear_s* h, size_t bytes, size_t with_all) {
+    return ensure_stage(&h->d_work, &h->work_bytes, with_all, nullptr, &h->retired) ||
+           (bytes < with_all && ensure_stage(&h->d_work, &h->work_bytes, bytes, nullptr, &h->retired));
 }
 }  // namespace
 
@@ -587,7 +638,7 @@ int tq_linear_reserve(tq_linear_t h, int max_batch) {
         if (!h || max_batch <= 0) { set_error("tq_linear_reserve: bad argument"); return 1; }
         if (max_batch < 2) return 0;                       // one row uses no workspace
         if (h->has_plane_views) {                          // two planes, each a layer of its own, plus their fp32 results
-            size_t work = 0, part = 0;
+            size_t work = 0, part = 0, split = 0;
             for (int k = 0; k < 2; ++k) {
                 const tq::LayerView& P = h->plane_view[k];
                 const int rows = max_batch < tq::kSkinnyMaxRows ? max_batch : tq::kSkinnyMaxRows;
@@ -596,9 +647,11 @@ int tq_linear_reserve(tq_linear_t h, int max_batch) {
                 const size_t big = max_batch >= 16 ? tq::prefill_reserve_bytes(P, max_batch, device_cu_count()) : 0;
                 work = std::max(work, std::max(small, big));
                 work = std::max(work, few_reserve_bytes(P, max_batch));
+                split = std::max(split, split_reserve_bytes(P, max_batch));
                 if (sk) part = std::max(part, tq::skinny_partial_bytes(P, rows));
             }
-            if (!reserve_work(h, work, std::max(work, tq::prefill_compose_reserve_bytes(h->view, max_batch, device_cu_count())))) return 1;
+            const size_t composed = tq::prefill_compose_reserve_bytes(h->view, max_batch, device_cu_count());
+            if (!reserve_work(h, work, std::max(work, std::max(split, composed)))) return 1;
             if (!ensure_stage(&h->d_partial, &h->partial_bytes, part, nullptr, &h->retired)) return 1;
             if (!ensure_stage(&h->d_sum, &h->sum_bytes, plane_sum_bytes(h, max_batch, tq::kBF16), nullptr, &h->retired)) return 1;
             return 0;
@@ -613,7 +666,7 @@ int tq_linear_reserve(tq_linear_t h, int max_batch) {
         const size_t few = few_reserve_bytes(V, max_batch);
         const size_t work = std::max(few, std::max(small, big));
         const size_t composed = pf ? tq::prefill_compose_reserve_bytes(V, max_batch, device_cu_count()) : 0;
-        if (!reserve_work(h, work, std::max(work, composed))) return 1;
+        if (!reserve_work(h, work, std::max(work, std::max(split_reserve_bytes(V, max_batch), composed)))) return 1;
         if (sk && !ensure_stage(&h->d_partial, &h->partial_bytes, tq::skinny_partial_bytes(V, rows), nullptr, &h->retired)) return 1;
         return 0;
     } catch (...) { set_error("tq_linear_reserve: exception"); return 1; }

@@ -57,5 +57,11 @@ int prefill_tile_shape(const LayerView& L, int batch, int num_cus);
 size_t prefill_tile_workspace_bytes(const LayerView& L, int batch);
 hipError_t launch_prefill_tile(const LayerView& L, int shape, const void* x, int x_dtype, int batch, void* y, int y_dtype,
                                void* workspace, hipStream_t stream);
+// The same kernel on operands of two fp16 parts each, for the calls of two and more rows that no fp16 path takes (fp32 precision).
+// Workspace: fragment images of both parts, then an exponent per row.
+bool prefill_split_supported(const LayerView& L, int batch);
+size_t prefill_split_workspace_bytes(const LayerView& L, int batch);
+hipError_t launch_prefill_split(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
+                                void* workspace, int num_cus, hipStream_t stream);
 
 }  // namespace tq

@@ -32,21 +32,28 @@ struct TileArgs {
     int M, N, K;
     int m_tiles, n_tiles;
     float out_scale;
+    const int* row_exp;        // two parts: rows of the images are times 2^-row_exp, entries of the table times 2^-table_exp
+    int table_exp;
 };
 
 }  // namespace
 
 // MB x NB blocks of 32 x 32 outputs per wave; KS waves share them along K, WN such groups stand side by side along N.
 // SUB: 64-column tiles that a lane's weights are loaded for at once (a whole number of them in a row).
-template <int MODE, int SUB, int MB, int NB, int KS, int WN>
+// PARTS = 2: every operand is the sum of two fp16 values, hi + lo, and a product the sum of four: fp32 precision at four matrix
+// instructions where v_mfma_f32_32x32x2_f32 would take the time of sixteen.  The images of the lo parts follow those of the hi
+// parts (zeros from K to a whole 64-column tile), the table is L.split_tables.
+template <int MODE, int SUB, int MB, int NB, int KS, int WN, int PARTS>
 __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileArgs a) {
     constexpr bool combined = (MODE == kSharedLut);
     constexpr int kPlanes = (MODE == kDual) ? 2 : 1;
     constexpr int kWaves = KS * WN;
     constexpr int kBlocks = MB * NB;
-    constexpr int kLut = 256 * 256;                        // lane-private table, 256 entries x 64 lanes x 4 bytes
+    constexpr bool split = PARTS == 2;
+    constexpr int kEntries = !split || combined ? 256 : 16 * kPlanes;
+    constexpr int kLut = kEntries * 256;                   // lane-private table, 64 lanes x 4 bytes per entry
     constexpr int kExchange = kWaves * kBlocks * 4096;     // [wave][block][register][lane] floats, over the table
-    constexpr int D = MB == 1 ? 4 : 2;
+    constexpr int D = (MB == 1 ? 4 : 2) / PARTS;
     constexpr int PV = combined ? 2 : 1;                   // 16-byte pieces of 32 columns
     constexpr int BV = SUB * PV;
     constexpr int BR = D / SUB > 2 ? D / SUB : 2;
@@ -64,10 +71,11 @@ __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileArgs 
     const int n0 = n_tile * (32 * NB * WN), m0 = m_tile * (32 * MB);
 
     // Weight tiles (64 SUB columns) of this wave, the second plane's after the first's.
-    const int T = (a.K >> 6) / SUB, total = T * kPlanes;
+    const int U = split ? ((a.K + 63) >> 6) * 4 : a.K >> 4;        // 16-column steps of an image
+    const int T = (U >> 2) / SUB, total = T * kPlanes;
     const int t_begin = total * ks / KS, t_end = total * (ks + 1) / KS;
 
-    const size_t plane_stride = (size_t)((a.M + 31) >> 5) * (a.K >> 4) * 1024;
+    const size_t part_stride = (size_t)((a.M + 31) >> 5) * U * 1024, plane_stride = PARTS * part_stride;
     // (uniform base addresses and 32-bit lane offsets throughout: with a 64-bit address per lane a third of the loop's
     // instructions computed addresses)
     const uint32_t aoff = (uint32_t)(g * (SUB * 2048) + l * 16);
@@ -76,7 +84,7 @@ __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileArgs 
     for (int i = 0; i < MB; ++i) {
         int rb = m_tile * MB + i;                          // row block; past the call: the last one again, never stored
         if (rb * 32 >= a.M) rb = (a.M - 1) >> 5;
-        ap[i] = a.xt + (size_t)rb * (a.K >> 4) * 1024;
+        ap[i] = a.xt + (size_t)rb * U * 1024;
     }
     uint32_t boff[NB];                                     // (prefill_supported: planes below 4 GB)
 #pragma unroll
@@ -86,20 +94,24 @@ __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileArgs 
         boff[j] = combined ? (uint32_t)n * (uint32_t)a.K + g * (32 * SUB) : (uint32_t)n * (uint32_t)(a.K >> 1) + g * (16 * SUB);
     }
 
-    f16x8 A[D][MB][4];
+    // (the upper half of the wave reads the lower half's columns again where the last tile has but 32: the images hold zeros)
+    const uint32_t tail = split && (a.K & 32) && g ? (combined ? 32u : 16u) : 0u;
+
+    f16x8 A[D][MB][4][PARTS];
     u32x4v B[BR][NB][BV];
     auto request_b = [&](u32x4v (&bv)[NB][BV], int st) {
         if (st >= t_end) st = t_end - 1;                   // (past the range: the last tile again, not used)
         if (st < 0) st = 0;                                // (a wave without tiles)
         const int p = (kPlanes == 2 && st >= T) ? 1 : 0;
         const uint8_t* const w = (p ? a.plane1 : a.plane0) + (size_t)(st - p * T) * (combined ? 64 * SUB : 32 * SUB);
+        const uint32_t back = split && st - p * T == T - 1 ? tail : 0u;
 #pragma unroll
         for (int j = 0; j < NB; ++j)
 #pragma unroll
-            for (int q = 0; q < BV; ++q) bv[j][q] = *reinterpret_cast<const u32x4v*>(w + q * 16 + boff[j]);
+            for (int q = 0; q < BV; ++q) bv[j][q] = *reinterpret_cast<const u32x4v*>(w + q * 16 + (boff[j] - back));
     };
     // Activations of piece q (32 columns of either half of the wave) of weight tile st.
-    auto request_a = [&](f16x8 (&av)[MB][4], int st, int q) {
+    auto request_a = [&](f16x8 (&av)[MB][4][PARTS], int st, int q) {
         if (st >= t_end) st = t_end - 1;
         if (st < 0) st = 0;
         const int p = (kPlanes == 2 && st >= T) ? 1 : 0;
@@ -108,7 +120,9 @@ __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileArgs 
         for (int i = 0; i < MB; ++i)
 #pragma unroll
             for (int s = 0; s < 4; ++s)
-                av[i][s] = *reinterpret_cast<const f16x8*>(ap[i] + at + ((s >> 1) * 1024 + (s & 1) * 512) + aoff);
+#pragma unroll
+                for (int h = 0; h < PARTS; ++h)
+                    av[i][s][h] = *reinterpret_cast<const f16x8*>(ap[i] + (at + h * part_stride) + ((s >> 1) * 1024 + (s & 1) * 512) + aoff);
     };
 #pragma unroll
     for (int b = 0; b < BR; ++b) request_b(B[b], t_begin + b);
@@ -117,8 +131,17 @@ __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileArgs 
 
     // The table, while those travel.  Shared rotation: fp16(lut[b]) in the upper half.  Nibble planes: the fp16 centroids
     // of both nibbles of byte b; with two planes lanes 0..31 of an entry hold the primary's and lanes 32..63 the
-    // residual's, and lanes l and l + 32 read the same column (the LDS serves a wave's reads in two halves).
-    {
+    // residual's, and lanes l and l + 32 read the same column (the LDS serves a wave's reads in two halves).  Two parts: both of
+    // an entry of the table in one dword; the second plane's 16 entries behind the first's.
+    if constexpr (split) {
+        typedef const __attribute__((address_space(4))) uint32_t cuint;
+        cuint* const src = (cuint*)reinterpret_cast<const uint32_t*>(a.tables);
+        uint32_t* const dst = reinterpret_cast<uint32_t*>(smem) + lane;
+        constexpr int kPer = (kEntries + kWaves - 1) / kWaves;
+        static_assert(kPer * kWaves == kEntries, "every wave writes as many entries");
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) dst[(wave * kPer + e) * 64] = src[wave * kPer + e];
+    } else {
         typedef const __attribute__((address_space(4))) float cfloat;
         cfloat* const src = (cfloat*)a.tables;
         uint32_t* const dst = reinterpret_cast<uint32_t*>(smem) + lane;
@@ -148,39 +171,96 @@ __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileArgs 
         for (int j = 0; j < NB; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    f32x16 sum[split ? MB : 1][split ? NB : 1];            // (two parts: the pieces that are done, acc what those additions left off)
+    if constexpr (split)
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) sum[i][j] = acc[i][j];
 
-    auto compute = [&](const f16x8 (&av)[MB][4], const u32x4v (&bv)[NB][BV], auto Qc, int st) {
-        constexpr int q = decltype(Qc)::value;
-        const uint32_t off = kPlanes == 2 ? (uint32_t)l * 4 + (st >= T ? 128u : 0u) : (uint32_t)lane * 4;
+    // The operands of step s of a piece (column block j of the wave), in PARTS parts.
+    auto decode = [&](const u32x4v (&bv)[NB][BV], int q, int s, int j, int st, f16x8 (&bf)[PARTS]) {
+        const uint32_t off = kPlanes == 2 && !split ? (uint32_t)l * 4 + (st >= T ? 128u : 0u) : (uint32_t)lane * 4;
+        uint32_t lv[8];                                    // entries of the operand's columns, or of pairs of them
+        if constexpr (combined) {
+            const u32x4v& piece = bv[j][q * PV + (s >> 1)];
+            const uint32_t w0 = piece[(s & 1) * 2], w1 = piece[(s & 1) * 2 + 1];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            f16x8 bf[NB];
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                u32x4v o;
-                if constexpr (combined) {
-                    const u32x4v& piece = bv[j][q * PV + (s >> 1)];
-                    const uint32_t w0 = piece[(s & 1) * 2], w1 = piece[(s & 1) * 2 + 1];
-                    uint32_t lv[8];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        lv[k] = *reinterpret_cast<const uint32_t*>(smem + gemm_entry_addr(w0, off, k));
-                        lv[4 + k] = *reinterpret_cast<const uint32_t*>(smem + gemm_entry_addr(w1, off, k));
-                    }
-                    o.x = pack_half2(lv[0], lv[1]); o.y = pack_half2(lv[2], lv[3]);
-                    o.z = pack_half2(lv[4], lv[5]); o.w = pack_half2(lv[6], lv[7]);
-                } else {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        o[k] = *reinterpret_cast<const uint32_t*>(smem + gemm_entry_addr(bv[j][q][s], off, k));
-                }
-                bf[j] = __builtin_bit_cast(f16x8, o);
+            for (int k = 0; k < 4; ++k) {
+                lv[k] = *reinterpret_cast<const uint32_t*>(smem + gemm_entry_addr(w0, off, k));
+                lv[4 + k] = *reinterpret_cast<const uint32_t*>(smem + gemm_entry_addr(w1, off, k));
             }
-            // (weights as the first operand: a lane's 16 results are 4 x 4 consecutive output columns of one token)
+        } else if constexpr (split) {
+            const uint32_t second = kPlanes == 2 && st >= T ? 0x10101010u : 0u;          // (the second plane's entries)
+            const uint32_t w = bv[j][q][s], even = (w & 0x0f0f0f0fu) | second, odd = ((w >> 4) & 0x0f0f0f0fu) | second;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                lv[2 * k] = *reinterpret_cast<const uint32_t*>(smem + gemm_entry_addr(even, off, k));
+                lv[2 * k + 1] = *reinterpret_cast<const uint32_t*>(smem + gemm_entry_addr(odd, off, k));
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) lv[k] = *reinterpret_cast<const uint32_t*>(smem + gemm_entry_addr(bv[j][q][s], off, k));
+        }
+        u32x4v o;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k] = combined || split ? pack_half2(lv[2 * k], lv[2 * k + 1]) : lv[k];
+        bf[0] = __builtin_bit_cast(f16x8, o);
+        if constexpr (split) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) o[k] = __builtin_amdgcn_perm(lv[2 * k + 1], lv[2 * k], 0x05040100u);      // the lower halves
+            bf[1] = __builtin_bit_cast(f16x8, o);
+        }
+    };
+    auto compute = [&](const f16x8 (&av)[MB][4][PARTS], const u32x4v (&bv)[NB][BV], auto Qc, int st) {
+        constexpr int q = decltype(Qc)::value;
+        // (weights as the first operand: a lane's 16 results are 4 x 4 consecutive output columns of one token)
+        auto mm = [&](f32x16& c, const f16x8& w, const f16x8& x) { c = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, x, c, 0, 0, 0); };
+        if constexpr (split) {
+            // One piece at a time: first the products with a lo part, whose sums are too small for their rounding to matter, then
+            // the four of hi parts, then the piece to the sum over pieces; what that addition rounds off is where the next
+            // piece starts from.  A matrix instruction rounds once, so a row's error does not grow with its length: 1.2e-7 (relative,
+            // against 64 bits) at any width where the fp32 kernels have 1.3e-7 to 1.5e-7 and one chain of all products 3.8e-7 at 8160.
+            f16x8 bf[4][NB][PARTS];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    decode(bv, q, s, j, st, bf[s][j]);
+#pragma unroll
+                    for (int i = 0; i < MB; ++i) {
+                        mm(acc[i][j], bf[s][j][1], av[i][s][1]);
+                        mm(acc[i][j], bf[s][j][1], av[i][s][0]);
+                        mm(acc[i][j], bf[s][j][0], av[i][s][1]);
+                    }
+                }
+                if constexpr (MB * NB == 4) __builtin_amdgcn_sched_barrier(0);      // (all decodes at once do not fit the registers)
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < MB; ++i)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) mm(acc[i][j], bf[s][j][0], av[i][s][0]);
 #pragma unroll
             for (int i = 0; i < MB; ++i)
 #pragma unroll
-                for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[j], av[i][s], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NB; ++j) {
+                    const f32x16 t = sum[i][j] + acc[i][j];
+                    acc[i][j] -= t - sum[i][j];
+                    sum[i][j] = t;
+                }
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                f16x8 bf[NB][PARTS];
+#pragma unroll
+                for (int j = 0; j < NB; ++j) decode(bv, q, s, j, st, bf[j]);
+#pragma unroll
+                for (int i = 0; i < MB; ++i)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) mm(acc[i][j], bf[j][0], av[i][s][0]);
+            }
         }
     };
     // Weight tile st + b with the activations that were requested D pieces ago; the slot of each piece is filled again.
@@ -224,23 +304,33 @@ __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileArgs 
 #pragma unroll
         for (int j = 0; j < NB; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) ex[((wave * kBlocks + i * NB + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+            for (int r = 0; r < 16; ++r) {
+                float v = acc[i][j][r];
+                if constexpr (split) v += sum[i][j][r];
+                ex[((wave * kBlocks + i * NB + j) * 16 + r) * 64 + lane] = v;
+            }
     __syncthreads();
     const bool vec = (a.N & 3) == 0;
     for (int u = wave; u < WN * kBlocks * 4; u += kWaves) {
         const int q = u & 3, b = (u >> 2) % kBlocks, w = (u >> 2) / kBlocks;
         const int row = m0 + (b / NB) * 32 + l, col = n0 + (w * NB + b % NB) * 32 + 8 * q + 4 * g;
-        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        std::conditional_t<split, double, float> t[4] = {};
 #pragma unroll
         for (int k = 0; k < KS; ++k)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] += ex[(((k * WN + w) * kBlocks + b) * 16 + 4 * q + e) * 64 + lane];
+            for (int e = 0; e < 4; ++e) t[e] += ex[(((k * WN + w) * kBlocks + b) * 16 + 4 * q + e) * 64 + lane];
         if (row >= a.M) continue;
+        const int x = split ? a.row_exp[row] + a.table_exp : 0;
+        auto scaled = [&](int e) -> float {                // (two parts: summed and scaled in 64 bits, one rounding)
+            if constexpr (split) return (float)(ldexp(t[e], x) * ((double)a.out_scale * a.norms[col + e]));
+            else return t[e] * (a.out_scale * a.norms[col + e]);
+        };
         const size_t at = (size_t)row * a.N + col;
         if (vec) {
             if (col >= a.N) continue;
+            float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] *= a.out_scale * a.norms[col + e];
+            for (int e = 0; e < 4; ++e) v[e] = scaled(e);
             if (a.y_dtype == kF32) {
                 const u32x4v o = {__builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1]),
                                   __builtin_bit_cast(uint32_t, v[2]), __builtin_bit_cast(uint32_t, v[3])};
@@ -256,7 +346,7 @@ __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileArgs 
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (col + e < a.N) store_scalar(a.y, a.y_dtype, at + e, v[e] * (a.out_scale * a.norms[col + e]));
+                if (col + e < a.N) store_scalar(a.y, a.y_dtype, at + e, scaled(e));
         }
     }
 }
@@ -265,18 +355,173 @@ namespace {
 
 struct TileShape { int mb, nb, ks, wn; };
 constexpr TileShape kTileShapes[] = {{1, 1, 8, 1}, {1, 2, 8, 1}, {2, 2, 8, 1}, {4, 2, 2, 2}};
+constexpr TileShape kSplitShapes[] = {{1, 1, 8, 1}, {1, 2, 8, 1}, {2, 2, 4, 2}};
 
 template <int MODE, int SUB>
 void launch_shape(int shape, const TileArgs& a, dim3 grid, hipStream_t stream) {
     switch (shape) {
-        case 0: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, SUB, 1, 1, 8, 1>), grid, dim3(512), 0, stream, a); break;
-        case 1: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, SUB, 1, 2, 8, 1>), grid, dim3(512), 0, stream, a); break;
-        case 2: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, SUB, 2, 2, 8, 1>), grid, dim3(512), 0, stream, a); break;
-        default: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, SUB, 4, 2, 2, 2>), grid, dim3(256), 0, stream, a); break;
+        case 0: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, SUB, 1, 1, 8, 1, 1>), grid, dim3(512), 0, stream, a); break;
+        case 1: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, SUB, 1, 2, 8, 1, 1>), grid, dim3(512), 0, stream, a); break;
+        case 2: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, SUB, 2, 2, 8, 1, 1>), grid, dim3(512), 0, stream, a); break;
+        default: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, SUB, 4, 2, 2, 2, 1>), grid, dim3(256), 0, stream, a); break;
     }
 }
 
+template <int MODE>
+void launch_split_shape(int shape, const TileArgs& a, dim3 grid, hipStream_t stream) {
+    switch (shape) {
+        case 0: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, 1, 1, 1, 8, 1, 2>), grid, dim3(512), 0, stream, a); break;
+        case 1: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, 1, 1, 2, 8, 1, 2>), grid, dim3(512), 0, stream, a); break;
+        default: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, 1, 2, 2, 4, 2, 2>), grid, dim3(512), 0, stream, a); break;
+    }
+}
+
+TileArgs tile_args(const LayerView& L, int batch, void* y, int y_dtype, const void* images, TileShape t) {
+    TileArgs a{};
+    a.xt = static_cast<const char*>(images);
+    a.plane0 = (L.mode == kSharedLut) ? L.packed_combined : L.packed_primary;
+    a.plane1 = L.packed_residual;
+    a.tables = L.tables;
+    a.norms = L.norms;
+    a.y = y; a.y_dtype = y_dtype;
+    a.M = batch; a.N = L.out_features; a.K = L.in_features;
+    a.m_tiles = (batch + 32 * t.mb - 1) / (32 * t.mb);
+    a.n_tiles = (a.N + 32 * t.nb * t.wn - 1) / (32 * t.nb * t.wn);
+    a.out_scale = L.inv_scale;                             // (1 / sqrt(bs) is in the rotated activations)
+    return a;
+}
+
+// The activations of tq_prefill_tile_kernel's operands in two parts: H (s (.) x) in fp32 as the fp32 kernels form it, times the power of
+// two that brings the largest of the row to [2^14, 2^15), rounded to fp16 (hi) and what that leaves off rounded again (lo).  A lane
+// has 32 consecutive columns, a wave 2048, a row `wpr` waves of one workgroup, which holds whole rows; both rotations of the
+// dual layout share the row's exponent.
+template <int PLANES>
+__global__ __launch_bounds__(1024) void tq_rotate_split_kernel(const void* __restrict__ x, int x_dtype, uint16_t* __restrict__ out,
+                                                               int* __restrict__ row_exp, int rows, int cols, int wpr,
+                                                               uint32_t seed, uint32_t seed2, uint32_t bs) {
+    __shared__ float wave_max[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int per = (int)(blockDim.x >> 6) / wpr;          // rows of a workgroup
+    const int in_wg = wave / wpr, row = (int)blockIdx.x * per + in_wg;
+    const int col = ((wave - in_wg * wpr) * 64 + lane) * 32;
+    const bool mine = in_wg < per && row < rows;
+    const bool active = mine && col < cols;
+    float v[PLANES][32], big = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 32; ++k) v[0][k] = 0.0f;
+    if (active) load_chunk(x, x_dtype, (size_t)row * cols + col, v[0]);
+#pragma unroll
+    for (int p = PLANES - 1; p >= 0; --p) {
+        const uint32_t sd = p ? seed2 : seed;
+#pragma unroll
+        for (int k = 0; k < 32; ++k) v[p][k] = v[0][k] * sign_of(sd, (uint32_t)(col + k) & (bs - 1));
+        fwht_lane32(v[p], bs, lane);
+#pragma unroll
+        for (int k = 0; k < 32; ++k) big = __builtin_fmaxf(big, __builtin_fabsf(v[p][k]));
+    }
+    big = __builtin_fmaxf(big, lane_xor<1>(big));
+    big = __builtin_fmaxf(big, lane_xor<2>(big));
+    big = __builtin_fmaxf(big, lane_xor<4>(big));
+    big = __builtin_fmaxf(big, lane_xor<8>(big));
+    big = __builtin_fmaxf(big, lane_xor<16>(big));
+    big = __builtin_fmaxf(big, lane_xor<32>(big));
+    if (lane == 0) wave_max[wave] = big;
+    __syncthreads();
+    if (!mine) return;
+    for (int w = 0; w < wpr; ++w) big = __builtin_fmaxf(big, wave_max[in_wg * wpr + w]);
+    const int e = __builtin_amdgcn_frexp_expf(big) - 15;   // (0, infinity: an exponent of 0)
+    if (col == 0) row_exp[row] = e;
+    const int U = ((cols + 63) >> 6) * 4;
+    if (col >= U * 16) return;
+    uint4* const img = reinterpret_cast<uint4*>(out) + (size_t)(row >> 5) * U * 64 + (row & 31) + (size_t)(col >> 4) * 64;
+    const size_t part = (size_t)((rows + 31) >> 5) * U * 64;
+#pragma unroll
+    for (int p = 0; p < PLANES; ++p)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            uint32_t h[4], l[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                uint16_t hb[2], lb[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const float s = ldexpf(v[p][8 * q + 2 * j + k], -e);
+                    const _Float16 hi = (_Float16)s, lo = (_Float16)(s - (float)hi);
+                    hb[k] = __builtin_bit_cast(uint16_t, hi);
+                    lb[k] = __builtin_bit_cast(uint16_t, lo);
+                }
+                h[j] = hb[0] | (uint32_t)hb[1] << 16;
+                l[j] = lb[0] | (uint32_t)lb[1] << 16;
+            }
+            uint4* const dst = img + 2 * p * part + (q >> 1) * 64 + (q & 1) * 32;
+            dst[0] = make_uint4(h[0], h[1], h[2], h[3]);
+            dst[part] = make_uint4(l[0], l[1], l[2], l[3]);
+        }
+}
+
 }  // namespace
+
+// The shape of a call with two parts: us of the rounds of workgroups on the CUs, each a fixed cost (table, first requests, sum over the
+// waves, stores) and a cost per 64-column tile of a wave, fitted to 24 calls of 2 to 1113 rows.  A wave's tile is a chain (table
+// reads, products with lo parts, products of hi parts, the sum over tiles): the matrix units are busy a third of the time.
+static int split_shape(const LayerView& L, int batch, int num_cus) {
+    static constexpr double kFirst[3] = {3.5, 6.3, 8.0}, kPerTile[3] = {1.28, 2.04, 3.6};
+    const double tiles64 = (L.mode == kDual ? 2.0 : 1.0) * ((L.in_features + 63) / 64);
+    double best = 0.0;
+    int shape = -1;
+    for (int s = 0; s < 3; ++s) {
+        const TileShape t = kSplitShapes[s];
+        const long long wgs = (long long)((batch + 32 * t.mb - 1) / (32 * t.mb)) * ((L.out_features + 32 * t.nb * t.wn - 1) / (32 * t.nb * t.wn));
+        const double cost = (double)((wgs + num_cus - 1) / num_cus) * (kFirst[s] + kPerTile[s] * tiles64 / t.ks);
+        if (shape < 0 || cost < best) { best = cost; shape = s; }
+    }
+    return shape;
+}
+
+// The calls that are left to the fp32 kernels otherwise: widths that are odd multiples of 32, nibble planes of odd multiples of 64 at
+// up to 15 rows, centroids beyond fp16.  Those kernels take four rows a launch, or one (dual rotation): few rows stay there.
+//   us per call before -> now, in x out, rows: shared rotation 1056 x 7017 at 8 / 33 / 1113 rows 27 / 110 / 3699 -> 12 / 16 / 130; 2080 x 7168 at
+//   1051 rows 5295 -> 175; dual rotation 3872 x 18432 at 12 rows 207 -> 61 (35 at 2 rows, where this takes 56); primary alone
+//   1696 x 8960 at 125 rows 476 -> 32 (16.2 at 4 rows, as long as this).
+bool prefill_split_supported(const LayerView& L, int batch) {
+    if (batch < (L.mode == kDual ? 4 : 5) || !L.split_tables || !shape_supported(L.in_features, L.block_size)) return false;
+    if (L.mode != kSharedLut && L.mode != kDual && L.mode != kPrimaryOnly) return false;
+    return (unsigned long long)L.out_features * (unsigned long long)L.in_features < (1ull << 32);      // (32-bit offsets into a plane)
+}
+
+static size_t split_image_bytes(const LayerView& L, int batch) {
+    return (L.mode == kDual ? 4 : 2) * (((size_t)batch + 31) / 32) * 32 * (((size_t)L.in_features + 63) / 64 * 64) * sizeof(uint16_t);
+}
+size_t prefill_split_workspace_bytes(const LayerView& L, int batch) { return split_image_bytes(L, batch) + (size_t)batch * sizeof(int); }
+
+hipError_t launch_prefill_split(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
+                                void* workspace, int num_cus, hipStream_t stream) {
+    uint16_t* const images = static_cast<uint16_t*>(workspace);
+    int* const row_exp = reinterpret_cast<int*>(static_cast<char*>(workspace) + split_image_bytes(L, batch));
+    const int wpr = (L.in_features + kSlab - 1) / kSlab, waves = wpr < 4 ? 4 : wpr, per = waves / wpr;
+    const dim3 rgrid((unsigned)((batch + per - 1) / per));
+    if (L.mode == kDual)
+        hipLaunchKernelGGL(tq_rotate_split_kernel<2>, rgrid, dim3(waves * 64), 0, stream, x, x_dtype, images, row_exp, batch,
+                           L.in_features, wpr, L.seed_primary, L.seed_residual, L.block_size);
+    else
+        hipLaunchKernelGGL(tq_rotate_split_kernel<1>, rgrid, dim3(waves * 64), 0, stream, x, x_dtype, images, row_exp, batch,
+                           L.in_features, wpr, L.seed_primary, 0u, L.block_size);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const int shape = split_shape(L, batch, num_cus);
+    TileArgs a = tile_args(L, batch, y, y_dtype, workspace, kSplitShapes[shape]);
+    a.tables = reinterpret_cast<const float*>(L.split_tables);
+    a.out_scale = L.inv_scale * L.inv_sqrt_bs;
+    a.row_exp = row_exp;
+    a.table_exp = L.split_exp;
+    const dim3 grid((unsigned)((a.n_tiles + 7) / 8 * 8 * a.m_tiles));
+    switch (L.mode) {
+        case kSharedLut: launch_split_shape<kSharedLut>(shape, a, grid, stream); break;
+        case kDual: launch_split_shape<kDual>(shape, a, grid, stream); break;
+        default: launch_split_shape<kPrimaryOnly>(shape, a, grid, stream); break;
+    }
+    return hipGetLastError();
+}
 
 size_t prefill_tile_workspace_bytes(const LayerView& L, int batch) {
     const size_t planes = (L.mode == kDual) ? 2 : 1;
@@ -320,18 +565,7 @@ hipError_t launch_prefill_tile(const LayerView& L, int shape, const void* x, int
                                void* workspace, hipStream_t stream) {
     hipError_t e = launch_rotate_tiles(L, x, x_dtype, batch, workspace, stream, kBlockImage);
     if (e != hipSuccess) return e;
-    const TileShape t = kTileShapes[shape];
-    TileArgs a{};
-    a.xt = static_cast<const char*>(workspace);
-    a.plane0 = (L.mode == kSharedLut) ? L.packed_combined : L.packed_primary;
-    a.plane1 = L.packed_residual;
-    a.tables = L.tables;
-    a.norms = L.norms;
-    a.y = y; a.y_dtype = y_dtype;
-    a.M = batch; a.N = L.out_features; a.K = L.in_features;
-    a.m_tiles = (batch + 32 * t.mb - 1) / (32 * t.mb);
-    a.n_tiles = (a.N + 32 * t.nb * t.wn - 1) / (32 * t.nb * t.wn);
-    a.out_scale = L.inv_scale;                             // (1 / sqrt(bs) is in the rotated activations)
+    const TileArgs a = tile_args(L, batch, y, y_dtype, workspace, kTileShapes[shape]);
     const dim3 grid((unsigned)((a.n_tiles + 7) / 8 * 8 * a.m_tiles));
     // Two 64-column tiles of a nibble plane at a time where the width allows it: 64 bytes of a row per pair of requests
     // instead of 32 (4864 x 896 at 512 rows 40.6 -> 38.0 us, 7680 x 565 55.0 -> 49.6; four tiles cost registers: 58).  The
