@@ -121,15 +121,29 @@ hipError_t device_malloc(void** p, size_t bytes);
 struct QuantArgsHost {
     const float* w; float* orig_norm; double* recon_partial; float* scaled_out;
     uint8_t* packed_primary; uint8_t* packed_residual;
-    const float* tables;     // device: [0..31] cP, [32..62] bP, [64..79] cR, [80..94] bR
+    const uint32_t* seeds;   // device: of the primary's and the residual's rotation
+    float tables[96];        // [0..31] cP, [32..62] bP, [64..79] cR, [80..94] bR
+    float* tables_out;       // samples: tables[0..63] are written here as well, where not NULL
+    uint32_t* absmax;        // samples: one largest |sample| (its bits) per wave, quantize_sample_waves of them; or NULL
     int out, in, n_primary, n_residual, primary_bits, residual_bits, shared_rotation;
-    uint32_t bs, seed_p, seed_r;
+    uint32_t bs;
     float scale_factor, inv_scale, inv_sqrt_bs;
     int quantize;            // 0: only emit the rotated * sqrt(in) samples
+    int sorted;              // both codebooks' boundaries are in order
 };
 hipError_t launch_row_norms(const float* w, float* norms, int out, int in, hipStream_t stream);
 hipError_t launch_derive_seeds(const float* w, size_t n_floats, uint32_t* seeds_dev, hipStream_t stream);
 hipError_t launch_quantize_rows(const QuantArgsHost& h, hipStream_t stream);
+// Waves of a launch over chunks of 32 columns (lanes_supported): tiles of 64 chunks, 4 waves to a workgroup, as many workgroups
+// as 256 CUs hold at once; every wave walks the same number of tiles, or one less.
+constexpr int kQWaves = 4;
+inline uint32_t quantize_workgroups(uint32_t tiles, uint32_t resident) {
+    const uint32_t each = (tiles + resident * kQWaves - 1) / (resident * kQWaves);
+    return (tiles + each * kQWaves - 1) / (each * kQWaves);
+}
+inline int quantize_sample_waves(int out, int in) {
+    return kQWaves * (int)quantize_workgroups((uint32_t)(((long long)out * (in / kChunk) + kWave - 1) / kWave), 768);
+}
 int quantize_partials_per_row(int in, uint32_t bs);      // doubles per row of recon_partial / launch_finish_norms' `slabs`
 hipError_t launch_finish_norms(const float* orig, const double* partial, float* norms, int out, int slabs,
                                hipStream_t stream);
@@ -144,7 +158,11 @@ hipError_t launch_lloyd_pass(const float* data, size_t n, const float* bounds_de
 // codebook p left the cells whose samples were kept, after state->steps[p] steps: call again with first_round == false
 // and the same workspace (another expectation, from there on), or with everything == true, which cannot miss and
 // needs a larger workspace of its own (first_round == true again).  With one problem the second's fields are not written.
-struct FitCodebooks { int nc[2]; float init[2][32]; };
+struct FitCodebooks {
+    int nc[2];
+    float init[2][32];
+    const uint32_t* absmax; int absmax_parts;    // device: bits of the largest |sample| in parts; or NULL: a pass of its own finds it
+};
 struct FitResult { float cent[2][32]; int steps[2]; int bad; int coarse[2]; int missed[2]; unsigned kept[2]; };
 bool fit_supported(size_t n);
 bool fit_predicts(size_t n);         // large enough that keeping only the expected cells pays
@@ -206,7 +224,8 @@ __device__ __forceinline__ float sign_of(uint32_t seed, uint32_t index) {
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+    // (no lane of these permutations is without a source: nothing is kept of the destination, no register is cleared for it)
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
 // Value held by lane (lane ^ MASK), without touching LDS:
@@ -236,13 +255,42 @@ __device__ __forceinline__ float lane_xor(float v) {
 }
 
 // One cross-lane butterfly stage over N values per lane: the lower lane of a pair
-// gets a+b, the upper lane a-b.  fma(v, +-1, partner) is exact, so the result is
-// bit-identical to the add/sub of the CPU butterfly.
+// gets a+b, the upper lane a-b.  v * +-1 is exact, so the result is bit-identical to
+// the add/sub of the CPU butterfly.  (A product and a sum, not an fma: the sum takes the partner's value through its
+// own DPP operand and is written in place, two instructions; an fma has no DPP operand for its addend: a move, the
+// fma and, where the stage is under a branch, half a copy.)
+// Four at a time, products before sums: a DPP instruction waits two issue slots for a register that the instruction before it
+// wrote, and left to itself the compiler puts the two side by side with a wait between them.
+template <int N, typename F>
+__device__ __forceinline__ void butterfly_pairs(float (&v)[N], float sgn, F partner) {
+    constexpr int G = N < 4 ? N : 4;
+    static_assert(N % G == 0, "whole groups");
+#pragma unroll
+    for (int k = 0; k < N; k += G) {
+        float own[G];
+#pragma unroll
+        for (int j = 0; j < G; ++j) own[j] = v[k + j] * sgn;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < G; ++j) v[k + j] = partner(v[k + j]) + own[j];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 template <int MASK, int N>
 __device__ __forceinline__ void butterfly_lanes(float (&v)[N], int lane) {
     const float sgn = (lane & MASK) ? -1.0f : 1.0f;
-#pragma unroll
-    for (int k = 0; k < N; ++k) v[k] = __builtin_fmaf(v[k], sgn, lane_xor<MASK>(v[k]));
+    butterfly_pairs<N>(v, sgn, [](float x) { return lane_xor<MASK>(x); });
+}
+
+// A numbering of the lanes under which the partner of lane ^ 4 is the mirror image within eight lanes (hardware lane ^ 7),
+// one DPP operand where lane ^ 4 takes two moves; 1, 2, 8, 16 and 32 stay what they are.  For kernels whose lanes
+// find their data by number: the butterfly below takes this number for `lane`.
+__device__ __forceinline__ int mirrored_lane(int lane) { return (lane & 4) ? lane ^ 3 : lane; }
+template <int N>
+__device__ __forceinline__ void butterfly_mirror(float (&v)[N], int lane) {
+    const float sgn = (lane & 4) ? -1.0f : 1.0f;
+    butterfly_pairs<N>(v, sgn, [](float x) { return dpp_mov<0x141>(x); });          // row_half_mirror
 }
 
 // Unnormalised natural-order Walsh-Hadamard butterfly over a block that is
@@ -250,7 +298,7 @@ __device__ __forceinline__ void butterfly_lanes(float (&v)[N], int lane) {
 // entirely inside the lane when bs <= N).  Stage order and the (a+b, a-b)
 // convention are those of reference src/rotation.cpp:14-25, so the result is
 // bit-identical to the CPU butterfly.
-template <int N>
+template <int N, bool MIRRORED = false>
 __device__ __forceinline__ void fwht_lanes(float (&v)[N], uint32_t bs, int lane) {
 #pragma unroll
     for (int h = 1; h < N; h <<= 1) {
@@ -268,7 +316,10 @@ __device__ __forceinline__ void fwht_lanes(float (&v)[N], uint32_t bs, int lane)
     }
     if ((uint32_t)N * 1 < bs) butterfly_lanes<1, N>(v, lane);
     if ((uint32_t)N * 2 < bs) butterfly_lanes<2, N>(v, lane);
-    if ((uint32_t)N * 4 < bs) butterfly_lanes<4, N>(v, lane);
+    if ((uint32_t)N * 4 < bs) {
+        if constexpr (MIRRORED) butterfly_mirror<N>(v, lane);
+        else butterfly_lanes<4, N>(v, lane);
+    }
     if ((uint32_t)N * 8 < bs) butterfly_lanes<8, N>(v, lane);
     if ((uint32_t)N * 16 < bs) butterfly_lanes<16, N>(v, lane);
     if ((uint32_t)N * 32 < bs) butterfly_lanes<32, N>(v, lane);

@@ -4,7 +4,7 @@
 // per step costs 200 passes for the two codebooks of a layer.  Here the samples are put in coarse value order once and
 // a step looks at the few thousand samples around each boundary only:
 //
-//   tq_fit_absmax_kernel    largest |sample|: fixes the scale of the value cells
+//   tq_fit_absmax_kernel    largest |sample|: fixes the scale of the value cells (the kernel that makes a layer's samples knows it)
 //   tq_fit_hist_kernel      per tile of the samples: how many fall into each of kFitCells value cells, and the sum of
 //                           their offsets inside the cell
 //   tq_fit_offsets_kernel   the tiles' counts become positions; the cells' totals
@@ -700,8 +700,9 @@ hipError_t launch_fit(const float* samples, size_t n, int problems, const float*
     const dim3 grid((unsigned)tiles, (unsigned)problems);
     if (first_round) {
         const unsigned parts = (unsigned)(n / 16384 < 1 ? 1 : (n / 16384 > 1024 ? 1024 : n / 16384));
-        hipLaunchKernelGGL(tq_fit_absmax_kernel, dim3(parts), dim3(256), 0, stream, samples, n, part);
-        hipLaunchKernelGGL(tq_fit_absmax_fold_kernel, dim3(1), dim3(256), 0, stream, part, (int)parts, fp, problems, P, cb, state);
+        if (!cb.absmax) hipLaunchKernelGGL(tq_fit_absmax_kernel, dim3(parts), dim3(256), 0, stream, samples, n, part);
+        hipLaunchKernelGGL(tq_fit_absmax_fold_kernel, dim3(1), dim3(256), 0, stream, cb.absmax ? cb.absmax : part,
+                           cb.absmax ? cb.absmax_parts : (int)parts, fp, problems, P, cb, state);
         hipLaunchKernelGGL(tq_fit_hist_kernel, grid, dim3(kFitThreads), 0, stream, fp, P, tile, hist);
         hipLaunchKernelGGL(tq_fit_offsets_kernel, dim3(kFitCells / 256, problems), dim3(256), 0, stream, P, (int)tiles, hist, first,
                            cell_n, cell_q);

@@ -8,28 +8,33 @@
 // reference leaves to its tensor runtime (row sums of squares) are accumulated in double in a
 // fixed order and rounded once.
 //
-// One wave handles one (row, 2048-column slab); a lane owns 32 consecutive columns, so the block
-// butterflies are the same in-register / cross-lane code the forward kernels use.
+// A lane owns 32 consecutive columns, so the block butterflies are the same in-register / cross-lane code the
+// forward kernels use.
+#include <cstring>
+
 #include "tq_device.h"
 
 namespace tq {
 
-constexpr int kQWaves = 4;
-
 struct QuantArgs {
     const float* w;          // [out, in] fp32
     float* orig_norm;        // [out]
-    double* recon_partial;   // [out, slabs] sum of squares of the reconstruction
-    float* scaled_out;       // optional [out, in]: rotated * sqrt(in) samples (codebook fitting), or NULL
+    double* recon_partial;   // [out, partials per row] sums of squares of the reconstruction
+    float* scaled_out;       // [out, in]: rotated * sqrt(in) samples (codebook fitting; nothing else is written then)
     uint8_t* packed_primary; // [out, in/2] or [out, in]
     uint8_t* packed_residual;// [out, in/2]
-    const float* tables;     // [0..31] primary centroids, [32..62] primary boundaries,
+    const uint32_t* seeds;
+    float tables[96];        // [0..31] primary centroids, [32..62] primary boundaries,
                              // [64..79] residual centroids, [80..94] residual boundaries
-    int out, in, chunks, slabs;
+    float* tables_out;       // kSamples: see QuantArgsHost
+    uint32_t* absmax;
+    int out, in, chunks;             // chunks of 32 columns in a row, ..
+    int units;                       // (blocks of at most 16 columns: units of a row)
+    uint32_t total_chunks, tiles;    // .. in the matrix, and tiles of 64 of them
     int n_primary, n_residual;       // centroid counts
     int primary_bits, residual_bits;
     int shared_rotation;
-    uint32_t bs, seed_p, seed_r;
+    uint32_t bs;
     float scale_factor, inv_scale, inv_sqrt_bs;
     int quantize;            // 0: only write scaled_out
 };
@@ -40,18 +45,36 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
     return v;
 }
 
-// Row sums of squares -> L2 norms (src/quantizer.cpp:56-58).  One wave per row; every lane adds
-// its strided elements in order, then a fixed shuffle tree.
+// Row sums of squares -> L2 norms (src/quantizer.cpp:56-58).  One wave per row; every lane adds its strided elements in
+// order into four sums, then a fixed shuffle tree.  VEC: 16 bytes per lane and load, four loads in flight; rows that do
+// not start on 16 bytes are read element by element.  Reads only: 18944 x 3584 (272 MB) 92 us one element per load, 42 to 57 us now.
+template <bool VEC>
 __global__ __launch_bounds__(256) void tq_row_norm_kernel(const float* __restrict__ w, float* __restrict__ norms,
                                                           int out, int in) {
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= out) return;
     const float* p = w + (size_t)row * in;
-    double acc = 0.0;
-    for (int j = lane; j < in; j += kWave) { const float sq = p[j] * p[j]; acc += (double)sq; }
-    acc = wave_sum_f64(acc);
-    if (lane == 0) norms[row] = sqrtf((float)acc);
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    if (VEC) {
+        const float4* q = reinterpret_cast<const float4*>(p);
+        const int n4 = in >> 2;
+        for (int j = lane; j < n4; j += 4 * kWave) {
+            float4 v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = q[j + k * kWave < n4 ? j + k * kWave : j];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float t[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) { const float sq = t[i] * t[i]; acc[i] += j + k * kWave < n4 ? (double)sq : 0.0; }
+            }
+        }
+    } else {
+        for (int j = lane; j < in; j += kWave) { const float sq = p[j] * p[j]; acc[0] += (double)sq; }
+    }
+    const double sum = wave_sum_f64((acc[0] + acc[1]) + (acc[2] + acc[3]));
+    if (lane == 0) norms[row] = sqrtf((float)sum);
 }
 
 // std::lower_bound over the boundaries: number of boundaries strictly below v (src/codebook.cpp:295-297).
@@ -61,156 +84,218 @@ __device__ __forceinline__ uint32_t bin_of(float v, const float* bounds, int nb)
     return idx;
 }
 
-__device__ __forceinline__ void inverse_rotate(float (&v)[kChunk], uint32_t bs, int lane, uint32_t seed,
-                                               uint32_t col0, float inv_sqrt_bs) {
-    fwht_lane32(v, bs, lane);
+// The same count by bisection where the boundaries are in order: `heap` holds them as a binary tree (node 1 the middle
+// one, node n's children 2n and 2n + 1; +inf past the last), so a level is one comparison, its result added into the
+// next node's number.  Levels 1 and 2 come from registers, the others from LDS (32 entries in as many banks: no
+// conflicts).  L = 4: 12 vector instructions and two LDS reads, where 15 comparisons take 30.
+template <int L>
+struct BinTree {
+    float root, left, right;
+    const char* heap;
+    __device__ __forceinline__ explicit BinTree(const float* h) : root(h[1]), left(h[2]), right(h[3]), heap(reinterpret_cast<const char*>(h)) {}
+    // Four times (2^L + the count): what addresses the next level's entry.
+    __device__ __forceinline__ uint32_t find(float v) const {
+        const bool upper = root < v;
+        uint32_t n = (upper ? 24u : 16u) + (((upper ? right : left) < v) ? 4u : 0u);
 #pragma unroll
-    for (int k = 0; k < kChunk; ++k) v[k] *= inv_sqrt_bs * sign_of(seed, (col0 + k) & (bs - 1));
+        for (int l = 2; l < L; ++l) n = 2u * n + ((*reinterpret_cast<const float*>(heap + n) < v) ? 4u : 0u);
+        return n;
+    }
+};
+
+// Boundary of a tree node: node 2^l + j of L levels is the one with (2j + 1) 2^(L-1-l) - 1 boundaries below it.
+__device__ __forceinline__ float tree_bound(int node, int levels, const float* bounds, int nb) {
+    if (node < 1 || node >= (1 << levels)) return __builtin_inff();
+    const int l = 31 - __builtin_clz((unsigned)node);
+    const int i = ((2 * (node - (1 << l)) + 1) << (levels - 1 - l)) - 1;
+    return i < nb ? bounds[i] : __builtin_inff();
 }
 
-__device__ __forceinline__ void forward_rotate(float (&v)[kChunk], uint32_t bs, int lane, uint32_t seed,
-                                               uint32_t col0, float inv_sqrt_bs) {
+// 32 indices, a byte each, as nibbles: lo nibble = even column (src/quantizer.cpp:33-39).
+__device__ __forceinline__ uint4 nibbles_of(const uint32_t (&b)[8]) {
+    uint32_t r[4];
 #pragma unroll
-    for (int k = 0; k < kChunk; ++k) v[k] *= sign_of(seed, (col0 + k) & (bs - 1));
-    fwht_lane32(v, bs, lane);
-#pragma unroll
-    for (int k = 0; k < kChunk; ++k) v[k] *= inv_sqrt_bs;
+    for (int d = 0; d < 4; ++d) {
+        const uint32_t lo = b[2 * d] & 0x0f0f0f0fu, hi = b[2 * d + 1] & 0x0f0f0f0fu;
+        r[d] = __builtin_amdgcn_perm(hi | (hi >> 4), lo | (lo >> 4), 0x06040200u);
+    }
+    return make_uint4(r[0], r[1], r[2], r[3]);
 }
 
-__global__ __launch_bounds__(kQWaves* kWave) void tq_quantize_kernel(QuantArgs a) {
-    __shared__ float tab[96];
-    for (int i = threadIdx.x; i < 96; i += blockDim.x) tab[i] = a.tables[i];
-    __syncthreads();
-    const float* cP = tab;
-    const float* bP = tab + 32;
-    const float* cR = tab + 64;
-    const float* bR = tab + 80;
+enum { kSamples = 0, kPrimaryPlane = 1, kSharedPlanes = 2, kDualPlanes = 3 };
 
-    const int lane = threadIdx.x & 63;
-    const long long wid = (long long)blockIdx.x * kQWaves + (threadIdx.x >> 6);
-    const int row = (int)(wid / a.slabs);
-    const int slab = (int)(wid % a.slabs);
-    if (row >= a.out) return;
-    const int chunk = slab * kWave + lane;
-    const bool active = chunk < a.chunks;
+// A wave takes 64 chunks of 32 columns of the matrix read as one row after the other, whatever the width: blocks are
+// whole groups of lanes (the chunks of a row are a multiple of a block's).  The signs of a lane's columns are the same in
+// every tile of 64 chunks, so they are hashed once per workgroup, 64 per ballot, and stay in registers; a workgroup
+// walks tiles of its own.  (Lanes are numbered so that each stage of a butterfly over 512 columns that leaves the lane
+// costs two instructions.)  MODE: samples alone (codebook fitting), or which planes.  LEVELS: of the primary's tree
+// (16 or 32 centroids); 0 where boundaries are in no order and are counted one by one.
+//
+// 18944 x 3584, two rotations: 880 us with one row's 2048-column slab per wave, signs hashed per element and use and
+// boundaries compared one by one (a loop over LDS, 64 of them per weight) -> 281 us.  What is left is vector work:
+// five butterflies, an IEEE division, two trees and a sum in doubles are about 150 instruction slots per weight.
+template <int MODE, int LEVELS>
+__global__ __launch_bounds__(kQWaves* kWave, MODE == kDualPlanes ? 2 : 3) void tq_quantize_kernel(QuantArgs a) {
+    constexpr int kTree = LEVELS == 4 ? 4 : 5;
+    __shared__ uint32_t sign_words[2][64];
+    __shared__ float heap_p[32], heap_r[16], cent_r[16], bounds[2][32];
+    __shared__ float cent_p[64];                         // the centroids; the centroids scaled back
+    const int tid = threadIdx.x;
+    const int lane = mirrored_lane(tid & 63), wave = tid >> 6;
     const uint32_t bs = a.bs;
-    const uint32_t col0 = ((uint32_t)chunk * kChunk) & (bs - 1);
-    const size_t elem0 = (size_t)row * a.in + (size_t)chunk * kChunk;
-
-    // normalise (src/quantizer.cpp:62-66), rotate and scale (:74-79)
-    float v[kChunk];
-    if (active) {
-        load_chunk(a.w, kF32, elem0, v);
-        const float nrm = a.orig_norm[row];
-        const float safe = nrm > 1e-10f ? nrm : 1e-10f;
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) v[k] = v[k] / safe;
+    const uint32_t period = bs < 64 ? 64 : bs;
+    for (uint32_t b = wave; b < period / 64; b += kQWaves) {
+        const uint32_t col = (b * 64 + (tid & 63)) & (bs - 1);
+        const unsigned long long p = __ballot(sign_of(a.seeds[0], col) > 0.0f);
+        const unsigned long long r = __ballot(MODE == kDualPlanes && sign_of(a.seeds[1], col) > 0.0f);
+        if (lane < 2) {
+            sign_words[0][2 * b + lane] = (uint32_t)(p >> (32 * lane));
+            sign_words[1][2 * b + lane] = (uint32_t)(r >> (32 * lane));
+        }
+    }
+    if (MODE == kSamples) {
+        if (a.tables_out && blockIdx.x == 0 && tid < 64) a.tables_out[tid] = a.tables[tid];
     } else {
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) v[k] = 0.0f;
-    }
-    forward_rotate(v, bs, lane, a.seed_p, col0, a.inv_sqrt_bs);
-#pragma unroll
-    for (int k = 0; k < kChunk; ++k) v[k] *= a.scale_factor;
-
-    if (a.scaled_out && active) {
-        float4* dst = reinterpret_cast<float4*>(a.scaled_out + elem0);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) dst[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-    }
-    if (!a.quantize) return;
-
-    // primary indices (:82-84), clamp as the reference does (codebook.cpp:297)
-    uint32_t ip[kChunk], ir[kChunk];
-    const int nbp = a.n_primary - 1, nbr = a.n_residual - 1;
-#pragma unroll
-    for (int k = 0; k < kChunk; ++k) {
-        uint32_t idx = bin_of(v[k], bP, nbp);
-        ip[k] = idx >= (uint32_t)a.n_primary ? a.n_primary - 1 : idx;
-        ir[k] = 0;
-    }
-
-    float rec[kChunk];                  // reconstruction in normalised space
-    if (a.residual_bits > 0) {
-        float res[kChunk];
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) res[k] = v[k] - cP[ip[k]];                  // :114-119
-        if (!a.shared_rotation) {                                                     // :131-145
-#pragma unroll
-            for (int k = 0; k < kChunk; ++k) res[k] *= a.inv_scale;
-            inverse_rotate(res, bs, lane, a.seed_p, col0, a.inv_sqrt_bs);
-            forward_rotate(res, bs, lane, a.seed_r, col0, a.inv_sqrt_bs);
-#pragma unroll
-            for (int k = 0; k < kChunk; ++k) res[k] *= a.scale_factor;
-        }
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) {
-            uint32_t idx = bin_of(res[k], bR, nbr);
-            ir[k] = idx >= (uint32_t)a.n_residual ? a.n_residual - 1 : idx;
-        }
-    }
-
-    // reconstruction (:166-234)
-    if (a.residual_bits > 0 && a.shared_rotation) {
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) {
-            const float combined = cP[ip[k]] + cR[ir[k] & 15u];
-            rec[k] = active ? combined * a.inv_scale : 0.0f;
-        }
-        inverse_rotate(rec, bs, lane, a.seed_p, col0, a.inv_sqrt_bs);
-    } else {
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) rec[k] = active ? cP[ip[k]] * a.inv_scale : 0.0f;
-        inverse_rotate(rec, bs, lane, a.seed_p, col0, a.inv_sqrt_bs);
-        if (a.residual_bits > 0) {
-            float r2[kChunk];
-#pragma unroll
-            for (int k = 0; k < kChunk; ++k) r2[k] = active ? cR[ir[k] & 15u] * a.inv_scale : 0.0f;
-            inverse_rotate(r2, bs, lane, a.seed_r, col0, a.inv_sqrt_bs);
-#pragma unroll
-            for (int k = 0; k < kChunk; ++k) rec[k] = rec[k] + r2[k];
-        }
-    }
-    double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < kChunk; ++k) { const float sq = rec[k] * rec[k]; acc += (double)sq; }
-    acc = wave_sum_f64(acc);
-    if (lane == 0) a.recon_partial[(size_t)row * a.slabs + slab] = acc;
-
-    // pack (src/quantizer.cpp:33-39,93-107,151-156)
-    if (active) {
-        if (a.primary_bits <= 4) {
-            uint32_t w4[4];
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                uint32_t w = 0;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    w |= ((ip[8 * d + 2 * j] & 15u) | ((ip[8 * d + 2 * j + 1] & 15u) << 4)) << (8 * j);
-                w4[d] = w;
+        const float* t = a.tables;
+        if (tid < 32) {
+            heap_p[tid] = tree_bound(tid, kTree, t + 32, a.n_primary - 1);
+            cent_p[tid] = t[tid];
+            cent_p[32 + tid] = t[tid] * a.inv_scale;
+            bounds[0][tid] = tid < 31 ? t[32 + tid] : 0.0f;
+            bounds[1][tid] = tid < 15 ? t[80 + tid] : 0.0f;
+            if (tid < 16) {
+                heap_r[tid] = tree_bound(tid, 4, t + 80, a.n_residual - 1);
+                cent_r[tid] = MODE == kSharedPlanes ? t[64 + tid] : t[64 + tid] * a.inv_scale;
             }
-            *reinterpret_cast<uint4*>(a.packed_primary + (size_t)row * (a.in >> 1) + (size_t)chunk * 16) =
-                make_uint4(w4[0], w4[1], w4[2], w4[3]);
+        }
+    }
+    __syncthreads();
+    const BinTree<kTree> tree_p(heap_p);
+    const BinTree<4> tree_r(heap_r);
+
+    float sp[kChunk], sr[kChunk];
+    {
+        const uint32_t w = ((uint32_t)lane * kChunk & (period - 1)) / kChunk;
+        const uint32_t wp = sign_words[0][w], wr = sign_words[1][w];
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+            sp[k] = (wp >> k & 1u) ? 1.0f : -1.0f;
+            sr[k] = (wr >> k & 1u) ? 1.0f : -1.0f;
+        }
+    }
+    const uint32_t group = bs < (uint32_t)kChunk ? 1u : bs / kChunk;             // lanes of a block
+    const float inv = a.inv_sqrt_bs;
+    uint32_t largest = 0;                                                        // (of the samples, as bits)
+
+    for (uint32_t tile = blockIdx.x * kQWaves + wave; tile < a.tiles; tile += gridDim.x * kQWaves) {
+        const uint32_t chunk = tile * kWave + lane;
+        const bool active = chunk < a.total_chunks;
+        const uint32_t row = chunk / (uint32_t)a.chunks;
+        const size_t elem0 = (size_t)chunk * kChunk;
+
+        // normalise (src/quantizer.cpp:62-66), rotate and scale (:74-79)
+        float v[kChunk];
+        if (active) {
+            load_chunk(a.w, kF32, elem0, v);
+            const float nrm = a.orig_norm[row];
+            const float safe = nrm > 1e-10f ? nrm : 1e-10f;
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) v[k] = v[k] / safe;
         } else {
-            uint32_t w8[8];
 #pragma unroll
-            for (int d = 0; d < 8; ++d)
-                w8[d] = ip[4 * d] | (ip[4 * d + 1] << 8) | (ip[4 * d + 2] << 16) | (ip[4 * d + 3] << 24);
-            uint4* dst = reinterpret_cast<uint4*>(a.packed_primary + (size_t)row * a.in + (size_t)chunk * 32);
-            dst[0] = make_uint4(w8[0], w8[1], w8[2], w8[3]);
-            dst[1] = make_uint4(w8[4], w8[5], w8[6], w8[7]);
+            for (int k = 0; k < kChunk; ++k) v[k] = 0.0f;
         }
-        uint32_t r4[4];
 #pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            uint32_t w = 0;
+        for (int k = 0; k < kChunk; ++k) v[k] *= sp[k];
+        fwht_lanes<kChunk, true>(v, bs, lane);
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                w |= ((ir[8 * d + 2 * j] & 15u) | ((ir[8 * d + 2 * j + 1] & 15u) << 4)) << (8 * j);
-            r4[d] = w;
+        for (int k = 0; k < kChunk; ++k) v[k] = v[k] * inv * a.scale_factor;
+
+        if (MODE == kSamples) {
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) largest = max(largest, __builtin_bit_cast(uint32_t, v[k]) & 0x7fffffffu);
+            if (active) {
+                float4* dst = reinterpret_cast<float4*>(a.scaled_out + elem0);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) dst[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+            }
+            continue;
         }
-        *reinterpret_cast<uint4*>(a.packed_residual + (size_t)row * (a.in >> 1) + (size_t)chunk * 16) =
-            make_uint4(r4[0], r4[1], r4[2], r4[3]);
+
+        // primary indices (:82-84), packed (:33-39,93-107), their centroids and the residual (:114-119)
+        float rec[kChunk];                  // reconstruction in normalised space
+        uint32_t pk[8];
+#pragma unroll
+        for (int d = 0; d < 8; ++d) pk[d] = 0;
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+            const uint32_t i = LEVELS ? tree_p.find(v[k]) : 4u * bin_of(v[k], bounds[0], a.n_primary - 1) + (4u << kTree);
+            pk[k >> 2] += (k & 3) ? i << (8 * (k & 3) - 2) : i >> 2;
+            const float* c = reinterpret_cast<const float*>(reinterpret_cast<const char*>(cent_p) + i) - (1 << kTree);
+            v[k] = v[k] - c[0];
+            rec[k] = c[MODE == kSharedPlanes ? 0 : 32];
+        }
+#pragma unroll
+        for (int d = 0; d < 8; ++d) pk[d] -= 0x01010101u << kTree;
+        if (active) {
+            if (a.primary_bits <= 4) {
+                *reinterpret_cast<uint4*>(a.packed_primary + (size_t)chunk * 16) = nibbles_of(pk);
+            } else {
+                uint4* dst = reinterpret_cast<uint4*>(a.packed_primary + elem0);
+                dst[0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+                dst[1] = make_uint4(pk[4], pk[5], pk[6], pk[7]);
+            }
+        }
+        if (MODE != kSharedPlanes) {                                                  // :166-234
+            fwht_lanes<kChunk, true>(rec, bs, lane);
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) rec[k] = rec[k] * inv * sp[k];
+        }
+        uint4 rk = make_uint4(0, 0, 0, 0);
+        if (MODE >= kSharedPlanes) {
+            if (MODE == kDualPlanes) {                                                // :131-145
+#pragma unroll
+                for (int k = 0; k < kChunk; ++k) v[k] *= a.inv_scale;
+                fwht_lanes<kChunk, true>(v, bs, lane);
+#pragma unroll
+                for (int k = 0; k < kChunk; ++k) v[k] = v[k] * inv * sp[k] * sr[k];
+                fwht_lanes<kChunk, true>(v, bs, lane);
+#pragma unroll
+                for (int k = 0; k < kChunk; ++k) v[k] = v[k] * inv * a.scale_factor;
+            }
+#pragma unroll
+            for (int d = 0; d < 8; ++d) pk[d] = 0;
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) {
+                const uint32_t i = LEVELS ? tree_r.find(v[k]) : 4u * bin_of(v[k], bounds[1], a.n_residual - 1) + 64u;
+                pk[k >> 2] += (k & 3) ? i << (8 * (k & 3) - 2) : i >> 2;
+                v[k] = *(reinterpret_cast<const float*>(reinterpret_cast<const char*>(cent_r) + i) - 16);
+            }
+#pragma unroll
+            for (int d = 0; d < 8; ++d) pk[d] -= 0x10101010u;
+            rk = nibbles_of(pk);
+            if (MODE == kSharedPlanes) {
+#pragma unroll
+                for (int k = 0; k < kChunk; ++k) rec[k] = (rec[k] + v[k]) * a.inv_scale;
+                fwht_lanes<kChunk, true>(rec, bs, lane);
+#pragma unroll
+                for (int k = 0; k < kChunk; ++k) rec[k] = rec[k] * inv * sp[k];
+            } else {
+                fwht_lanes<kChunk, true>(v, bs, lane);
+#pragma unroll
+                for (int k = 0; k < kChunk; ++k) rec[k] = rec[k] + v[k] * inv * sr[k];
+            }
+        }
+        if (active) *reinterpret_cast<uint4*>(a.packed_residual + (size_t)chunk * 16) = rk;
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) { const float sq = rec[k] * rec[k]; acc += (double)sq; }
+        for (uint32_t m = group >> 1; m >= 1; m >>= 1) acc += __shfl_xor(acc, (int)m, kWave);
+        if (active && (lane & (group - 1)) == 0) a.recon_partial[chunk / group] = acc;
+    }
+    if (MODE == kSamples && a.absmax) {
+        for (int m = 32; m >= 1; m >>= 1) largest = max(largest, (uint32_t)__shfl_xor((int)largest, m, kWave));
+        if (lane == 0) a.absmax[blockIdx.x * kQWaves + wave] = largest;
     }
 }
 
@@ -259,7 +344,9 @@ __global__ __launch_bounds__(256) void tq_quantize_small_kernel(QuantArgs a) {
     const float* bP = tab + 32;
     const float* cR = tab + 64;
     const float* bR = tab + 80;
-    const int units = a.in / U;                     // a.slabs == units: one partial sum of squares per unit
+    if (a.tables_out && blockIdx.x == 0 && threadIdx.x < 64) a.tables_out[threadIdx.x] = a.tables[threadIdx.x];
+    const uint32_t seed_p = a.seeds[0], seed_r = a.seeds[1];
+    const int units = a.units;                      // in / U: one partial sum of squares per unit
     const long long id = (long long)blockIdx.x * 256 + threadIdx.x;
     const int row = (int)(id / units);
     const int unit = (int)(id - (long long)row * units);
@@ -272,7 +359,7 @@ __global__ __launch_bounds__(256) void tq_quantize_small_kernel(QuantArgs a) {
 #pragma unroll
     for (int k = 0; k < U; ++k) v[k] = a.w[elem0 + k] / safe;
 #pragma unroll
-    for (int b = 0; b < NB; ++b) small_forward<BS>(v + b * BS, a.seed_p, a.inv_sqrt_bs);
+    for (int b = 0; b < NB; ++b) small_forward<BS>(v + b * BS, seed_p, a.inv_sqrt_bs);
 #pragma unroll
     for (int k = 0; k < U; ++k) v[k] *= a.scale_factor;
     if (a.scaled_out) {
@@ -299,8 +386,8 @@ __global__ __launch_bounds__(256) void tq_quantize_small_kernel(QuantArgs a) {
             for (int k = 0; k < U; ++k) res[k] *= a.inv_scale;
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                small_inverse<BS>(res + b * BS, a.seed_p, a.inv_sqrt_bs);
-                small_forward<BS>(res + b * BS, a.seed_r, a.inv_sqrt_bs);
+                small_inverse<BS>(res + b * BS, seed_p, a.inv_sqrt_bs);
+                small_forward<BS>(res + b * BS, seed_r, a.inv_sqrt_bs);
             }
 #pragma unroll
             for (int k = 0; k < U; ++k) res[k] *= a.scale_factor;
@@ -315,18 +402,18 @@ __global__ __launch_bounds__(256) void tq_quantize_small_kernel(QuantArgs a) {
 #pragma unroll
         for (int k = 0; k < U; ++k) rec[k] = (cP[ip[k]] + cR[ir[k] & 15u]) * a.inv_scale;
 #pragma unroll
-        for (int b = 0; b < NB; ++b) small_inverse<BS>(rec + b * BS, a.seed_p, a.inv_sqrt_bs);
+        for (int b = 0; b < NB; ++b) small_inverse<BS>(rec + b * BS, seed_p, a.inv_sqrt_bs);
     } else {
 #pragma unroll
         for (int k = 0; k < U; ++k) rec[k] = cP[ip[k]] * a.inv_scale;
 #pragma unroll
-        for (int b = 0; b < NB; ++b) small_inverse<BS>(rec + b * BS, a.seed_p, a.inv_sqrt_bs);
+        for (int b = 0; b < NB; ++b) small_inverse<BS>(rec + b * BS, seed_p, a.inv_sqrt_bs);
         if (a.residual_bits > 0) {
             float r2[U];
 #pragma unroll
             for (int k = 0; k < U; ++k) r2[k] = cR[ir[k] & 15u] * a.inv_scale;
 #pragma unroll
-            for (int b = 0; b < NB; ++b) small_inverse<BS>(r2 + b * BS, a.seed_r, a.inv_sqrt_bs);
+            for (int b = 0; b < NB; ++b) small_inverse<BS>(r2 + b * BS, seed_r, a.inv_sqrt_bs);
 #pragma unroll
             for (int k = 0; k < U; ++k) rec[k] = rec[k] + r2[k];
         }
@@ -363,18 +450,78 @@ __global__ void tq_finish_norms_kernel(const float* __restrict__ orig, const dou
     norms[r] = orig[r] / safe;
 }
 
-// FNV-1a over sampled bytes of the fp32 weight, salts 0 and 1 (src/quantizer.cpp:12-28).
+// FNV-1a over sampled bytes of the fp32 weight, salts 0 and 1 (src/quantizer.cpp:12-28): h = (h ^ byte) * P, modulo 2^32,
+// byte after byte.  One thread per salt took 50 us for 4096 bytes (a chain of xor and multiply).  Here all bytes at once:
+//   The exclusive or only touches the low byte, and the low byte of h depends on low bytes alone.  P is odd, so bit k of
+//   (x * P) is bit k of x, flipped by something that the bits of x below k decide: with the bits below k of every
+//   step known, bit k of every step is a running parity.  Eight such scans give the low byte l before each step.
+//   Then h' = (h + d) * P with d = (l ^ byte) - l known, and the hash is h0 P^n + sum of d_i P^(n-i): a plain sum.
+// 18944 x 3584: 20 us, of which most is the samples' way from memory (one byte in 66 KB, a page each).
+constexpr uint32_t kFnvPrime = 16777619u;
+constexpr int kSeedOwn = 8;                                    // bytes of a thread: 4096 to 8191 of them in all, or fewer
+__device__ __forceinline__ uint32_t fnv_power(uint32_t n) {
+    uint32_t r = 1, b = kFnvPrime;
+    for (; n; n >>= 1, b *= b) if (n & 1u) r *= b;
+    return r;
+}
 __global__ __launch_bounds__(1024) void tq_derive_seed_kernel(const uint8_t* __restrict__ bytes, size_t byte_count,
                                                               uint32_t* __restrict__ seeds_out) {
-    __shared__ uint8_t sample[8192];
+    __shared__ uint32_t parity[2][16];                         // of a wave's steps; bit s: salt s
+    __shared__ uint32_t sums[2][16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const size_t stride = (byte_count > 4096) ? (byte_count / 4096) : 1;
-    const size_t count = (byte_count + stride - 1) / stride;       // < 8192
-    for (size_t i = threadIdx.x; i < count; i += blockDim.x) sample[i] = bytes[i * stride];
+    const uint32_t count = (uint32_t)((byte_count + stride - 1) / stride);       // < 8192
+    const uint32_t first = (uint32_t)tid * kSeedOwn;
+    uint32_t byte[kSeedOwn], low[2][kSeedOwn];
+#pragma unroll
+    for (int i = 0; i < kSeedOwn; ++i) {
+        byte[i] = first + i < count ? bytes[(size_t)(first + i) * stride] : 0u;
+        low[0][i] = low[1][i] = 0u;
+    }
+    const uint32_t start[2] = {2166136261u, 2166136261u ^ 1u};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        uint32_t flip[2] = {0u, 0u};                           // bit i: step i turns bit k over
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int i = 0; i < kSeedOwn; ++i) {
+                const uint32_t x = (low[s][i] ^ byte[i]) & ((1u << k) - 1u);
+                flip[s] |= ((((x * kFnvPrime) ^ byte[i]) >> k) & 1u) << i;
+            }
+        const unsigned long long b0 = __ballot(__popc(flip[0]) & 1), b1 = __ballot(__popc(flip[1]) & 1);
+        const unsigned long long below = (1ull << lane) - 1ull;
+        uint32_t run[2] = {(uint32_t)__popcll(b0 & below), (uint32_t)__popcll(b1 & below)};
+        if (lane == 0) parity[k & 1][wave] = (uint32_t)(__popcll(b0) & 1) | (uint32_t)(__popcll(b1) & 1) << 1;
+        __syncthreads();                                       // (two sets: the next bit's are written beside a late reader's)
+        uint32_t before = 0;
+        for (int w = 0; w < wave; ++w) before ^= parity[k & 1][w];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            uint32_t bit = (run[s] + (before >> s) + (start[s] >> k)) & 1u;
+#pragma unroll
+            for (int i = 0; i < kSeedOwn; ++i) {
+                low[s][i] |= bit << k;
+                bit ^= (flip[s] >> i) & 1u;
+            }
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        uint32_t h = 0;
+        uint32_t own = 0;
+#pragma unroll
+        for (int i = 0; i < kSeedOwn; ++i)
+            if (first + i < count) { h = (h + ((low[s][i] ^ byte[i]) - low[s][i])) * kFnvPrime; ++own; }
+        if (own) h *= fnv_power(count - first - own);
+        for (int m = 32; m >= 1; m >>= 1) h += (uint32_t)__shfl_xor((int)h, m, kWave);
+        if (lane == 0) sums[s][wave] = h;
+    }
     __syncthreads();
-    if (threadIdx.x < 2) {
-        uint32_t hash = 2166136261u ^ (uint32_t)threadIdx.x;
-        for (size_t i = 0; i < count; ++i) { hash ^= sample[i]; hash *= 16777619u; }
-        seeds_out[threadIdx.x] = hash;
+    if (tid < 2) {
+        uint32_t h = start[tid] * fnv_power(count);
+        for (int w = 0; w < 16; ++w) h += sums[tid][w];
+        seeds_out[tid] = h;
     }
 }
 
@@ -477,7 +624,9 @@ hipError_t launch_codebook_lookup(const uint8_t* indices, size_t n, const float*
 }
 
 hipError_t launch_row_norms(const float* w, float* norms, int out, int in, hipStream_t stream) {
-    hipLaunchKernelGGL(tq_row_norm_kernel, dim3((out + 3) / 4), dim3(256), 0, stream, w, norms, out, in);
+    const bool vec = in % 4 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0;
+    if (vec) hipLaunchKernelGGL(tq_row_norm_kernel<true>, dim3((out + 3) / 4), dim3(256), 0, stream, w, norms, out, in);
+    else hipLaunchKernelGGL(tq_row_norm_kernel<false>, dim3((out + 3) / 4), dim3(256), 0, stream, w, norms, out, in);
     return hipGetLastError();
 }
 
@@ -488,27 +637,37 @@ hipError_t launch_derive_seeds(const float* w, size_t n_floats, uint32_t* seeds_
 }
 
 // Partial sums of squares per row that launch_quantize_rows writes (what recon_partial must hold and
-// launch_finish_norms is told): 2048-column slabs, or for blocks of at most 16 columns on widths the lane
+// launch_finish_norms is told): blocks, of 32 columns at least, or for blocks of at most 16 columns on widths the lane
 // kernel does not take, units of max(block, 2) columns.
 int quantize_partials_per_row(int in, uint32_t bs) {
-    if (lanes_supported(in, bs)) return (in / kChunk + kWave - 1) / kWave;
+    if (lanes_supported(in, bs)) return in / (int)(bs < (uint32_t)kChunk ? kChunk : bs);
     return in / (int)(bs < 2 ? 2 : bs);
+}
+
+template <int LEVELS>
+static void launch_quantize_mode(const QuantArgs& a, dim3 grid, hipStream_t stream) {
+    const dim3 block(kQWaves * kWave);
+    if (a.residual_bits == 0) hipLaunchKernelGGL((tq_quantize_kernel<kPrimaryPlane, LEVELS>), grid, block, 0, stream, a);
+    else if (a.shared_rotation) hipLaunchKernelGGL((tq_quantize_kernel<kSharedPlanes, LEVELS>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((tq_quantize_kernel<kDualPlanes, LEVELS>), grid, block, 0, stream, a);
 }
 
 hipError_t launch_quantize_rows(const QuantArgsHost& h, hipStream_t stream) {
     QuantArgs a{};
     a.w = h.w; a.orig_norm = h.orig_norm; a.recon_partial = h.recon_partial; a.scaled_out = h.scaled_out;
-    a.packed_primary = h.packed_primary; a.packed_residual = h.packed_residual; a.tables = h.tables;
-    a.out = h.out; a.in = h.in; a.chunks = h.in / kChunk; a.slabs = (a.chunks + kWave - 1) / kWave;
+    a.packed_primary = h.packed_primary; a.packed_residual = h.packed_residual;
+    std::memcpy(a.tables, h.tables, sizeof(a.tables));
+    if (!h.quantize) { a.tables_out = h.tables_out; a.absmax = h.absmax; }
+    a.out = h.out; a.in = h.in; a.chunks = h.in / kChunk;
     a.n_primary = h.n_primary; a.n_residual = h.n_residual;
     a.primary_bits = h.primary_bits; a.residual_bits = h.residual_bits; a.shared_rotation = h.shared_rotation;
-    a.bs = h.bs; a.seed_p = h.seed_p; a.seed_r = h.seed_r;
+    a.bs = h.bs; a.seeds = h.seeds;
     a.scale_factor = h.scale_factor; a.inv_scale = h.inv_scale; a.inv_sqrt_bs = h.inv_sqrt_bs;
     a.quantize = h.quantize;
     if (!lanes_supported(h.in, h.bs)) {                 // blocks of 1 to 16 columns, in registers
         if (!layout_valid(h.in, h.bs) || h.bs > 16) return hipErrorInvalidValue;
-        a.slabs = quantize_partials_per_row(h.in, h.bs);
-        const long long threads = (long long)a.out * a.slabs;
+        a.units = quantize_partials_per_row(h.in, h.bs);
+        const long long threads = (long long)a.out * a.units;
         const long long g = (threads + 255) / 256;
         if (g > 0x7fffffffLL) return hipErrorInvalidValue;
         const dim3 grid((unsigned)g), block(256);
@@ -521,10 +680,17 @@ hipError_t launch_quantize_rows(const QuantArgsHost& h, hipStream_t stream) {
         }
         return hipGetLastError();
     }
-    const long long waves = (long long)a.out * a.slabs;
-    const long long grid = (waves + kQWaves - 1) / kQWaves;
-    if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(tq_quantize_kernel, dim3((unsigned)grid), dim3(kQWaves * kWave), 0, stream, a);
+    const long long chunks = (long long)a.out * a.chunks;
+    if (chunks > 0xffffffffLL - kWave) return hipErrorInvalidValue;
+    a.total_chunks = (uint32_t)chunks;
+    a.tiles = (a.total_chunks + kWave - 1) / kWave;
+    // (what runs at once is three workgroups on each of 256 CUs, two where both planes have a rotation: 240 registers)
+    const bool two = a.quantize && a.residual_bits > 0 && !a.shared_rotation;
+    const dim3 grid(quantize_workgroups(a.tiles, two ? 512 : 768));
+    if (!a.quantize) hipLaunchKernelGGL((tq_quantize_kernel<kSamples, 0>), grid, dim3(kQWaves * kWave), 0, stream, a);
+    else if (!h.sorted) launch_quantize_mode<0>(a, grid, stream);
+    else if (a.n_primary <= 16) launch_quantize_mode<4>(a, grid, stream);
+    else launch_quantize_mode<5>(a, grid, stream);
     return hipGetLastError();
 }
 

@@ -138,6 +138,21 @@ struct DevBuf {
     template <typename T> T* as() { return static_cast<T*>(p); }
 };
 
+// The small buffers of one call in one block: one allocation and one free instead of one each per buffer.
+class SmallBuffers {
+    DevBuf block_;
+    size_t used_ = 0;
+
+public:
+    bool alloc(size_t total, const char* what) { return block_.alloc(total, what); }
+    template <typename T> T* take(size_t n) {
+        T* p = reinterpret_cast<T*>(static_cast<unsigned char*>(block_.p) + used_);
+        used_ += room<T>(n);
+        return p;
+    }
+    template <typename T> static size_t room(size_t n) { return (n * sizeof(T) + 255) & ~(size_t)255; }
+};
+
 bool check_shape(int out, int in, uint32_t bs, const char* who) {
     if (out <= 0 || in <= 0) { set_error(std::string(who) + ": bad dimensions"); return false; }
     if (bs == 0 || in % (int)bs != 0) {
@@ -160,6 +175,12 @@ void fill_tables(const float* cbp, int np, const float* cbr, int nr, float* t) {
     midpoints(cbp, np, t + 32);
     std::memcpy(t + 64, cbr, nr * sizeof(float));
     midpoints(cbr, nr, t + 80);
+}
+
+bool ascending(const float* b, int n) {
+    for (int i = 1; i < n; ++i)
+        if (!(b[i - 1] <= b[i])) return false;
+    return true;
 }
 
 // generate_codebook_from_data_cpu (src/codebook.cpp:99-143), one pass over all samples per step: samples that are not
@@ -206,9 +227,10 @@ bool lloyd_max(const float* samples_dev, size_t n, int bits, int iterations, boo
 
 // The codebook of the samples and, with residual_bits > 0, the one of their residuals against the global codebook
 // (gtab_dev: [0..31] centroids, [32..62] boundaries), each from the analytic start (src/codebook.cpp:99-143,
-// src/converter.cpp:345-357).
+// src/converter.cpp:345-357).  absmax: bits of the largest |sample| in so many parts, or NULL; result: room on the device.
 bool fit_codebooks(const float* samples_dev, size_t n, int primary_bits, int residual_bits, int iterations,
-                   const float* gtab_dev, int ngc, float* cbp_out, float* cbr_out) {
+                   const float* gtab_dev, int ngc, const uint32_t* absmax, int absmax_parts, tq::FitResult* result, float* cbp_out,
+                   float* cbr_out) {
     const int problems = residual_bits > 0 ? 2 : 1;
     if (tq::fit_supported(n)) {
         tq::FitCodebooks cb{};
@@ -217,9 +239,9 @@ bool fit_codebooks(const float* samples_dev, size_t n, int primary_bits, int res
             cb.nc[p] = tq_generate_codebook(bits[p], cb.init[p], nullptr);
             if (cb.nc[p] < 0) { set_error("tq_fit_layer_codebooks: unsupported bit width"); return false; }
         }
-        DevBuf res;
+        cb.absmax = absmax;
+        cb.absmax_parts = absmax_parts;
         tq::FitResult r{};
-        if (!res.alloc(sizeof(r), "hipMalloc(fit result)")) return false;      // (the passes need as much)
         for (bool everything = !tq::fit_predicts(n);; everything = true) {
             DevBuf work;
             if (!work.alloc(tq::fit_workspace_bytes(n, problems, everything), "hipMalloc(fit)")) break;    // (the passes below need none)
@@ -228,8 +250,8 @@ bool fit_codebooks(const float* samples_dev, size_t n, int primary_bits, int res
             bool missed = true, passes = false;
             for (int round = 0; missed && !passes && round < (everything ? 1 : 4); ++round) {
                 if (!hip_ok(tq::launch_fit(samples_dev, n, problems, gtab_dev, ngc, cb, iterations, round == 0, everything, work.p,
-                                           res.as<tq::FitResult>(), nullptr), "fit launch") ||
-                    !hip_ok(hipMemcpy(&r, res.p, sizeof(r), hipMemcpyDeviceToHost), "copy centroids"))
+                                           result, nullptr), "fit launch") ||
+                    !hip_ok(hipMemcpy(&r, result, sizeof(r), hipMemcpyDeviceToHost), "copy centroids"))
                     return false;
                 missed = r.missed[0] || (problems == 2 && r.missed[1]);
                 passes = r.bad || r.coarse[0] || (problems == 2 && r.coarse[1]);
@@ -302,36 +324,33 @@ int tq_quantize_weight(const float* weight_dev, int out, int in,
             set_error("tq_quantize_weight: bad codebook sizes or bit widths"); return 1;
         }
         const int slabs = tq::quantize_partials_per_row(in, block_size);
-        DevBuf d_orig, d_partial, d_tables, d_seeds;
-        float tables[96];
-        fill_tables(cbp, np, cbr, nr, tables);
+        SmallBuffers small;
+        if (!small.alloc(SmallBuffers::room<float>(out) + SmallBuffers::room<double>((size_t)out * slabs) + SmallBuffers::room<uint32_t>(2),
+                         "hipMalloc(norms)")) return 1;
+        float* const orig = small.take<float>(out);
+        double* const partial = small.take<double>((size_t)out * slabs);
+        uint32_t* const d_seeds = small.take<uint32_t>(2);
         uint32_t seeds[2] = {0, 0};
-        if (!d_orig.alloc((size_t)out * sizeof(float), "hipMalloc(norms)") ||
-            !d_partial.alloc((size_t)out * slabs * sizeof(double), "hipMalloc(partials)") ||
-            !d_tables.alloc(sizeof(tables), "hipMalloc(tables)") ||
-            !d_seeds.alloc(2 * sizeof(uint32_t), "hipMalloc(seeds)") ||
-            !hip_ok(hipMemcpy(d_tables.p, tables, sizeof(tables), hipMemcpyHostToDevice), "copy tables") ||
-            !hip_ok(tq::launch_derive_seeds(weight_dev, (size_t)out * in, d_seeds.as<uint32_t>(), nullptr), "derive_seed") ||
-            !hip_ok(hipMemcpy(seeds, d_seeds.p, sizeof(seeds), hipMemcpyDeviceToHost), "copy seeds") ||
-            !hip_ok(tq::launch_row_norms(weight_dev, d_orig.as<float>(), out, in, nullptr), "row norms"))
+        if (!hip_ok(tq::launch_derive_seeds(weight_dev, (size_t)out * in, d_seeds, nullptr), "derive_seed") ||
+            !hip_ok(tq::launch_row_norms(weight_dev, orig, out, in, nullptr), "row norms"))
             return 1;
-        if (residual_bits == 0 &&
-            !hip_ok(hipMemset(pr_dev, 0, (size_t)out * (in / 2)), "zero residual plane")) return 1;
 
         tq::QuantArgsHost a{};
-        a.w = weight_dev; a.orig_norm = d_orig.as<float>(); a.recon_partial = d_partial.as<double>();
+        a.w = weight_dev; a.orig_norm = orig; a.recon_partial = partial;
         a.scaled_out = nullptr; a.packed_primary = pp_dev; a.packed_residual = pr_dev;
-        a.tables = d_tables.as<float>();
+        fill_tables(cbp, np, cbr, nr, a.tables);
+        a.seeds = d_seeds;
         a.out = out; a.in = in; a.n_primary = np; a.n_residual = nr;
         a.primary_bits = primary_bits; a.residual_bits = residual_bits; a.shared_rotation = shared_rotation ? 1 : 0;
-        a.bs = block_size; a.seed_p = seeds[0]; a.seed_r = seeds[1];
+        a.bs = block_size;
         a.scale_factor = std::sqrt(static_cast<float>(in));                     // src/quantizer.cpp:51
         a.inv_scale = 1.0f / a.scale_factor;                                    // :52
         a.inv_sqrt_bs = 1.0f / std::sqrt(static_cast<float>(block_size));       // src/rotation.cpp:301
         a.quantize = 1;
+        a.sorted = ascending(a.tables + 32, np - 1) && ascending(a.tables + 80, nr - 1);
         if (!hip_ok(tq::launch_quantize_rows(a, nullptr), "quantize rows") ||
-            !hip_ok(tq::launch_finish_norms(d_orig.as<float>(), d_partial.as<double>(), norms_dev, out, slabs, nullptr),
-                    "finish norms") ||
+            !hip_ok(tq::launch_finish_norms(orig, partial, norms_dev, out, slabs, nullptr), "finish norms") ||
+            !hip_ok(hipMemcpy(seeds, d_seeds, sizeof(seeds), hipMemcpyDeviceToHost), "copy seeds") ||     // (waits for all of it)
             !hip_ok(hipDeviceSynchronize(), "quantize sync"))
             return 1;
         seeds_host[0] = seeds[0];
@@ -352,37 +371,36 @@ int tq_fit_layer_codebooks(const float* weight_dev, int out, int in, uint32_t bl
         if (!check_shape(out, in, block_size, "tq_fit_layer_codebooks")) return 1;
         if (ngc < 2 || ngc > 32) { set_error("tq_fit_layer_codebooks: bad global codebook"); return 1; }
         const size_t n = (size_t)out * in;
-        DevBuf d_orig, d_scaled, d_tables, d_seeds, d_g;
-        float tables[96];
-        fill_tables(gcp, ngc, gcp, ngc > 16 ? 16 : ngc, tables);
-        float gtab[64];
-        std::memset(gtab, 0, sizeof(gtab));
-        std::memcpy(gtab, gcp, ngc * sizeof(float));
-        midpoints(gcp, ngc, gtab + 32);
-        uint32_t seeds[2];
-        if (!d_orig.alloc((size_t)out * sizeof(float), "hipMalloc(norms)") ||
-            !d_scaled.alloc(n * sizeof(float), "hipMalloc(samples)") ||
-            !d_tables.alloc(sizeof(tables), "hipMalloc(tables)") ||
-            !d_g.alloc(sizeof(gtab), "hipMalloc(global codebook)") ||
-            !d_seeds.alloc(2 * sizeof(uint32_t), "hipMalloc(seeds)") ||
-            !hip_ok(hipMemcpy(d_tables.p, tables, sizeof(tables), hipMemcpyHostToDevice), "copy tables") ||
-            !hip_ok(hipMemcpy(d_g.p, gtab, sizeof(gtab), hipMemcpyHostToDevice), "copy global codebook") ||
-            !hip_ok(tq::launch_derive_seeds(weight_dev, n, d_seeds.as<uint32_t>(), nullptr), "derive_seed") ||
-            !hip_ok(hipMemcpy(seeds, d_seeds.p, sizeof(seeds), hipMemcpyDeviceToHost), "copy seeds") ||
-            !hip_ok(tq::launch_row_norms(weight_dev, d_orig.as<float>(), out, in, nullptr), "row norms"))
+        DevBuf d_scaled;
+        SmallBuffers small;
+        const bool lanes = tq::lanes_supported(in, block_size);
+        const int waves = lanes ? tq::quantize_sample_waves(out, in) : 0;
+        if (!d_scaled.alloc(n * sizeof(float), "hipMalloc(samples)") ||
+            !small.alloc(SmallBuffers::room<float>(out) + SmallBuffers::room<float>(64) + SmallBuffers::room<uint32_t>(2) +
+                         SmallBuffers::room<uint32_t>(waves) + SmallBuffers::room<tq::FitResult>(1), "hipMalloc(norms)")) return 1;
+        float* const orig = small.take<float>(out);
+        float* const gtab = small.take<float>(64);
+        uint32_t* const d_seeds = small.take<uint32_t>(2);
+        uint32_t* const absmax = small.take<uint32_t>(waves);
+        tq::FitResult* const result = small.take<tq::FitResult>(1);
+        if (!hip_ok(tq::launch_derive_seeds(weight_dev, n, d_seeds, nullptr), "derive_seed") ||
+            !hip_ok(tq::launch_row_norms(weight_dev, orig, out, in, nullptr), "row norms"))
             return 1;
         tq::QuantArgsHost a{};
-        a.w = weight_dev; a.orig_norm = d_orig.as<float>(); a.scaled_out = d_scaled.as<float>();
-        a.tables = d_tables.as<float>();
+        a.w = weight_dev; a.orig_norm = orig; a.scaled_out = d_scaled.as<float>();
+        fill_tables(gcp, ngc, gcp, ngc > 16 ? 16 : ngc, a.tables);           // ([0..63]: what the fit reads)
+        a.tables_out = gtab;
+        a.seeds = d_seeds;
+        a.absmax = lanes ? absmax : nullptr;
         a.out = out; a.in = in; a.n_primary = ngc; a.n_residual = 2;
-        a.primary_bits = primary_bits; a.bs = block_size; a.seed_p = seeds[0]; a.seed_r = seeds[1];
+        a.primary_bits = primary_bits; a.bs = block_size;
         a.scale_factor = std::sqrt(static_cast<float>(in));
         a.inv_scale = 1.0f / a.scale_factor;
         a.inv_sqrt_bs = 1.0f / std::sqrt(static_cast<float>(block_size));
         a.quantize = 0;
         if (!hip_ok(tq::launch_quantize_rows(a, nullptr), "rotate samples")) return 1;
-        return fit_codebooks(d_scaled.as<float>(), n, primary_bits, residual_bits, iterations, d_g.as<float>(), ngc, cbp_out,
-                             cbr_out) ? 0 : 1;
+        return fit_codebooks(d_scaled.as<float>(), n, primary_bits, residual_bits, iterations, gtab, ngc, lanes ? absmax : nullptr, waves,
+                             result, cbp_out, cbr_out) ? 0 : 1;
     } catch (...) { set_error("tq_fit_layer_codebooks: exception"); return 1; }
 }
 
@@ -432,10 +450,10 @@ int tq_generate_codebook_from_data_host(const float* data_host, size_t n, int bi
         if (!centroids_out || (n > 0 && !data_host)) { set_error("tq_generate_codebook_from_data: NULL argument"); return -1; }
         if (n == 0) return tq_generate_codebook(bits, centroids_out, boundaries_out);   // src/codebook.cpp:101-103
         if (bits < 1 || bits > 5) { set_error("Unsupported bit width; must be 1-5"); return -1; }
-        DevBuf d;
-        if (!d.alloc(n * sizeof(float), "hipMalloc(samples)") ||
+        DevBuf d, res;
+        if (!d.alloc(n * sizeof(float), "hipMalloc(samples)") || !res.alloc(sizeof(tq::FitResult), "hipMalloc(fit result)") ||
             !hip_ok(hipMemcpy(d.p, data_host, n * sizeof(float), hipMemcpyHostToDevice), "copy samples") ||
-            !fit_codebooks(d.as<float>(), n, bits, 0, iterations, nullptr, 0, centroids_out, nullptr))
+            !fit_codebooks(d.as<float>(), n, bits, 0, iterations, nullptr, 0, nullptr, 0, res.as<tq::FitResult>(), centroids_out, nullptr))
             return -1;
         if (boundaries_out) midpoints(centroids_out, 1 << bits, boundaries_out);
         return 1 << bits;
