@@ -25,8 +25,8 @@
 // that) the fit says so and is left to the pass per step.
 //
 // 18944 x 3584 (68 M samples, 2 x 100 steps).  One pass over all samples per step took 230 ms, 1.1 ms each (thread-private
-// bins in 96 KB of LDS, one wave per SIMD) and a copy of the partial sums to the host; the kernels here take 1.13 ms:
-// scatter 320 us, iterate 304, refine 143, hist 140, predict 99, absmax 58, offsets 45, scan 23.  What bounds them is
+// bins in 96 KB of LDS, one wave per SIMD) and a copy of the partial sums to the host; the kernels here take 1.04 ms:
+// scatter 320 us, iterate 264, refine 138, hist 140, predict 99, offsets 45, scan 23.  What bounds them is
 // said at each.  Sorting every sample instead of the expected 15 % took 1840 us in the scatter kernel and 870 in refine.
 #include "tq_bins.h"
 #include "tq_device.h"
@@ -72,6 +72,16 @@ __device__ __forceinline__ void fit_cell(float v, float scale, uint32_t& cell, u
     off = lin ? lo : (d & 0x1fffu);
     if (i >= (uint32_t)kFitHalf) { i = (uint32_t)kFitHalf - 1; off = 0x1fffu; }   // (a boundary beyond all samples)
     cell = v < 0.0f ? (uint32_t)kFitHalf - 1u - i : (uint32_t)kFitHalf + i;
+}
+
+// The offset of a sample whose cell is known, one or four instructions: the scale is a power of two and leaves the mantissa
+// as it is.  `whole`: the linear cell's number.
+__device__ __forceinline__ uint32_t fit_log_offset(float v) { return __builtin_bit_cast(uint32_t, v) & 0x1fffu; }
+__device__ __forceinline__ uint32_t fit_linear_offset(float v, float scale, float whole) {
+    return (uint32_t)((__builtin_fabsf(v) * scale * 65536.0f - whole) * 4194304.0f);
+}
+__device__ __forceinline__ float fit_cell_whole(uint32_t cell) {
+    return (float)(cell < (uint32_t)kFitHalf ? (uint32_t)kFitHalf - 1u - cell : cell - (uint32_t)kFitHalf);
 }
 
 // Magnitude of a cell's lower end, and how far its offsets are shifted, in units of 2^-38 of the scale.
@@ -474,9 +484,9 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_refine_kernel(const FitPar
     float* dst = fine + fit_region(kept, p) + at;
     uint64_t base; int shift; bool neg;
     fit_cell_base((uint32_t)cell, base, shift, neg);
+    const float whole = fit_cell_whole((uint32_t)cell);
     auto part_of = [&](float v, uint32_t& o) {
-        uint32_t c;
-        fit_cell(v, scale, c, o);
+        o = shift ? fit_log_offset(v) : fit_linear_offset(v, scale, whole);
         return fit_part(o, shift);
     };
     uint32_t cnt = 0;                                                 // wave 0: of part `tid`
@@ -535,7 +545,31 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_refine_kernel(const FitPar
 
 // All Lloyd-Max steps of one codebook (src/codebook.cpp:105-136): one workgroup, a wave per boundary.  out->missed[p]:
 // a boundary came to a cell that was not kept; out->cent and out->steps say how far the fit has come.  A step is a chain
-// of three latencies (the cell's entries, its samples, the workgroup's sums): 3 us.
+// of latencies (the cell's entries, its samples, the workgroup's sums).  The entries stay in the wave's registers, a part per
+// lane, as long as the boundary stays in its cell; a sample's offset comes from its mantissa, the cell being known; no more
+// rounds of 64 samples run than there are samples for (four waves share a SIMD: what a wave issues counts), and sums over a
+// wave go through DPP operands: 3.0 us a step -> 2.6.
+struct FitCut {                                       // a boundary's cell
+    uint32_t cell, at, s0;
+    i128 q0;                                          // of the samples below the cell
+    uint32_t n_part, n_all;                           // lane l: samples and offset sums below part l; of all
+    unsigned long long o_part, o_all;
+    uint64_t base; int shift; bool neg;
+};
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
+    auto step = [&](auto other) { v += __builtin_bit_cast(uint32_t, other(__builtin_bit_cast(float, v))); };
+    step([](float x) { return lane_xor<1>(x); });
+    step([](float x) { return lane_xor<2>(x); });
+    step([](float x) { return lane_xor<4>(x); });
+    step([](float x) { return lane_xor<8>(x); });
+    step([](float x) { return lane_xor<16>(x); });
+    step([](float x) { return lane_xor<32>(x); });
+    return v;
+}
+__device__ __forceinline__ unsigned long long lane_value(unsigned long long v, int l) {
+    return (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32 |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
+}
 __global__ __launch_bounds__(kFitThreads) void tq_fit_iterate_kernel(const FitParams* __restrict__ P, size_t n, int iterations,
                                                                      const uint32_t* __restrict__ start_all,
                                                                      const i128* __restrict__ below_all,
@@ -571,44 +605,70 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_iterate_kernel(const FitPa
     __syncthreads();
     const unsigned long long cut_lo = start[kFitHalf - kFitCut], cut_hi = start[kFitHalf + kFitCut];
     int iter = out->steps[p];
+    constexpr int kCuts = 2;                                          // boundaries of a wave: 31 of them, 16 waves
+    FitCut cuts[kCuts];
+#pragma unroll
+    for (int u = 0; u < kCuts; ++u) cuts[u].cell = kFitAbsent;
     for (; iter < iterations; ++iter) {
-        for (int k = wave; k < nc - 1; k += kFitThreads / kWave) {
+#pragma unroll
+        for (int u = 0; u < kCuts; ++u) {
+            const int k = wave + u * (kFitThreads / kWave);
+            if (k >= nc - 1) continue;
+            FitCut& c = cuts[u];
             const float b = (cent[k] + cent[k + 1]) * 0.5f;
             uint32_t cell, boff;
             fit_cell(b, scale, cell, boff);
-            uint64_t base; int shift; bool neg;
-            fit_cell_base(cell, base, shift, neg);
-            const uint32_t part = fit_part(boff, shift);
-            const size_t q = ((size_t)p * kFitCells + cell) * (kFitParts + 1);
-            const uint32_t at = place[cell], s0 = start[cell];
-            const i128 q0 = below[cell];
-            const uint32_t n0 = part_n[q + part], n1 = part_n[q + part + 1], n_all = part_n[q + kFitParts];
-            const unsigned long long o0 = part_o[q + part], o1 = part_o[q + part + 1], o_all = part_o[q + kFitParts];
-            if (at == kFitAbsent) { if (lane == 0) missed = 1; continue; }
+            cell = (uint32_t)__builtin_amdgcn_readfirstlane((int)cell);
+            boff = (uint32_t)__builtin_amdgcn_readfirstlane((int)boff);
+            if (cell != c.cell) {
+                const size_t q = ((size_t)p * kFitCells + cell) * (kFitParts + 1);
+                c.cell = cell;
+                c.at = place[cell];
+                c.s0 = start[cell];
+                c.q0 = below[cell];
+                c.n_part = part_n[q + lane];
+                c.n_all = part_n[q + kFitParts];
+                c.o_part = part_o[q + lane];
+                c.o_all = part_o[q + kFitParts];
+                fit_cell_base(cell, c.base, c.shift, c.neg);
+            }
+            if (c.at == kFitAbsent) { if (lane == 0) missed = 1; continue; }
+            const int part = (int)fit_part(boff, c.shift);
+            const uint32_t n0 = (uint32_t)__builtin_amdgcn_readlane((int)c.n_part, part);
+            const uint32_t n1 = part + 1 < kFitParts ? (uint32_t)__builtin_amdgcn_readlane((int)c.n_part, (part + 1) & 63) : c.n_all;
             // larger magnitudes are smaller values below zero: the parts above are the ones to the left there
             uint32_t cnt = 0;
             unsigned long long off = 0;
-            for (uint32_t i = at + n0 + lane; i < at + n1; i += kWave * 8) {      // eight loads at once: a step is a chain of latencies
+            const float whole = fit_cell_whole(cell);
+            for (uint32_t i = n0; i < n1; i += kWave * 8) {                               // eight loads at once: a step is a chain of latencies
+                const float* src = fine + c.at + i;
+                const uint32_t left = n1 - i;                                            // (no more rounds of 64 than samples fill)
                 float v[8];
+                uint32_t own = 0;                                                        // (8 offsets of 22 bits, 64 lanes: below 2^31)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = fine[i + j * kWave < at + n1 ? i + j * kWave : i];
+                for (int j = 0; j < 8; ++j)
+                    if (j * kWave < left) v[j] = src[j * kWave + lane < left ? j * kWave + lane : 0];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    uint32_t c, o;
-                    fit_cell(v[j], scale, c, o);
-                    if (i + j * kWave < at + n1 && !(b < v[j])) { cnt += 1; off += o; }
-                }
+                for (int j = 0; j < 8; ++j)
+                    if (j * kWave < left) {
+                        const bool below_b = j * kWave + lane < left && !(b < v[j]);
+                        const uint32_t o = c.shift ? fit_log_offset(v[j]) : fit_linear_offset(v[j], scale, whole);
+                        cnt += (uint32_t)__popcll(__ballot(below_b));
+                        own += below_b ? o : 0u;
+                    }
+                off += wave_sum_u32(own);
             }
-            for (int m = 32; m >= 1; m >>= 1) {
-                cnt += (uint32_t)__shfl_xor((int)cnt, m, kWave);
-                off += (unsigned long long)__shfl_xor((long long)off, m, kWave);
+            if (c.neg) {
+                cnt += c.n_all - n1;
+                off += c.o_all - (part + 1 < kFitParts ? lane_value(c.o_part, (part + 1) & 63) : c.o_all);
+            } else {
+                cnt += n0;
+                off += lane_value(c.o_part, part);
             }
-            cnt += neg ? n_all - n1 : n0;
-            off += neg ? o_all - o1 : o0;
             if (lane == 0) {
-                const i128 t = (i128)cnt * (i128)base + ((i128)off << shift);
-                left_n[k + 1] = s0 + (unsigned long long)cnt;
-                left_q[k + 1] = q0 + (neg ? -t : t);
+                const i128 t = (i128)cnt * (i128)c.base + ((i128)off << c.shift);
+                left_n[k + 1] = c.s0 + (unsigned long long)cnt;
+                left_q[k + 1] = c.q0 + (c.neg ? -t : t);
             }
         }
         __syncthreads();
