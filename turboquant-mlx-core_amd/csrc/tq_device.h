@@ -260,7 +260,8 @@ __device__ __forceinline__ float lane_xor(float v) {
 // own DPP operand and is written in place, two instructions; an fma has no DPP operand for its addend: a move, the
 // fma and, where the stage is under a branch, half a copy.)
 // Four at a time, products before sums: a DPP instruction waits two issue slots for a register that the instruction before it
-// wrote, and left to itself the compiler puts the two side by side with a wait between them.
+// wrote, and left to itself the compiler puts the two side by side with a wait between them.  (Up to eight values, the kernels
+// of few rows: left to the compiler, which has other work to put there; kept apart 1 % slower.)
 template <int N, typename F>
 __device__ __forceinline__ void butterfly_pairs(float (&v)[N], float sgn, F partner) {
     constexpr int G = N < 4 ? N : 4;
@@ -270,10 +271,10 @@ __device__ __forceinline__ void butterfly_pairs(float (&v)[N], float sgn, F part
         float own[G];
 #pragma unroll
         for (int j = 0; j < G; ++j) own[j] = v[k + j] * sgn;
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (N > 8) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < G; ++j) v[k + j] = partner(v[k + j]) + own[j];
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (N > 8) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
