@@ -101,12 +101,45 @@ void two_parts() {
     expect(poor.forward(40) == 0 && !Layer::ran("tq_rotate_split") && !dev.launched.empty(), "no memory");
 }
 
+// Layers on the same activations: one launch where their tiles do not fill the chip one layer at a time, captured too once they
+// are reserved, in the workspaces their own calls need; layer by layer where those cannot be had, or where a layer comes twice.
+void groups() {
+    const struct { int in; uint32_t bs, seed; int outs[3], rows; const char* kernel; size_t launches; } cases[] = {
+        {896, 128, 1234, {896, 130, 128}, 33, "tq_prefill_tile_kernel", 2},
+        {960, 64, 0, {512, 96, 33}, 40, "tq_prefill_tile_kernel", 2},
+        {1024, 512, 0, {3456, 300, 257}, 2000, "tq_prefill_panel_kernel", 2},
+        {2560, 512, 1234, {5120, 512, 514}, 1600, "tq_prefill_panel_kernel", 5}};       // (three are composed)
+    for (const auto& c : cases) {
+        std::vector<Layer*> ls;
+        tq_linear_t hs[3];
+        void* ys[3];
+        for (int j = 0; j < 3; ++j) {
+            ls.push_back(new Layer(c.in, c.outs[j], c.rows, 4, true, c.seed, c.bs));
+            hs[j] = ls[j]->h;
+            ys[j] = ls[j]->y.data();
+            expect(tq_linear_reserve(hs[j], c.rows) == 0, tq_last_error(), c.in);
+        }
+        auto run = [&]() {
+            dev.launched.clear();
+            return tq_linear_forward_group(hs, 3, ls[0]->x.data(), TQ_DTYPE_F32, c.rows, ys, TQ_DTYPE_F32, reinterpret_cast<void*>(&dev));
+        };
+        dev.capturing = true;
+        expect(run() == 0, tq_last_error(), c.in);
+        expect(Layer::ran(c.kernel) && dev.launched.size() == c.launches, "shared launches", dev.launched.size());
+        dev.capturing = false;
+        hs[2] = hs[1];
+        expect(run() == 0 && dev.launched.size() > c.launches, "a layer twice: one by one", dev.launched.size());
+        for (Layer* l : ls) delete l;
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const fake::Check checks[] = {{"compose_without_memory", compose_without_memory},
                                   {"reserve_without_memory", reserve_without_memory},
                                   {"five_bit_one_row", five_bit_one_row},
-                                  {"two_parts", two_parts}};
+                                  {"two_parts", two_parts},
+                                  {"groups", groups}};
     return fake::run(checks, argc, argv);
 }

@@ -1,0 +1,75 @@
+"""Layers that share the prefill launches (q, k, v or gate, up on 33 and more rows), and the gated block's product formed where the
+rows are rotated or the chunks added.  References: the dequantised weights (bit-exact elsewhere) in 64 bits."""
+import numpy as np
+import pytest
+
+from test_gpu_mlp import _Hip, _rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def tq():
+    import __graft_entry__ as entry
+    pkg = entry.load_package()
+    pkg.lib()
+    return pkg
+
+
+def _layer(tq, out_f, in_f, bs, mode, seed):
+    w = (np.random.default_rng(seed).standard_normal((out_f, in_f)) * 0.02).astype(np.float32)
+    cb = tq.generate_codebook(4)
+    qw = tq.quantize_weight(w, cb, cb, 4, 0 if mode == "primary_only" else 4, bs, mode == "shared")
+    layer = tq.TurboQuantLinear(in_f, out_f, qw, cb, cb, bs)
+    return layer, layer.dequantize().astype(np.float64)
+
+
+@pytest.mark.parametrize("mode,outs,in_f,bs,batch", [
+    ("dual", (896, 130, 128), 896, 128, 33),              # small tiles, pairs of 64-column tiles; a ragged weight tile
+    ("dual", (200, 64), 1088, 64, 77),                    # ... an odd number of 64-column tiles, two layers
+    ("shared", (512, 96, 33), 960, 64, 40),
+    ("primary_only", (640, 128, 128), 1536, 512, 130),
+    ("shared", (3456, 300, 257), 1024, 512, 2000),        # panels that k and v do not fill; ragged panel and weight tiles
+    ("dual", (5120, 512, 514), 2560, 512, 1600),          # ... through composed planes
+])
+def test_group_of_prefill_layers(tq, mode, outs, in_f, bs, batch):
+    """fp16 weights and rotated activations, sums in fp32: 2e-4 to 4e-4, so 1e-3 as for the layers by themselves."""
+    hip = _Hip()
+    made = [_layer(tq, o, in_f, bs, mode, 50 + j) for j, o in enumerate(outs)]
+    x = np.random.default_rng(batch).standard_normal((batch, in_f)).astype(np.float32)
+    dx, ys = hip.upload(x), [hip.alloc(batch * o * 4) for o in outs]
+    for _ in range(2):                                     # (workspaces are used again)
+        tq.forward_group_device([m[0] for m in made], dx, tq.F32, batch, ys, tq.F32)
+    for o, y, (_, w) in zip(outs, ys, made):
+        assert _rel(hip.download(y, (batch, o), np.float32), x.astype(np.float64) @ w.T) < 1e-3
+    hip.free(dx, *ys)
+    for layer, _ in made:
+        layer.close()
+
+
+@pytest.mark.parametrize("mode,hidden,inter,bs,batch", [
+    ("dual", 512, 1088, 64, 37),                          # gate and up in one launch; product formed with two rows per wave
+    ("shared", 256, 5120, 256, 700),                      # ... with eight, the last of them past the rows
+    ("primary_only", 512, 1250, 2, 20),                   # blocks of two columns: a launch of its own forms the product
+    ("shared", 512, 1090, 512, 5), ("shared", 512, 896, 128, 9),      # chunk sums of one column per lane, and of four:
+    ("dual", 512, 16384, 512, 16),
+])
+def test_gated_block_product(tq, mode, hidden, inter, bs, batch):
+    """Three layers of 2e-4 to 4e-4 each, independent: 1e-3."""
+    hip = _Hip()
+    bs_down = tq.best_block_size(inter)
+    bs_up = min(bs, tq.best_block_size(hidden))
+    (gate, wg), (up, wu) = (_layer(tq, inter, hidden, bs_up, mode, 60 + j) for j in range(2))
+    down, wd = _layer(tq, hidden, inter, bs_down, mode, 62)
+    mlp = tq.TurboQuantMLP(gate, up, down, max_batch=batch)
+    x = np.random.default_rng(batch).standard_normal((batch, hidden)).astype(np.float32)
+    dx, dy = hip.upload(x), hip.alloc(batch * hidden * 4)
+    mlp.forward_device(dx, tq.F32, batch, dy, tq.F32)
+    x64 = x.astype(np.float64)
+    g = x64 @ wg.T
+    want = (g / (1.0 + np.exp(-g)) * (x64 @ wu.T)) @ wd.T
+    assert _rel(hip.download(dy, (batch, hidden), np.float32), want) < 1e-3
+    mlp.close()
+    hip.free(dx, dy)
+    for layer in (gate, up, down):
+        layer.close()

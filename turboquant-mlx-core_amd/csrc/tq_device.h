@@ -77,8 +77,14 @@ hipError_t launch_prefill(const LayerView& L, const void* x, int x_dtype, int ba
 // Images of the rotated activations: 256-row tiles as tq_prefill_gemm_kernel keeps them in LDS, or fragment images of 512
 // rows (tq_prefill_panel_kernel) or 32 rows (tq_prefill_tile_kernel).
 enum : int { kTileImage = 0, kPanelImage = 1, kBlockImage = 2 };
+// gate: the activations are silu(gate) * x (both fp32), where rotate_takes_gate() (fragment images only).
 hipError_t launch_rotate_tiles(const LayerView& L, const void* x, int x_dtype, int batch, void* workspace,
-                               hipStream_t stream, int layout = kTileImage);
+                               hipStream_t stream, int layout = kTileImage, const float* gate = nullptr);
+// Layers of equal width, block and mode on the same activations, each into its own workspace, one launch where fragment
+// images of blocks of up to 512 columns are written.
+hipError_t launch_rotate_group(const LayerView* Ls, int n, const void* x, int x_dtype, const float* gate, int batch,
+                               void* const* workspaces, hipStream_t stream, int layout);
+bool rotate_takes_gate(const LayerView& L);
 // Small batches (tq_skinny.hip): 2..32 rows (any activation type) on shared-rotation layers, batch rows as
 // the M side of 16x16x32 MFMAs.  xt_workspace as for launch_prefill; partial: skinny_partial_bytes() for this batch.
 constexpr int kSkinnyMaxRows = 32;
@@ -87,10 +93,11 @@ size_t skinny_partial_bytes(const LayerView& L, int batch);
 size_t skinny_workspace_bytes(const LayerView& L, int batch);
 hipError_t launch_skinny(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,
                          void* xt_workspace, float* partial, int num_cus, hipStream_t stream);
-// Two or three shared-rotation layers of equal width on the same activation rows: both launches shared.
+// Two or three layers of equal width and mode on the same activation rows: both launches shared.  gated (two layers of as
+// many rows): silu(layer 0) * layer 1 is written to ys[0] alone, fp32.
 bool skinny_group_supported(const LayerView* Ls, int n, int x_dtype, int batch, int num_cus);
 hipError_t launch_skinny_group(const LayerView* Ls, int n, const void* x, int x_dtype, int batch, void* const* ys,
-                               int y_dtype, float* const* partials, int num_cus, hipStream_t stream);
+                               int y_dtype, float* const* partials, int num_cus, hipStream_t stream, bool gated = false);
 // Two to twelve rows (tq_gemv_few.hip): the batch-1 kernel's shape (whole weight rows per
 // stream, no cut along K, no second kernel), four weight rows by four activation rows per 4x4x4 matrix block.
 // workspace: gemv_few_workspace_bytes() (0 for most calls of up to four rows: the workgroups rotate the rows

@@ -410,9 +410,18 @@ static bool takes_compose(tq_linear_s* h, const tq::LayerView& V, int batch, hip
                                       stream, &h->retired));
 }
 static int run_compose(tq_linear_s* h, const tq::LayerView& V, const void* x_dev, int x_dtype, int batch, void* y_dev, int y_dtype,
-                       hipStream_t stream, void* static_ws, size_t capacity) {
+                       hipStream_t stream, void* static_ws, size_t capacity, const float* x_gate) {
     return hip_ok(tq::launch_prefill_compose(V, x_dev, x_dtype, batch, y_dev, y_dtype, static_ws ? static_ws : h->d_work, capacity,
-                                             device_cu_count(), stream), "tq_prefill_compose launch") ? 0 : 1;
+                                             device_cu_count(), stream, x_gate), "tq_prefill_compose launch") ? 0 : 1;
+}
+
+// Activations that are silu(gate) * x, gate and x fp32 (the middle of a gated block): where a kernel that rotates forms the product
+// it takes the gate; for the others it is formed in `out`, [batch, in] fp32, first.
+struct GatedRows { const float* gate; float* out; };
+static bool form_gated(const GatedRows& gated, const void** x_dev, size_t n, hipStream_t stream) {
+    if (!hip_ok(tq::launch_silu_mul(gated.gate, static_cast<const float*>(*x_dev), gated.out, tq::kF32, n, stream), "silu_mul launch")) return false;
+    *x_dev = gated.out;
+    return true;
 }
 
 // Shared by tq_linear_forward, tq_linear_forward_static and the MLP block.  gate: optional fp32
@@ -422,8 +431,19 @@ static int run_compose(tq_linear_s* h, const tq::LayerView& V, const void* x_dev
 // One layer view through the tuned kernels (or the generic ones where they do not take its shape).
 // static_ws / static_cap: the caller's share of the static array, or NULL: the handle's own workspaces.
 int forward_view(tq_linear_s* h, const tq::LayerView& V, bool generic_only, const void* x_dev, int x_dtype, int batch,
-                 void* y_dev, int y_dtype, hipStream_t stream, const float* gate, void* static_ws, size_t static_cap) {
+                 void* y_dev, int y_dtype, hipStream_t stream, const float* gate, void* static_ws, size_t static_cap,
+                 const GatedRows* gated = nullptr) {
     const bool lanes = !generic_only && tq::lanes_supported(V.in_features, V.block_size);
+    // (the matrix-core prefill kernels; large tiles keep images that another kernel writes)
+    const bool fragments = lanes && !gate && !tq::skinny_supported(V, x_dtype, batch) && tq::prefill_supported(V, x_dtype, batch) &&
+                           !tq::gemv_few_supported(V, batch, device_cu_count()) && tq::rotate_takes_gate(V) &&
+                           (tq::prefill_tile_shape(V, batch, device_cu_count()) >= 0 ||
+                            tq::prefill_panel_supported(V, batch, device_cu_count(), ~(size_t)0));
+    if (gated && !fragments) {
+        if (!form_gated(*gated, &x_dev, (size_t)batch * V.in_features, stream)) return 1;
+        gated = nullptr;
+    }
+    const float* const x_gate = gated ? gated->gate : nullptr;
     // (the gated store is a feature of the one-row kernels; 16..32 rows: the small-batch kernel where it takes the layer)
     // (two to twelve rows: whole weight rows per stream, 4 x 4 x 4 matrix blocks; a
     // workspace only where the rows are rotated by a kernel of their own)
@@ -459,7 +479,7 @@ int forward_view(tq_linear_s* h, const tq::LayerView& V, bool generic_only, cons
     float* partial = nullptr;
     tq::PrefillPlan plan{};
     if (prefill && takes_compose(h, V, batch, stream, static_ws, static_ws ? static_cap : ~(size_t)0))
-        return run_compose(h, V, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws, static_ws ? static_cap : ~(size_t)0);
+        return run_compose(h, V, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws, static_ws ? static_cap : ~(size_t)0, x_gate);
     // (few output tiles: small ones, tq_prefill_tile.hip; a static workspace too small for its images goes on)
     const int tile = prefill ? tq::prefill_tile_shape(V, batch, device_cu_count()) : -1;
     if (tile >= 0) {
@@ -470,7 +490,7 @@ int forward_view(tq_linear_s* h, const tq::LayerView& V, bool generic_only, cons
             ws = h->d_work;
         }
         if (!static_ws || need <= static_cap)
-            return hip_ok(tq::launch_prefill_tile(V, tile, x_dev, x_dtype, batch, y_dev, y_dtype, ws, stream),
+            return hip_ok(tq::launch_prefill_tile(V, tile, x_dev, x_dtype, batch, y_dev, y_dtype, ws, stream, x_gate),
                           "tq_prefill_tile launch") ? 0 : 1;
     }
     // (more than 256 rows and enough output tiles: 512-row activation panels, tq_prefill_panel.hip)
@@ -500,7 +520,7 @@ int forward_view(tq_linear_s* h, const tq::LayerView& V, bool generic_only, cons
     if (panel)
         return hip_ok(tq::launch_prefill_panel(V, x_dev, x_dtype, batch, y_dev, y_dtype, work,
                                                tq::prefill_panel_workspace_bytes(V, batch, device_cu_count(), static_ws ? static_cap : ~(size_t)0),
-                                               device_cu_count(), stream),
+                                               device_cu_count(), stream, x_gate),
                       "tq_prefill_panel launch") ? 0 : 1;
     if (prefill) {
         // Dense contraction: rotate once, dequantise tiles to fp16 in LDS, MFMA.
@@ -522,7 +542,7 @@ size_t plane_sum_bytes(const tq_linear_s* h, int batch, int y_dtype) {
 }
 
 int forward_impl(tq_linear_s* h, const void* x_dev, int x_dtype, int batch, void* y_dev, int y_dtype,
-                 hipStream_t stream, const float* gate, void* static_ws = nullptr) {
+                 hipStream_t stream, const float* gate, void* static_ws = nullptr, const GatedRows* gated = nullptr) {
     // 5-bit primaries with their own residual rotation or a 4-bit residual keep their two planes.  One
     // row runs both planes in one pass (tq_gemv_five.hip, tq_generic.hip); more rows run each plane through
     // the tuned kernels as a layer of its own and add the two results: y = P x~p + R x~r, the same sum the
@@ -531,8 +551,10 @@ int forward_impl(tq_linear_s* h, const void* x_dev, int x_dtype, int batch, void
     const bool two_plane5 = h->view.mode >= tq::kShared5 && !h->has_fwd_view;
     const size_t cap = (size_t)TQ_STATIC_SCRATCH_BYTES;
     if (two_plane5 && !gate && h->has_plane_views && takes_compose(h, h->view, batch, stream, static_ws, static_ws ? cap : ~(size_t)0))
-        return run_compose(h, h->view, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws, static_ws ? cap : ~(size_t)0);
+        return run_compose(h, h->view, x_dev, x_dtype, batch, y_dev, y_dtype, stream, static_ws, static_ws ? cap : ~(size_t)0,
+                           gated ? gated->gate : nullptr);
     if (two_plane5 && batch >= 2 && !gate && h->has_plane_views) {
+        if (gated && !form_gated(*gated, &x_dev, (size_t)batch * h->view.in_features, stream)) return 1;      // (once for both planes)
         const size_t one = align256((size_t)batch * h->view.out_features * sizeof(float));
         const size_t need = plane_sum_bytes(h, batch, y_dtype);
         unsigned char* sums = nullptr;
@@ -557,7 +579,50 @@ int forward_impl(tq_linear_s* h, const void* x_dev, int x_dtype, int batch, void
         return hip_ok(tq::launch_add(t0, t1, y_dev, y_dtype, (size_t)batch * h->view.out_features, stream), "tq_add launch") ? 0 : 1;
     }
     const tq::LayerView& V = h->has_fwd_view ? h->fwd_view : h->view;
-    return forward_view(h, V, two_plane5, x_dev, x_dtype, batch, y_dev, y_dtype, stream, gate, static_ws, static_ws ? cap : 0);
+    return forward_view(h, V, two_plane5, x_dev, x_dtype, batch, y_dev, y_dtype, stream, gate, static_ws, static_ws ? cap : 0, gated);
+}
+
+// Layers on the same activations through the prefill kernels in one launch (and one that rotates), where their tiles do not
+// fill the chip one layer at a time.  0: done, 1: failed, -1: not such a group (or no workspace for it): layer by layer.
+// Every layer's images, and its composed weight, lie in its own workspace, which does not grow past what a call of its own
+// with as many rows asks for.
+static int forward_prefill_group(tq_linear_s* const* hs, const tq::LayerView* views, int n, const void* x_dev, int x_dtype, int batch,
+                                 void* const* ys, int y_dtype, hipStream_t stream) {
+    const int cus = device_cu_count();
+    for (int j = 0; j < n; ++j) {
+        const tq::LayerView& V = views[j];
+        for (int i = 0; i < j; ++i) if (hs[i] == hs[j]) return -1;           // (one workspace)
+        if (V.mode != tq::kSharedLut && V.mode != tq::kDual && V.mode != tq::kPrimaryOnly) return -1;
+        if (!tq::lanes_supported(V.in_features, V.block_size) || tq::gemv_few_supported(V, batch, cus) ||
+            tq::skinny_supported(V, x_dtype, batch) || !tq::prefill_supported(V, x_dtype, batch)) return -1;
+    }
+    void* ws[3] = {nullptr, nullptr, nullptr};
+    for (bool may_compose : {true, false}) {
+        const int how = tq::prefill_panel_group(views, n, batch, cus, may_compose);
+        if (how == tq::kGroupNone) break;
+        bool room = true;
+        for (int j = 0; j < n && room; ++j) {
+            const tq::LayerView& V = views[j];
+            const size_t need = tq::prefill_panel_group_bytes(V, batch, how);
+            if (how == tq::kGroupComposed && need > hs[j]->work_bytes)
+                room = need <= std::max(tq::prefill_reserve_bytes(V, batch, cus), tq::prefill_compose_reserve_bytes(V, batch, cus));
+            room = room && ensure_stage(&hs[j]->d_work, &hs[j]->work_bytes, need, stream, &hs[j]->retired);
+            ws[j] = hs[j]->d_work;
+        }
+        if (room)
+            return hip_ok(tq::launch_prefill_panel_group(views, n, how, x_dev, x_dtype, batch, ys, y_dtype, ws, stream),
+                          "tq_prefill_panel group launch") ? 0 : 1;
+        if (how != tq::kGroupComposed) break;
+    }
+    const int shape = tq::prefill_tile_group_shape(views, n, batch, cus);
+    if (shape < 0) return -1;
+    for (int j = 0; j < n; ++j) {
+        if (tq::prefill_compose_supported(views[j], batch, cus, ~(size_t)0)) return -1;
+        if (!ensure_stage(&hs[j]->d_work, &hs[j]->work_bytes, tq::prefill_tile_workspace_bytes(views[j], batch), stream, &hs[j]->retired)) return 1;
+        ws[j] = hs[j]->d_work;
+    }
+    return hip_ok(tq::launch_prefill_tile_group(views, n, shape, x_dev, x_dtype, batch, ys, y_dtype, ws, stream, nullptr),
+                  "tq_prefill_tile group launch") ? 0 : 1;
 }
 
 extern "C" {
@@ -735,6 +800,10 @@ int tq_linear_forward_group(const tq_linear_t* hs, int n, const void* x_dev, int
             return hip_ok(tq::launch_skinny_group(views, n, x_dev, x_dtype, batch, y_devs, y_dtype, partials,
                                                   device_cu_count(), st), "tq_skinny group launch") ? 0 : 1;
         }
+        if (plain && n > 1) {
+            const int done = forward_prefill_group(hs, views, n, x_dev, x_dtype, batch, y_devs, y_dtype, st);
+            if (done >= 0) return done;
+        }
         for (int j = 0; j < n; ++j)
             if (forward_impl(hs[j], x_dev, x_dtype, batch, y_devs[j], y_dtype, st, nullptr) != 0) return 1;
         return 0;
@@ -879,7 +948,6 @@ int tq_mlp_forward(tq_mlp_t m, const void* x_dev, int x_dtype, int batch, void* 
             set_error("tq_mlp_forward: bad batch (larger than max_batch?) or dtype"); return 1;
         }
         hipStream_t st = static_cast<hipStream_t>(stream);
-        const size_t n = (size_t)batch * m->gate->view.out_features;
         if (batch == 1 && !m->gate->has_fwd_view && !m->up->has_fwd_view && !m->down->has_fwd_view &&
             m->gate->view.mode < tq::kShared5 && m->up->view.mode < tq::kShared5 && m->down->view.mode < tq::kShared5) {
             // One row, gate and up of equal width and mode, an intermediate row wider than 16384 columns:
@@ -906,8 +974,8 @@ int tq_mlp_forward(tq_mlp_t m, const void* x_dev, int x_dtype, int batch, void* 
             if (forward_impl(m->up, x_dev, x_dtype, batch, m->d_act, tq::kF32, st, m->d_gate) != 0) return 1;
             return forward_impl(m->down, m->d_act, tq::kF32, batch, y_dev, y_dtype, st, nullptr);
         }
-        // two or more rows: matrix-core paths for all three layers (small-batch or prefill kernel), one
-        // elementwise kernel; the activation is handed to the down projection as fp32
+        // two or more rows: matrix-core paths for all three layers (small-batch or prefill kernel); silu(gate) * up is
+        // formed in fp32, by the kernel that rotates for the down projection or by an elementwise one
         const tq::LayerView both[2] = {m->gate->has_fwd_view ? m->gate->fwd_view : m->gate->view,
                                        m->up->has_fwd_view ? m->up->fwd_view : m->up->view};
         const bool plain = !(m->gate->view.mode >= tq::kShared5 && !m->gate->has_fwd_view) &&
@@ -923,18 +991,23 @@ int tq_mlp_forward(tq_mlp_t m, const void* x_dev, int x_dtype, int batch, void* 
                                                   need ? m->gate->d_work : nullptr, device_cu_count(), st),
                         "tq_gemv_few group launch")) return 1;
         } else if (plain && !any_few && tq::skinny_group_supported(both, 2, x_dtype, batch, device_cu_count())) {
-            // gate and up share the small-batch kernel and its reduction (workspaces sized by tq_mlp_create)
-            void* outs[2] = {m->d_gate, m->d_up};
+            // gate and up share the small-batch kernel and its reduction, which forms silu(gate) * up (workspaces sized by
+            // tq_mlp_create)
+            void* outs[2] = {m->d_act, nullptr};
             float* partials[2] = {static_cast<float*>(m->gate->d_partial), static_cast<float*>(m->up->d_partial)};
             if (!hip_ok(tq::launch_skinny_group(both, 2, x_dev, x_dtype, batch, outs, tq::kF32, partials,
-                                                device_cu_count(), st), "tq_skinny group launch")) return 1;
+                                                device_cu_count(), st, true), "tq_skinny group launch")) return 1;
+            return forward_impl(m->down, m->d_act, tq::kF32, batch, y_dev, y_dtype, st, nullptr);
         } else {
-            if (forward_impl(m->gate, x_dev, x_dtype, batch, m->d_gate, tq::kF32, st, nullptr) != 0) return 1;
-            if (forward_impl(m->up, x_dev, x_dtype, batch, m->d_up, tq::kF32, st, nullptr) != 0) return 1;
+            void* outs[2] = {m->d_gate, m->d_up};
+            tq_linear_s* const layers[2] = {m->gate, m->up};
+            const int done = plain ? forward_prefill_group(layers, both, 2, x_dev, x_dtype, batch, outs, tq::kF32, st) : -1;
+            if (done > 0) return 1;
+            if (done < 0 && (forward_impl(m->gate, x_dev, x_dtype, batch, m->d_gate, tq::kF32, st, nullptr) != 0 ||
+                             forward_impl(m->up, x_dev, x_dtype, batch, m->d_up, tq::kF32, st, nullptr) != 0)) return 1;
         }
-        const int act_dtype = tq::kF32;
-        if (!hip_ok(tq::launch_silu_mul(m->d_gate, m->d_up, m->d_act, act_dtype, n, st), "silu_mul launch")) return 1;
-        return forward_impl(m->down, m->d_act, act_dtype, batch, y_dev, y_dtype, st, nullptr);
+        const GatedRows gated = {m->d_gate, static_cast<float*>(m->d_act)};
+        return forward_impl(m->down, m->d_up, tq::kF32, batch, y_dev, y_dtype, st, nullptr, nullptr, &gated);
     } catch (...) { set_error("tq_mlp_forward: exception"); return 1; }
 }
 

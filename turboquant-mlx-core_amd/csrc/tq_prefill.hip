@@ -479,16 +479,22 @@ __global__ __launch_bounds__(256) void tq_rotate_f16_kernel(const void* __restri
 // wave-private piece of LDS so that a store instruction writes eight whole 128-byte lines.  R = 2, for calls
 // with few rows (less than two waves of 8 rows per SIMD): the launch is as long as one wave's chain of loads,
 // butterflies and stores, so the waves are kept short and store their 2 x 16 bytes themselves.
-// planes = 2: both rotations of the dual layout from one read of the activations (images out and out2).
+// planes = 2: both rotations of the dual layout from one read of the activations (images out and out2).  blockIdx.y: the
+// layer of a group on the same activations.  GATED (x fp32): the activations are silu(gate) * x, formed as they are read,
+// in fp32 as tq_silu_mul_kernel forms them: 2048 rows of 27648 columns 136 us where that kernel and this one took 139 + 77.
 // (The same kernel writing the 256-row tile images of tq_prefill_gemm_kernel was measured and not kept: there a lane of
 // tq_rotate_f16_kernel already stores the 64 contiguous bytes of its chunk; 512 x 27648 took 25.5 us instead of 19.8,
 // 1024 x 5120 9.4 instead of 10.0.)
 constexpr int kRotPitch = 144;                 // bytes of a lane's 8 x 16 B in LDS, padded: 16-byte accesses spread over the banks
-template <int R>
-__global__ __launch_bounds__(256) void tq_rotate_panel_kernel(const void* __restrict__ x, int x_dtype,
-                                                               uint16_t* __restrict__ out, uint16_t* __restrict__ out2,
-                                                               int rows, int cols, int segs, int planes, int blocks,
-                                                               uint32_t seed, uint32_t seed2, uint32_t bs, float scale) {
+struct RotateGroup {
+    uint16_t* out[3];
+    uint16_t* out2[3];
+    uint32_t seed[3], seed2[3];
+};
+template <int R, bool GATED>
+__global__ __launch_bounds__(256) void tq_rotate_panel_kernel(const void* __restrict__ x, int x_dtype, const float* __restrict__ gate,
+                                                               RotateGroup group, int rows, int cols, int segs, int planes,
+                                                               int blocks, uint32_t bs, float scale) {
     __shared__ __align__(16) char stage_all[R == 8 ? 4 * kWave * kRotPitch : 16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     char* const stage = stage_all + (R == 8 ? wave * (kWave * kRotPitch) : 0);
@@ -504,25 +510,45 @@ __global__ __launch_bounds__(256) void tq_rotate_panel_kernel(const void* __rest
     for (int r = 0; r < R; ++r) {
         const int row = row0 + r < rows ? row0 + r : rows - 1;
         const size_t e = (size_t)row * cols + (active ? col : 0);
-        if (x_dtype == kF32) {
+        if (GATED || x_dtype == kF32) {
             const uint4* p = reinterpret_cast<const uint4*>(static_cast<const float*>(x) + e);
             raw[r][0] = p[0]; raw[r][1] = p[1];
         } else {
             raw[r][0] = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(x) + e);
         }
     }
+    if constexpr (GATED) {
+        uint4 graw[R][2];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int row = row0 + r < rows ? row0 + r : rows - 1;
+            const uint4* p = reinterpret_cast<const uint4*>(gate + (size_t)row * cols + (active ? col : 0));
+            graw[r][0] = p[0]; graw[r][1] = p[1];
+        }
+        auto gated = [](uint32_t u, uint32_t g) {
+            const float gf = __builtin_bit_cast(float, g);
+            return __builtin_bit_cast(uint32_t, gf / (1.0f + expf(-gf)) * __builtin_bit_cast(float, u));
+        };
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                raw[r][h].x = gated(raw[r][h].x, graw[r][h].x); raw[r][h].y = gated(raw[r][h].y, graw[r][h].y);
+                raw[r][h].z = gated(raw[r][h].z, graw[r][h].z); raw[r][h].w = gated(raw[r][h].w, graw[r][h].w);
+            }
+    }
     const int U_all = cols >> 4, ustep = blocks ? 64 : 1024;
     const int g_own = seg * 64 + lane;                                 // this lane's 8-column group of the row
     for (int plane = 0; plane < planes; ++plane) {
-        const uint32_t sd = plane ? seed2 : seed;
-        uint4* const img = reinterpret_cast<uint4*>(plane ? out2 : out);
+        const uint32_t sd = plane ? group.seed2[blockIdx.y] : group.seed[blockIdx.y];
+        uint4* const img = reinterpret_cast<uint4*>(plane ? group.out2[blockIdx.y] : group.out[blockIdx.y]);
         float sg[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) sg[j] = active ? sign_of(sd, (uint32_t)(col + j) & (bs - 1)) : 0.0f;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             float v[8];
-            if (x_dtype == kF32) {
+            if (GATED || x_dtype == kF32) {
                 const uint32_t w[8] = {raw[r][0].x, raw[r][0].y, raw[r][0].z, raw[r][0].w, raw[r][1].x, raw[r][1].y, raw[r][1].z, raw[r][1].w};
 #pragma unroll
                 for (int j = 0; j < 8; ++j) v[j] = __builtin_bit_cast(float, w[j]);
@@ -644,8 +670,9 @@ size_t prefill_reserve_bytes(const LayerView& L, int max_batch, int num_cus) {
     look(16); look(kSkinnyMaxRows); look(kSkinnyMaxRows + 1); look(128); look(129);
     for (int rows = kBM; rows < max_batch + kBM; rows += kBM) { look(rows); look(rows + 1); }
     look(max_batch);
-    // (small tiles, whichever row counts take them: images of 32 rows)
+    // (small tiles, whichever row counts take them: images of 32 rows; the panels of a group: images of 512)
     if (max_batch >= 16) need = std::max(need, prefill_tile_workspace_bytes(L, max_batch));
+    if (max_batch > kSkinnyMaxRows) need = std::max(need, prefill_panel_workspace_bytes(L, max_batch, num_cus, 0));
     return need;
 }
 
@@ -659,42 +686,56 @@ bool prefill_supported(const LayerView& L, int x_dtype, int batch) {
     return L.in_features % kKLoad == 0;
 }
 
-// Rotated activations of `batch` rows as fp16 images in `workspace` (both rotations for dual mode).
-hipError_t launch_rotate_tiles(const LayerView& L, const void* x, int x_dtype, int batch, void* workspace,
-                               hipStream_t stream, int layout) {
+// Rotated activations of `batch` rows as fp16 images in the layers' workspaces (both rotations for dual mode).  Layers of
+// one group: equal width, block and mode.  gate: the activations are silu(gate) * x (x fp32; rotate_takes_gate).
+bool rotate_takes_gate(const LayerView& L) { return L.block_size <= 512; }
+hipError_t launch_rotate_group(const LayerView* Ls, int n, const void* x, int x_dtype, const float* gate, int batch,
+                               void* const* workspaces, hipStream_t stream, int layout) {
+    const LayerView& L = Ls[0];
     const int K = L.in_features, M = batch;
-    uint16_t* xt = static_cast<uint16_t*>(workspace);
-    const int chunks = K / kChunk;
-    const dim3 rgrid((unsigned)(((long long)M * chunks + 4 * kWave - 1) / (4 * kWave)));   // 256 chunks per workgroup
+    const int planes = L.mode == kDual ? 2 : 1;
     const int tile_m = layout == kPanelImage ? kPanelM : layout == kBlockImage ? 32 : kBM;   // rows of one image
-    uint16_t* const xt2 = xt + (size_t)((M + tile_m - 1) / tile_m) * tile_m * K;
+    RotateGroup g{};
+    for (int j = 0; j < n; ++j) {
+        g.out[j] = static_cast<uint16_t*>(workspaces[j]);
+        g.out2[j] = g.out[j] + (size_t)((M + tile_m - 1) / tile_m) * tile_m * K;
+        g.seed[j] = Ls[j].seed_primary;
+        g.seed2[j] = Ls[j].seed_residual;
+    }
     if (layout != kTileImage && L.block_size <= 512) {
-        const int segs = (K + 511) / 512;
-        const int planes = L.mode == kDual ? 2 : 1;
-        const int blocks = layout == kBlockImage;
-        const long long tasks8 = (long long)((M + 7) / 8) * segs;
-        if (tasks8 >= 2048) {
-            hipLaunchKernelGGL(tq_rotate_panel_kernel<8>, dim3((unsigned)((tasks8 + 3) / 4)), dim3(256), 0, stream, x, x_dtype,
-                               xt, xt2, M, K, segs, planes, blocks, L.seed_primary, L.seed_residual, L.block_size, L.inv_sqrt_bs);
-        } else {
-            const long long tasks2 = (long long)((M + 1) / 2) * segs;
-            hipLaunchKernelGGL(tq_rotate_panel_kernel<2>, dim3((unsigned)((tasks2 + 3) / 4)), dim3(256), 0, stream, x, x_dtype,
-                               xt, xt2, M, K, segs, planes, blocks, L.seed_primary, L.seed_residual, L.block_size, L.inv_sqrt_bs);
-        }
+        const int segs = (K + 511) / 512, blocks = layout == kBlockImage;
+        const long long tasks8 = (long long)((M + 7) / 8) * segs, tasks2 = (long long)((M + 1) / 2) * segs;
+        const bool eight = tasks8 * n >= 2048;
+        const dim3 grid((unsigned)(((eight ? tasks8 : tasks2) + 3) / 4), n);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, x_dtype, gate, g, M, K, segs, planes, blocks, L.block_size,
+                               L.inv_sqrt_bs);
+        };
+        if (gate) eight ? go(tq_rotate_panel_kernel<8, true>) : go(tq_rotate_panel_kernel<2, true>);
+        else eight ? go(tq_rotate_panel_kernel<8, false>) : go(tq_rotate_panel_kernel<2, false>);
         return hipGetLastError();
     }
+    if (gate) return hipErrorInvalidValue;
+    const int chunks = K / kChunk;
+    const dim3 rgrid((unsigned)(((long long)M * chunks + 4 * kWave - 1) / (4 * kWave)));   // 256 chunks per workgroup
     auto rotate = [&](auto Layout, uint16_t* to, uint32_t seed) {
         hipLaunchKernelGGL(tq_rotate_f16_kernel<decltype(Layout)::value>, rgrid, dim3(256), 0, stream, x, x_dtype, to, M, K, chunks,
                            seed, L.block_size, L.inv_sqrt_bs);
     };
-    for (int p = 0; p < (L.mode == kDual ? 2 : 1); ++p) {
-        uint16_t* const to = p ? xt2 : xt;
-        const uint32_t seed = p ? L.seed_residual : L.seed_primary;
-        if (layout == kPanelImage) rotate(std::integral_constant<int, kPanelImage>{}, to, seed);
-        else if (layout == kBlockImage) rotate(std::integral_constant<int, kBlockImage>{}, to, seed);
-        else rotate(std::integral_constant<int, kTileImage>{}, to, seed);
-    }
+    for (int j = 0; j < n; ++j)
+        for (int p = 0; p < planes; ++p) {
+            uint16_t* const to = p ? g.out2[j] : g.out[j];
+            const uint32_t seed = p ? g.seed2[j] : g.seed[j];
+            if (layout == kPanelImage) rotate(std::integral_constant<int, kPanelImage>{}, to, seed);
+            else if (layout == kBlockImage) rotate(std::integral_constant<int, kBlockImage>{}, to, seed);
+            else rotate(std::integral_constant<int, kTileImage>{}, to, seed);
+        }
     return hipGetLastError();
+}
+
+hipError_t launch_rotate_tiles(const LayerView& L, const void* x, int x_dtype, int batch, void* workspace,
+                               hipStream_t stream, int layout, const float* gate) {
+    return launch_rotate_group(&L, 1, x, x_dtype, gate, batch, &workspace, stream, layout);
 }
 
 hipError_t launch_prefill(const LayerView& L, const void* x, int x_dtype, int batch, void* y, int y_dtype,

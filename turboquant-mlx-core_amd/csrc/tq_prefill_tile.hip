@@ -15,6 +15,7 @@
 // row block of 32 rows, 2 for two and four) and of BR weight tiles; what bounds it is said at prefill_tile_shape.
 #include "tq_prefill_common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace tq {
@@ -36,6 +37,12 @@ struct TileArgs {
     int table_exp;
 };
 
+// Layers on the same activations, one launch: layer j owns the workgroups first[j] .. first[j + 1] - 1 (whole rounds of the XCDs).
+struct TileGroup {
+    TileArgs a[3];
+    int first[4];
+};
+
 }  // namespace
 
 // MB x NB blocks of 32 x 32 outputs per wave; KS waves share them along K, WN such groups stand side by side along N.
@@ -44,7 +51,10 @@ struct TileArgs {
 // instructions where v_mfma_f32_32x32x2_f32 would take the time of sixteen.  The images of the lo parts follow those of the hi
 // parts (zeros from K to a whole 64-column tile), the table is L.split_tables.
 template <int MODE, int SUB, int MB, int NB, int KS, int WN, int PARTS>
-__global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileArgs a) {
+__global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileGroup group) {
+    const int layer = (int)blockIdx.x >= group.first[2] ? 2 : ((int)blockIdx.x >= group.first[1] ? 1 : 0);
+    const TileArgs& a = group.a[layer];
+    const int block = (int)blockIdx.x - group.first[layer];
     constexpr bool combined = (MODE == kSharedLut);
     constexpr int kPlanes = (MODE == kDual) ? 2 : 1;
     constexpr int kWaves = KS * WN;
@@ -65,7 +75,7 @@ __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileArgs 
     const int l = lane & 31, g = lane >> 5;
 
     // Workgroup ids go round the XCDs (id % 8): the row tiles that share a tile of weights run on one XCD.
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int xcd = block & 7, slot = block >> 3;
     const int n_tile = (slot / a.m_tiles) * 8 + xcd, m_tile = slot % a.m_tiles;
     if (n_tile >= a.n_tiles) return;                       // whole workgroup leaves together
     const int n0 = n_tile * (32 * NB * WN), m0 = m_tile * (32 * MB);
@@ -358,7 +368,7 @@ constexpr TileShape kTileShapes[] = {{1, 1, 8, 1}, {1, 2, 8, 1}, {2, 2, 8, 1}, {
 constexpr TileShape kSplitShapes[] = {{1, 1, 8, 1}, {1, 2, 8, 1}, {2, 2, 4, 2}};
 
 template <int MODE, int SUB>
-void launch_shape(int shape, const TileArgs& a, dim3 grid, hipStream_t stream) {
+void launch_shape(int shape, const TileGroup& a, dim3 grid, hipStream_t stream) {
     switch (shape) {
         case 0: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, SUB, 1, 1, 8, 1, 1>), grid, dim3(512), 0, stream, a); break;
         case 1: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, SUB, 1, 2, 8, 1, 1>), grid, dim3(512), 0, stream, a); break;
@@ -368,7 +378,7 @@ void launch_shape(int shape, const TileArgs& a, dim3 grid, hipStream_t stream) {
 }
 
 template <int MODE>
-void launch_split_shape(int shape, const TileArgs& a, dim3 grid, hipStream_t stream) {
+void launch_split_shape(int shape, const TileGroup& a, dim3 grid, hipStream_t stream) {
     switch (shape) {
         case 0: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, 1, 1, 1, 8, 1, 2>), grid, dim3(512), 0, stream, a); break;
         case 1: hipLaunchKernelGGL((tq_prefill_tile_kernel<MODE, 1, 1, 2, 8, 1, 2>), grid, dim3(512), 0, stream, a); break;
@@ -389,6 +399,17 @@ TileArgs tile_args(const LayerView& L, int batch, void* y, int y_dtype, const vo
     a.n_tiles = (a.N + 32 * t.nb * t.wn - 1) / (32 * t.nb * t.wn);
     a.out_scale = L.inv_scale;                             // (1 / sqrt(bs) is in the rotated activations)
     return a;
+}
+
+int tile_workgroups(const TileArgs& a) { return (a.n_tiles + 7) / 8 * 8 * a.m_tiles; }
+
+TileGroup tile_group(const TileArgs* a, int n) {
+    TileGroup g{};
+    for (int j = 0; j < 3; ++j) {
+        if (j < n) g.a[j] = a[j];
+        g.first[j + 1] = j < n ? g.first[j] + tile_workgroups(a[j]) : 1 << 30;          // (no workgroup reaches an unused slot)
+    }
+    return g;
 }
 
 // The activations of tq_prefill_tile_kernel's operands in two parts: H (s (.) x) in fp32 as the fp32 kernels form it, times the power of
@@ -514,11 +535,12 @@ hipError_t launch_prefill_split(const LayerView& L, const void* x, int x_dtype, 
     a.out_scale = L.inv_scale * L.inv_sqrt_bs;
     a.row_exp = row_exp;
     a.table_exp = L.split_exp;
-    const dim3 grid((unsigned)((a.n_tiles + 7) / 8 * 8 * a.m_tiles));
+    const dim3 grid((unsigned)tile_workgroups(a));
+    const TileGroup g = tile_group(&a, 1);
     switch (L.mode) {
-        case kSharedLut: launch_split_shape<kSharedLut>(shape, a, grid, stream); break;
-        case kDual: launch_split_shape<kDual>(shape, a, grid, stream); break;
-        default: launch_split_shape<kPrimaryOnly>(shape, a, grid, stream); break;
+        case kSharedLut: launch_split_shape<kSharedLut>(shape, g, grid, stream); break;
+        case kDual: launch_split_shape<kDual>(shape, g, grid, stream); break;
+        default: launch_split_shape<kPrimaryOnly>(shape, g, grid, stream); break;
     }
     return hipGetLastError();
 }
@@ -537,51 +559,94 @@ size_t prefill_tile_workspace_bytes(const LayerView& L, int batch) {
 //   us per call before -> now, bf16:  dual rotation, in x out: 896 x 4864 at 77 rows 57.7 -> 17.9, at 512 rows 60.3 -> 36.2;
 //   4864 x 896 at 77 rows 72.7 -> 25.3; 7680 x 565 at 160 rows 82.2 -> 37.2; 5120 x 5120 at 77 rows 68.2 -> 34.6, at 1024 rows
 //   138.6 (not taken).  Shared rotation: 896 x 4864 at 77 rows 34.9 -> 13.5; 2048 x 2048 at 512 rows 43.2 -> 22.4.
-int prefill_tile_shape(const LayerView& L, int batch, int num_cus) {
-    if (!prefill_supported(L, kBF16, batch)) return -1;    // (up to 32 rows: what the small-batch kernels leave)
-    if (prefill_panel_supported(L, batch, num_cus, ~(size_t)0)) return -1;
-    static constexpr double kFirst[4] = {5.0, 5.0, 5.0, 12.0}, kMore[4] = {2.4, 6.5, 7.0, 16.0};
-    static constexpr double kPerTile[3][4] = {{0.094, 0.125, 0.17, 0.45}, {0.107, 0.164, 0.24, 0.60}, {0.07, 0.12, 0.17, 0.45}};
-    const double* const per_tile = kPerTile[L.mode == kDual ? 0 : (L.mode == kSharedLut ? 1 : 2)];
+namespace {
+
+double large_tile_us(const LayerView& L, int batch, int num_cus) {
     const int planes = L.mode == kDual ? 2 : 1;
-    const double tiles64 = (double)planes * (L.in_features / 64);
     const PrefillPlan p = prefill_plan(L, batch, num_cus, ~(size_t)0);
     const long long big = (long long)((batch + 255) / 256) * ((L.out_features + 255) / 256) * p.splits;
-    double best = (double)((big + num_cus - 1) / num_cus) * 0.8 * planes * p.steps_per_split;
-    if (p.splits > 1) best += 5.0 + (double)p.splits * batch * L.out_features * 8.0 / 5.0e6;
-    best *= 0.95;
+    double us = (double)((big + num_cus - 1) / num_cus) * 0.8 * planes * p.steps_per_split;
+    if (p.splits > 1) us += 5.0 + (double)p.splits * batch * L.out_features * 8.0 / 5.0e6;
+    return 0.95 * us;
+}
+
+// The cheapest shape for layers of equal width and mode in one launch.
+int small_tile_shape(const LayerView* Ls, int n, int batch, int num_cus, double* us) {
+    static constexpr double kFirst[4] = {5.0, 5.0, 5.0, 12.0}, kMore[4] = {2.4, 6.5, 7.0, 16.0};
+    static constexpr double kPerTile[3][4] = {{0.094, 0.125, 0.17, 0.45}, {0.107, 0.164, 0.24, 0.60}, {0.07, 0.12, 0.17, 0.45}};
+    const int mode = Ls[0].mode;
+    const double* const per_tile = kPerTile[mode == kDual ? 0 : (mode == kSharedLut ? 1 : 2)];
+    const double tiles64 = (double)(mode == kDual ? 2 : 1) * (Ls[0].in_features / 64);
     int shape = -1;
     for (int s = 0; s < 4; ++s) {
         const TileShape t = kTileShapes[s];
-        const long long wgs = (long long)((batch + 32 * t.mb - 1) / (32 * t.mb)) * ((L.out_features + 32 * t.nb * t.wn - 1) / (32 * t.nb * t.wn));
+        long long wgs = 0;
+        for (int j = 0; j < n; ++j)
+            wgs += (long long)((batch + 32 * t.mb - 1) / (32 * t.mb)) * ((Ls[j].out_features + 32 * t.nb * t.wn - 1) / (32 * t.nb * t.wn));
         const double rounds = (double)((wgs + num_cus - 1) / num_cus);
         const double cost = kFirst[s] + (rounds - 1.0) * kMore[s] + rounds * per_tile[s] * tiles64;
-        if (cost < best) { best = cost; shape = s; }
+        if (shape < 0 || cost < *us) { *us = cost; shape = s; }
     }
     return shape;
 }
 
-hipError_t launch_prefill_tile(const LayerView& L, int shape, const void* x, int x_dtype, int batch, void* y, int y_dtype,
-                               void* workspace, hipStream_t stream) {
-    hipError_t e = launch_rotate_tiles(L, x, x_dtype, batch, workspace, stream, kBlockImage);
+}  // namespace
+
+int prefill_tile_shape(const LayerView& L, int batch, int num_cus) {
+    if (!prefill_supported(L, kBF16, batch)) return -1;    // (up to 32 rows: what the small-batch kernels leave)
+    if (prefill_panel_supported(L, batch, num_cus, ~(size_t)0)) return -1;
+    double us;
+    const int shape = small_tile_shape(&L, 1, batch, num_cus, &us);
+    return us < large_tile_us(L, batch, num_cus) ? shape : -1;
+}
+
+double prefill_tile_us(const LayerView& L, int batch, int num_cus) {
+    double us;
+    small_tile_shape(&L, 1, batch, num_cus, &us);
+    return std::min(us, large_tile_us(L, batch, num_cus));
+}
+
+int prefill_tile_group_shape(const LayerView* Ls, int n, int batch, int num_cus) {
+    for (int j = 0; j < n; ++j) {
+        if (Ls[j].in_features != Ls[0].in_features || Ls[j].block_size != Ls[0].block_size || Ls[j].mode != Ls[0].mode) return -1;
+        if (prefill_tile_shape(Ls[j], batch, num_cus) < 0) return -1;
+    }
+    double us;
+    return small_tile_shape(Ls, n, batch, num_cus, &us);
+}
+
+hipError_t launch_prefill_tile_group(const LayerView* Ls, int n, int shape, const void* x, int x_dtype, int batch, void* const* ys,
+                                     int y_dtype, void* const* workspaces, hipStream_t stream, const float* gate) {
+    hipError_t e = launch_rotate_group(Ls, n, x, x_dtype, gate, batch, workspaces, stream, kBlockImage);
     if (e != hipSuccess) return e;
-    const TileArgs a = tile_args(L, batch, y, y_dtype, workspace, kTileShapes[shape]);
-    const dim3 grid((unsigned)((a.n_tiles + 7) / 8 * 8 * a.m_tiles));
+    TileArgs a[3];
+    int wgs = 0;
+    for (int j = 0; j < n; ++j) {
+        a[j] = tile_args(Ls[j], batch, ys[j], y_dtype, workspaces[j], kTileShapes[shape]);
+        wgs += tile_workgroups(a[j]);
+    }
+    const TileGroup g = tile_group(a, n);
+    const dim3 grid((unsigned)wgs);
     // Two 64-column tiles of a nibble plane at a time where the width allows it: 64 bytes of a row per pair of requests
     // instead of 32 (4864 x 896 at 512 rows 40.6 -> 38.0 us, 7680 x 565 55.0 -> 49.6; four tiles cost registers: 58).  The
     // combined plane's tile is 64 bytes already (two tiles at a time: 5 to 30 % slower).
-    const bool pairs = a.K % 128 == 0;
+    const bool pairs = Ls[0].in_features % 128 == 0;
     auto go = [&](auto Mode) {
         constexpr int M = decltype(Mode)::value;
-        if constexpr (M != kSharedLut) { if (pairs) { launch_shape<M, 2>(shape, a, grid, stream); return; } }
-        launch_shape<M, 1>(shape, a, grid, stream);
+        if constexpr (M != kSharedLut) { if (pairs) { launch_shape<M, 2>(shape, g, grid, stream); return; } }
+        launch_shape<M, 1>(shape, g, grid, stream);
     };
-    switch (L.mode) {
+    switch (Ls[0].mode) {
         case kSharedLut: go(std::integral_constant<int, kSharedLut>{}); break;
         case kDual: go(std::integral_constant<int, kDual>{}); break;
         default: go(std::integral_constant<int, kPrimaryOnly>{}); break;
     }
     return hipGetLastError();
+}
+
+hipError_t launch_prefill_tile(const LayerView& L, int shape, const void* x, int x_dtype, int batch, void* y, int y_dtype,
+                               void* workspace, hipStream_t stream, const float* gate) {
+    return launch_prefill_tile_group(&L, 1, shape, x, x_dtype, batch, &y, y_dtype, &workspace, stream, gate);
 }
 
 }  // namespace tq

@@ -429,42 +429,54 @@ __global__ __launch_bounds__(kSkThreads) __attribute__((amdgpu_waves_per_eu(2, 2
 }
 
 // y[b, n] = norm[n] * out_scale * sum over chunks of partial[c][b][n]
-// grid = blocks of 64 columns x batch rows.  The four waves of a block share the chunks of those 64
+// grid = blocks of 64 V columns x batch rows, V columns per lane.  The four waves of a block share the chunks of those
 // columns (wave w takes chunks w, w + 4, ..., eight loads in flight at a time) and add up through
 // LDS: a single thread per output walking all chunks four at a time spent one memory latency per
-// four chunks, 4.5 us for a kernel that moves a few hundred KB.
-__device__ __forceinline__ void skinny_reduce_body(const float* __restrict__ partial, const float* __restrict__ norms,
-                                                   void* __restrict__ y, int y_dtype, int N, int chunks,
-                                                   float out_scale, const int block) {
-    __shared__ float part[4][64];
+// four chunks, 4.5 us for a kernel that moves a few hundred KB.  V = 4 (16 bytes per load) where N is a multiple of four and
+// a block per CU is left: 2 x 27648 columns of 8 rows in 20 chunks (35 MB) with their product 8.9 us, where 12.4 us and a launch of 4.9 for the product stood.
+template <int V>
+__device__ __forceinline__ void skinny_sum(const float* __restrict__ partial, int N, int chunks, int n, bool live, float (*part)[64 * V],
+                                           float (&t)[V]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int b = blockIdx.y;
-    const int n = block * 64 + lane;
-    const bool live = n < N;
-    const float nrm = live ? norms[n] : 0.0f;
-    const float* p = partial + (size_t)b * N + (live ? n : 0);
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const float* p = partial + (size_t)blockIdx.y * N + (live ? n : 0);
     const size_t step = (size_t)gridDim.y * N;          // one chunk: [batch][N]
-    float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    vec s[8] = {};
     int c = wave;
     for (; c + 28 < chunks; c += 32) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) s[k] += p[(size_t)(c + 4 * k) * step];
+        for (int k = 0; k < 8; ++k) s[k] += *reinterpret_cast<const vec*>(p + (size_t)(c + 4 * k) * step);
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-        if (c + 4 * k < chunks) s[k] += p[(size_t)(c + 4 * k) * step];
-    part[wave][lane] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+        if (c + 4 * k < chunks) s[k] += *reinterpret_cast<const vec*>(p + (size_t)(c + 4 * k) * step);
+    *reinterpret_cast<vec*>(&part[wave][lane * V]) = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
     __syncthreads();
-    if (wave == 0 && live) {
-        const float t = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
-        store_scalar(y, y_dtype, (size_t)b * N + n, t * (out_scale * nrm));
-    }
+#pragma unroll
+    for (int e = 0; e < V; ++e)
+        t[e] = (part[0][lane * V + e] + part[1][lane * V + e]) + (part[2][lane * V + e] + part[3][lane * V + e]);
 }
 
+template <int V>
+__device__ __forceinline__ void skinny_reduce_body(const float* __restrict__ partial, const float* __restrict__ norms,
+                                                   void* __restrict__ y, int y_dtype, int N, int chunks,
+                                                   float out_scale, const int block) {
+    __shared__ __align__(16) float part[4][64 * V];
+    const int n = block * (64 * V) + (int)(threadIdx.x & 63) * V;
+    const bool live = n < N;
+    float t[V];
+    skinny_sum<V>(partial, N, chunks, n, live, part, t);
+    if (threadIdx.x < 64 && live)
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+            store_scalar(y, y_dtype, (size_t)blockIdx.y * N + n + e, t[e] * (out_scale * norms[n + e]));
+}
+
+template <int V>
 __global__ __launch_bounds__(256) void tq_skinny_reduce_kernel(const float* __restrict__ partial,
                                                                const float* __restrict__ norms, void* __restrict__ y,
                                                                int y_dtype, int batch, int N, int chunks, float out_scale) {
-    skinny_reduce_body(partial, norms, y, y_dtype, N, chunks, out_scale, (int)blockIdx.x);
+    skinny_reduce_body<V>(partial, norms, y, y_dtype, N, chunks, out_scale, (int)blockIdx.x);
 }
 
 struct SkinnyReduceGroup {
@@ -476,10 +488,38 @@ struct SkinnyReduceGroup {
     int first[4];              // layer j owns blockIdx.x in first[j] .. first[j + 1] - 1
     int y_dtype, chunks;
 };
+template <int V>
 __global__ __launch_bounds__(256) void tq_skinny_reduce_group_kernel(SkinnyReduceGroup r) {
     const int b = (int)blockIdx.x;
     const int j = b >= r.first[2] ? 2 : (b >= r.first[1] ? 1 : 0);
-    skinny_reduce_body(r.partial[j], r.norms[j], r.y[j], r.y_dtype, r.N[j], r.chunks, r.out_scale[j], b - r.first[j]);
+    skinny_reduce_body<V>(r.partial[j], r.norms[j], r.y[j], r.y_dtype, r.N[j], r.chunks, r.out_scale[j], b - r.first[j]);
+}
+
+// Gate and up of a gated block: silu(sum of layer 0) * sum of layer 1 in one pass (a launch of its own for the product: 5 us).
+template <int V>
+__global__ __launch_bounds__(256) void tq_skinny_reduce_gated_kernel(SkinnyReduceGroup r) {
+    __shared__ __align__(16) float part[2][4][64 * V];
+    const int N = r.N[0], n = (int)blockIdx.x * (64 * V) + (int)(threadIdx.x & 63) * V;
+    const bool live = n < N;
+    float g[V], u[V];
+    skinny_sum<V>(r.partial[0], N, r.chunks, n, live, part[0], g);
+    skinny_sum<V>(r.partial[1], N, r.chunks, n, live, part[1], u);
+    if (threadIdx.x < 64 && live)
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            const float gate = g[e] * (r.out_scale[0] * r.norms[0][n + e]), up = u[e] * (r.out_scale[1] * r.norms[1][n + e]);
+            static_cast<float*>(r.y[0])[(size_t)blockIdx.y * N + n + e] = gate / (1.0f + expf(-gate)) * up;
+        }
+}
+
+static void launch_skinny_reduce(const float* partial, const float* norms, void* y, int y_dtype, int batch, int N, int chunks,
+                                 float out_scale, hipStream_t stream) {
+    if (N % 4 == 0 && (long long)N * batch >= 262144)
+        hipLaunchKernelGGL(tq_skinny_reduce_kernel<4>, dim3((unsigned)((N + 255) / 256), batch), dim3(256), 0, stream, partial, norms, y,
+                           y_dtype, batch, N, chunks, out_scale);
+    else
+        hipLaunchKernelGGL(tq_skinny_reduce_kernel<1>, dim3((unsigned)((N + 63) / 64), batch), dim3(256), 0, stream, partial, norms, y,
+                           y_dtype, batch, N, chunks, out_scale);
 }
 
 static bool skinny_nibble(const LayerView& L) {
@@ -534,9 +574,7 @@ hipError_t launch_skinny(const LayerView& L, const void* x, int x_dtype, int bat
         else hipLaunchKernelGGL((tq_skinny_nibble_kernel<1, false>), grid_n, dim3(kSkThreads), 0, stream, n);
         hipError_t en = hipGetLastError();
         if (en != hipSuccess) return en;
-        const unsigned blocks_n = (unsigned)((L.out_features + 63) / 64);
-        hipLaunchKernelGGL(tq_skinny_reduce_kernel, dim3(blocks_n, batch), dim3(256), 0, stream,
-                           partial, L.norms, y, y_dtype, batch, L.out_features, n.units, L.inv_scale);
+        launch_skinny_reduce(partial, L.norms, y, y_dtype, batch, L.out_features, n.units, L.inv_scale, stream);
         return hipGetLastError();
     }
     const bool fused = L.block_size <= (uint32_t)kSkChunk;
@@ -568,9 +606,7 @@ hipError_t launch_skinny(const LayerView& L, const void* x, int x_dtype, int bat
     else hipLaunchKernelGGL((tq_skinny_kernel<false, 1, false>), grid, dim3(kSkThreads), 0, stream, a);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const unsigned blocks = (unsigned)((L.out_features + 63) / 64);
-    hipLaunchKernelGGL(tq_skinny_reduce_kernel, dim3(blocks, batch), dim3(256), 0, stream,
-                       partial, L.norms, y, y_dtype, batch, L.out_features, a.chunks, L.inv_scale);
+    launch_skinny_reduce(partial, L.norms, y, y_dtype, batch, L.out_features, a.chunks, L.inv_scale, stream);
     return hipGetLastError();
 }
 
@@ -590,13 +626,16 @@ bool skinny_group_supported(const LayerView* Ls, int n, int x_dtype, int batch, 
 }
 
 hipError_t launch_skinny_group(const LayerView* Ls, int n, const void* x, int x_dtype, int batch, void* const* ys,
-                               int y_dtype, float* const* partials, int num_cus, hipStream_t stream) {
+                               int y_dtype, float* const* partials, int num_cus, hipStream_t stream, bool gated) {
     const bool nibble = Ls[0].mode == kDual || Ls[0].mode == kPrimaryOnly;
     const int planes = Ls[0].mode == kDual ? 2 : 1;
     const int K = Ls[0].in_features, chunks = (K + kSkChunk - 1) / kSkChunk * planes;   // work units: (chunk, plane)
     const int total_wgs = num_cus / chunks;                       // workgroups per unit, all layers together
     long long rows = 0;
-    for (int j = 0; j < n; ++j) rows += Ls[j].out_features;
+    bool fours = true;                                            // columns per lane of the reduction
+    for (int j = 0; j < n; ++j) { rows += Ls[j].out_features; fours = fours && Ls[j].out_features % 4 == 0; }
+    fours = fours && rows * batch >= 262144;                       // (a thousand blocks; fewer: 5.8 us where one column each takes 4.0)
+    const int reduce_cols = fours ? 256 : 64;
     int wgs[3] = {0, 0, 0}, used = 0;
     for (int j = 0; j < n; ++j) {
         wgs[j] = (int)((long long)total_wgs * Ls[j].out_features / rows);
@@ -642,7 +681,7 @@ hipError_t launch_skinny_group(const LayerView* Ls, int n, const void* x, int x_
             r.partial[j] = partials[j]; r.norms[j] = L.norms; r.y[j] = ys[j]; r.N[j] = L.out_features;
             r.out_scale[j] = L.inv_scale;
             g.first[j + 1] = g.first[j] + wgs[j];
-            r.first[j + 1] = r.first[j] + (L.out_features + 63) / 64;
+            r.first[j + 1] = r.first[j] + (L.out_features + reduce_cols - 1) / reduce_cols;
         } else {
             g.first[j] = 1 << 30; g.first[j + 1] = 1 << 30;       // no workgroup reaches an unused slot
             gn.first[j] = 1 << 30; gn.first[j + 1] = 1 << 30;
@@ -650,7 +689,7 @@ hipError_t launch_skinny_group(const LayerView* Ls, int n, const void* x, int x_
         }
     }
     int reduce_blocks = 0;
-    for (int j = 0; j < n; ++j) reduce_blocks += (Ls[j].out_features + 63) / 64;
+    for (int j = 0; j < n; ++j) reduce_blocks += (Ls[j].out_features + reduce_cols - 1) / reduce_cols;
     r.y_dtype = y_dtype; r.chunks = chunks;
     const dim3 grid(chunks, used);
     const bool two = batch > 16, ragged = K % kSkChunk != 0;
@@ -667,7 +706,11 @@ hipError_t launch_skinny_group(const LayerView* Ls, int n, const void* x, int x_
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(tq_skinny_reduce_group_kernel, dim3(reduce_blocks, batch), dim3(256), 0, stream, r);
+    const dim3 rgrid((unsigned)(gated ? r.first[1] : reduce_blocks), batch);
+    if (gated && fours) hipLaunchKernelGGL(tq_skinny_reduce_gated_kernel<4>, rgrid, dim3(256), 0, stream, r);
+    else if (gated) hipLaunchKernelGGL(tq_skinny_reduce_gated_kernel<1>, rgrid, dim3(256), 0, stream, r);
+    else if (fours) hipLaunchKernelGGL(tq_skinny_reduce_group_kernel<4>, rgrid, dim3(256), 0, stream, r);
+    else hipLaunchKernelGGL(tq_skinny_reduce_group_kernel<1>, rgrid, dim3(256), 0, stream, r);
     return hipGetLastError();
 }
 
