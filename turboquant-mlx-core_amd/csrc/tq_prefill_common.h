@@ -27,6 +27,34 @@ __device__ __forceinline__ uint32_t pack_half2(uint32_t lo_val, uint32_t hi_val)
     return __builtin_amdgcn_perm(hi_val, lo_val, 0x07060302u);   // {lo.b2, lo.b3, hi.b2, hi.b3}
 }
 
+// The decode table of the prefill kernels on nibble planes: 256 entries of 64 lane-private dwords, entry b the fp16 centroids
+// of both nibbles of byte b (low nibble = even column); a wave writes PER of them (wave w: from w PER on), every lane its own column.
+// A wave asks for the centroids once, one per lane, before its other requests (loads come back in order), and hands them
+// round in registers: with two to four scalar loads per entry the table took 3 to 10 us of a call (dual rotation, 896 ->
+// 4864 twice at 77 rows in one launch: 25.7 -> 17.3 us; 4864 -> 896 17.9 -> 14.5).  (The byte planes' table, one scalar load per
+// entry and eight of them at once, is no slower than this.)
+template <int N>
+__device__ __forceinline__ uint32_t row_value(uint32_t v) {          // of lane N of each row of 16 lanes
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x150 + N, 0xf, 0xf, true);
+}
+// `centroid`: lane l that of l % 16, may differ between rows of 16 lanes.
+template <int PER>
+__device__ __forceinline__ void fill_pair_table(char* table, float centroid, int wave, int lane) {
+    static_assert(PER % 16 == 0, "whole rows of the table");
+    const uint32_t c = (uint32_t)float_to_f16_bits(centroid);
+    uint32_t* const dst = reinterpret_cast<uint32_t*>(table) + wave * (PER * 64) + lane;
+#pragma unroll
+    for (int r = 0; r < PER / 16; ++r) {
+        const uint32_t high = (uint32_t)__shfl((int)c, (lane & 48) + wave * (PER / 16) + r, kWave) << 16;
+        uint32_t* const d = dst + r * (16 * 64);
+        d[0 * 64] = high | row_value<0>(c); d[1 * 64] = high | row_value<1>(c); d[2 * 64] = high | row_value<2>(c);
+        d[3 * 64] = high | row_value<3>(c); d[4 * 64] = high | row_value<4>(c); d[5 * 64] = high | row_value<5>(c);
+        d[6 * 64] = high | row_value<6>(c); d[7 * 64] = high | row_value<7>(c); d[8 * 64] = high | row_value<8>(c);
+        d[9 * 64] = high | row_value<9>(c); d[10 * 64] = high | row_value<10>(c); d[11 * 64] = high | row_value<11>(c);
+        d[12 * 64] = high | row_value<12>(c); d[13 * 64] = high | row_value<13>(c); d[14 * 64] = high | row_value<14>(c);
+        d[15 * 64] = high | row_value<15>(c);
+    }
+}
 // The panel kernel (tq_prefill_panel.hip): 512-row activation panels, activations read from global memory in
 // MFMA operand order.  Its rotated activations are "fragment images" (rotate_panel_kernel writes them).
 constexpr int kPanelM = 512;

@@ -76,12 +76,9 @@ struct PanelArgs {
     float* partial;
 };
 
-// Layers on the same activations, one launch (all tiles whole): layer j owns the workgroups first[j] .. first[j + 1] - 1
-// (whole rounds of the XCDs).
-struct PanelGroup {
-    PanelArgs a[3];
-    int first[4];
-};
+// Layers on the same activations, one launch (all tiles whole): blockIdx.y.  blockIdx.x and first_part_wg reach as far as
+// the largest layer needs; what a smaller one has no tile for ends at once.
+struct PanelGroup { PanelArgs a[3]; };
 
 // Waits for this wave's LDS traffic, then the workgroup barrier.  Written out because __syncthreads() also
 // waits for every global load in flight, and the activation ring lives on loads that stay in flight.
@@ -111,8 +108,8 @@ template <int PIECES> struct TileBytes { u32x4v v[PIECES]; };   // index bytes (
 // Both groups run the same number of sub-steps, so they meet at every barrier.
 template <int MODE, int NBLK, int KG = 1>
 __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelGroup group) {
-    const int layer = (int)blockIdx.x >= group.first[2] ? 2 : ((int)blockIdx.x >= group.first[1] ? 1 : 0);
-    const PanelArgs& a = group.a[layer];
+    const PanelArgs& a = group.a[blockIdx.y];
+    const int id = (int)blockIdx.x;
     static_assert(KG == 1 || (KG == 2 && NBLK == 1), "a second wave group: one row block per wave");
     constexpr int kExchange = 4 * 64 * 272;            // past the epilogue's stage: the second group's products
     __shared__ __align__(16) char smem[KG == 2 ? (kPLut + 4 * kWTile) : kPSmem];
@@ -132,7 +129,6 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelG
     constexpr int kPlanes = (MODE == kDual) ? 2 : 1;
     constexpr int kRing = dense ? 2 : 4;                   // tiles of index bytes in registers
     const int U_all = a.K / kSubK;                         // sub-steps of a row (a multiple of kUnroll)
-    const int id = (int)blockIdx.x - group.first[layer];
     int panel, n_tile, part = -1, part_slot = 0;            // part_slot: index of the part's fp32 product
     int u_begin = 0, u_end = U_all, plane_begin = 0, plane_end = kPlanes;
     if (id < a.first_part_wg) {
@@ -257,6 +253,11 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelG
                 Bf[s][j] = *reinterpret_cast<const f16x8*>(bfrag + buf * kWTile + j * 32 * kWPitch + ks * 32);
         };
 
+        float value = 0.0f;                                // of the nibble planes' table
+        if constexpr (!dense && !combined) {
+            value = a.tables[(plane == 0 ? 0 : 16) + (lane & 15)];
+            __builtin_amdgcn_sched_barrier(0);
+        }
         // Requests first: index bytes of the first four tiles, activations of the first seven sub-steps.
         const int t_begin = u_begin >> 2;
         load_bytes(std::integral_constant<int, 0>{}, t_begin);
@@ -273,21 +274,16 @@ __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelG
         load_a(std::integral_constant<int, 5>{}, u_begin + 5);
         load_a(std::integral_constant<int, 6>{}, u_begin + 6);
 
-        // The table, while those travel: wave w writes entries 64 w .. 64 w + 63, lane l into bytes 4 l .. of each
-        // entry's 256.  Values come through scalar loads.  Shared rotation: entry b = fp16(lut[b]) in the upper half.
-        // Nibble planes: entry b = the fp16 centroids of both nibbles of byte b (low nibble = even column).
-        if constexpr (!dense) {
+        // The table, while those travel.  Shared rotation: entry b = fp16(lut[b]) in the upper half.  Nibble planes: the
+        // fp16 centroids of both nibbles of byte b.
+        if constexpr (combined) {                          // (values through scalar loads, the same for all lanes)
             typedef const __attribute__((address_space(4))) float cfloat;
-            cfloat* const src = (cfloat*)(a.tables + (plane == 0 ? 0 : 16));
-            uint32_t* const dst = reinterpret_cast<uint32_t*>(smem) + lane;
+            cfloat* const src = (cfloat*)a.tables + (kg * 4 + wave) * (64 / KG);
+            uint32_t* const dst = reinterpret_cast<uint32_t*>(smem) + (kg * 4 + wave) * (64 / KG) * 64 + lane;
 #pragma unroll 8
-            for (int e = 0; e < 64 / KG; ++e) {
-                const int entry = (kg * 4 + wave) * (64 / KG) + e;
-                uint32_t v;
-                if constexpr (combined) v = (uint32_t)float_to_f16_bits(src[entry]) << 16;
-                else v = (uint32_t)float_to_f16_bits(src[entry & 15]) | ((uint32_t)float_to_f16_bits(src[entry >> 4]) << 16);
-                dst[entry * 64] = v;
-            }
+            for (int e = 0; e < 64 / KG; ++e) dst[e * 64] = (uint32_t)float_to_f16_bits(src[e]) << 16;
+        } else if constexpr (!dense) {
+            fill_pair_table<64 / KG>(smem, value, kg * 4 + wave, lane);
         }
         lds_barrier();
         // Tile 0 and the first quarter of tile 1, then the first fragments.
@@ -740,15 +736,6 @@ PanelArgs panel_args(const LayerView& L, int batch, void* y, int y_dtype, void* 
     return a;
 }
 
-PanelGroup panel_group(const PanelArgs* a, int n) {
-    PanelGroup g{};
-    for (int j = 0; j < 3; ++j) {
-        if (j < n) g.a[j] = a[j];
-        g.first[j + 1] = j + 1 < n ? g.first[j] + a[j].first_part_wg : 1 << 30;
-    }
-    return g;
-}
-
 // Row blocks per wave: a single panel of at most 384 rows is run by the kernel that multiplies only the blocks
 // that hold tokens.
 void launch_panel_kernel(int mode, int batch, bool whole_tiles, int K, const PanelGroup& g, dim3 grid, hipStream_t stream) {
@@ -788,7 +775,7 @@ hipError_t launch_prefill_panel(const LayerView& L, const void* x, int x_dtype, 
     a.first_part_wg = plan.tail_tiles == a.panels * a.n_tiles ? 0 : 8 * a.n_per_xcd * a.panels;
     a.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + plan.xt_bytes);
     const dim3 grid((unsigned)(a.first_part_wg + a.tail_tiles * a.parts));
-    launch_panel_kernel(L.mode, batch, a.tail_tiles == 0, a.K, panel_group(&a, 1), grid, stream);
+    launch_panel_kernel(L.mode, batch, a.tail_tiles == 0, a.K, PanelGroup{{a}}, grid, stream);
     e = hipGetLastError();
     if (e != hipSuccess || a.tail_tiles == 0) return e;
     hipLaunchKernelGGL(tq_prefill_panel_sum_kernel, dim3((unsigned)(a.tail_tiles * 16)), dim3(256), 0, stream, a);
@@ -1003,7 +990,7 @@ hipError_t launch_prefill_compose(const LayerView& L, const void* x, int x_dtype
         a.first_part_wg = q.tail_tiles == a.panels * a.n_tiles ? 0 : 8 * a.n_per_xcd * a.panels;
         a.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + q.xt_bytes);
         hipLaunchKernelGGL((tq_prefill_panel_kernel<kDense, 4>), dim3((unsigned)(a.first_part_wg + a.tail_tiles * a.parts)),
-                           dim3(kPThreads), 0, stream, panel_group(&a, 1));
+                           dim3(kPThreads), 0, stream, PanelGroup{{a}});
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if (a.tail_tiles) {
             hipLaunchKernelGGL(tq_prefill_panel_sum_kernel, dim3((unsigned)(a.tail_tiles * 16)), dim3(256), 0, stream, a);
@@ -1074,8 +1061,9 @@ size_t prefill_panel_group_bytes(const LayerView& L, int batch, int how) {
 hipError_t launch_prefill_panel_group(const LayerView* Ls, int n, int how, const void* x, int x_dtype, int batch, void* const* ys,
                                       int y_dtype, void* const* workspaces, hipStream_t stream) {
     LayerView views[3];
-    PanelArgs a[3];
-    unsigned wgs = 0;
+    PanelGroup g{};
+    PanelArgs* const a = g.a;
+    int wgs = 0;
     for (int j = 0; j < n; ++j) views[j] = how == kGroupComposed ? slab_view(Ls[j], Ls[j].out_features) : Ls[j];
     hipError_t e = launch_rotate_group(views, n, x, x_dtype, nullptr, batch, workspaces, stream, kPanelImage);
     if (e != hipSuccess) return e;
@@ -1088,13 +1076,14 @@ hipError_t launch_prefill_panel_group(const LayerView* Ls, int n, int how, const
             a[j].plane1 = nullptr;
             a[j].out_scale = Ls[j].inv_scale / Ls[j].compose_scale;
         }
-        wgs += (unsigned)a[j].first_part_wg;
+        wgs = std::max(wgs, a[j].first_part_wg);
     }
-    const PanelGroup g = panel_group(a, n);
+    for (int j = 0; j < n; ++j) a[j].first_part_wg = wgs;
+    const dim3 grid((unsigned)wgs, (unsigned)n);
     if (how == kGroupComposed)
-        hipLaunchKernelGGL((tq_prefill_panel_kernel<kDense, 4>), dim3(wgs), dim3(kPThreads), 0, stream, g);
+        hipLaunchKernelGGL((tq_prefill_panel_kernel<kDense, 4>), grid, dim3(kPThreads), 0, stream, g);
     else
-        launch_panel_kernel(Ls[0].mode, batch, true, Ls[0].in_features, g, dim3(wgs), stream);
+        launch_panel_kernel(Ls[0].mode, batch, true, Ls[0].in_features, g, grid, stream);
     return hipGetLastError();
 }
 

@@ -37,11 +37,9 @@ struct TileArgs {
     int table_exp;
 };
 
-// Layers on the same activations, one launch: layer j owns the workgroups first[j] .. first[j + 1] - 1 (whole rounds of the XCDs).
-struct TileGroup {
-    TileArgs a[3];
-    int first[4];
-};
+// Layers on the same activations, one launch: blockIdx.y (a number that has to be read from the arguments first costs a trip to
+// host memory, 0.4 us).  blockIdx.x reaches as far as the largest layer needs; what a smaller one has no tile for ends at once.
+struct TileGroup { TileArgs a[3]; };
 
 }  // namespace
 
@@ -52,9 +50,8 @@ struct TileGroup {
 // parts (zeros from K to a whole 64-column tile), the table is L.split_tables.
 template <int MODE, int SUB, int MB, int NB, int KS, int WN, int PARTS>
 __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileGroup group) {
-    const int layer = (int)blockIdx.x >= group.first[2] ? 2 : ((int)blockIdx.x >= group.first[1] ? 1 : 0);
-    const TileArgs& a = group.a[layer];
-    const int block = (int)blockIdx.x - group.first[layer];
+    const TileArgs& a = group.a[blockIdx.y];
+    const int block = (int)blockIdx.x;
     constexpr bool combined = (MODE == kSharedLut);
     constexpr int kPlanes = (MODE == kDual) ? 2 : 1;
     constexpr int kWaves = KS * WN;
@@ -134,6 +131,13 @@ __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileGroup
                 for (int h = 0; h < PARTS; ++h)
                     av[i][s][h] = *reinterpret_cast<const f16x8*>(ap[i] + (at + h * part_stride) + ((s >> 1) * 1024 + (s & 1) * 512) + aoff);
     };
+    constexpr int kPer = kEntries / kWaves;                // entries of the table that a wave writes
+    static_assert(kPer * kWaves == kEntries, "every wave writes as many entries");
+    float value = 0.0f;                                    // of the nibble planes' table
+    if constexpr (!combined && !split) {
+        value = a.tables[(kPlanes == 2 ? 16 * g : 0) + (lane & 15)];
+        __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int b = 0; b < BR; ++b) request_b(B[b], t_begin + b);
 #pragma unroll
@@ -143,34 +147,17 @@ __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileGroup
     // of both nibbles of byte b; with two planes lanes 0..31 of an entry hold the primary's and lanes 32..63 the
     // residual's, and lanes l and l + 32 read the same column (the LDS serves a wave's reads in two halves).  Two parts: both of
     // an entry of the table in one dword; the second plane's 16 entries behind the first's.
-    if constexpr (split) {
+    if constexpr (combined || split) {
         typedef const __attribute__((address_space(4))) uint32_t cuint;
         cuint* const src = (cuint*)reinterpret_cast<const uint32_t*>(a.tables);
         uint32_t* const dst = reinterpret_cast<uint32_t*>(smem) + lane;
-        constexpr int kPer = (kEntries + kWaves - 1) / kWaves;
-        static_assert(kPer * kWaves == kEntries, "every wave writes as many entries");
-#pragma unroll
-        for (int e = 0; e < kPer; ++e) dst[(wave * kPer + e) * 64] = src[wave * kPer + e];
-    } else {
-        typedef const __attribute__((address_space(4))) float cfloat;
-        cfloat* const src = (cfloat*)a.tables;
-        uint32_t* const dst = reinterpret_cast<uint32_t*>(smem) + lane;
 #pragma unroll 8
-        for (int e = 0; e < 256 / kWaves; ++e) {
-            const int entry = wave * (256 / kWaves) + e;
-            uint32_t v;
-            if constexpr (combined) {
-                v = (uint32_t)float_to_f16_bits(src[entry]) << 16;
-            } else {
-                v = (uint32_t)float_to_f16_bits(src[entry & 15]) | ((uint32_t)float_to_f16_bits(src[entry >> 4]) << 16);
-                if constexpr (kPlanes == 2) {
-                    const uint32_t r = (uint32_t)float_to_f16_bits(src[16 + (entry & 15)]) |
-                                       ((uint32_t)float_to_f16_bits(src[16 + (entry >> 4)]) << 16);
-                    v = g ? r : v;
-                }
-            }
-            dst[entry * 64] = v;
+        for (int e = 0; e < kPer; ++e) {
+            const uint32_t v = src[wave * kPer + e];
+            dst[(wave * kPer + e) * 64] = split ? v : (uint32_t)float_to_f16_bits(__builtin_bit_cast(float, v)) << 16;
         }
+    } else {
+        fill_pair_table<kPer>(smem, value, wave, lane);
     }
     __syncthreads();
 
@@ -403,15 +390,6 @@ TileArgs tile_args(const LayerView& L, int batch, void* y, int y_dtype, const vo
 
 int tile_workgroups(const TileArgs& a) { return (a.n_tiles + 7) / 8 * 8 * a.m_tiles; }
 
-TileGroup tile_group(const TileArgs* a, int n) {
-    TileGroup g{};
-    for (int j = 0; j < 3; ++j) {
-        if (j < n) g.a[j] = a[j];
-        g.first[j + 1] = j < n ? g.first[j] + tile_workgroups(a[j]) : 1 << 30;          // (no workgroup reaches an unused slot)
-    }
-    return g;
-}
-
 // The activations of tq_prefill_tile_kernel's operands in two parts: H (s (.) x) in fp32 as the fp32 kernels form it, times the power of
 // two that brings the largest of the row to [2^14, 2^15), rounded to fp16 (hi) and what that leaves off rounded again (lo).  A lane
 // has 32 consecutive columns, a wave 2048, a row `wpr` waves of one workgroup, which holds whole rows; both rotations of the
@@ -536,7 +514,7 @@ hipError_t launch_prefill_split(const LayerView& L, const void* x, int x_dtype, 
     a.row_exp = row_exp;
     a.table_exp = L.split_exp;
     const dim3 grid((unsigned)tile_workgroups(a));
-    const TileGroup g = tile_group(&a, 1);
+    const TileGroup g = {{a}};
     switch (L.mode) {
         case kSharedLut: launch_split_shape<kSharedLut>(shape, g, grid, stream); break;
         case kDual: launch_split_shape<kDual>(shape, g, grid, stream); break;
@@ -619,14 +597,13 @@ hipError_t launch_prefill_tile_group(const LayerView* Ls, int n, int shape, cons
                                      int y_dtype, void* const* workspaces, hipStream_t stream, const float* gate) {
     hipError_t e = launch_rotate_group(Ls, n, x, x_dtype, gate, batch, workspaces, stream, kBlockImage);
     if (e != hipSuccess) return e;
-    TileArgs a[3];
+    TileGroup g{};
     int wgs = 0;
     for (int j = 0; j < n; ++j) {
-        a[j] = tile_args(Ls[j], batch, ys[j], y_dtype, workspaces[j], kTileShapes[shape]);
-        wgs += tile_workgroups(a[j]);
+        g.a[j] = tile_args(Ls[j], batch, ys[j], y_dtype, workspaces[j], kTileShapes[shape]);
+        wgs = std::max(wgs, tile_workgroups(g.a[j]));
     }
-    const TileGroup g = tile_group(a, n);
-    const dim3 grid((unsigned)wgs);
+    const dim3 grid((unsigned)wgs, (unsigned)n);
     // Two 64-column tiles of a nibble plane at a time where the width allows it: 64 bytes of a row per pair of requests
     // instead of 32 (4864 x 896 at 512 rows 40.6 -> 38.0 us, 7680 x 565 55.0 -> 49.6; four tiles cost registers: 58).  The
     // combined plane's tile is 64 bytes already (two tiles at a time: 5 to 30 % slower).
