@@ -25,8 +25,8 @@
 // that) the fit says so and is left to the pass per step.
 //
 // 18944 x 3584 (68 M samples, 2 x 100 steps).  One pass over all samples per step took 230 ms, 1.1 ms each (thread-private
-// bins in 96 KB of LDS, one wave per SIMD) and a copy of the partial sums to the host; the kernels here take 1.04 ms:
-// scatter 320 us, iterate 264, refine 138, hist 140, predict 99, offsets 45, scan 23.  What bounds them is
+// bins in 96 KB of LDS, one wave per SIMD) and a copy of the partial sums to the host; the kernels here take 0.95 ms:
+// scatter 260 to 320 us, iterate 246, hist 140, refine 115, predict 84, offsets 45, scan 23.  What bounds them is
 // said at each.  Sorting every sample instead of the expected 15 % took 1840 us in the scatter kernel and 870 in refine.
 #include "tq_bins.h"
 #include "tq_device.h"
@@ -373,8 +373,7 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_predict_kernel(const FitPa
                 move = fabsf(nv - c);
                 c = nv;
             }
-            for (int m = 32; m >= 1; m >>= 1) move = fmaxf(move, __shfl_xor(move, m, kWave));
-            if (move < 1e-7f) break;
+            if (__ballot(move >= 1e-7f) == 0) break;                  // (a maximum over the wave: six LDS latencies a step)
         }
     }
     __syncthreads();
@@ -463,8 +462,11 @@ constexpr int kFitParts = 64;
 __device__ __forceinline__ uint32_t fit_part(uint32_t off, int shift) { return shift ? off >> 7 : off >> 16; }
 
 // One workgroup per (cell, problem): its samples in the order of the parts, from `sorted` to `fine`, and the parts'
-// first positions and offset sums.
-__global__ __launch_bounds__(kFitThreads) void tq_fit_refine_kernel(const FitParams* __restrict__ P,
+// first positions and offset sums.  A cell is a chain of latencies (its entries, its samples, the counters, its samples again),
+// so four workgroups share a CU.  Cells of up to kRefineLds samples are put in order in LDS and written in whole lines: written
+// where they belong one by one, every sample is a request to the L2 of its own, 20 M of them in 18944 x 3584 (138 us -> 115).
+constexpr int kRefineThreads = 512, kRefineLds = 8192;
+__global__ __launch_bounds__(kRefineThreads) void tq_fit_refine_kernel(const FitParams* __restrict__ P,
                                                                     const uint32_t* __restrict__ start_all,
                                                                     const uint32_t* __restrict__ place,
                                                                     const uint32_t* __restrict__ kept, size_t capacity,
@@ -473,6 +475,7 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_refine_kernel(const FitPar
                                                                     unsigned long long* __restrict__ part_o) {
     __shared__ unsigned long long both[kFitParts];                    // counts (upper 23 bits) and offset sums, as in the tiles
     __shared__ uint32_t pos[kFitParts];
+    __shared__ float ordered[kRefineLds];
     const int p = blockIdx.y, cell = blockIdx.x, tid = threadIdx.x;
     if (P->bad || !fit_room(kept, gridDim.y, capacity)) return;
     const uint32_t at = place[(size_t)p * kFitCells + cell];
@@ -495,15 +498,15 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_refine_kernel(const FitPar
         const uint32_t hi = lo + kFitMaxTile < n ? lo + kFitMaxTile : n;
         if (tid < kFitParts) both[tid] = 0;
         __syncthreads();
-        for (uint32_t i = lo + tid; i < hi; i += 4 * kFitThreads) {
+        for (uint32_t i = lo + tid; i < hi; i += 4 * kRefineThreads) {
             float v[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = src[i + j * kFitThreads < hi ? i + j * kFitThreads : i];
+            for (int j = 0; j < 4; ++j) v[j] = src[i + j * kRefineThreads < hi ? i + j * kRefineThreads : i];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 uint32_t o;
                 const uint32_t k = part_of(v[j], o);
-                if (i + j * kFitThreads < hi) atomicAdd(&both[k], (1ull << 41) | (unsigned long long)o);
+                if (i + j * kRefineThreads < hi) atomicAdd(&both[k], (1ull << 41) | (unsigned long long)o);
             }
         }
         __syncthreads();
@@ -527,20 +530,26 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_refine_kernel(const FitPar
         pos[tid] = a - cnt;
     }
     __syncthreads();
-    for (uint32_t i = tid; i < n; i += 4 * kFitThreads) {
+    const bool in_lds = n <= (uint32_t)kRefineLds;
+    for (uint32_t i = tid; i < n; i += 4 * kRefineThreads) {
         float v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = src[i + j * kFitThreads < n ? i + j * kFitThreads : i];
+        for (int j = 0; j < 4; ++j) v[j] = src[i + j * kRefineThreads < n ? i + j * kRefineThreads : i];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             uint32_t o;
             const uint32_t k = part_of(v[j], o);
-            if (i + j * kFitThreads < n) {
+            if (i + j * kRefineThreads < n) {
                 const uint32_t to = atomicAdd(&pos[k], 1u);
-                if (to < n) dst[to] = v[j];
+                if (to >= n) continue;
+                if (in_lds) ordered[to] = v[j];
+                else dst[to] = v[j];
             }
         }
     }
+    if (!in_lds) return;
+    __syncthreads();
+    for (uint32_t i = tid; i < n; i += kRefineThreads) dst[i] = ordered[i];
 }
 
 // All Lloyd-Max steps of one codebook (src/codebook.cpp:105-136): one workgroup, a wave per boundary.  out->missed[p]:
@@ -548,7 +557,7 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_refine_kernel(const FitPar
 // of latencies (the cell's entries, its samples, the workgroup's sums).  The entries stay in the wave's registers, a part per
 // lane, as long as the boundary stays in its cell; a sample's offset comes from its mantissa, the cell being known; no more
 // rounds of 64 samples run than there are samples for (four waves share a SIMD: what a wave issues counts), and sums over a
-// wave go through DPP operands: 3.0 us a step -> 2.6.
+// wave go through DPP operands, whether a centroid moved is a ballot: 3.0 us a step -> 2.5.
 struct FitCut {                                       // a boundary's cell
     uint32_t cell, at, s0;
     i128 q0;                                          // of the samples below the cell
@@ -684,8 +693,8 @@ __global__ __launch_bounds__(kFitThreads) void tq_fit_iterate_kernel(const FitPa
                     cent[lane] = nv;
                 }
             }
-            for (int m = 32; m >= 1; m >>= 1) shift = fmaxf(shift, __shfl_xor(shift, m, kWave));
-            if (lane == 0) stop = shift < 1e-6f ? 1 : 0;                             // src/codebook.cpp:132
+            const bool moves = __ballot(shift >= 1e-6f) != 0;                        // src/codebook.cpp:132
+            if (lane == 0) stop = moves ? 0 : 1;
         } else if (wave == 1 && lane < nc) {
             // each of a bin's samples around zero may have lost up to one unit; the centroid again, beside wave 0
             const unsigned long long from = max(left_n[lane], cut_lo), to = min(left_n[lane + 1], cut_hi);
@@ -771,7 +780,7 @@ hipError_t launch_fit(const float* samples, size_t n, int problems, const float*
     hipLaunchKernelGGL(tq_fit_predict_kernel, dim3(problems), dim3(kFitThreads), 0, stream, P, iterations, start, below, cb,
                        state, everything ? 1 : 0, place, kept);
     hipLaunchKernelGGL(tq_fit_scatter_kernel, grid, dim3(kFitThreads), 0, stream, fp, P, tile, first, place, kept, cap, sorted);
-    hipLaunchKernelGGL(tq_fit_refine_kernel, dim3(kFitCells, problems), dim3(kFitThreads), 0, stream, P, start, place, kept, cap, sorted,
+    hipLaunchKernelGGL(tq_fit_refine_kernel, dim3(kFitCells, problems), dim3(kRefineThreads), 0, stream, P, start, place, kept, cap, sorted,
                        fine, part_n, part_o);
     hipLaunchKernelGGL(tq_fit_iterate_kernel, dim3(problems), dim3(kFitThreads), 0, stream, P, n, iterations, start, below, place,
                        kept, cap, fine, part_n, part_o, cb, state);
