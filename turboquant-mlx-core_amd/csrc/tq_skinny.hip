@@ -410,9 +410,9 @@ __device__ __forceinline__ void skinny_nibble_body(const SkinnyNibbleArgs& a, co
     }
 }
 
-// grid = units x workgroups per unit
-template <int SETS, bool RAGGED>
-__global__ __launch_bounds__(kSkThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void tq_skinny_nibble_kernel(SkinnyNibbleArgs a) {
+// grid = units x workgroups per unit.  TWO: two workgroups share a CU (half the registers each).
+template <int SETS, bool RAGGED, bool TWO = false>
+__global__ __launch_bounds__(kSkThreads) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 2, TWO ? 4 : 2))) void tq_skinny_nibble_kernel(SkinnyNibbleArgs a) {
     skinny_nibble_body<SETS, RAGGED>(a, (int)blockIdx.x, (int)blockIdx.y);
 }
 
@@ -421,8 +421,8 @@ struct SkinnyNibbleGroup {
     SkinnyNibbleArgs a[3];
     int first[4];
 };
-template <int SETS, bool RAGGED>
-__global__ __launch_bounds__(kSkThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void tq_skinny_nibble_group_kernel(SkinnyNibbleGroup g) {
+template <int SETS, bool RAGGED, bool TWO = false>
+__global__ __launch_bounds__(kSkThreads) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 2, TWO ? 4 : 2))) void tq_skinny_nibble_group_kernel(SkinnyNibbleGroup g) {
     const int b = (int)blockIdx.y;
     const int j = b >= g.first[2] ? 2 : (b >= g.first[1] ? 1 : 0);
     skinny_nibble_body<SETS, RAGGED>(g.a[j], (int)blockIdx.x, b - g.first[j]);
@@ -526,6 +526,15 @@ static bool skinny_nibble(const LayerView& L) {
     return (L.mode == kDual || L.mode == kPrimaryOnly) && L.block_size <= (uint32_t)kSkChunk;
 }
 
+// Workgroups of a launch on nibble planes.  Up to 16 rows two fit a CU (80 KB of LDS, 124 registers): where a wave has 12 groups of 16
+// weight rows and more, the second one's loads fill the first one's decode (2 x 27648 x 5120 at eight rows 71.2 -> 69.9 us, a
+// 6656 x 17408 block at 15 rows 127.7 -> 121).  With fewer groups its table and rotation cost more than that: 10782 x 1024
+// at five rows 10.1 -> 12.6.
+static int nibble_workgroups(long long groups, int units, int batch, int num_cus) {
+    const long long waves = (long long)(num_cus / units > 0 ? num_cus / units : 1) * (kSkThreads / 64);
+    return batch <= 16 && groups >= 12 * waves ? 2 * num_cus : num_cus;
+}
+
 bool skinny_supported(const LayerView& L, int x_dtype, int batch) {
     if (batch < 2 || batch > kSkMaxRows) return false;                                   // (any activation type)
     // whole 64-column pieces (nibble planes: 128-column pieces); a row that does not fill its last 512-column
@@ -562,7 +571,8 @@ hipError_t launch_skinny(const LayerView& L, const void* x, int x_dtype, int bat
         n.planes = L.mode == kDual ? 2 : 1;
         n.units = (L.in_features + kSkChunk - 1) / kSkChunk * n.planes;
         n.groups = (L.out_features + 15) / 16;
-        n.wgs_per_unit = num_cus / n.units > 0 ? num_cus / n.units : 1;   // one workgroup per CU
+        const int slots = nibble_workgroups(n.groups, n.units, batch, num_cus);
+        n.wgs_per_unit = slots / n.units > 0 ? slots / n.units : 1;
         const int workers_n = n.wgs_per_unit * (kSkThreads / 64);
         n.groups_q = n.groups / workers_n;
         n.groups_rem = n.groups % workers_n;
@@ -570,6 +580,8 @@ hipError_t launch_skinny(const LayerView& L, const void* x, int x_dtype, int bat
         const bool two = batch > 16, ragged = L.in_features % kSkChunk != 0;
         if (two && ragged) hipLaunchKernelGGL((tq_skinny_nibble_kernel<2, true>), grid_n, dim3(kSkThreads), 0, stream, n);
         else if (two) hipLaunchKernelGGL((tq_skinny_nibble_kernel<2, false>), grid_n, dim3(kSkThreads), 0, stream, n);
+        else if (slots > num_cus && ragged) hipLaunchKernelGGL((tq_skinny_nibble_kernel<1, true, true>), grid_n, dim3(kSkThreads), 0, stream, n);
+        else if (slots > num_cus) hipLaunchKernelGGL((tq_skinny_nibble_kernel<1, false, true>), grid_n, dim3(kSkThreads), 0, stream, n);
         else if (ragged) hipLaunchKernelGGL((tq_skinny_nibble_kernel<1, true>), grid_n, dim3(kSkThreads), 0, stream, n);
         else hipLaunchKernelGGL((tq_skinny_nibble_kernel<1, false>), grid_n, dim3(kSkThreads), 0, stream, n);
         hipError_t en = hipGetLastError();
@@ -630,10 +642,11 @@ hipError_t launch_skinny_group(const LayerView* Ls, int n, const void* x, int x_
     const bool nibble = Ls[0].mode == kDual || Ls[0].mode == kPrimaryOnly;
     const int planes = Ls[0].mode == kDual ? 2 : 1;
     const int K = Ls[0].in_features, chunks = (K + kSkChunk - 1) / kSkChunk * planes;   // work units: (chunk, plane)
-    const int total_wgs = num_cus / chunks;                       // workgroups per unit, all layers together
     long long rows = 0;
     bool fours = true;                                            // columns per lane of the reduction
     for (int j = 0; j < n; ++j) { rows += Ls[j].out_features; fours = fours && Ls[j].out_features % 4 == 0; }
+    const int slots = nibble ? nibble_workgroups(rows / 16, chunks, batch, num_cus) : num_cus;
+    const int total_wgs = slots / chunks;                         // workgroups per unit, all layers together
     fours = fours && rows * batch >= 262144;                       // (a thousand blocks; fewer: 5.8 us where one column each takes 4.0)
     const int reduce_cols = fours ? 256 : 64;
     int wgs[3] = {0, 0, 0}, used = 0;
@@ -696,6 +709,8 @@ hipError_t launch_skinny_group(const LayerView* Ls, int n, const void* x, int x_
     if (nibble) {
         if (two && ragged) hipLaunchKernelGGL((tq_skinny_nibble_group_kernel<2, true>), grid, dim3(kSkThreads), 0, stream, gn);
         else if (two) hipLaunchKernelGGL((tq_skinny_nibble_group_kernel<2, false>), grid, dim3(kSkThreads), 0, stream, gn);
+        else if (slots > num_cus && ragged) hipLaunchKernelGGL((tq_skinny_nibble_group_kernel<1, true, true>), grid, dim3(kSkThreads), 0, stream, gn);
+        else if (slots > num_cus) hipLaunchKernelGGL((tq_skinny_nibble_group_kernel<1, false, true>), grid, dim3(kSkThreads), 0, stream, gn);
         else if (ragged) hipLaunchKernelGGL((tq_skinny_nibble_group_kernel<1, true>), grid, dim3(kSkThreads), 0, stream, gn);
         else hipLaunchKernelGGL((tq_skinny_nibble_group_kernel<1, false>), grid, dim3(kSkThreads), 0, stream, gn);
     } else {
