@@ -485,9 +485,7 @@ static int split_shape(const LayerView& L, int batch, int num_cus) {
 bool prefill_split_supported(const LayerView& L, int batch) {
     if (batch < (L.mode == kDual ? 4 : 5) || !L.split_tables || !shape_supported(L.in_features, L.block_size)) return false;
     if (L.mode != kSharedLut && L.mode != kDual && L.mode != kPrimaryOnly) return false;
-    const unsigned long long weights = (unsigned long long)L.out_features * (unsigned long long)L.in_features;
-    if (L.mode == kPrimaryOnly && batch <= 8 && weights < (1u << 20)) return false;        // (two fp32 launches: 1216 x 669 at 5 rows 10.8 us, this 11.6)
-    return weights < (1ull << 32);                                                         // (32-bit offsets into a plane)
+    return (unsigned long long)L.out_features * (unsigned long long)L.in_features < (1ull << 32);      // (32-bit offsets into a plane)
 }
 
 static size_t split_image_bytes(const LayerView& L, int batch) {
