@@ -478,7 +478,7 @@ __global__ __launch_bounds__(256) void tq_rotate_f16_kernel(const void* __restri
 // consecutive bytes of the image (rows r % 32 = 8 j .. 8 j + 7 of lane group g); they change lanes through a
 // wave-private piece of LDS so that a store instruction writes eight whole 128-byte lines.  R = 2, for calls
 // with few rows (less than two waves of 8 rows per SIMD): the launch is as long as one wave's chain of loads,
-// butterflies and stores, so the waves are kept short and store their 2 x 16 bytes themselves.
+// butterflies and stores, so the waves are kept short, store their 2 x 16 bytes themselves and take one rotation each.
 // planes = 2: both rotations of the dual layout from one read of the activations (images out and out2).  blockIdx.y: the
 // layer of a group on the same activations.  GATED (x fp32): the activations are silu(gate) * x, formed as they are read,
 // in fp32 as tq_silu_mul_kernel forms them: 2048 rows of 27648 columns 136 us where that kernel and this one took 139 + 77.
@@ -539,7 +539,9 @@ __global__ __launch_bounds__(256) void tq_rotate_panel_kernel(const void* __rest
     }
     const int U_all = cols >> 4, ustep = blocks ? 64 : 1024;
     const int g_own = seg * 64 + lane;                                 // this lane's 8-column group of the row
-    for (int plane = 0; plane < planes; ++plane) {
+    // (few rows: a plane per workgroup)
+    const int plane0 = gridDim.z > 1 ? (int)blockIdx.z : 0, plane1 = gridDim.z > 1 ? plane0 + 1 : planes;
+    for (int plane = plane0; plane < plane1; ++plane) {
         const uint32_t sd = plane ? group.seed2[blockIdx.y] : group.seed[blockIdx.y];
         uint4* const img = reinterpret_cast<uint4*>(plane ? group.out2[blockIdx.y] : group.out[blockIdx.y]);
         float sg[8];
@@ -706,7 +708,7 @@ hipError_t launch_rotate_group(const LayerView* Ls, int n, const void* x, int x_
         const int segs = (K + 511) / 512, blocks = layout == kBlockImage;
         const long long tasks8 = (long long)((M + 7) / 8) * segs, tasks2 = (long long)((M + 1) / 2) * segs;
         const bool eight = tasks8 * n >= 2048;
-        const dim3 grid((unsigned)(((eight ? tasks8 : tasks2) + 3) / 4), n);
+        const dim3 grid((unsigned)(((eight ? tasks8 : tasks2) + 3) / 4), n, eight ? 1 : planes);
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, x_dtype, gate, g, M, K, segs, planes, blocks, L.block_size,
                                L.inv_sqrt_bs);
