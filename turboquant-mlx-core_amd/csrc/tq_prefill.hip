@@ -498,6 +498,8 @@ __global__ __launch_bounds__(256) void tq_rotate_panel_kernel(const void* __rest
     __shared__ __align__(16) char stage_all[R == 8 ? 4 * kWave * kRotPitch : 16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     char* const stage = stage_all + (R == 8 ? wave * (kWave * kRotPitch) : 0);
+    const uint32_t seeds[2] = {group.seed[blockIdx.y], group.seed2[blockIdx.y]};
+    uint16_t* const outs[2] = {group.out[blockIdx.y], group.out2[blockIdx.y]};
     const long long task = (long long)blockIdx.x * 4 + wave;           // (row group, segment), segment fastest
     const int rg = (int)(task / segs), seg = (int)(task - (long long)rg * segs);
     const int row0 = rg * R;
@@ -542,8 +544,8 @@ __global__ __launch_bounds__(256) void tq_rotate_panel_kernel(const void* __rest
     // (few rows: a plane per workgroup)
     const int plane0 = gridDim.z > 1 ? (int)blockIdx.z : 0, plane1 = gridDim.z > 1 ? plane0 + 1 : planes;
     for (int plane = plane0; plane < plane1; ++plane) {
-        const uint32_t sd = plane ? group.seed2[blockIdx.y] : group.seed[blockIdx.y];
-        uint4* const img = reinterpret_cast<uint4*>(plane ? group.out2[blockIdx.y] : group.out[blockIdx.y]);
+        const uint32_t sd = plane ? seeds[1] : seeds[0];
+        uint4* const img = reinterpret_cast<uint4*>(plane ? outs[1] : outs[0]);
         float sg[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) sg[j] = active ? sign_of(sd, (uint32_t)(col + j) & (bs - 1)) : 0.0f;

@@ -108,7 +108,7 @@ template <int PIECES> struct TileBytes { u32x4v v[PIECES]; };   // index bytes (
 // Both groups run the same number of sub-steps, so they meet at every barrier.
 template <int MODE, int NBLK, int KG = 1>
 __global__ __launch_bounds__(kPThreads * KG) void tq_prefill_panel_kernel(PanelGroup group) {
-    const PanelArgs& a = group.a[blockIdx.y];
+    const PanelArgs a = group.a[blockIdx.y];               // (all of it at once)
     const int id = (int)blockIdx.x;
     static_assert(KG == 1 || (KG == 2 && NBLK == 1), "a second wave group: one row block per wave");
     constexpr int kExchange = 4 * 64 * 272;            // past the epilogue's stage: the second group's products

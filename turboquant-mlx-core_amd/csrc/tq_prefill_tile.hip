@@ -50,7 +50,7 @@ struct TileGroup { TileArgs a[3]; };
 // parts (zeros from K to a whole 64-column tile), the table is L.split_tables.
 template <int MODE, int SUB, int MB, int NB, int KS, int WN, int PARTS>
 __global__ __launch_bounds__(64 * KS * WN) void tq_prefill_tile_kernel(TileGroup group) {
-    const TileArgs& a = group.a[blockIdx.y];
+    const TileArgs a = group.a[blockIdx.y];                // (all of it at once)
     const int block = (int)blockIdx.x;
     constexpr bool combined = (MODE == kSharedLut);
     constexpr int kPlanes = (MODE == kDual) ? 2 : 1;
