@@ -1,8 +1,8 @@
 // Bin of a value among sorted boundaries, for the codebook fit.
 //
 // std::lower_bound over the boundaries (reference src/codebook.cpp:295-297) is the number of boundaries strictly below
-// the value.  Comparing with each of them is two vector instructions per boundary and value (30 for 4 bits; what the
-// quantizer does); here 256 equally wide cells over the boundaries' range say how many boundaries lie
+// the value.  Comparing with each of them is two vector instructions per boundary and value (30 for 4 bits; the
+// quantizer bisects a tree of them, 12 and two LDS reads); here 256 equally wide cells over the boundaries' range say how many boundaries lie
 // in the cells below, and only the boundaries of the value's own cell (one at most for any codebook whose
 // boundaries are 1/253 of the range apart) are compared.  The cell is a monotone function of the value, rounding included,
 // and the boundaries' own cells come from the same function, so the result is the exact count.
